@@ -7,14 +7,11 @@ are exact.
 """
 import functools
 import math
-import os
-import sys
 
 import numpy as np
 import torch
 
-sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
-import __graft_entry__  # noqa: E402
+import __graft_entry__
 
 __graft_entry__.load_package()
 from cvm_runtime_amd import graphgen, hipops, runtime  # noqa: E402
