@@ -4,7 +4,8 @@ The product is the shared library `libcvm_runtime_hip.so` built from csrc/:
 hand-written HIP kernels behind the operator-level C ABI
 (include/cvm_hip_ops.h) and a C++ graph runtime behind the reference's model
 C API (include/cvm_c_api.h).  This Python package is only a loader plus thin
-ctypes wrappers; torch is used for device memory and streams, nothing else.
+wrappers (ctypes, and csrc/binding for the operators a node-by-node caller issues
+most); torch is used for device memory and streams, nothing else.
 
 There is no CPU fallback: if the library is missing or no GPU is present the
 wrappers raise.
@@ -14,7 +15,9 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libcvm_runtime_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "_hipops_native.so")
 _lib = None
+_native = None
 
 
 class CvmHipError(RuntimeError):
@@ -37,6 +40,23 @@ def lib():
                      "cvmhip_packed_weight_bytes", "cvmhip_packed_act_bytes", "cvmhip_packed_depthwise_bytes"):
             getattr(_lib, name).restype = ctypes.c_size_t
     return _lib
+
+
+def native():
+    """The native half of hipops.py (raises if it has not been built)."""
+    global _native
+    if _native is None:
+        lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise CvmHipError("%s is missing: build it with `python cvm-runtime_amd/build.py`" % NATIVE_PATH)
+        import importlib.util
+        import torch  # noqa: F401  (its libraries are what the module links to)
+        spec = importlib.util.spec_from_file_location("_hipops_native", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.setup(CvmHipError)
+        _native = mod
+    return _native
 
 
 def check(rc):

@@ -3,18 +3,22 @@
 Every .hip / .cc file under csrc/ is compiled with hipcc for gfx950 and linked
 into cvm-runtime_amd/libcvm_runtime_hip.so, the one library that exports both
 the operator-level C ABI (include/cvm_hip_ops.h) and the model-level C ABI
-(include/cvm_c_api.h).
+(include/cvm_c_api.h).  csrc/binding/ becomes _hipops_native.so, the native half of
+hipops.py; it is the only object that knows torch, and the library does not need it.
 """
 import glob
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libcvm_runtime_hip.so")
+BINDING = os.path.join(HERE, "_hipops_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-fsigned-char", "-fvisibility=hidden", "-I" + os.path.join(HERE, "..", "include")]
@@ -37,15 +41,29 @@ def _compile(src):
     return obj
 
 
+def _build_binding():
+    torch = os.path.dirname(importlib.util.find_spec("torch").origin)
+    inc = [os.path.join(torch, "include"), os.path.join(torch, "include", "torch", "csrc", "api", "include"),
+           os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"), sysconfig.get_paths()["include"]]
+    cmd = (["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"] +
+           ["-I" + d for d in inc] + [os.path.join(CSRC, "binding", "hipops_native.cc"), "-o", BINDING, "-L" + HERE,
+            "-l:" + os.path.basename(LIB), "-L" + os.path.join(torch, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+            "-lc10_hip", "-Wl,-rpath,$ORIGIN"])
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("binding failed: %s\n%s" % (" ".join(cmd), r.stdout))
+
+
 def build(verbose=False):
     os.makedirs(OBJ, exist_ok=True)
-    srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "**", "*.cc"), recursive=True))
+    srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "runtime", "*.cc")))
     with ThreadPoolExecutor(max_workers=8) as ex:
         objs = list(ex.map(_compile, srcs))
     cmd = [HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB] + objs + ["-Wl,-Bsymbolic"]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout)
+    _build_binding()
     if verbose:
         print("built", LIB)
     return LIB

@@ -1,16 +1,18 @@
-"""Thin ctypes wrappers over the operator-level C ABI (include/cvm_hip_ops.h).
+"""Thin wrappers over the operator-level C ABI (include/cvm_hip_ops.h).
 
 Arguments and results are int32 torch tensors on the GPU (torch only supplies
 the device memory and the stream).  The names and argument meaning follow the
 reference's operators (`cvm.runtime.<dev>.<op>`, src/runtime/cpu/ops), so a
-parity test reads like the reference's tests/test_op.cc cases.
+parity test reads like the reference's tests/test_op.cc cases.  The operators
+of a node-by-node inference go through the native half of this module
+(csrc/binding/hipops_native.cc), the others through ctypes.
 """
 import ctypes
 import os
 
 import torch
 
-from . import check, lib
+from . import check, lib, native
 
 _i32p = ctypes.POINTER(ctypes.c_int32)
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -38,8 +40,12 @@ def _apply_conv_tuning():
 
 
 def _stream():
-    _apply_conv_tuning()
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def _conv_stream():
+    _apply_conv_tuning()
+    return _stream()
 
 
 def _shape(s):
@@ -61,73 +67,47 @@ def conv_out_hw(h, w, kh, kw, sh, sw, ph, pw, dh, dw):
 
 
 def conv2d(x, w, b=None, strides=(1, 1), padding=(0, 0), dilation=(1, 1), groups=1):
-    n, ic, h, wd = x.shape
-    oc, _, kh, kw = w.shape
-    oh, ow = conv_out_hw(h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1], dilation[0], dilation[1])
-    y = _new((n, oc, oh, ow), x)
-    L = lib()
-    nbytes = L.cvmhip_conv2d_workspace_bytes(n, ic, h, wd, oc, kh, kw, groups)
-    ws = _workspace(nbytes, x.device)
-    check(L.cvmhip_conv2d(_ptr(x), _ptr(w), _ptr(b), _ptr(y), n, ic, h, wd, oc, kh, kw,
-                          strides[0], strides[1], padding[0], padding[1], dilation[0], dilation[1],
-                          groups, ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(ws.numel()), _stream()))
-    return y
+    return native().conv2d(x, w, b, strides, padding, dilation, groups)
 
 
 def dense(x, w, b=None, operand_bits=8):
-    m, k = x.shape
-    n = w.shape[0]
-    y = _new((m, n), x)
-    L = lib()
-    ws = _workspace(L.cvmhip_dense_workspace_bytes(m, k, n), x.device)
-    check(L.cvmhip_dense(_ptr(x), _ptr(w), _ptr(b), _ptr(y), m, k, n, operand_bits,
-                         ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(ws.numel()), _stream()))
-    return y
-
-
-def _unary(fn, x, *args, out=None):
-    y = torch.empty_like(x) if out is None else out
-    check(fn(_ptr(x), _ptr(y), ctypes.c_int64(x.numel()), *args, _stream()))
-    return y
+    return native().dense(x, w, b, operand_bits)
 
 
 def relu(x, out=None):
-    return _unary(lib().cvmhip_relu, x, out=out)
+    return native().unary(0, x, out, 0, 0)
 
 
 def cvm_clip(x, precision, out=None):
-    return _unary(lib().cvmhip_cvm_clip, x, int(precision), out=out)
+    return native().unary(1, x, out, int(precision), 0)
 
 
 def cvm_right_shift(x, precision, shift_bit, out=None):
-    return _unary(lib().cvmhip_cvm_right_shift, x, int(precision), int(shift_bit), out=out)
+    return native().unary(2, x, out, int(precision), int(shift_bit))
 
 
 def cvm_left_shift(x, precision, shift_bit, out=None):
-    return _unary(lib().cvmhip_cvm_left_shift, x, int(precision), int(shift_bit), out=out)
+    return native().unary(3, x, out, int(precision), int(shift_bit))
 
 
 def clip(x, a_min, a_max, out=None):
-    return _unary(lib().cvmhip_clip, x, ctypes.c_int32(a_min), ctypes.c_int32(a_max), out=out)
+    return native().unary(4, x, out, a_min, a_max)
 
 
 def abs_(x, out=None):
-    return _unary(lib().cvmhip_abs, x, out=out)
+    return native().unary(5, x, out, 0, 0)
 
 
 def negative(x, out=None):
-    return _unary(lib().cvmhip_negative, x, out=out)
+    return native().unary(6, x, out, 0, 0)
 
 
 def cvm_precision(x, out=None):
-    return _unary(lib().cvmhip_cvm_precision, x, out=out)
+    return native().unary(7, x, out, 0, 0)
 
 
 def elemwise(op, a, b, out=None):
-    c = torch.empty_like(a) if out is None else out
-    check(lib().cvmhip_elemwise(0 if op == "elemwise_add" else 1, _ptr(a), _ptr(b), _ptr(c),
-                                ctypes.c_int64(a.numel()), _stream()))
-    return c
+    return native().elemwise(0 if op == "elemwise_add" else 1, a, b, out)
 
 
 def broadcast_shape(sa, sb):
@@ -138,11 +118,7 @@ def broadcast_shape(sa, sb):
 
 
 def broadcast(op, a, b):
-    cs = broadcast_shape(a.shape, b.shape)
-    c = _new(cs, a)
-    check(lib().cvmhip_broadcast(BCAST[op], _ptr(a), _shape(a.shape), a.dim(), _ptr(b), _shape(b.shape),
-                                 b.dim(), _ptr(c), _shape(cs), len(cs), _stream()))
-    return c
+    return native().broadcast(BCAST[op], a, b)
 
 
 def pool_out(h, k, s, p, ceil_mode):
@@ -152,16 +128,7 @@ def pool_out(h, k, s, p, ceil_mode):
 
 
 def max_pool2d(x, pool_size, strides=(1, 1), padding=(0, 0), ceil_mode=False):
-    n, c, h, w = x.shape
-    pad = list(padding)
-    if len(pad) == 1:
-        pad = [pad[0], pad[0]]
-    oh = pool_out(h, pool_size[0], strides[0], pad[0], ceil_mode)
-    ow = pool_out(w, pool_size[1], strides[1], pad[1], ceil_mode)
-    y = _new((n, c, oh, ow), x)
-    check(lib().cvmhip_max_pool2d(_ptr(x), _ptr(y), n, c, h, w, oh, ow, pool_size[0], pool_size[1],
-                                  strides[0], strides[1], pad[0], pad[1], _stream()))
-    return y
+    return native().max_pool2d(x, pool_size, strides, padding, ceil_mode)
 
 
 def reduce_shape(shape, axes, keepdims, exclude):
@@ -183,12 +150,7 @@ def reduce_shape(shape, axes, keepdims, exclude):
 
 
 def reduce(op, x, axes=(), keepdims=False, exclude=False):
-    ys = reduce_shape(x.shape, list(axes), keepdims, exclude)
-    y = _new(ys, x)
-    ax = _shape(list(axes)) if len(axes) else None
-    check(lib().cvmhip_reduce(0 if op == "sum" else 1, _ptr(x), _shape(x.shape), x.dim(), _ptr(y),
-                              ctypes.c_int64(y.numel()), ax, len(axes), int(bool(exclude)), _stream()))
-    return y
+    return native().reduce(0 if op == "sum" else 1, x, reduce_shape(x.shape, axes, keepdims, exclude), axes, int(bool(exclude)))
 
 
 def copy(x, shape):
@@ -280,27 +242,14 @@ def where(cond, x, y, out):
 
 
 def get_valid_counts(x, score_threshold):
-    b, n, k = x.shape
-    vc = _new((b,), x)
-    y = torch.empty_like(x)
-    L = lib()
-    ws = _workspace(L.cvmhip_get_valid_counts_workspace_bytes(b, n), x.device)
-    check(L.cvmhip_get_valid_counts(_ptr(x), _ptr(vc), _ptr(y), b, n, k, ctypes.c_int32(score_threshold),
-                                    ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(ws.numel()), _stream()))
-    return vc, y
+    return native().get_valid_counts(x, score_threshold)
 
 
 def non_max_suppression(x, valid_count, y, iou_threshold=50, force_suppress=False, top_k=-1,
                         id_index=0, coord_start=2, score_index=1, max_output_size=-1):
     """In place on y; x is mutated exactly as the reference mutates it."""
-    b, n, k = x.shape
-    L = lib()
-    ws = _workspace(L.cvmhip_nms_workspace_bytes(b, n, k), x.device)
-    check(L.cvmhip_non_max_suppression(_ptr(x), _ptr(valid_count), _ptr(y), b, n, k, max_output_size,
-                                       iou_threshold, top_k, coord_start, score_index, id_index,
-                                       int(bool(force_suppress)), ctypes.c_void_p(ws.data_ptr()),
-                                       ctypes.c_size_t(ws.numel()), _stream()))
-    return y
+    return native().non_max_suppression(x, valid_count, y, iou_threshold, force_suppress, top_k, id_index, coord_start,
+                                        score_index, max_output_size)
 
 
 def non_max_suppression_static(x, valid_count, y, iou_threshold=50, force_suppress=False, top_k=-1,
@@ -372,27 +321,27 @@ def _act_buffer(npix, c, dev):
 def pack_act_i8(x):
     n, c, h, w = x.shape
     xp = _act_buffer(n * h * w, c, x.device)
-    check(lib().cvmhip_pack_nhwc_i8(_ptr(x), _vp(xp), n, c, h * w, _stream()))
+    check(lib().cvmhip_pack_nhwc_i8(_ptr(x), _vp(xp), n, c, h * w, _conv_stream()))
     return xp
 
 
 def flatten_act_i8(xp, n, c, hw):
     """int8 act tensor of n images x hw pixels x c channels -> act tensor of n pixels x hw * c channels (cvmhip_flatten_act_i8)"""
     yp = _act_buffer(n, hw * c, xp.device)
-    check(lib().cvmhip_flatten_act_i8(_vp(xp), _vp(yp), n, c, hw, _stream()))
+    check(lib().cvmhip_flatten_act_i8(_vp(xp), _vp(yp), n, c, hw, _conv_stream()))
     return yp
 
 
 def unpack_act_i8(xp, n, c, h, w):
     x = torch.empty((n, c, h, w), dtype=torch.int32, device=xp.device)
-    check(lib().cvmhip_unpack_nhwc_i8(_vp(xp), _ptr(x), n, c, h * w, _stream()))
+    check(lib().cvmhip_unpack_nhwc_i8(_vp(xp), _ptr(x), n, c, h * w, _conv_stream()))
     return x
 
 
 def pack_weights(w):
     oc, ic, kh, kw = w.shape
     wp = _workspace(lib().cvmhip_packed_weight_bytes(oc, ic, kh, kw), w.device)
-    check(lib().cvmhip_pack_weights(_ptr(w), _vp(wp), oc, ic, kh, kw, _stream()))
+    check(lib().cvmhip_pack_weights(_ptr(w), _vp(wp), oc, ic, kh, kw, _conv_stream()))
     return wp
 
 
@@ -406,7 +355,7 @@ def conv2d_i8(xp, n, ic, h, w, wp, oc, kh, kw, bias=None, chain1=None, residual=
     check(lib().cvmhip_conv2d_i8(_vp(xp), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None,
                                  _vp(residual), ctypes.byref(chain2) if chain2 else None, _vp(out), int(out_is_i8),
                                  n, ic, h, w, oc, kh, kw, strides[0], strides[1], padding[0], padding[1],
-                                 dilation[0], dilation[1], _stream()))
+                                 dilation[0], dilation[1], _conv_stream()))
     return out
 
 
@@ -421,7 +370,7 @@ def conv2d_pool2_i8(xp, n, ic, h, w, wp, oc, kh, kw, bias=None, chain1=None, str
     out = _act_buffer(n * (oh // 2) * (ow // 2), oc, xp.device)
     check(lib().cvmhip_conv2d_pool2_i8(_vp(xp), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None, _vp(out),
                                        n, ic, h, w, oc, kh, kw, strides[0], strides[1], padding[0], padding[1],
-                                       dilation[0], dilation[1], _stream()))
+                                       dilation[0], dilation[1], _conv_stream()))
     return out
 
 
@@ -441,7 +390,7 @@ def conv2d_i8_ws(xp, n, ic, h, w, wp, oc, kh, kw, bias=None, chain1=None, out_is
         out = torch.empty((n, oc, oh, ow), dtype=torch.int32, device=xp.device)
     check(L.cvmhip_conv2d_i8_ws(_vp(xp), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None, None, None,
                                 _vp(out), int(out_is_i8), n, ic, h, w, oc, kh, kw, strides[0], strides[1],
-                                padding[0], padding[1], dilation[0], dilation[1], _vp(ws), ctypes.c_size_t(need), _stream()))
+                                padding[0], padding[1], dilation[0], dilation[1], _vp(ws), ctypes.c_size_t(need), _conv_stream()))
     return out, need
 
 
@@ -452,7 +401,7 @@ def conv2d_i8_nhwc(xp, n, ic, h, w, wp, oc, kh, kw, out, offset, image_stride, b
     check(lib().cvmhip_conv2d_i8_nhwc(_vp(xp), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None,
                                       ctypes.c_void_p(out.data_ptr() + 4 * offset), ctypes.c_int64(image_stride),
                                       n, ic, h, w, oc, kh, kw, strides[0], strides[1], padding[0], padding[1],
-                                      dilation[0], dilation[1], _stream()))
+                                      dilation[0], dilation[1], _conv_stream()))
     return out
 
 
@@ -471,12 +420,12 @@ def conv2d_stem_pool3_i8(x, w, bias, chain1, strides, padding, pool_oh, pool_ow)
     L.cvmhip_packed_stem_weight_bytes.restype = ctypes.c_size_t
     xs = _workspace(L.cvmhip_stem_input_bytes(n, h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1]), x.device)
     wp = _workspace(L.cvmhip_packed_stem_weight_bytes(oc, kh, kw), x.device)
-    check(L.cvmhip_pack_stem_input(_ptr(x), _vp(xs), n, c, h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1], _stream()))
-    check(L.cvmhip_pack_stem_weights(_ptr(w), _vp(wp), oc, c, kh, kw, _stream()))
+    check(L.cvmhip_pack_stem_input(_ptr(x), _vp(xs), n, c, h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1], _conv_stream()))
+    check(L.cvmhip_pack_stem_weights(_ptr(w), _vp(wp), oc, c, kh, kw, _conv_stream()))
     out = _act_buffer(n * pool_oh * pool_ow, oc, x.device)
     check(L.cvmhip_conv2d_stem_pool3_i8(_vp(xs), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None, _vp(out),
                                         n, c, h, wd, oc, kh, kw, strides[0], strides[1], padding[0], padding[1],
-                                        pool_oh, pool_ow, _stream()))
+                                        pool_oh, pool_ow, _conv_stream()))
     return out
 
 
@@ -487,7 +436,7 @@ def pack_weights_pair(w_a, w_b):
     oc_b = w_b.shape[0]
     L.cvmhip_packed_weight_pair_bytes.restype = ctypes.c_size_t
     wp = _workspace(L.cvmhip_packed_weight_pair_bytes(oc_a, oc_b, ic, kh, kw), w_a.device)
-    check(L.cvmhip_pack_weights_pair(_ptr(w_a), oc_a, _ptr(w_b), oc_b, _vp(wp), ic, kh, kw, _stream()))
+    check(L.cvmhip_pack_weights_pair(_ptr(w_a), oc_a, _ptr(w_b), oc_b, _vp(wp), ic, kh, kw, _conv_stream()))
     return wp
 
 
@@ -498,7 +447,7 @@ def conv2d_i8_nhwc_pair(xp, n, ic, h, w, wp, kh, kw, out_a, offset_a, stride_a, 
                                            ctypes.c_void_p(out_a.data_ptr() + 4 * offset_a), ctypes.c_int64(stride_a), oc_a,
                                            ctypes.c_void_p(out_b.data_ptr() + 4 * offset_b), ctypes.c_int64(stride_b), oc_b,
                                            n, ic, h, w, kh, kw, strides[0], strides[1], padding[0], padding[1],
-                                           dilation[0], dilation[1], _stream()))
+                                           dilation[0], dilation[1], _conv_stream()))
 
 
 class HeadGroup:
@@ -560,17 +509,17 @@ class HeadGroup:
     def launch(self, i8=False):
         dev = torch.frombuffer(bytearray(self.table), dtype=torch.uint8).to(self.device)
         if i8:
-            check(lib().cvmhip_conv_group_launch_i8(_vp(dev), self.count, self.blocks, ctypes.c_double(0), ctypes.c_double(0), _stream()))
+            check(lib().cvmhip_conv_group_launch_i8(_vp(dev), self.count, self.blocks, ctypes.c_double(0), ctypes.c_double(0), _conv_stream()))
             torch.cuda.synchronize()
             return
-        check(lib().cvmhip_conv_group_launch(_vp(dev), self.count, self.blocks, ctypes.c_double(0), ctypes.c_double(0), _stream()))
+        check(lib().cvmhip_conv_group_launch(_vp(dev), self.count, self.blocks, ctypes.c_double(0), ctypes.c_double(0), _conv_stream()))
         torch.cuda.synchronize()
 
 
 def pack_depthwise_weights(w):
     c, one, kh, kw = w.shape
     wp = _workspace(lib().cvmhip_packed_depthwise_bytes(c, kh, kw), w.device)
-    check(lib().cvmhip_pack_depthwise_weights(_ptr(w), _vp(wp), c, kh, kw, _stream()))
+    check(lib().cvmhip_pack_depthwise_weights(_ptr(w), _vp(wp), c, kh, kw, _conv_stream()))
     return wp
 
 
@@ -583,7 +532,7 @@ def pack_depthwise_weights_mfma(w):
     L = lib()
     L.cvmhip_packed_depthwise_mfma_bytes.restype = ctypes.c_size_t
     wp = _workspace(L.cvmhip_packed_depthwise_mfma_bytes(c, kh, kw), w.device)
-    check(L.cvmhip_pack_depthwise_weights_mfma(_ptr(w), _vp(wp), c, kh, kw, _stream()))
+    check(L.cvmhip_pack_depthwise_weights_mfma(_ptr(w), _vp(wp), c, kh, kw, _conv_stream()))
     return wp
 
 
@@ -598,7 +547,7 @@ def depthwise_conv2d_mfma_i8(xp, n, c, h, w, wp, kh, kw, bias=None, chain1=None,
         out = torch.empty((n, c, oh, ow), dtype=torch.int32, device=xp.device)
     check(lib().cvmhip_depthwise_conv2d_mfma_i8(_vp(xp), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None,
                                                 _vp(out), int(out_is_i8), n, c, h, w, kh, kw, strides[0], strides[1],
-                                                padding[0], padding[1], dilation[0], dilation[1], _stream()))
+                                                padding[0], padding[1], dilation[0], dilation[1], _conv_stream()))
     return out
 
 
@@ -611,7 +560,7 @@ def depthwise_conv2d_i8(xp, n, c, h, w, wp, kh, kw, bias=None, chain1=None, out_
         out = torch.empty((n, c, oh, ow), dtype=torch.int32, device=xp.device)
     check(lib().cvmhip_depthwise_conv2d_i8(_vp(xp), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None,
                                            _vp(out), int(out_is_i8), n, c, h, w, kh, kw, strides[0], strides[1],
-                                           padding[0], padding[1], dilation[0], dilation[1], _stream()))
+                                           padding[0], padding[1], dilation[0], dilation[1], _conv_stream()))
     return out
 
 
@@ -623,7 +572,7 @@ def add_i8(a, b, n, c, h, w, chain1=None, out_is_i8=True, out=None):
     else:
         out = torch.empty((n, c, h, w), dtype=torch.int32, device=a.device)
     check(lib().cvmhip_add_i8(_vp(a), _vp(b), ctypes.byref(chain1) if chain1 else None, _vp(out), int(out_is_i8),
-                              n, c, h * w, _stream()))
+                              n, c, h * w, _conv_stream()))
     return out
 
 
@@ -631,7 +580,7 @@ def max_pool2d_i8(xp, n, c, h, w, pool_size, strides, padding, oh, ow, out=None)
     if out is None:
         out = _act_buffer(n * oh * ow, c, xp.device)
     check(lib().cvmhip_max_pool2d_i8(_vp(xp), _vp(out), n, c, h, w, oh, ow, pool_size[0], pool_size[1],
-                                     strides[0], strides[1], padding[0], padding[1], _stream()))
+                                     strides[0], strides[1], padding[0], padding[1], _conv_stream()))
     return out
 
 
@@ -643,7 +592,7 @@ def sum_hw_i8(xp, n, c, hw, chain1=None, out_is_i8=False, out=None):
     else:
         out = torch.empty((n, c), dtype=torch.int32, device=xp.device)
     check(lib().cvmhip_sum_hw_i8(_vp(xp), ctypes.byref(chain1) if chain1 else None, _vp(out), int(out_is_i8),
-                                 n, c, hw, _stream()))
+                                 n, c, hw, _conv_stream()))
     return out
 
 
@@ -657,8 +606,8 @@ def conv2d_stem_i8(x, w, bias=None, chain1=None, out_is_i8=True, strides=(1, 1),
     assert L.cvmhip_stem_eligible(c, kh, kw, 1, 1)
     xs = _workspace(L.cvmhip_stem_input_bytes(n, h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1]), x.device)
     wp = _workspace(L.cvmhip_packed_stem_weight_bytes(oc, kh, kw), x.device)
-    check(L.cvmhip_pack_stem_input(_ptr(x), _vp(xs), n, c, h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1], _stream()))
-    check(L.cvmhip_pack_stem_weights(_ptr(w), _vp(wp), oc, c, kh, kw, _stream()))
+    check(L.cvmhip_pack_stem_input(_ptr(x), _vp(xs), n, c, h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1], _conv_stream()))
+    check(L.cvmhip_pack_stem_weights(_ptr(w), _vp(wp), oc, c, kh, kw, _conv_stream()))
     oh, ow = conv_out_hw(h, wd, kh, kw, strides[0], strides[1], padding[0], padding[1], 1, 1)
     if out_is_i8:
         out = _act_buffer(n * oh * ow, oc, x.device)
@@ -666,5 +615,5 @@ def conv2d_stem_i8(x, w, bias=None, chain1=None, out_is_i8=True, strides=(1, 1),
         out = torch.empty((n, oc, oh, ow), dtype=torch.int32, device=x.device)
     check(L.cvmhip_conv2d_stem_i8(_vp(xs), _vp(wp), _ptr(bias), ctypes.byref(chain1) if chain1 else None, _vp(out),
                                   int(out_is_i8), n, c, h, wd, oc, kh, kw, strides[0], strides[1], padding[0], padding[1],
-                                  _stream()))
+                                  _conv_stream()))
     return out
