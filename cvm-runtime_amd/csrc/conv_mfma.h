@@ -215,6 +215,8 @@ StemGeom stem_geom(int n, int h, int w, int kh, int kw, int sh, int sw, int ph, 
 size_t packed_stem_weight_bytes(int oc, int kp);
 int pack_stem_input(const int32_t* x, int8_t* xs, int n, int c, int h, int w, int kh, int kw, int sh, int sw, int ph,
                     int pw, hipStream_t s);
+int pack_stem_input_i8(const int8_t* x, int range, int8_t* xs, int n, int c, int h, int w, int kh, int kw, int sh, int sw, int ph,
+                       int pw, hipStream_t s);
 int pack_stem_weights(const int32_t* w, int8_t* wp, int oc, int c, int kh, int kw, hipStream_t s);
 // Row-window convolution + chain + max_pool2d(3x3, stride 2, padding 1) in one launch (k_stem_pool): xs from
 // pack_stem_input, wp from pack_stem_weights, out the pooled int8 tensor (n, oc, qh, qw); oc 32 or 64.

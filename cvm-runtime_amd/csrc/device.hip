@@ -14,6 +14,7 @@ using namespace cvmhip;
   } while (0)
 
 #include <string.h>
+#include <chrono>
 #include <map>
 #include <string>
 #include <vector>
@@ -123,6 +124,109 @@ int cvmhip_copy_kernel(void* dst, const void* src, size_t bytes, void* stream) {
   if (blocks > 256 * 32) blocks = 256 * 32;
   k_copy16<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(reinterpret_cast<const int4*>(src), reinterpret_cast<int4*>(dst), count);
   return check_launch("copy_kernel");
+}
+
+// Pinned host memory -> device.  Bound by the bus: four 16-byte requests per thread in flight move 46 GB/s (one request
+// per thread: 42); the copy engine moves 59 GB/s, but the first kernel behind it waits about 10 us for its signal, and a
+// piece costs the engine 5 us (2.4 MB in four pieces behind the host's copy of each: 65 us to the first kernel here, 90 us
+// with the engine; 150 KB: 7 against 17 us).
+__global__ void __launch_bounds__(256) k_import(const int4* __restrict__ src, int4* __restrict__ dst, int64_t count, int tail) {
+  const int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+  int4 v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) v[u] = src[i + u * 256 < count ? i + u * 256 : count - 1];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (i + u * 256 < count) dst[i + u * 256] = v[u];
+  if (blockIdx.x == 0 && (int)threadIdx.x < tail)
+    reinterpret_cast<int8_t*>(dst + count)[threadIdx.x] = reinterpret_cast<const int8_t*>(src + count)[threadIdx.x];
+}
+
+__global__ void __launch_bounds__(64) k_import_small(const int8_t* __restrict__ src, int8_t* __restrict__ dst, int count) {
+  if ((int)threadIdx.x < count) dst[threadIdx.x] = src[threadIdx.x];
+}
+
+int cvmhip_import_bytes(void* dst, const void* src_host, size_t bytes, void* stream) {
+  if (bytes == 0) return CVMHIP_OK;
+  if (!dst || !src_host || ((uintptr_t)dst & 15) || ((uintptr_t)src_host & 15)) return arg_error("import_bytes");
+  const int64_t count = (int64_t)(bytes / 16);
+  const int tail = (int)(bytes % 16);
+  if (count == 0)
+    k_import_small<<<1, 64, 0, as_stream(stream)>>>(reinterpret_cast<const int8_t*>(src_host), reinterpret_cast<int8_t*>(dst), tail);
+  else
+    k_import<<<(unsigned)((count + 1023) / 1024), 256, 0, as_stream(stream)>>>(reinterpret_cast<const int4*>(src_host),
+                                                                               reinterpret_cast<int4*>(dst), count, tail);
+  return check_launch("import_bytes");
+}
+
+// Device -> pinned host memory, and a word that says so.  Every workgroup makes its stores visible to the host before it
+// counts itself out; the last one to count stores the ticket.  The host polls that word instead of waiting for the
+// stream (7.5 us from launch to seen, against 11.7 us for a launch and a stream synchronisation, and no copy calls).
+struct ExportArgs {
+  const int32_t* src[CVMHIP_EXPORT_MAX];
+  int32_t* dst[CVMHIP_EXPORT_MAX];
+  int64_t words[CVMHIP_EXPORT_MAX];
+  int count;
+};
+
+__global__ void __launch_bounds__(256) k_export(ExportArgs a, const uint32_t* __restrict__ status, uint32_t* __restrict__ status_host,
+                                                uint32_t* __restrict__ counter, uint32_t* __restrict__ flag, uint32_t ticket) {
+  const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+  for (int k = 0; k < a.count; ++k) {
+    const int64_t granules = a.words[k] / 4;
+    const int4* s = reinterpret_cast<const int4*>(a.src[k]);
+    int4* d = reinterpret_cast<int4*>(a.dst[k]);
+    for (int64_t i = first; i < granules; i += stride) d[i] = s[i];
+    const int64_t at = granules * 4 + first;
+    if (at < a.words[k]) a.dst[k][at] = a.src[k][at];
+  }
+  if (status && blockIdx.x == 0 && threadIdx.x == 0) *status_host = *status;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    if (before == gridDim.x - 1) {
+      *counter = 0;
+      __hip_atomic_store(flag, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+}
+
+int cvmhip_export_words(const void* const* src, void* const* dst_host, const int64_t* words, int count, const uint32_t* status,
+                        uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, uint32_t ticket, void* stream) {
+  if (!src || !dst_host || !words || count < 0 || count > CVMHIP_EXPORT_MAX || !counter || !flag_host || (status && !status_host))
+    return arg_error("export_words");
+  ExportArgs a{};
+  int64_t most = 0;
+  a.count = count;
+  for (int k = 0; k < count; ++k) {
+    if (!src[k] || !dst_host[k] || words[k] < 0 || ((uintptr_t)src[k] & 15) || ((uintptr_t)dst_host[k] & 15)) return arg_error("export_words");
+    a.src[k] = reinterpret_cast<const int32_t*>(src[k]);
+    a.dst[k] = reinterpret_cast<int32_t*>(dst_host[k]);
+    a.words[k] = words[k];
+    if (words[k] > most) most = words[k];
+  }
+  // 64 workgroups fill the bus
+  int64_t blocks = (most / 4 + 255) / 256;
+  if (blocks < 1) blocks = 1;
+  if (blocks > 64) blocks = 64;
+  k_export<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(a, status, status_host, counter, flag_host, ticket);
+  return check_launch("export_words");
+}
+
+int cvmhip_export_wait(const uint32_t* flag_host, uint32_t ticket, void* stream) {
+  if (!flag_host) return arg_error("export_wait");
+  // a run is milliseconds at most; past 50 ms the wait goes to the runtime, which also sees errors
+  const auto began = std::chrono::steady_clock::now();
+  for (uint32_t spin = 1;; ++spin) {
+    if (__atomic_load_n(flag_host, __ATOMIC_ACQUIRE) == ticket) return CVMHIP_OK;
+    if ((spin & 1023u) == 0 && std::chrono::steady_clock::now() - began > std::chrono::milliseconds(50)) break;
+    __builtin_ia32_pause();
+  }
+  HIP_TRY(hipStreamSynchronize(as_stream(stream)), "export_wait");
+  if (__atomic_load_n(flag_host, __ATOMIC_ACQUIRE) == ticket) return CVMHIP_OK;
+  set_error("export_wait: the stream ended without the outputs");
+  return CVMHIP_ERR_RUNTIME;
 }
 
 int cvmhip_copy_h2d(void* dst, const void* src, size_t bytes, void* stream) {

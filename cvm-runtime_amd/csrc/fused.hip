@@ -530,6 +530,15 @@ int cvmhip_pack_stem_input(const int32_t* x, void* xs, int n, int c, int h, int 
   return pack_stem_input(x, reinterpret_cast<int8_t*>(xs), n, c, h, w, kh, kw, stride_h, stride_w, pad_h, pad_w, as_stream(stream));
 }
 
+int cvmhip_pack_stem_input_i8(const void* x, int32_t range, void* xs, int n, int c, int h, int w, int kh, int kw,
+                              int stride_h, int stride_w, int pad_h, int pad_w, void* stream) {
+  if (!x || !xs || ((uintptr_t)xs & 15) || range < 0 || !stem_eligible(c, kh, kw, 1, 1) ||
+      cvmhip_stem_input_bytes(n, h, w, kh, kw, stride_h, stride_w, pad_h, pad_w) == 0)
+    return arg_error("pack_stem_input_i8");
+  return pack_stem_input_i8(reinterpret_cast<const int8_t*>(x), range, reinterpret_cast<int8_t*>(xs), n, c, h, w, kh, kw, stride_h,
+                            stride_w, pad_h, pad_w, as_stream(stream));
+}
+
 size_t cvmhip_packed_stem_weight_bytes(int oc, int kh, int kw) {
   if (oc < 1 || kh < 1 || kw < 1 || kw > 8) return 0;
   const int rb = kw * 4 <= 16 ? 16 : 32;

@@ -714,6 +714,24 @@ void HipGraphRuntime::BuildPlan() {
   }
   plan_ = std::move(plan);
   fused_ = true;
+  // An int8 input that only row-window convolutions read is packed for them from the caller's bytes.
+  data_stays_i8_ = false;
+  if (GetInputPrecision() <= 8) {
+    const uint32_t de = entry_id(input_nodes_[GetInputIndex("data")], 0);
+    bool only_stems = !is_head[de];
+    for (const PlanStep& st : plan_) {
+      if (st.kind == PlanStep::STEMPACK) {
+        if (st.src == de) data_stays_i8_ = true;
+      } else if (st.kind == PlanStep::NODE) {
+        for (const DevTensor& t : execs_[st.exec_index].call.in) only_stems = only_stems && t.data != entry_ptr_[de];
+      } else if (st.kind == PlanStep::PACK) {
+        only_stems = only_stems && st.src != de;
+      }
+    }
+    data_stays_i8_ = data_stays_i8_ && only_stems;
+    data_range_ = static_cast<int32_t>((static_cast<uint32_t>(1) << (precision_[de] - 1)) - 1);
+    if (data_stays_i8_) AllocInputStage();   // its address is part of the captured launches
+  }
   if (hooks_.fold_bias) FoldRequant();
   if (hooks_.seq) BuildSequences();
   BuildGroups();
@@ -934,6 +952,11 @@ void HipGraphRuntime::RunStep(PlanStep& st) {
       Check(cvmhip_unpack_nhwc_i8(i8_ptr_[st.src], entry_ptr_[st.dst], st.n, st.c, st.h, stream_), "unpack");
       break;
     case PlanStep::STEMPACK:
+      if (data_stays_i8_ && entry_ptr_[st.src] == DataDevicePtr()) {
+        Check(cvmhip_pack_stem_input_i8(in_stage_dev_, data_range_, static_cast<DeviceBuffer*>(st.aux.get())->ptr, st.n, st.c, st.h, st.w,
+                                        st.kh, st.kw, st.sh, st.sw, st.ph, st.pw, stream_), "pack_stem_input_i8");
+        break;
+      }
       Check(cvmhip_pack_stem_input(entry_ptr_[st.src], static_cast<DeviceBuffer*>(st.aux.get())->ptr, st.n, st.c, st.h, st.w,
                                    st.kh, st.kw, st.sh, st.sw, st.ph, st.pw, stream_), "pack_stem_input");
       break;

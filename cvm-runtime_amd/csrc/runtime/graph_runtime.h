@@ -216,8 +216,14 @@ class HipGraphRuntime {
   size_t workspace_bytes_ = 0;
   void* stream_ = nullptr;
   void* in_stage_host_ = nullptr;  // pinned staging copy of an int8 input
-  void* in_stage_dev_ = nullptr;   // its device copy before widening
-  void* out_stage_host_ = nullptr; // pinned copies of the outputs, back to back
+  void* in_stage_dev_ = nullptr;   // its device copy
+  bool in_stage_busy_ = false;     // the device may still read in_stage_host_
+  bool data_stays_i8_ = false;     // fused: nothing reads `data` as int32, the row-window packing takes in_stage_dev_
+  int32_t data_range_ = 0;         // clamp of the input
+  void AllocInputStage();
+  void* out_stage_host_ = nullptr; // pinned: ticket and status words, then the outputs back to back
+  void* out_counter_ = nullptr;    // device word of cvmhip_export_words
+  uint32_t ticket_ = 0;
   std::vector<const int32_t*> out_host_;
   std::vector<int32_t*> entry_ptr_;
   struct Exec { uint32_t nid; const OpKernel* kernel; OpCall call; };

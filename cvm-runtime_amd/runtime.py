@@ -91,10 +91,20 @@ def CVMAPIGetPreprocessMethod(net):
     return buf.value.decode()
 
 
+# bytes object of n bytes that are not initialised: the library writes a result straight into it, before anyone else has
+# seen it (a zeroed buffer and its copy into a bytes object cost 100 us for a detector's 600 KB)
+_new_bytes = ctypes.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.restype, _new_bytes.argtypes = ctypes.py_object, [ctypes.c_void_p, ctypes.c_ssize_t]
+
+
+def _inference(net, input_data, output_length):
+    out = _new_bytes(None, output_length)
+    _ck(lib().CVMAPIInference(net, ctypes.c_char_p(input_data), ctypes.c_int(len(input_data)), ctypes.c_char_p(out)), "CVMAPIInference")
+    return out
+
+
 def CVMAPIInference(net, input_data):
-    out = ctypes.create_string_buffer(CVMAPIGetOutputLength(net))
-    _ck(lib().CVMAPIInference(net, ctypes.c_char_p(input_data), ctypes.c_int(len(input_data)), out), "CVMAPIInference")
-    return out.raw
+    return _inference(net, input_data, CVMAPIGetOutputLength(net))
 
 
 class HipModel:
@@ -117,7 +127,7 @@ class HipModel:
             pass
 
     def inference(self, input_data):
-        return CVMAPIInference(self.net, input_data)
+        return _inference(self.net, input_data, self.output_length)
 
     def set_input(self, input_data):
         _ck(lib().CVMHIPSetInput(self.net, ctypes.c_char_p(input_data), ctypes.c_int(len(input_data))), "CVMHIPSetInput")

@@ -175,6 +175,18 @@ int cvmhip_host_free(void* ptr);
 /* int8 bytes already on the device -> the int32 `data` tensor, clamped to [-range, range]: the input
  * path of CvmRuntime::SetInput (src/runtime/graph_runtime.cc:317-397) without widening on the host */
 int cvmhip_widen_clamp_i8(const void* src, int32_t* dst, int64_t count, int32_t range, void* stream);
+/* Host <-> device through kernels on memory from cvmhip_host_alloc, for the two ends of an inference: no copy engine, and
+ * so no signal between an engine and the kernels around it.
+ * import: `bytes` from pinned host memory to the device (both 16-byte aligned; the last granule may be partial).
+ * export: up to CVMHIP_EXPORT_MAX device arrays of 32-bit words (sources and destinations 16-byte aligned), then `*status`
+ * (may be NULL) to status_host, then `ticket` to *flag_host, which the host may poll: when it reads the ticket, everything
+ * before it has arrived.  `counter` is one zeroed device word, left zero. */
+#define CVMHIP_EXPORT_MAX 8
+int cvmhip_import_bytes(void* dst, const void* src_host, size_t bytes, void* stream);
+int cvmhip_export_words(const void* const* src, void* const* dst_host, const int64_t* words, int count, const uint32_t* status,
+                        uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, uint32_t ticket, void* stream);
+/* Waits until *flag_host is `ticket`, and returns an error if the stream comes to its end without that. */
+int cvmhip_export_wait(const uint32_t* flag_host, uint32_t ticket, void* stream);
 int cvmhip_copy_h2d(void* dst, const void* src, size_t bytes, void* stream);
 int cvmhip_copy_d2h(void* dst, const void* src, size_t bytes, void* stream);
 int cvmhip_copy_d2d(void* dst, const void* src, size_t bytes, void* stream);
@@ -413,6 +425,9 @@ int cvmhip_stem_eligible(int c, int kh, int kw, int dil_h, int dil_w);
 size_t cvmhip_stem_input_bytes(int n, int h, int w, int kh, int kw, int stride_h, int stride_w, int pad_h, int pad_w);
 int cvmhip_pack_stem_input(const int32_t* x, void* xs, int n, int c, int h, int w, int kh, int kw,
                            int stride_h, int stride_w, int pad_h, int pad_w, void* stream);
+/* the same from int8 NCHW, every value first clamped to [-range, range] (the input clamp of the graph runtime) */
+int cvmhip_pack_stem_input_i8(const void* x, int32_t range, void* xs, int n, int c, int h, int w, int kh, int kw,
+                              int stride_h, int stride_w, int pad_h, int pad_w, void* stream);
 size_t cvmhip_packed_stem_weight_bytes(int oc, int kh, int kw);
 int cvmhip_pack_stem_weights(const int32_t* w, void* wp, int oc, int c, int kh, int kw, void* stream);
 int cvmhip_conv2d_stem_i8(const void* xs, const void* wp, const int32_t* bias, const cvmhip_chain* chain,

@@ -1,0 +1,50 @@
+"""The two ends of CVMAPIInference: the caller's bytes through the pinned buffer (pieces, odd sizes, the clamp) into the
+row-window or the plain layout, and the outputs with their ticket back -- against the oracle's graph executor."""
+import numpy as np
+import pytest
+
+import oracle.graph as og
+from cvm_runtime_amd import graphgen, runtime, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,c,h,w,k,stride,precision,second_reader", [
+    (1, 1, 1, 1, 1, 1, 8, False),       # one byte in
+    (1, 3, 5, 7, 3, 1, 6, False),       # rows that are not whole stores, values beyond the input's precision
+    (2, 4, 17, 13, 7, 2, 8, False),
+    (1, 3, 9, 33, 5, 2, 7, True),       # a second reader of the input: it exists as int32 too
+    (3, 32, 6, 6, 3, 1, 8, False),      # not a row-window layer
+    (7, 3, 224, 225, 3, 2, 8, False),   # several pieces, the last one ragged
+])
+def test_inference_ends(n, c, h, w, k, stride, precision, second_reader, dev):
+    g = graphgen.GraphBuilder("io-%d-%d-%d" % (n, c, w))
+    x = g.var("data", (n, c, h, w), precision)
+    heads = [g.conv_relu_q(x, 32, k, stride, k // 2)]
+    if second_reader:
+        heads = [g.reshape(heads[0], (n, 1, int(np.prod(g.shape(heads[0])[1:])))), g.reshape(g.clip8(x), (n, 1, c * h * w))]
+    js, pb = g.build(heads)
+    model = runtime.HipModel(js, pb)
+    params = graphgen.load_params(pb)
+    top = (1 << (precision - 1)) - 1
+    for call in range(3):   # eager, capture, replay, each on another input
+        data = synth.tensor("io", "x%d" % call, (n, c, h, w), -128, 127)
+        want = og.run_graph(js, params, np.clip(data, -top, top))
+        want = want[0].ravel() if len(want) == 1 else np.concatenate([v.reshape(n, -1) for v in want], axis=1).ravel()
+        got = np.frombuffer(model.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want), "call %d" % call
+    model.close()
+
+
+def test_many_calls_in_a_row(dev):
+    """Past the 64 calls after which the stream itself is waited for; outputs of several kilobytes."""
+    g, heads = graphgen.conv_op_graph(n=1, c=32, h=9, w=9, oc=40)
+    js, pb = g.build(heads)
+    model = runtime.HipModel(js, pb)
+    params = graphgen.load_params(pb)
+    inputs = [synth.tensor("io-many", str(i), (1, 32, 9, 9), -127, 127) for i in range(3)]
+    want = [og.run_graph(js, params, v)[0].ravel() for v in inputs]
+    for i in range(140):
+        got = np.frombuffer(model.inference(inputs[i % 3].astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want[i % 3]), i
+    model.close()
