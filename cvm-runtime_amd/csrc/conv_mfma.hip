@@ -2083,32 +2083,82 @@ __global__ void __launch_bounds__(256) k_pack_act(const int32_t* __restrict__ x,
 // has nch + 1 chunks; the last one is all zero (a K range that ends early reads
 // it instead of branching).  Layout: [OCp/32][nch + 1][64][16].
 // row_bytes > 0 selects the row-window K order k = kh*row_bytes + kw*4 + c (conv_mfma.h: StemGeom).
+__device__ __forceinline__ void pack_weight_dword(const int32_t* __restrict__ w, int8_t* __restrict__ wp, int64_t i,
+                                                  int oc, int ic, int taps, int cp, int nch, int row_bytes, int kw_taps) {
+  const int d = (int)(i & 3);
+  const int lane = (int)((i >> 2) & 63);
+  const int64_t t = i >> 8;
+  const int chunk = (int)(t % (nch + 1));
+  const int64_t tile = t / (nch + 1);
+  const int64_t o = tile * 32 + (lane & 31);
+  const int k = chunk * 32 + (lane >> 5) * 16 + d * 4;
+  int tap = k / cp, c = k - tap * cp;
+  if (row_bytes > 0) {
+    const int r = k / row_bytes, s4 = (k - r * row_bytes) >> 2;   // filter row, tap inside the window
+    tap = s4 < kw_taps ? r * kw_taps + s4 : taps;                  // window bytes past the last tap multiply by zero
+    c = 0;
+  }
+  uint32_t pack = 0;
+  if (o < oc && tap < taps && chunk < nch) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int32_t v = (c + j < ic) ? w[((int64_t)o * ic + c + j) * taps + tap] : 0;
+      pack |= (uint32_t)(uint8_t)(int8_t)v << (8 * j);
+    }
+  }
+  reinterpret_cast<uint32_t*>(wp)[i] = pack;
+}
+
 __global__ void __launch_bounds__(256) k_pack_weights(const int32_t* __restrict__ w, int8_t* __restrict__ wp, int64_t total,
                                                       int oc, int ic, int taps, int cp, int nch, int row_bytes, int kw_taps) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const int d = (int)(i & 3);
-    const int lane = (int)((i >> 2) & 63);
-    const int64_t t = i >> 8;
-    const int chunk = (int)(t % (nch + 1));
-    const int64_t tile = t / (nch + 1);
-    const int64_t o = tile * 32 + (lane & 31);
-    const int k = chunk * 32 + (lane >> 5) * 16 + d * 4;
-    int tap = k / cp, c = k - tap * cp;
-    if (row_bytes > 0) {
-      const int r = k / row_bytes, s4 = (k - r * row_bytes) >> 2;   // filter row, tap inside the window
-      tap = s4 < kw_taps ? r * kw_taps + s4 : taps;                  // window bytes past the last tap multiply by zero
-      c = 0;
-    }
-    uint32_t pack = 0;
-    if (o < oc && tap < taps && chunk < nch) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride)
+    pack_weight_dword(w, wp, i, oc, ic, taps, cp, nch, row_bytes, kw_taps);
+}
+
+// Pixel-blocked activations (Cp % 32 == 0), one 16-channel granule of a pixel per thread: a wavefront reads 64
+// consecutive pixels of a channel (256 bytes) in each of 16 loads, all in flight, and stores two runs of 512 bytes.
+// `lin` counts pixels (rounded up to whole wavefronts) inside channel granules.  Bound by memory: the three inputs of a
+// bottleneck at batch 16 (51, 13 and 13 MB) with their filters take 7.0 us on average, against 8.3 us with a dword of the
+// destination per thread (64-byte pieces of four channels per load) and 3.5 us for the filter's own launch.
+__device__ __forceinline__ void pack_act_granule(const int32_t* __restrict__ x, int8_t* __restrict__ xp, int64_t lin, int64_t npix,
+                                                 int64_t wave_pix, int c, int hw, int cp, FastDiv div_hw) {
+  const int granule = (int)(lin / wave_pix);   // the same for a whole wavefront
+  const int64_t p = lin - granule * wave_pix;
+  if (p >= npix) return;
+  const int64_t n = fastdiv((unsigned)p, div_hw);
+  const int32_t* xc = x + n * c * hw + (p - n * hw);
+  const int c0 = granule * 16;
+  int32_t v[16];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int32_t v = (c + j < ic) ? w[((int64_t)o * ic + c + j) * taps + tap] : 0;
-        pack |= (uint32_t)(uint8_t)(int8_t)v << (8 * j);
-      }
-    }
-    reinterpret_cast<uint32_t*>(wp)[i] = pack;
+  for (int j = 0; j < 16; ++j) v[j] = xc[(int64_t)(c0 + j < c ? c0 + j : c - 1) * hw];
+  __builtin_amdgcn_sched_barrier(0);
+  uint32_t d[4];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) v[j] = c0 + j < c ? v[j] : 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) d[q] = pack_bytes(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+  *reinterpret_cast<uint4*>(xp + act_offset(p, c0, cp)) = make_uint4(d[0], d[1], d[2], d[3]);
+}
+
+__global__ void __launch_bounds__(256) k_pack_act16(const int32_t* __restrict__ x, int8_t* __restrict__ xp, int64_t total, int64_t npix,
+                                                    int64_t wave_pix, int c, int hw, int cp, FastDiv div_hw) {
+  const int64_t lin = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (lin < total) pack_act_granule(x, xp, lin, npix, wave_pix, c, hw, cp, div_hw);
+}
+
+// Both operands of a convolution called on int32 tensors, one launch: the first act_blocks workgroups pack the
+// activations, the others the filter.  Neither reads what the other writes, and a launch is 2.3 us.
+__global__ void __launch_bounds__(256) k_pack_both(const int32_t* __restrict__ x, int8_t* __restrict__ xp, int64_t act_total,
+                                                   unsigned act_blocks, int64_t npix, int64_t wave_pix, int c, int hw, int cp,
+                                                   FastDiv div_hw, const int32_t* __restrict__ w, int8_t* __restrict__ wp,
+                                                   int64_t w_total, int oc, int taps, int nch) {
+  if (blockIdx.x < act_blocks) {
+    const int64_t lin = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (lin < act_total) pack_act_granule(x, xp, lin, npix, wave_pix, c, hw, cp, div_hw);
+  } else {
+    const int64_t i = (int64_t)(blockIdx.x - act_blocks) * 256 + threadIdx.x;
+    if (i < w_total) pack_weight_dword(w, wp, i, oc, c, taps, cp, nch, 0, 0);
   }
 }
 
@@ -2225,6 +2275,67 @@ k_conv_grouped(const int32_t* __restrict__ x, const int32_t* __restrict__ w, con
       }
     }
     y[i] = wadd(acc, bias ? bias[o] : 0);
+  }
+}
+
+// One input channel per group (depthwise, with or without a channel multiplier), filter rows of KW taps: four
+// neighbouring outputs of a row per thread, so a row of the window is read once for four outputs, and the filter, which is
+// the same for a whole workgroup (one output plane), comes through the scalar cache.  Same exact int32 products.
+// Bound by the 32-bit multiplies (a quarter of the rate of an add: 36 of them, 3.3 us of the chip for 4 x 96 x 75 x 75) and
+// by the masks of the border: 13.4 us there against 23 us for one output per thread.
+template <int KH, int KW, bool UNIT>
+__global__ void __launch_bounds__(256)
+k_conv_planes(const int32_t* __restrict__ x, const int32_t* __restrict__ w, const int32_t* __restrict__ bias, int32_t* __restrict__ y,
+              int planes, int ic, int h, int wd, int oc, int oh, int ow, int sh, int sw, int ph, int pw, int dh, int dw, int ocg,
+              FastDiv div_quads) {
+  const int quads = (ow + 3) >> 2;
+  for (int plane = blockIdx.y; plane < planes; plane += gridDim.y) {
+    const int b = plane / oc, o = plane - b * oc;
+    const int32_t* xc = x + ((int64_t)b * ic + o / ocg) * h * wd;
+    const int32_t* wc = w + (int64_t)o * KH * KW;
+    const int32_t b0 = bias ? bias[o] : 0;
+    const int lin = blockIdx.x * 256 + threadIdx.x;
+    if (lin >= oh * quads) continue;
+    const int p = (int)fastdiv((unsigned)lin, div_quads), q = (lin - p * quads) * 4;
+    // every load of the window is issued, from the nearest pixel inside, and masked afterwards; at stride 1 the windows
+    // of the four outputs share their columns
+    constexpr int COLS = UNIT ? KW + 3 : 4 * KW;
+    int32_t v[KH][COLS];
+#pragma unroll
+    for (int r = 0; r < KH; ++r) {
+      const int ih = p * sh + r * dh - ph;
+      const int32_t* xr = xc + (int64_t)(ih < 0 ? 0 : (ih < h ? ih : h - 1)) * wd;
+#pragma unroll
+      for (int e = 0; e < COLS; ++e) {
+        const int iw = UNIT ? q + e - pw : (q + e / KW) * sw + (e % KW) * dw - pw;
+        v[r][e] = xr[iw < 0 ? 0 : (iw < wd ? iw : wd - 1)];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    int32_t acc[4] = {b0, b0, b0, b0};
+#pragma unroll
+    for (int r = 0; r < KH; ++r) {
+      const int ih = p * sh + r * dh - ph;
+      const bool row = ih >= 0 && ih < h;
+#pragma unroll
+      for (int e = 0; e < COLS; ++e) {
+        const int iw = UNIT ? q + e - pw : (q + e / KW) * sw + (e % KW) * dw - pw;
+        v[r][e] = row && iw >= 0 && iw < wd ? v[r][e] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int t = 0; t < KW; ++t) acc[u] = wadd(acc[u], wmul(v[r][UNIT ? u + t : u * KW + t], wc[r * KW + t]));
+    }
+    int32_t* yr = y + (int64_t)plane * oh * ow + (int64_t)p * ow + q;
+    typedef int v4i __attribute__((ext_vector_type(4), aligned(4)));   // rows need not start on 16 bytes
+    if (q + 3 < ow) {
+      *reinterpret_cast<v4i*>(yr) = v4i{acc[0], acc[1], acc[2], acc[3]};
+    } else {
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        if (q + u < ow) yr[u] = acc[u];
+    }
   }
 }
 
@@ -2362,6 +2473,13 @@ int pack_activations(const int32_t* x, int8_t* xp, int n, int c, int hw, hipStre
   const int64_t total = act_bytes(npix, cp) / 4;
   if (total == 0) return CVMHIP_OK;
   KernelTimer timer("k_pack_act", (double)n * c * hw * 5.0, s);  // bytes: 4 read + 1 written per element
+  if (cp % 32 == 0 && npix < INT32_MAX) {
+    const int64_t wave_pix = (npix + 63) / 64 * 64, lins = wave_pix * (cp / 16), grid = (lins + 255) / 256;
+    if (grid <= INT32_MAX) {
+      k_pack_act16<<<(unsigned)grid, 256, 0, s>>>(x, xp, lins, npix, wave_pix, c, hw, cp, make_fastdiv((uint32_t)hw));
+      return check_launch("pack_act");
+    }
+  }
   k_pack_act<<<grid_for(total, 256), 256, 0, s>>>(x, reinterpret_cast<uint32_t*>(xp), total, npix, c, hw, cp);
   return check_launch("pack_act");
 }
@@ -2380,6 +2498,25 @@ int pack_weights(const int32_t* w, int8_t* wp, int oc, int ic, int kh, int kw, h
   const int64_t total = (int64_t)(ocp / 32) * (nch + 1) * 256;  // dwords
   k_pack_weights<<<grid_for(total, 256), 256, 0, s>>>(w, wp, total, oc, ic, kh * kw, pad_channels(ic), nch, 0, kw);
   return check_launch("pack_weights");
+}
+
+// pack_activations and pack_weights for one convolution
+static int pack_operands(const int32_t* x, int8_t* xp, int n, int ic, int hw, const int32_t* w, int8_t* wp, int oc, int kh, int kw,
+                         hipStream_t s) {
+  const int cp = pad_channels(ic);
+  const int64_t npix = (int64_t)n * hw, wave_pix = (npix + 63) / 64 * 64, act_total = wave_pix * (cp / 16);
+  int ocp, kp;
+  weight_dims(oc, ic, kh, kw, &ocp, &kp);
+  const int nch = kp / 32;
+  const int64_t w_total = (int64_t)(ocp / 32) * (nch + 1) * 256;
+  const int64_t act_blocks = (act_total + 255) / 256, w_blocks = (w_total + 255) / 256;
+  if (cp % 32 != 0 || npix >= INT32_MAX || act_blocks + w_blocks > INT32_MAX) {   // few channels: kept as NHWC, packed by dwords
+    const int rc = pack_activations(x, xp, n, ic, hw, s);
+    return rc ? rc : pack_weights(w, wp, oc, ic, kh, kw, s);
+  }
+  k_pack_both<<<(unsigned)(act_blocks + w_blocks), 256, 0, s>>>(x, xp, act_total, (unsigned)act_blocks, npix, wave_pix, ic, hw, cp,
+                                                               make_fastdiv((uint32_t)hw), w, wp, w_total, oc, kh * kw, nch);
+  return check_launch("pack_operands");
 }
 
 bool stem_eligible(int c, int kh, int kw, int dil_h, int dil_w) {
@@ -3205,6 +3342,18 @@ int cvmhip_conv2d(const int32_t* x, const int32_t* w, const int32_t* bias, int32
   hipStream_t s = as_stream(stream);
   if (groups > 1) {
     const int64_t total = (int64_t)n * oc * oh * ow;
+    const int64_t quads = (int64_t)oh * ((ow + 3) / 4), planes = (int64_t)n * oc;
+    if (ic == groups && kh == 3 && kw == 3 && planes < INT32_MAX && quads < INT32_MAX && (int64_t)h * wd < INT32_MAX) {
+      const dim3 grid((unsigned)((quads + 255) / 256), (unsigned)(planes < 65535 ? planes : 65535));
+      const FastDiv div_quads = make_fastdiv((uint32_t)((ow + 3) / 4));
+      if (stride_w == 1 && dil_w == 1)
+        k_conv_planes<3, 3, true><<<grid, 256, 0, s>>>(x, w, bias, y, (int)planes, ic, h, wd, oc, oh, ow, stride_h, stride_w, pad_h,
+                                                       pad_w, dil_h, dil_w, oc / groups, div_quads);
+      else
+        k_conv_planes<3, 3, false><<<grid, 256, 0, s>>>(x, w, bias, y, (int)planes, ic, h, wd, oc, oh, ow, stride_h, stride_w, pad_h,
+                                                        pad_w, dil_h, dil_w, oc / groups, div_quads);
+      return check_launch("conv_planes");
+    }
     k_conv_grouped<<<grid_for(total, 256, 1 << 20), 256, 0, s>>>(x, w, bias, y, total, ic, h, wd, oc, oh, ow, kh, kw,
                                                                stride_h, stride_w, pad_h, pad_w, dil_h, dil_w,
                                                                ic / groups, oc / groups);
@@ -3214,9 +3363,7 @@ int cvmhip_conv2d(const int32_t* x, const int32_t* w, const int32_t* bias, int32
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return arg_error("conv2d workspace");
   int8_t* xp = reinterpret_cast<int8_t*>(workspace);
   int8_t* wp = xp + packed_act_bytes((int64_t)n * h * wd, ic);
-  int rc = pack_activations(x, xp, n, ic, h * wd, s);
-  if (rc) return rc;
-  rc = pack_weights(w, wp, oc, ic, kh, kw, s);
+  const int rc = pack_operands(x, xp, n, ic, h * wd, w, wp, oc, kh, kw, s);
   if (rc) return rc;
   ConvGeom g = {};
   g.N = n; g.H = h; g.W = wd; g.Cp = pad_channels(ic); g.C = ic;
@@ -3247,9 +3394,7 @@ int cvmhip_dense(const int32_t* x, const int32_t* w, const int32_t* bias, int32_
   // x[m][k] is already "NHWC" with one pixel per row; the filter is OC x K x 1 x 1
   int8_t* xp = reinterpret_cast<int8_t*>(workspace);
   int8_t* wp = xp + packed_act_bytes(m, k);
-  int rc = pack_activations(x, xp, m, k, 1, s);
-  if (rc) return rc;
-  rc = pack_weights(w, wp, n, k, 1, 1, s);
+  const int rc = pack_operands(x, xp, m, k, 1, w, wp, n, 1, 1, s);
   if (rc) return rc;
   ConvGeom g = {};
   g.N = m; g.H = 1; g.W = 1; g.Cp = pad_channels(k); g.C = k;

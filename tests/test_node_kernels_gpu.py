@@ -1,0 +1,47 @@
+"""Kernels of the int32 operator contract at the edges of their splits, against the oracle: long reductions, operand packing
+of a convolution, depthwise planes."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from cvm_runtime_amd import hipops, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def T(a, dev):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+
+
+@pytest.mark.parametrize("op", ["sum", "max"])
+@pytest.mark.parametrize("outputs,run", [(1, 513), (3, 1023), (2, 1024), (5, 1025), (7, 4099), (300, 3136), (1, 70001)])
+def test_long_runs(op, outputs, run, dev):
+    x = synth.tensor("runs", "%d-%d" % (outputs, run), (outputs, run), -2 ** 31, 2 ** 31 - 1)
+    x[0] = -np.abs(x[0] // 2) - 1   # all negative
+    got = hipops.reduce(op, T(x, dev), (1,)).cpu().numpy()
+    assert np.array_equal(got, oracle.reduce(op, x, (1,)))
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,k", [(1, 17, 1, 1, 5, 1), (2, 33, 7, 9, 40, 3), (3, 64, 5, 13, 32, 1), (1, 100, 8, 8, 130, 3)])
+def test_conv_operand_packing(n, c, h, w, oc, k, dev):
+    x = synth.tensor("packing", "x%d" % c, (n, c, h, w), -300, 300)   # narrowed like the reference narrows
+    wt = synth.tensor("packing", "w%d" % c, (oc, c, k, k), -127, 127)
+    got = hipops.conv2d(T(x, dev), T(wt, dev), None, (1, 1), (k // 2, k // 2)).cpu().numpy()
+    assert np.array_equal(got, oracle.conv2d(x, wt, None, (1, 1), (k // 2, k // 2)))
+
+
+@pytest.mark.parametrize("n,c,mult,h,w,strides,padding,dilation", [
+    (1, 2, 1, 3, 3, (1, 1), (0, 0), (1, 1)),       # one output
+    (2, 3, 2, 5, 7, (1, 1), (1, 1), (1, 1)),       # a channel multiplier; rows that are not whole quads
+    (1, 5, 1, 9, 6, (2, 2), (1, 1), (1, 1)),
+    (1, 4, 1, 12, 11, (1, 2), (2, 3), (2, 1)),
+    (1, 4, 1, 12, 70, (2, 1), (0, 2), (1, 3)),
+    (3, 130, 1, 33, 64, (1, 1), (1, 1), (1, 1)),   # several workgroups per plane
+])
+def test_depthwise_planes(n, c, mult, h, w, strides, padding, dilation, dev):
+    x = synth.tensor("planes", "x%d-%d" % (c, w), (n, c, h, w), -2 ** 31, 2 ** 31 - 1)   # exact and wrapping
+    wt = synth.tensor("planes", "w%d-%d" % (c, w), (c * mult, 1, 3, 3), -2 ** 31, 2 ** 31 - 1)
+    b = synth.tensor("planes", "b%d" % c, (c * mult,), -32768, 32768)
+    got = hipops.conv2d(T(x, dev), T(wt, dev), T(b, dev), strides, padding, dilation, groups=c).cpu().numpy()
+    assert np.array_equal(got, oracle.conv2d(x, wt, b, strides, padding, dilation, groups=c))
