@@ -733,6 +733,7 @@ void HipGraphRuntime::BuildPlan() {
     if (data_stays_i8_) AllocInputStage();   // its address is part of the captured launches
   }
   if (hooks_.fold_bias) FoldRequant();
+  BuildResident();
   if (hooks_.seq) BuildSequences();
   BuildGroups();
 }
@@ -809,6 +810,7 @@ void HipGraphRuntime::BuildSequences() {
         r.bytes += static_cast<double>(st.n) * st.h * st.w * st.c + static_cast<double>(st.oc) * st.c * st.kh * st.kw +
                    px * st.oc * (st.src2 != kNone ? 2.0 : 1.0);
       }
+      for (ResidentRun& q : residents_) q.under_seq = q.under_seq || (q.first < j && q.last >= i);
       for (size_t k = 0; k < count; ++k) r.cfgs.push_back(cvmhip_conv_seq_layer_config(table.data(), static_cast<int>(k)));
       seq_at_[i] = static_cast<int>(seqs_.size());
       seqs_.push_back(r);
@@ -842,7 +844,7 @@ void HipGraphRuntime::BuildGroups() {
     size_t j = i;
     for (; j < plan_.size(); ++j) {
       const PlanStep& st = plan_[j];
-      if (st.kind != PlanStep::CONV || !st.nhwc || st.stem) break;
+      if (in_resident_[j] || st.kind != PlanStep::CONV || !st.nhwc || st.stem) break;
       table.resize((j - i + 1) * entry);
       int nb = 0;
       const int32_t* bias = st.pair ? static_cast<const int32_t*>(static_cast<DeviceBuffer*>(st.pair_bias.get())->ptr) : st.bias;
@@ -893,7 +895,7 @@ void HipGraphRuntime::BuildGroups() {
     size_t j = i;
     for (; j < plan_.size(); ++j) {
       const PlanStep& st = plan_[j];
-      if (st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
+      if (in_resident_[j] || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
       bool reads_member = false;
       for (uint32_t w : written) reads_member = reads_member || st.src == w || st.src2 == w;
       if (reads_member) break;

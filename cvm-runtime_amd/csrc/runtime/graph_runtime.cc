@@ -446,6 +446,10 @@ HipGraphRuntime::HipGraphRuntime(const std::string& graph_json, int device_id, b
 void HipGraphRuntime::ReadHooks() {
   auto env = [](const char* name) { const char* v = std::getenv(name); return std::string(v ? v : ""); };
   hooks_.fuse = env("CVM_HIP_FUSE") != "0";
+  hooks_.resident = env("CVM_HIP_RESIDENT") != "0";
+  for (const char* other : {"CVM_HIP_SEQ", "CVM_HIP_SEQCFG", "CVM_HIP_DW", "CVM_HIP_POOLFUSE", "CVM_HIP_HEADPAIR", "CVM_HIP_HEADGROUP",
+                            "CVM_HIP_CONVGROUP", "CVM_HIP_FLATDENSE", "CVM_HIP_CONV", "CVM_HIP_WAVECFG", "CVM_HIP_TILE"})
+    hooks_.resident = hooks_.resident && env(other).empty();
   hooks_.fold_bias = env("CVM_HIP_FOLDBIAS") != "0";
   hooks_.graph = env("CVM_HIP_GRAPH") != "0";
   hooks_.seq = env("CVM_HIP_SEQ") != "0";
@@ -495,6 +499,7 @@ void HipGraphRuntime::Release() {
   if (seq_counted_) { CountSequenceModel(-1); seq_counted_ = false; }
   seqs_.clear();
   groups_.clear();
+  residents_.clear();
   if (seq_sync_) { cvmhip_free(seq_sync_); seq_sync_ = nullptr; }
   if (seq_error_host_) { cvmhip_host_free(seq_error_host_); seq_error_host_ = nullptr; }
   execs_.clear();  // releases per-node device state before the stream goes away
@@ -712,7 +717,8 @@ void HipGraphRuntime::LoadParams(const std::string& blob) {
   }
 }
 
-// Layer-sequence launches pay for layers that are bound by latency and cost a little where layers are large:
+// Layer-sequence launches pay for layers that are bound by latency and cost a little where layers are large, and steps that
+// could also run with their maps in LDS have a third form, which the other two leave room for:
 // which way a model runs faster is measured once, when it is loaded (a few replays each way; timing does not
 // depend on the values in the tensors, so whatever the storage holds will do), unless CVM_HIP_SEQ=1 forces them.
 void HipGraphRuntime::CalibrateSequences() {
@@ -771,7 +777,11 @@ void HipGraphRuntime::Launch() {
   if (fused_) {
     const bool seq = seq_mode_;
     for (size_t i = 0; i < plan_.size();) {
-      if (seq && seq_at_[i] >= 0) {   // (a sequence launch covers whatever grouped launches lie inside its run)
+      if (resident_at_[i] >= 0 && !(seq && residents_[resident_at_[i]].under_seq)) {
+        const ResidentRun& r = residents_[resident_at_[i]];
+        HipCheck(cvmhip_resident_launch(r.table, r.nlayers, r.images, r.lds, r.ops, r.bytes, stream_), "layers in LDS");
+        i = r.last + 1;
+      } else if (seq && seq_at_[i] >= 0) {   // (a sequence launch covers whatever grouped launches lie inside its run)
         const SeqRun& r = seqs_[seq_at_[i]];
         HipCheck(cvmhip_conv_seq_launch(r.table, r.nlayers, seq_sync_, r.ops, r.bytes, stream_), "layer-sequence launch");
         seq_ran_ = true;

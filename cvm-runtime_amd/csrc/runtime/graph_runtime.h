@@ -176,6 +176,8 @@ class HipGraphRuntime {
     int extra = 0;   // steps of two launches: a dense layer over a whole map behind the copy that flattens the map
     if (fused_)
       for (const PlanStep& st : plan_) extra += st.flat ? 1 : 0;
+    for (const ResidentRun& r : residents_)
+      if (!(r.under_seq && SeqNow())) grouped += static_cast<int>(r.last - r.first);
     if (launches) *launches = static_cast<int>(NumSteps()) - lay + seq - (fused_ ? grouped : 0) + extra;
     if (sequences) *sequences = seq;
     if (layers) *layers = lay;
@@ -242,6 +244,9 @@ class HipGraphRuntime {
     int conv_kernel = 0, wave_cfg = -1, tile_wm = 0, tile_wn = 0;
     // layer-sequence launches: CVM_HIP_SEQ_SPIN=<polls> patience of a wait at a layer boundary (0: every wait gives up at once)
     int seq_spin = 2000000;
+    // CVM_HIP_RESIDENT=0: no launches with the maps in LDS.  Off as well when another launch form is asked for by name
+    // (any of the switches of the planner or of the kernel choice is set): those name forms of single layers.
+    bool resident = true;
     bool flat_dense = true;   // CVM_HIP_FLATDENSE=0: a dense layer over a whole map gathers its operand from the map as it lies
     bool seq_chains = true;   // CVM_HIP_SEQ_CHAIN=0: no 1x1 layers chained behind the layer that feeds them (cvmhip_conv_seq_link)
     std::vector<std::pair<int, int>> seq_layer_cfg;   // CVM_HIP_SEQCFG: (layer of a sequence, configuration)
@@ -290,6 +295,24 @@ class HipGraphRuntime {
     double ops = 0, bytes = 0;
   };
   void BuildGroups();
+  // Runs of steps whose maps fit in LDS, one workgroup per image (resident_plan.cc)
+  struct ResidentRun {
+    size_t first = 0, last = 0;         // plan_ indices, inclusive
+    std::shared_ptr<void> owner;        // table, filters and biases (device)
+    void* table = nullptr;
+    int nlayers = 0, images = 0;
+    size_t lds = 0;
+    bool under_seq = false;             // shares steps with a sequence launch, which runs instead where sequences are in use
+    double ops = 0, bytes = 0;
+  };
+  struct ResidentDraft;
+  void BuildResident();
+  bool ResidentEligible(const PlanStep& st) const;
+  double ResidentGain(const PlanStep& st) const;      // microseconds saved by the step inside such a launch, estimated
+  ResidentDraft DraftResident(size_t first, size_t last) const;
+  std::vector<ResidentRun> residents_;
+  std::vector<int> resident_at_;        // per plan_ index: the run that starts there, or -1
+  std::vector<bool> in_resident_;       // per plan_ index: inside such a run
   std::vector<GroupRun> groups_;
   std::vector<int> group_at_;           // per plan_ index: the group that starts there, or -1
   void CalibrateSequences();            // measures a run with and without sequence launches, keeps the faster

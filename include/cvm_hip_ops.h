@@ -444,6 +444,37 @@ int cvmhip_conv2d_stem_pool3_i8_eligible(int n, int c, int h, int wd, int oc, in
 int cvmhip_conv2d_stem_pool3_i8(const void* xs, const void* wp, const int32_t* bias, const cvmhip_chain* chain, void* out,
                                 int n, int c, int h, int wd, int oc, int kh, int kw, int stride_h, int stride_w,
                                 int pad_h, int pad_w, int pool_oh, int pool_ow, void* stream);
+/* A run of layers whose maps fit in LDS in one launch, a workgroup per image.  The table (nlayers entries of
+ * cvmhip_resident_layer_bytes, filled on the host, read on the device at a 64-byte aligned address) holds the loads of what
+ * the run reads (kind 0: int8 NCHW image clamped to +-range, 1: int8 act tensor), convolutions (2: filter from
+ * cvmhip_resident_pack_filter, `bias` as many values as the output has channels in LDS: 16 or the next multiple of 32;
+ * v = chain(acc + bias), with a residual chain2(v + residual)), sums over the map (3, with chain) and max-pools (4).  A map
+ * lies at byte `at` of LDS (a multiple of 16, below cvmhip_resident_lds_limit; -1: not in LDS) with a border of zeros as wide
+ * as the padding of the convolutions that read it; maps that are alive together must not overlap.  out_mode: 0 the result
+ * stays in LDS, 1 it (also) goes to an int8 act tensor, 2 to int32 NCHW.  Maps with their borders are at most 255 x 255. */
+typedef struct cvmhip_resident_map {
+  int32_t at, c, h, w, border_y, border_x;
+} cvmhip_resident_map;
+typedef struct cvmhip_resident_desc {
+  int32_t kind;
+  cvmhip_resident_map src, res, dst;
+  int32_t kh, kw, sh, sw, ph, pw, dh, dw;
+  int32_t range, out_mode;
+  int32_t border_clean;   /* the border of dst is zero already: the last map at this place had the same extent and border */
+  const void* in;
+  const void* filter;
+  const int32_t* bias;
+  void* out;
+  cvmhip_chain chain, chain2;
+} cvmhip_resident_desc;
+size_t cvmhip_resident_layer_bytes(void);
+size_t cvmhip_resident_lds_limit(void);
+size_t cvmhip_resident_tensor_bytes(int c, int h, int w, int border_y, int border_x);
+size_t cvmhip_resident_filter_bytes(int oc, int c, int kh, int kw);
+int cvmhip_resident_pack_filter(const int32_t* w, void* dst, int oc, int c, int kh, int kw, int dil_h, int dil_w,
+                                int stored_w /* row of the input map in LDS, with its border */, void* stream);
+int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* desc);
+int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_t lds_bytes, double ops, double bytes, void* stream);
 /* depthwise conv2d (groups == channels == out channels) on int8 act tensors, filter packed by
  * cvmhip_pack_depthwise_weights into [kh*kw][cp] int8 */
 size_t cvmhip_packed_depthwise_bytes(int c, int kh, int kw);

@@ -1,0 +1,70 @@
+"""Layers whose maps stay in LDS, one launch for all of them, against the oracle running the graph node by node."""
+import numpy as np
+import pytest
+
+import oracle.graph as og
+from cvm_runtime_amd import graphgen, runtime, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _net(case, batch):
+    """A few layers with the forms that a launch tells apart; every case ends in sum and dense."""
+    name, c, h, w, widths = case
+    g = graphgen.GraphBuilder("resident-" + name)
+    x = g.var("data", (batch, c, h, w), 8)
+    x = g.conv_relu_q(x, widths[0], 3, 1, 1)
+    for i, oc in enumerate(widths[1:]):
+        y, k = g.conv(x, oc, 3, 1 + i % 2, 1 + (name == "dilated"), dilation=2 if name == "dilated" else 1)
+        if name == "multiply":
+            y = g.rshift(g.op("broadcast_mul", [y, g.param("m%d" % i, (1,), 3, 3, 3)], {}, [g.shape(y)])[0], graphgen.shift_for(k) + 2)
+        else:
+            y = g.rshift(g.relu(y), graphgen.shift_for(k))
+        z = g.conv_relu_q(y, oc, 1, relu=False)
+        x = g.rshift(g.relu(g.add(z, y)), 1)
+        if name == "pooled":
+            x = g.max_pool(x, 2, 2) if i % 2 else g.max_pool(x, 3, 2, 1)
+    s, _ = g.global_sum(x)
+    y, _ = g.dense(g.flatten(g.rshift(s, 4)), 7)
+    return g, [y]
+
+
+CASES = [
+    ("tile", 3, 16, 16, (16, 16, 32)),            # whole tiles of 16 pixels in a row
+    ("odd", 1, 7, 13, (5, 20, 33)),               # rows, channels and tiles with remainders
+    ("small", 3, 4, 3, (16, 48)),                 # fewer tiles than wavefronts
+    ("wide", 3, 8, 8, (64, 130, 96)),             # filters longer than what is requested ahead
+    ("dilated", 2, 12, 11, (24, 24, 24)),
+    ("multiply", 3, 10, 16, (16, 16, 16)),        # a chain that is no shift and clip
+    ("pooled", 3, 18, 22, (16, 24, 40)),
+]
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_small_maps_stay_in_lds(case, batch, dev):
+    g, heads = _net(case, batch)
+    js, pb = g.build(heads)
+    x = synth.tensor("resident-" + case[0], "data", (batch,) + case[1:4], -127, 127).astype(np.int8)
+    m = runtime.HipModel(js, pb)
+    steps = m.launch_counts()[0]
+    assert steps <= 3, steps          # the packed image, the launch, and at most what its last layer leaves
+    got = [np.frombuffer(m.inference(x.tobytes()), np.int32) for _ in range(3)]
+    m.close()
+    want = og.run_graph(js, graphgen.load_params(pb), x.astype(np.int32))[0].ravel()
+    for v in got:
+        assert np.array_equal(v, want)
+
+
+def test_images_in_rounds(dev):
+    """More images than compute units, and a partial last group of eight for the workgroups that fetch the filters."""
+    g, heads = _net(CASES[0], 261)
+    js, pb = g.build(heads)
+    x = synth.tensor("resident-rounds", "data", (261, 3, 16, 16), -127, 127).astype(np.int8)
+    m = runtime.HipModel(js, pb)
+    got = np.frombuffer(m.inference(x.tobytes()), np.int32).reshape(261, -1)
+    m.close()
+    for i in (0, 1, 255, 256, 260):
+        one, heads1 = _net(CASES[0], 1)
+        j1, p1 = one.build(heads1)
+        assert np.array_equal(got[i], og.run_graph(j1, graphgen.load_params(p1), x[i:i + 1].astype(np.int32))[0].ravel())
