@@ -1,6 +1,7 @@
 #include "graph_runtime.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -452,7 +453,8 @@ void HipGraphRuntime::ReadHooks() {
     hooks_.resident = hooks_.resident && env(other).empty();
   hooks_.fold_bias = env("CVM_HIP_FOLDBIAS") != "0";
   hooks_.graph = env("CVM_HIP_GRAPH") != "0";
-  hooks_.seq = env("CVM_HIP_SEQ") != "0";
+  hooks_.graph_forced = !env("CVM_HIP_GRAPH").empty();
+  hooks_.seq = env("CVM_HIP_SEQ") != "0" && env("CVM_HIP_RESIDENT") != "1";
   hooks_.seq_forced = env("CVM_HIP_SEQ") == "1";
   hooks_.seq_chains = env("CVM_HIP_SEQ_CHAIN") != "0";
   hooks_.flat_dense = env("CVM_HIP_FLATDENSE") != "0";
@@ -715,6 +717,33 @@ void HipGraphRuntime::LoadParams(const std::string& blob) {
     if (SeqNow()) CalibrateSequences();
     else seq_calibration_pending_ = true;
   }
+  ChooseSubmission();
+}
+
+// A graph is one submission, and saves the host what it costs to issue every launch (2.8 to 4 us each); but it reaches the
+// device about 7 us later than a launch does, and what follows it waits as long (calls of CVMAPIInference: ResNet-20, one
+// launch between input and output, 61 us as a graph, 54 without; SSD-512, 35 launches, 312 and 293; VGG-16 at batch 16 484
+// and 475; ResNet-50 at batch 50 1020 and 999).  Where the host is hardly faster than the device, its every delay shows:
+// ResNet-50 at batch 1, 52 launches of 4.7 us, took 264 us without a graph in one process and 299 in the next, and 270 to 277
+// with one in all.  So a few calls are made when the model is loaded, and launches are issued one by one where a call has 6 us
+// or more for each of them (SSD at 300 x 300 6.6, SSD-512 8.4, ResNet-50 5.2 at batch 1 and 6.4 at batch 6).
+// CVM_HIP_GRAPH=0 or 1 names a form (and with CVM_HIP_SEQ=1 nothing runs before the first call).
+void HipGraphRuntime::ChooseSubmission() {
+  if (!fused_ || !hooks_.graph || hooks_.graph_forced || hooks_.seq_forced || GetInputPrecision() > 8) return;
+  const std::vector<int8_t> input(static_cast<size_t>(shape_size(InputShape())), 0);
+  std::vector<double> us;
+  for (int i = 0; i < 11; ++i) {
+    const auto begin = std::chrono::steady_clock::now();
+    SetDataI8(input.data(), InputShape());
+    seq_mode_ = SeqNow();
+    Launch();
+    FetchOutputs();
+    us.push_back(1e6 * std::chrono::duration<double>(std::chrono::steady_clock::now() - begin).count());
+  }
+  std::nth_element(us.begin(), us.begin() + 5, us.end());
+  int launches = 0;
+  LaunchCounts(&launches, nullptr, nullptr);
+  hooks_.graph = us[5] < 6.0 * launches;
 }
 
 // Layer-sequence launches pay for layers that are bound by latency and cost a little where layers are large, and steps that
@@ -802,7 +831,8 @@ void HipGraphRuntime::Launch() {
 
 // The launches of a run never change (shapes, pointers and attributes are
 // fixed at load time), so after one eager run they are captured into an
-// executable graph and replayed with a single submission.  Per-kernel timing
+// executable graph and replayed with a single submission, unless issuing them one
+// by one measured faster (ChooseSubmission).  Per-kernel timing
 // needs the eager path (its event pairs must not end up inside a graph);
 // CVM_HIP_GRAPH=0 keeps it for good.
 void HipGraphRuntime::Run() {

@@ -42,10 +42,11 @@ CASES = [
 
 @pytest.mark.parametrize("batch", [1, 3])
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
-def test_small_maps_stay_in_lds(case, batch, dev):
+def test_small_maps_stay_in_lds(case, batch, dev, monkeypatch):
     g, heads = _net(case, batch)
     js, pb = g.build(heads)
     x = synth.tensor("resident-" + case[0], "data", (batch,) + case[1:4], -127, 127).astype(np.int8)
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "1")
     m = runtime.HipModel(js, pb)
     steps = m.launch_counts()[0]
     assert steps <= 3, steps          # the packed image, the launch, and at most what its last layer leaves
