@@ -1403,7 +1403,8 @@ k_conv_big(const int8_t* __restrict__ xp, const int8_t* __restrict__ wf, void* _
   constexpr int NA = BM / 32, NB = BN / 32;               // 32-row blocks of the two operands
   constexpr int AF = NA * 2, BF = NB * 2;                  // fragments per stage (two 32-byte chunks of K)
   constexpr int STAGE = (AF + BF) * 1024;
-  constexpr int NST = TM * TN <= 8 ? 3 : (STAGE * 4 <= 147456 ? 4 : 3);   // two workgroups per CU share the LDS when the tile is small
+  // two workgroups per CU share the LDS when the tile is small
+  constexpr int NST = TM * TN <= 4 ? 4 : TM * TN <= 8 ? 3 : (STAGE * 4 <= 147456 ? 4 : 3);
   constexpr int LA = AF / 4, LB = BF / 4;                  // requests per wavefront and stage
   constexpr int LPW = LA + LB;
   constexpr int PXW = NB / 4;                              // pixel blocks whose rows a wavefront gathers
@@ -1540,7 +1541,7 @@ k_conv_big(const int8_t* __restrict__ xp, const int8_t* __restrict__ wf, void* _
   // inside those 32 clocks is free.  (In blocks between groups of MFMAs the same instructions left the pipe idle
   // for half of a step when the workgroup had the CU to itself.)
   constexpr int H1 = LPW / 2, H2 = LPW - H1, NM = TM * TN;
-  static_assert(H2 <= NM - 3 && TM + TN <= NM, "a half step has an MFMA for every request, LDS read and piece of address arithmetic");
+  static_assert((H2 <= NM - 3 || (NM == 4 && H2 == 2)) && TM + TN <= NM, "a half step has an MFMA for every request, LDS read and piece of address arithmetic");
   auto lds16 = [&](const int8_t* p) __attribute__((always_inline)) { return *reinterpret_cast<const v4i*>(p + lane * 16); };
 #pragma unroll
   for (int st = 0; st < NST; ++st) {
@@ -2704,13 +2705,13 @@ static int choose_wave_cfg_base(const ConvGeom& g, int cus) {
 
 // ---- large-tile kernel: tile shapes and choice
 struct BigCfg { int wgm, wgn, tm, tn; };
-static const BigCfg kBigCfgs[] = {{2, 2, 4, 4}, {2, 2, 2, 4}, {1, 4, 2, 4}};   // 256x256, 128x256, 64x512 (channels x pixels)
+static const BigCfg kBigCfgs[] = {{2, 2, 4, 4}, {2, 2, 2, 4}, {1, 4, 2, 4}, {2, 2, 2, 2}};   // 256x256, 128x256, 64x512, 128x128 (channels x pixels)
 static int64_t big_cfg_blocks(const BigCfg& c, const ConvGeom& g) {
   const int bm = c.wgm * c.tm * 32, bn = c.wgn * c.tn * 32;
   return (int64_t)((g.OC + bm - 1) / bm) * ((g.P + bn - 1) / bn);
 }
 // The largest tile that does not reach past the layer's channels and still gives most compute units a tile; -1 when
-// the layer is too small for this kernel (fewer than 160 tiles of the smallest fitting shape, or a short K).
+// the layer is too small for this kernel (fewer than 144 tiles of the smallest fitting shape, or a short K).
 static int choose_big_cfg(const ConvGeom& g) {
   // K >= 512: with K = 256 (the 1x1 layers of a ResNet's second stage) the ring never fills and the wavefront
   // kernel is faster (7.5 us against 11.6 for 256 -> 128 channels over 16 x 56 x 56 pixels)
@@ -2719,7 +2720,12 @@ static int choose_big_cfg(const ConvGeom& g) {
   // 1.05-1.2 for the wavefront kernel); the 256 x 256 tile (one workgroup, 1.4) and the 64 x 512 one (0.65, below the
   // wavefront kernel's 0.96 on 64 -> 64 channels) are kept for forced use
   if (g.OC <= 64) return -1;
-  return big_cfg_blocks(kBigCfgs[1], g) >= 160 ? 1 : -1;
+  // From 144 tiles on, nine of sixteen compute units, the ring beats the wavefront kernel's own operand streams (ResNet-50 at
+  // batch 50, 154 tiles each: 20.7 -> 16.3 us for 128 -> 128 channels 3x3/2, 16.2 -> 12.7 for 1024 -> 512; batch 16, 100
+  // tiles: 7.4 -> 8.9 for the latter).  Where only the 128 x 128 tile has that many it takes the layer (14 x 14 pixels, 50
+  // images: 11.2 -> 9.5 us for 1024 -> 256, 19.4 -> 16.3 for 256 -> 256 3x3/2); with both the larger one is the faster
+  // (13.1 against 15.8 us for 512 -> 256 at 28 x 28).
+  return big_cfg_blocks(kBigCfgs[1], g) >= 144 ? 1 : big_cfg_blocks(kBigCfgs[3], g) >= 144 ? 3 : -1;
 }
 template <int OUT>
 static void launch_big_out(int cfg, unsigned grid, hipStream_t s, const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g,
@@ -2734,7 +2740,8 @@ static void launch_big_out(int cfg, unsigned grid, hipStream_t s, const int8_t* 
   }
   if (cfg == 0) k_conv_big<2, 2, 4, 4, OUT><<<grid, 256, 0, s>>>(xp, wp, out, g, ep);
   else if (cfg == 1) k_conv_big<2, 2, 2, 4, OUT><<<grid, 256, 0, s>>>(xp, wp, out, g, ep);
-  else k_conv_big<1, 4, 2, 4, OUT><<<grid, 256, 0, s>>>(xp, wp, out, g, ep);
+  else if (cfg == 2) k_conv_big<1, 4, 2, 4, OUT><<<grid, 256, 0, s>>>(xp, wp, out, g, ep);
+  else k_conv_big<2, 2, 2, 2, OUT><<<grid, 256, 0, s>>>(xp, wp, out, g, ep);
 }
 
 static void launch_wave(int cfg, int mode, unsigned grid, hipStream_t s, const int8_t* xp, const int8_t* wp, void* out,
@@ -2945,7 +2952,7 @@ int conv_igemm_ws(const int8_t* xp, const int8_t* wp, void* out, ConvGeom g, con
     int bcfg = big;
     if (tune.kernel == CONV_KERNEL_BIG && bcfg < 0 && !g.dw && !rows && (g.Cp % 32) == 0 && g.KH <= 32 && g.KW <= 32)
       bcfg = g.OC > 128 ? 0 : g.OC > 64 ? 1 : 2;   // forced: any size
-    if (tune.kernel == CONV_KERNEL_BIG && tune.tile_wm >= 1 && tune.tile_wm <= 3 && bcfg >= 0) bcfg = tune.tile_wm - 1;
+    if (tune.kernel == CONV_KERNEL_BIG && tune.tile_wm >= 1 && tune.tile_wm <= 4 && bcfg >= 0) bcfg = tune.tile_wm - 1;
     if (bcfg >= 0 && kslices <= 1) {
       const BigCfg& c = kBigCfgs[bcfg];
       if (pool_in_registers && c.tn == 4) ep.pool = 2;
