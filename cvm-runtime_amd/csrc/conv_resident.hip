@@ -101,7 +101,8 @@ __device__ __forceinline__ uint32_t res_pack(const int32_t (&v)[4]) {
 }
 
 // four channels of pixel p of this image, to LDS byte `at` and wherever else the layer wants them
-__device__ __forceinline__ void res_store(const ResHead& h, ResTable L, char* lds, int img, int p, int at, int oc, const int32_t (&v)[4]) {
+__device__ __forceinline__ void res_store(const ResHead& h, ResTable L, char* lds, int32_t* out_host, int img, int p, int at, int oc,
+                                          const int32_t (&v)[4]) {
   uint32_t d = res_pack(v);
   if (h.flags & RES_MASK) {
     const int left = L->OC - oc;
@@ -114,10 +115,13 @@ __device__ __forceinline__ void res_store(const ResHead& h, ResTable L, char* ld
       if (oc < gcp) res_write(reinterpret_cast<int8_t*>(L->out) + act_offset((int64_t)img * h.P + p, oc, gcp), d);
     } else {
       const int OC = L->OC;
-      int32_t* y = reinterpret_cast<int32_t*>(L->out) + ((int64_t)img * OC + oc) * h.P + p;
+      const int64_t first = ((int64_t)img * OC + oc) * h.P + p;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (oc + e < OC) res_write(y + (int64_t)e * h.P, v[e]);
+        if (oc + e < OC) {
+          res_write(reinterpret_cast<int32_t*>(L->out) + first + (int64_t)e * h.P, v[e]);
+          if (out_host) res_write(out_host + first + (int64_t)e * h.P, v[e]);
+        }
     }
   }
 }
@@ -215,7 +219,7 @@ __device__ __forceinline__ void res_border(const ResHead& h, ResTable L, char* l
 // The kernel is bound by instructions (a 16-channel layer has three products per 16 results of a lane group), so the
 // regular case keeps everything that does not differ between lanes in scalar registers and knows its tiles' distances.
 template <int TP, bool PLAIN>
-__device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds, int img, int wave, int lane) {
+__device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds, int32_t* out_host, int img, int wave, int lane) {
   constexpr int AHEAD = TP == 4 ? 2 : 3;   // (four pixel tiles leave registers for two chunks)
   ResRing<AHEAD> r;
   int item = wave, group = (int)fastdiv((unsigned)wave, h.div_oct), ot = wave - group * h.octiles;
@@ -308,7 +312,7 @@ __device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds
           } else {
             res_requant(h, lds, q.res + oc, v);
           }
-          res_store(h, L, lds, img, p, q.dst + oc, oc + (lane >> 4) * 4, v);
+          res_store(h, L, lds, out_host, img, p, q.dst + oc, oc + (lane >> 4) * 4, v);
         }
       }
     }
@@ -331,7 +335,8 @@ __device__ __forceinline__ ResHead res_head(ResTable L) {
   return h;
 }
 
-__global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* table, int nlayers, int images) {
+__global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* table, int nlayers, int images,
+                                                               const cvmhip_resident_call call) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int img = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -366,30 +371,48 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
     if (h.kind == RES_CONV) {
       const bool plain = (h.flags & (RES_CHAIN | RES_CHAIN2 | RES_MASK | RES_OUT | RES_REGULAR)) == RES_REGULAR;
       if (plain) {
-        if (h.tp == 1) res_conv<1, true>(h, L, lds, img, wave, lane);
-        else if (h.tp == 2) res_conv<2, true>(h, L, lds, img, wave, lane);
-        else res_conv<4, true>(h, L, lds, img, wave, lane);
+        if (h.tp == 1) res_conv<1, true>(h, L, lds, call.out_host, img, wave, lane);
+        else if (h.tp == 2) res_conv<2, true>(h, L, lds, call.out_host, img, wave, lane);
+        else res_conv<4, true>(h, L, lds, call.out_host, img, wave, lane);
       } else {
-        if (h.tp == 1) res_conv<1, false>(h, L, lds, img, wave, lane);
-        else if (h.tp == 2) res_conv<2, false>(h, L, lds, img, wave, lane);
-        else res_conv<4, false>(h, L, lds, img, wave, lane);
+        if (h.tp == 1) res_conv<1, false>(h, L, lds, call.out_host, img, wave, lane);
+        else if (h.tp == 2) res_conv<2, false>(h, L, lds, call.out_host, img, wave, lane);
+        else res_conv<4, false>(h, L, lds, call.out_host, img, wave, lane);
       }
       continue;
     }
     res_barrier();
     res_border(h, L, lds, tid);
     if (h.kind == RES_IMAGE) {
-      const int W = L->W, C = L->C, range = L->range;
-      const int8_t* x = L->in + (int64_t)img * C * h.P;
-      for (int p = tid; p < h.P; p += RES_THREADS) {
-        const int oy = (int)fastdiv((unsigned)p, h.div_ow), at = h.dst + oy * h.dst_row + (p - oy * W) * h.ocp;
-        for (int c0 = 0; c0 < h.ocp; c0 += 4) {
-          int32_t v[4];
+      const int C = L->C, range = L->range;
+      const int8_t* x = (call.image_host ? reinterpret_cast<const int8_t*>(call.image_host) : L->in) + (int64_t)img * C * h.P;
+      if (C <= 4 && (h.P & 3) == 0) {
+        // four pixels to a thread: all of an image's bytes are requested at once (host memory is 1.5 us away)
+        for (int p = tid * 4; p < h.P; p += RES_THREADS * 4) {
+          uint32_t d[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = c0 < C ? res_load<int8_t>(x + (int64_t)(c0 + e < C ? c0 + e : C - 1) * h.P + p) : 0;
+          for (int c = 0; c < 4; ++c) d[c] = res_load<uint32_t>(x + (c < C ? c : C - 1) * h.P + p);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = c0 + e < C ? res_clamp(v[e], -range, range) : 0;
-          *reinterpret_cast<uint32_t*>(lds + at + c0) = res_pack(v);
+          for (int j = 0; j < 4; ++j) {
+            const int oy = (int)fastdiv((unsigned)(p + j), h.div_ow), at = h.dst + oy * h.dst_row + (p + j - oy * h.OW) * h.ocp;
+            int32_t v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = c < C ? res_clamp((int32_t)(int8_t)(d[c] >> (8 * j)), -range, range) : 0;
+            *reinterpret_cast<uint4*>(lds + at) = make_uint4(res_pack(v), 0, 0, 0);
+            for (int c = 16; c < h.ocp; c += 16) *reinterpret_cast<uint4*>(lds + at + c) = make_uint4(0, 0, 0, 0);
+          }
+        }
+      } else {
+        for (int p = tid; p < h.P; p += RES_THREADS) {
+          const int oy = (int)fastdiv((unsigned)p, h.div_ow), at = h.dst + oy * h.dst_row + (p - oy * h.OW) * h.ocp;
+          for (int c0 = 0; c0 < h.ocp; c0 += 4) {
+            int32_t v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = c0 < C ? res_load<int8_t>(x + (int64_t)(c0 + e < C ? c0 + e : C - 1) * h.P + p) : 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = c0 + e < C ? res_clamp(v[e], -range, range) : 0;
+            *reinterpret_cast<uint32_t*>(lds + at + c0) = res_pack(v);
+          }
         }
       }
     } else if (h.kind == RES_ACT) {
@@ -417,7 +440,7 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] += __shfl_xor(v[e], d, 64);
         res_chain(L->chain, v);
-        if (lane == 0) res_store(h, L, lds, img, 0, h.dst + q * 4, q * 4, v);
+        if (lane == 0) res_store(h, L, lds, call.out_host, img, 0, h.dst + q * 4, q * 4, v);
       }
     } else {
       const int quads = h.ocp >> 2, H = L->H, W = L->W, cp = L->cp, map = L->map, row = L->row;
@@ -437,7 +460,18 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
             for (int e = 0; e < 4; ++e) v[e] = max(v[e], (int32_t)(int8_t)(d >> (8 * e)));
           }
         }
-        res_store(h, L, lds, img, p, h.dst + oy * h.dst_row + ox * h.ocp + c, c, v);
+        res_store(h, L, lds, call.out_host, img, p, h.dst + oy * h.dst_row + ox * h.ocp + c, c, v);
+      }
+    }
+  }
+  if (call.flag_host) {
+    __threadfence_system();
+    __syncthreads();
+    if (tid == 0) {
+      const uint32_t before = __hip_atomic_fetch_add(call.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+      if (before == (uint32_t)images - 1) {
+        *call.counter = 0;
+        __hip_atomic_store(call.flag_host, call.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
   }
@@ -621,14 +655,18 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d)
   return CVMHIP_OK;
 }
 
-int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_t lds_bytes, double ops, double bytes, void* stream) {
+int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_t lds_bytes, const cvmhip_resident_call* call, double ops,
+                           double bytes, void* stream) {
   if (!dev_table || ((uintptr_t)dev_table & 63) || nlayers < 1 || images < 1 || lds_bytes < 16 || lds_bytes > RES_LDS_MOST)
     return arg_error("resident_launch");
+  if (call && (!call->image_host || ((uintptr_t)call->image_host & 3) || !call->out_host || !call->counter || !call->flag_host))
+    return arg_error("resident_launch call");
   char desc[64] = "";
   if (kernel_timing_enabled()) snprintf(desc, sizeof(desc), "%d layers in LDS, %d images", nlayers, images);
   KernelTimer timer("k_conv_resident", ops, as_stream(stream), bytes, desc);
   const int grid = ((images + 7) & ~7) + 8 * RES_HELPERS;
-  k_conv_resident<<<(unsigned)grid, RES_THREADS, lds_bytes, as_stream(stream)>>>(reinterpret_cast<const ResLayer*>(dev_table), nlayers, images);
+  k_conv_resident<<<(unsigned)grid, RES_THREADS, lds_bytes, as_stream(stream)>>>(reinterpret_cast<const ResLayer*>(dev_table), nlayers, images,
+                                                                                call ? *call : cvmhip_resident_call{});
   return check_launch("conv_resident");
 }
 

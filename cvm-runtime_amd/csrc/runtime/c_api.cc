@@ -60,10 +60,7 @@ int CVMAPIInference(void* net, char* input_data, int input_len, char* output_dat
   NOT_NULL(net);
   NOT_NULL(input_data);
   NOT_NULL(output_data);
-  HipModel* model = static_cast<HipModel*>(net);
-  model->SetInput(input_data, input_len);
-  model->Run();
-  model->GetOutput(output_data);
+  static_cast<HipModel*>(net)->Inference(input_data, input_len, output_data);
   API_END();
 }
 

@@ -139,6 +139,8 @@ class HipGraphRuntime {
   void CopyOutputTo(int index, int32_t* host);  // synchronises the stream
   // every output copied into pinned host memory owned by the runtime (valid until the next call); one synchronisation
   const std::vector<const int32_t*>& FetchOutputs();
+  // SetDataI8, Run and FetchOutputs as one call
+  const std::vector<const int32_t*>& InferI8(const int8_t* host, const Shape& shape);
 
   // device-resident variants used to time Run() alone
   int32_t* DataDevicePtr();
@@ -220,8 +222,12 @@ class HipGraphRuntime {
   void* in_stage_host_ = nullptr;  // pinned staging copy of an int8 input
   void* in_stage_dev_ = nullptr;   // its device copy
   bool in_stage_busy_ = false;     // the device may still read in_stage_host_
+  bool in_stage_ahead_ = false;    // in_stage_host_ holds an input that in_stage_dev_ has not seen (InferI8)
   bool data_stays_i8_ = false;     // fused: nothing reads `data` as int32, the row-window packing takes in_stage_dev_
   int32_t data_range_ = 0;         // clamp of the input
+  uint32_t CheckData(const Shape& shape) const;   // the shape `data` must have; its entry
+  void AllocOutputStage();
+  void AwaitTicket();
   void AllocInputStage();
   void* out_stage_host_ = nullptr; // pinned: ticket and status words, then the outputs back to back
   void* out_counter_ = nullptr;    // device word of cvmhip_export_words
@@ -303,6 +309,7 @@ class HipGraphRuntime {
     void* table = nullptr;
     int nlayers = 0, images = 0;
     size_t lds = 0;
+    bool whole_call = false;            // all of the plan, from the int8 input to the model's only output
     bool under_seq = false;             // shares steps with a sequence launch, which runs instead where sequences are in use
     double ops = 0, bytes = 0;
   };

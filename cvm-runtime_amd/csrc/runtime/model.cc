@@ -58,6 +58,17 @@ void HipModel::SetInput(const void* input, int size) {
   }
 }
 
+void HipModel::Inference(const void* input, int size, char* mem) {
+  CVM_VERIFY(GetInputLength() == size);
+  if (input_bytes_ == 4) {
+    SetInput(input, size);
+    Run();
+    GetOutput(mem);
+  } else {
+    SaveTensor(rt_->InferI8(static_cast<const int8_t*>(input), in_shape_), mem);
+  }
+}
+
 void HipModel::GetOutput(char* mem) {
   SaveTensor(rt_->FetchOutputs(), mem);   // all heads in pinned host memory, one synchronisation
 }

@@ -26,6 +26,7 @@ class HipModel {
   std::string GetVersion() const { return version_; }
   std::string GetPostprocessMethod() const { return postprocess_; }
 
+  void Inference(const void* input, int size, char* mem);   // SetInput, Run and GetOutput
   void SetInput(const void* input, int size);  // PlanInput + set_input
   void Run() { rt_->Run(); }
   void GetOutput(char* mem);                   // get_output + SaveTensor

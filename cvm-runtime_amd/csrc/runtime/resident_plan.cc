@@ -369,6 +369,10 @@ void HipGraphRuntime::BuildResident() {
     }
     Check(cvmhip_copy_h2d(base, table.data(), table.size(), stream_), "resident table");
     Check(cvmhip_stream_sync(stream_), "resident table");   // the host copy goes away
+    const ResidentDraft::Layer& tail = d.layers.back();
+    r.whole_call = from == 0 && to + 1 == n && outputs_.size() == 1 && tail.d.out_mode == 2 && tail.d.out == entry_ptr_[entry_id(outputs_[0])];
+    for (size_t l = 0; l < d.layers.size(); ++l)
+      r.whole_call = r.whole_call && d.layers[l].d.kind != 1 && (l == 0) == (d.layers[l].d.kind == 0) && (d.layers[l].d.out_mode == 0 || l + 1 == d.layers.size());
     r.table = base;
     r.owner = buf;
     resident_at_[from] = static_cast<int>(residents_.size());

@@ -474,7 +474,17 @@ size_t cvmhip_resident_filter_bytes(int oc, int c, int kh, int kw);
 int cvmhip_resident_pack_filter(const int32_t* w, void* dst, int oc, int c, int kh, int kw, int dil_h, int dil_w,
                                 int stored_w /* row of the input map in LDS, with its border */, void* stream);
 int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* desc);
-int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_t lds_bytes, double ops, double bytes, void* stream);
+/* A whole call in that launch: the image comes from pinned host memory instead of `in`, the int32 result also goes to
+ * pinned memory, and `ticket` is stored to *flag_host behind it (cvmhip_export_wait; *counter is a zeroed device word). */
+typedef struct cvmhip_resident_call {
+  const void* image_host;
+  int32_t* out_host;
+  uint32_t* counter;
+  uint32_t* flag_host;
+  uint32_t ticket;
+} cvmhip_resident_call;
+int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_t lds_bytes, const cvmhip_resident_call* call /* or NULL */,
+                           double ops, double bytes, void* stream);
 /* depthwise conv2d (groups == channels == out channels) on int8 act tensors, filter packed by
  * cvmhip_pack_depthwise_weights into [kh*kw][cp] int8 */
 size_t cvmhip_packed_depthwise_bytes(int c, int kh, int kw);

@@ -51,6 +51,8 @@ def test_small_maps_stay_in_lds(case, batch, dev, monkeypatch):
     steps = m.launch_counts()[0]
     assert steps <= 3, steps          # the packed image, the launch, and at most what its last layer leaves
     got = [np.frombuffer(m.inference(x.tobytes()), np.int32) for _ in range(3)]
+    m.run()                           # the same input again, in the staged form
+    got.append(np.frombuffer(m.get_output(), np.int32))
     m.close()
     want = og.run_graph(js, graphgen.load_params(pb), x.astype(np.int32))[0].ravel()
     for v in got:
