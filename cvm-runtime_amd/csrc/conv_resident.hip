@@ -3,9 +3,8 @@
 // What bounds such layers when each is a launch is the launch: an empty kernel and its gap are 1.8 us, the chain of
 // prologue, first operands, reduction and drain inside it another 2-3 us, while the arithmetic of a 32 x 32 x 16 layer is a
 // few hundred clocks of one compute unit.  Here the activations of an image never leave the compute unit: a layer boundary
-// is a workgroup barrier, the filters stream from L2 straight into MFMA operands (the first ones of a layer are requested
-// before the barrier in front of it), and the batch spreads over the chip by images.  ResNet-20: 96 us in 23 launches at
-// batch 1, 41.5 us in one; 114 us at batch 64, 42.4 us.
+// is a workgroup barrier, and the batch spreads over the chip by images.  ResNet-20: 96 us in 23 launches at
+// batch 1, 39 us in one; 114 us at batch 64, 39.5 us.
 //
 // Arithmetic: v_mfma_i32_16x16x64_i8 with the filter as the first operand and 16 pixels as the second.  Lane l supplies
 // filter row l & 15 and pixel l & 15, both with the 16 bytes (l >> 4) of the 64 bytes of K, and receives channels
@@ -15,12 +14,15 @@
 // convolutions that read the map: the 16 bytes a lane needs of any tap are one ds_read_b128 at (pixel's place) + (tap's
 // place), and 16 neighbouring pixels of a 16-channel map are 256 contiguous bytes.  K is ordered tap by tap; the places of
 // the four 16-byte groups of every K step are a table behind the filter.
-// What bounds it now (clocks of a 32 x 32 x 16 layer of ResNet-20, 4.2 K in all): 1.5 K of LDS operand reads at 128 bytes a
-// clock, about as much of instructions for places and results (2 wavefronts to a SIMD), the rest from barrier to first
-// product.  What it took to get there, same network at batch 1: all operand reads of a chunk issued before its first product
-// instead of a read and a wait per product, 62 -> 52 us; requests for the first filters inside the loop that uses them, so
-// that they land in its registers, 54 -> 45; plain layers in a loop without the tests for the other forms, 45 -> 41.5.  Three
-// chunks ahead with four pixel tiles, or 1024 threads, run out of registers (79 us with 28 of them spilled).
+// The filter of a layer, its tap offsets, biases and the places of its tiles lie in LDS as well, fetched while the layer in
+// front of it is computed.
+// What bounds it now (ResNet-20, one workgroup, 98 K clocks in all): 46 K of LDS transfers at 128 bytes a clock, 34 K of vector
+// instructions, 14 K of scalar ones and 17 K of products on each SIMD, which hardly overlap: behind a barrier all wavefronts
+// read at the same time and then compute at the same time.  On the way, same network at batch 1: all operand reads of a
+// chunk before its first product instead of a read and a wait each 62 -> 52 us; filters requested inside the loop that uses
+// them 54 -> 45; plain layers without the tests for other forms 45 -> 41.5; filters and places from LDS (no scalar register
+// is spilled any more) and a sum without LDS shuffles 41.5 -> 39.  No difference: 1024 threads, another priority for half of
+// the wavefronts, pixels an odd number of granules apart.
 #include <string.h>
 
 #include "conv_mfma.h"
@@ -31,36 +33,48 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 constexpr int RES_THREADS = 512, RES_WAVES = RES_THREADS / 64;
 constexpr int RES_CHUNK = 3;        // K steps computed together (a 3 x 3 filter over 16, 64, 128, ... channels is whole chunks)
-constexpr int RES_HELPERS = 2;     // workgroups per XCD that only touch the filters
 constexpr int RES_LDS_MOST = 150 * 1024;
 
 enum { RES_IMAGE = 0, RES_ACT = 1, RES_CONV = 2, RES_SUM = 3, RES_POOL = 4 };
 // flags: a chain that is not one clamp and shift; channels past OC exist; the result goes to memory; its map has a border;
-// the pixels of every group of tiles exist and lie like the first group's
-enum { RES_CHAIN = 1, RES_CHAIN2 = 2, RES_MASK = 4, RES_OUT = 8, RES_BORDER = 16, RES_REGULAR = 32 };
+// none of these, and the pixels of every item exist: the places are in LDS (res_plain)
+enum { RES_CHAIN = 1, RES_CHAIN2 = 2, RES_MASK = 4, RES_OUT = 8, RES_BORDER = 16, RES_PLAIN = 32 };
 
 // What the common path of a layer needs, in scalar registers from the layer's first instruction on: read field by field
 // where it is used, every field was a trip through the scalar cache in a chain of them.
 struct ResHead {
-  int kind, tp, items, octiles, chunks, P, OW, flags;
-  FastDiv div_ow, div_oct;
-  int src, step_y, step_x;          // window of output pixel (0, 0), and bytes to the next row's and column's window
-  int dst, dst_row, ocp;            // output pixel (0, 0), bytes of a stored row (dst: -1 = not kept in LDS)
-  int res, res_row;                 // residual likewise (res: -1 = none)
+  int kind, tp, items, chunks;
+  int flags, w_at, taps_at, bias_at;   // in LDS: fragments [octile][chunk][step][64 lanes][16 bytes], byte offsets in the
+                                       // window of the groups [chunk][step][4], biases [octile][16]
+  int places_at, residual;             // RES_PLAIN: the lanes' ResPlace, then an ResItem for every item
   int lo, hi, shift, lo2, hi2, shift2;
-  const int8_t* filter;             // [octile][chunk][step][64 lanes][16 bytes]
-  const int* taps;                  // [chunk][step][4]: byte offset of the group in the window
-  const int32_t* bias;              // octiles * 16 values
-  // RES_REGULAR: bytes from a group's first tile to its tile j, in the input, the result and the residual
-  int src_off[4], dst_off[4], res_off[4], unused[4];
+  // border of the output map: start, bytes of a stored row, of the gap between two rows, in front of the first pixel; rows
+  int border_at, border_row, border_side, border_edge, border_rows;
+  // filter of the next convolution, to be fetched during this layer: KiB, where to, where from
+  int next_kb, next_at, unused;
+  const int8_t* next;
+  int unused2[6];
+};
+// Byte offsets of a lane's pixel of a tile, in LDS, without what the tile adds: first tap of the window, result, residual; and
+// the lane's bytes of a channel tile's biases.
+struct ResPlace {
+  int src, dst, res, bias;
+};
+// What the tiles of an item add to them, and the LDS byte of its filter and of its biases.
+struct ResItem {
+  int src[4], dst[4], res[4];
+  int filter, bias, unused[2];
 };
 struct __attribute__((aligned(64))) ResLayer {
   ResHead h;
+  int octiles, P, OW;
+  FastDiv div_ow, div_oct, div_w;
+  int src, step_y, step_x;          // window of output pixel (0, 0), and bytes to the next row's and column's window
+  int dst, dst_row, ocp;            // output pixel (0, 0), bytes of a stored row (dst: -1 = not kept in LDS)
+  int res, res_row;                 // residual likewise (res: -1 = none)
   int C, H, W, cp, map, row;        // IMAGE, ACT: the map; SUM, POOL: the input (map: pixel (0, 0), row: bytes of a stored row)
   int KH, KW, SH, SW, PH, PW, range;
   int OC, out_mode, gcp;            // out_mode: 0 LDS only, 1 int8 act tensor of gcp channels, 2 int32 (image, channel, pixel)
-  // border of the output map: start, bytes of a stored row, of the gap between two rows, in front of the first pixel; rows
-  int border_at, border_row, border_side, border_edge, border_rows;
   const int8_t* in;                 // IMAGE: int8 NCHW, ACT: act tensor of gcp channels
   void* out;
   DevChain chain, chain2;
@@ -75,6 +89,18 @@ template <typename T>
 __device__ __forceinline__ T res_load(const void* p) { return *(const RES_GLOBAL T*)p; }
 template <typename T>
 __device__ __forceinline__ void res_write(void* p, T v) { *(RES_GLOBAL T*)p = v; }
+
+// sum over the wavefront, in lane 63: 1, 2, 4 and 8 lanes to the right inside rows of 16, then the rows' last lanes onward
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int32_t res_add_from(int32_t v) { return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false); }
+__device__ __forceinline__ int32_t res_wave_sum(int32_t v) {
+  v = res_add_from<0x111, 0xf>(v);
+  v = res_add_from<0x112, 0xf>(v);
+  v = res_add_from<0x114, 0xf>(v);
+  v = res_add_from<0x118, 0xf>(v);
+  v = res_add_from<0x142, 0xa>(v);
+  return res_add_from<0x143, 0xc>(v);
+}
 
 // (lo <= hi)
 __device__ __forceinline__ int res_clamp(int v, int lo, int hi) {
@@ -100,111 +126,81 @@ __device__ __forceinline__ uint32_t res_pack(const int32_t (&v)[4]) {
   return __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
 }
 
+// where the pixels of a layer lie, for the forms that are not RES_PLAIN
+struct ResGeometry {
+  int P, OW;
+  FastDiv div_ow;
+  int src, step_y, step_x, dst, dst_row, ocp, res, res_row;
+};
+__device__ __forceinline__ ResGeometry res_geometry(ResTable L) {
+  return ResGeometry{L->P, L->OW, FastDiv{L->div_ow.m, L->div_ow.l}, L->src, L->step_y, L->step_x, L->dst, L->dst_row, L->ocp, L->res, L->res_row};
+}
+
 // four channels of pixel p of this image, to LDS byte `at` and wherever else the layer wants them
-__device__ __forceinline__ void res_store(const ResHead& h, ResTable L, char* lds, int32_t* out_host, int img, int p, int at, int oc,
+__device__ __forceinline__ void res_store(const ResHead& h, const ResGeometry& q, ResTable L, char* lds, int32_t* out_host, int img, int p, int at, int oc,
                                           const int32_t (&v)[4]) {
   uint32_t d = res_pack(v);
   if (h.flags & RES_MASK) {
     const int left = L->OC - oc;
     d = left >= 4 ? d : left <= 0 ? 0u : d & ((1u << (8 * left)) - 1u);
   }
-  if (h.dst >= 0) *reinterpret_cast<uint32_t*>(lds + at) = d;
+  if (q.dst >= 0) *reinterpret_cast<uint32_t*>(lds + at) = d;
   if (h.flags & RES_OUT) {
     if (L->out_mode == 1) {
       const int gcp = L->gcp;
-      if (oc < gcp) res_write(reinterpret_cast<int8_t*>(L->out) + act_offset((int64_t)img * h.P + p, oc, gcp), d);
+      if (oc < gcp) res_write(reinterpret_cast<int8_t*>(L->out) + act_offset((int64_t)img * q.P + p, oc, gcp), d);
     } else {
       const int OC = L->OC;
-      const int64_t first = ((int64_t)img * OC + oc) * h.P + p;
+      const int64_t first = ((int64_t)img * OC + oc) * q.P + p;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (oc + e < OC) {
-          res_write(reinterpret_cast<int32_t*>(L->out) + first + (int64_t)e * h.P, v[e]);
-          if (out_host) res_write(out_host + first + (int64_t)e * h.P, v[e]);
+          res_write(reinterpret_cast<int32_t*>(L->out) + first + (int64_t)e * q.P, v[e]);
+          if (out_host) res_write(out_host + first + (int64_t)e * q.P, v[e]);
         }
     }
   }
 }
 
-// filter fragments and tap offsets of a chunk
-struct ResChunk {
-  v4i a[RES_CHUNK];
-  int tap[RES_CHUNK];
-};
-// the chunks an item keeps in flight, and its bias
-template <int AHEAD>
-struct ResRing {
-  ResChunk c[AHEAD];
-  v4i bias;
-};
-
-// (addresses: a uniform base and the lane's own 32-bit offset)
-__device__ __forceinline__ void res_fetch(const ResHead& h, ResChunk& c, int ot, int chunk, int lane) {
-  const int8_t* f = h.filter + (unsigned)(ot * h.chunks + chunk) * (RES_CHUNK * 1024u);
-  const int8_t* t = reinterpret_cast<const int8_t*>(h.taps) + (unsigned)chunk * (RES_CHUNK * 16u);
+// A chunk of one item: all operand reads, then the products.  `w`: the lane's bytes of the chunk's first fragment.
+template <int TP>
+__device__ __forceinline__ void res_chunk(const char* lds, const char* w, const int (&tap)[RES_CHUNK], const int (&base)[TP], v4i (&acc)[TP]) {
+  v4i a[RES_CHUNK], x[RES_CHUNK][TP];
 #pragma unroll
   for (int u = 0; u < RES_CHUNK; ++u) {
-    c.a[u] = res_load<v4i>(f + (unsigned)lane * 16u + u * 1024);
-    c.tap[u] = res_load<int>(t + (unsigned)(lane >> 4) * 4u + u * 16);
+    a[u] = *reinterpret_cast<const v4i*>(w + u * 1024);
+#pragma unroll
+    for (int j = 0; j < TP; ++j) x[u][j] = *reinterpret_cast<const v4i*>(lds + (base[j] + tap[u]));
   }
-}
-
-template <int AHEAD>
-__device__ __forceinline__ void res_request(const ResHead& h, ResRing<AHEAD>& r, int ot, int lane) {
-#pragma unroll
-  for (int c = 0; c < AHEAD; ++c)
-    if (c < h.chunks) res_fetch(h, r.c[c], ot, c, lane);
-  r.bias = res_load<v4i>(reinterpret_cast<const int8_t*>(h.bias) + (unsigned)ot * 64u + (unsigned)(lane >> 4) * 16u);
-}
-
-// all operand reads before the first product
-template <int TP>
-__device__ __forceinline__ void res_chunk(const char* lds, const ResChunk& c, const int (&base)[TP], v4i (&acc)[TP]) {
-  v4i x[RES_CHUNK][TP];
-#pragma unroll
-  for (int u = 0; u < RES_CHUNK; ++u)
-#pragma unroll
-    for (int j = 0; j < TP; ++j) x[u][j] = *reinterpret_cast<const v4i*>(lds + (base[j] + c.tap[u]));
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int u = 0; u < RES_CHUNK; ++u)
 #pragma unroll
-    for (int j = 0; j < TP; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.a[u], x[u][j], acc[j], 0, 0, 0);
+    for (int j = 0; j < TP; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u], x[u][j], acc[j], 0, 0, 0);
 }
 
-// Byte offsets of lane (l & 15)'s pixel in the input window, the result and the residual.
-struct ResPlace {
-  int src, dst, res;
-};
 // pixel p; the channel of the lane's group inside a tile is added where the tile is written
-__device__ __forceinline__ ResPlace res_place(const ResHead& h, int p, int lane) {
-  const int y = (int)fastdiv((unsigned)p, h.div_ow), x = p - y * h.OW;
-  const int column = __mul24(x, h.ocp) + (lane >> 4) * 4;
-  ResPlace q;
-  q.src = h.src + __mul24(y, h.step_y) + __mul24(x, h.step_x);
-  q.dst = h.dst + __mul24(y, h.dst_row) + column;
-  q.res = h.res + __mul24(y, h.res_row) + column;
-  return q;
+__host__ __device__ inline ResPlace res_place(const ResGeometry& g, int p, int y, int lane) {
+  const int x = p - y * g.OW, column = x * g.ocp + (lane >> 4) * 4;
+  return ResPlace{g.src + y * g.step_y + x * g.step_x, g.dst + y * g.dst_row + column, g.res + y * g.res_row + column, (lane >> 4) * 16};
 }
 
-__device__ __forceinline__ void res_requant(const ResHead& h, const char* lds, int res, int32_t (&v)[4]) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = res_clamp(v[e], h.lo, h.hi) >> h.shift;
-  if (h.res >= 0) {
-    const uint32_t d = *reinterpret_cast<const uint32_t*>(lds + res);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = res_clamp(wadd(v[e], (int32_t)(int8_t)(d >> (8 * e))), h.lo2, h.hi2) >> h.shift2;
+// The end of a layer: its results and the next layer's filter are in LDS.  (The fetches of the filter are not known to the
+// compiler, which could not tell them from the operands it waits for.)
+__device__ __forceinline__ void res_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+__device__ __forceinline__ void res_fetch_next(const ResHead& h, uint32_t lds_base, int wave, int lane) {
+  for (int k = wave; k < h.next_kb; k += RES_WAVES) {
+    const int8_t* from = h.next + (unsigned)k * 1024u + (unsigned)lane * 16u;
+    // (the s_nop is the wait state between a scalar write to M0 and its use)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_base + (uint32_t)(h.next_at + k * 1024)) : "memory");
   }
 }
 
-// A barrier that orders LDS only: requests to memory stay in flight across it (what a layer stores to memory is not read
-// inside the launch).
-__device__ __forceinline__ void res_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-__device__ __forceinline__ void res_border(const ResHead& h, ResTable L, char* lds, int tid) {
+__device__ __forceinline__ void res_border(const ResHead& h, char* lds, int tid) {
   if (h.flags & RES_BORDER) {
     // the border is three runs: in front of the first pixel, behind the last one, and between the rows
-    const int row = L->border_row, side = L->border_side, edge = L->border_edge, rows = L->border_rows, at = L->border_at;
+    const int row = h.border_row, side = h.border_side, edge = h.border_edge, rows = h.border_rows, at = h.border_at;
     const uint4 zero = make_uint4(0, 0, 0, 0);
     for (int i = tid * 16; i < edge; i += RES_THREADS * 16) {
       *reinterpret_cast<uint4*>(lds + at + i) = zero;
@@ -215,122 +211,122 @@ __device__ __forceinline__ void res_border(const ResHead& h, ResTable L, char* l
   }
 }
 
-// The first item's operands are requested before the barrier in front of the layer.
-// The kernel is bound by instructions (a 16-channel layer has three products per 16 results of a lane group), so the
-// regular case keeps everything that does not differ between lanes in scalar registers and knows its tiles' distances.
-template <int TP, bool PLAIN>
-__device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds, int32_t* out_host, int img, int wave, int lane) {
-  constexpr int AHEAD = TP == 4 ? 2 : 3;   // (four pixel tiles leave registers for two chunks)
-  ResRing<AHEAD> r;
-  int item = wave, group = (int)fastdiv((unsigned)wave, h.div_oct), ot = wave - group * h.octiles;
-  if (item < h.items) res_request(h, r, ot, lane);
-  res_barrier();
-  res_border(h, L, lds, wave * 64 + lane);
-  if (item >= h.items) return;
-  const ResPlace own = res_place(h, lane & 15, lane);
-  const bool regular = PLAIN || (h.flags & RES_REGULAR);
-  for (;;) {
-    const int p0 = group * (TP * 16), y0 = (int)fastdiv((unsigned)p0, h.div_ow), x0 = p0 - y0 * h.OW;
-    int base[TP];
-    if (regular) {
-      const int s0 = y0 * h.step_y + x0 * h.step_x;
+template <int TP>
+__device__ __forceinline__ void res_products(const ResHead& h, const char* lds, const char* w, int lane, int (&tap)[RES_CHUNK],
+                                             const int (&base)[TP], v4i (&acc)[TP]) {
+  const char* taps = lds + (h.taps_at + (lane >> 4) * 4);
+  for (int c = 0; c < h.chunks; ++c) {
+    int now[RES_CHUNK];
+    const char* after = c + 1 == h.chunks ? taps : taps + (c + 1) * (RES_CHUNK * 16);   // (the next item starts over)
 #pragma unroll
-      for (int j = 0; j < TP; ++j) base[j] = own.src + (s0 + h.src_off[j]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < TP; ++j) {
-        const int p = p0 + j * 16 + (lane & 15);
-        base[j] = res_place(h, p < h.P ? p : 0, lane).src;   // pixels past the map are computed and dropped
-      }
+    for (int u = 0; u < RES_CHUNK; ++u) {
+      now[u] = tap[u];
+      tap[u] = *reinterpret_cast<const int*>(after + u * 16);
     }
-    const int oc = ot * 16;
+    res_chunk<TP>(lds, w + c * (RES_CHUNK * 1024), now, base, acc);
+  }
+}
+__device__ __forceinline__ void res_first_taps(const ResHead& h, const char* lds, int lane, int (&tap)[RES_CHUNK]) {
+#pragma unroll
+  for (int u = 0; u < RES_CHUNK; ++u) tap[u] = *reinterpret_cast<const int*>(lds + (h.taps_at + (lane >> 4) * 4 + u * 16));
+}
+
+// A convolution with nothing out of the ordinary.  The kernel is bound by instructions (a SIMD issues one in 4 clocks, a
+// 16-channel layer has three products per 16 results of a lane group): what differs between the lanes and between the
+// items comes from tables that were fetched with the filter, and a layer's own constants fit in scalar registers.
+template <int TP>
+__device__ __forceinline__ void res_plain_conv(const ResHead& h, char* lds, int wave, int lane) {
+  if (wave >= h.items) return;
+  const ResPlace own = *reinterpret_cast<const ResPlace*>(lds + (h.places_at + lane * 16));
+  const char* rec = lds + (h.places_at + 1024 + wave * 64);
+  int tap[RES_CHUNK];
+  res_first_taps(h, lds, lane, tap);
+  for (int item = wave;;) {
+    const v4i src = *reinterpret_cast<const v4i*>(rec), dst = *reinterpret_cast<const v4i*>(rec + 16);
+    const int filter = *reinterpret_cast<const int*>(rec + 48), bias_at = *reinterpret_cast<const int*>(rec + 52);
     uint32_t residual[TP];
-    if (PLAIN && h.res >= 0) {
-      const int r0 = y0 * h.res_row + x0 * h.ocp + oc;
+    if (h.residual) {
+      const v4i res = *reinterpret_cast<const v4i*>(rec + 32);
 #pragma unroll
-      for (int j = 0; j < TP; ++j) residual[j] = *reinterpret_cast<const uint32_t*>(lds + (own.res + (r0 + h.res_off[j])));
+      for (int j = 0; j < TP; ++j) residual[j] = *reinterpret_cast<const uint32_t*>(lds + (own.res + res[j]));
     }
+    int base[TP];
     v4i acc[TP];
+    const v4i bias = *reinterpret_cast<const v4i*>(lds + (bias_at + own.bias));
 #pragma unroll
-    for (int j = 0; j < TP; ++j) acc[j] = r.bias;
-    if (h.chunks <= AHEAD) {
-      res_chunk<TP>(lds, r.c[0], base, acc);
-      if (h.chunks > 1) res_chunk<TP>(lds, r.c[1], base, acc);
-      if (AHEAD > 2 && h.chunks > 2) res_chunk<TP>(lds, r.c[2], base, acc);
-    } else {
-      // a chunk's registers are requested again, for the chunk AHEAD further on, once it is used
-      const int last = h.chunks - 1;
-      for (int c = 0;; c += AHEAD) {
-        res_chunk<TP>(lds, r.c[0], base, acc);
-        if (c == last) break;
-        res_fetch(h, r.c[0], ot, min(c + AHEAD, last), lane);
-        res_chunk<TP>(lds, r.c[1], base, acc);
-        if (c + 1 == last) break;
-        res_fetch(h, r.c[1], ot, min(c + AHEAD + 1, last), lane);
-        if constexpr (AHEAD > 2) {
-          res_chunk<TP>(lds, r.c[2], base, acc);
-          if (c + 2 == last) break;
-          res_fetch(h, r.c[2], ot, min(c + AHEAD + 2, last), lane);
-        }
-      }
+    for (int j = 0; j < TP; ++j) {
+      base[j] = own.src + src[j];
+      acc[j] = bias;
     }
-    if constexpr (PLAIN) {
-      const int d0 = y0 * h.dst_row + x0 * h.ocp + oc;
-      if (h.res >= 0) {
-#pragma unroll
-        for (int j = 0; j < TP; ++j) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            acc[j][e] = res_clamp(wadd(res_clamp(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2) >> h.shift2;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < TP; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[j][e] = res_clamp(acc[j][e], h.lo, h.hi) >> h.shift;
-      }
+    res_products<TP>(h, lds, lds + (filter + lane * 16), lane, tap, base, acc);
+    if (h.residual) {
 #pragma unroll
       for (int j = 0; j < TP; ++j) {
-        const int32_t v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
-        *reinterpret_cast<uint32_t*>(lds + (own.dst + (d0 + h.dst_off[j]))) = res_pack(v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[j][e] = res_clamp(wadd(res_clamp(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2) >> h.shift2;
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < TP; ++j) {
-        const int p = p0 + j * 16 + (lane & 15);
-        if (p < h.P) {
-          const ResPlace q = res_place(h, p, lane);
-          int32_t v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
-          if (h.flags & (RES_CHAIN | RES_CHAIN2)) {
-            res_chain(L->chain, v);
-            if (h.res >= 0) {
-              const uint32_t d = *reinterpret_cast<const uint32_t*>(lds + (q.res + oc));
+      for (int j = 0; j < TP; ++j)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) v[e] = wadd(v[e], (int32_t)(int8_t)(d >> (8 * e)));
-              res_chain(L->chain2, v);
-            }
-          } else {
-            res_requant(h, lds, q.res + oc, v);
-          }
-          res_store(h, L, lds, out_host, img, p, q.dst + oc, oc + (lane >> 4) * 4, v);
-        }
-      }
+        for (int e = 0; e < 4; ++e) acc[j][e] = res_clamp(acc[j][e], h.lo, h.hi) >> h.shift;
+    }
+#pragma unroll
+    for (int j = 0; j < TP; ++j) {
+      const int32_t v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
+      *reinterpret_cast<uint32_t*>(lds + (own.dst + dst[j])) = res_pack(v);
     }
     item += RES_WAVES;
     if (item >= h.items) return;
-    const int before = ot;
-    group = (int)fastdiv((unsigned)item, h.div_oct);
-    ot = item - group * h.octiles;
-    if (ot != before || h.chunks > AHEAD) res_request(h, r, ot, lane);   // (else the ring still holds the whole filter)
+    rec += RES_WAVES * 64;
+  }
+}
+
+// any convolution, one pixel tile at a time
+__device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds, int32_t* out_host, int img, int wave, int lane) {
+  const ResGeometry g = res_geometry(L);
+  const FastDiv div_oct{L->div_oct.m, L->div_oct.l};
+  const int octiles = L->octiles;
+  int tap[RES_CHUNK];
+  res_first_taps(h, lds, lane, tap);
+  for (int item = wave; item < h.items; item += RES_WAVES) {
+    const int group = (int)fastdiv((unsigned)item, div_oct), ot = item - group * octiles, oc = ot * 16;
+    const int pixel = group * 16 + (lane & 15), p = pixel < g.P ? pixel : 0;   // pixels past the map are computed and dropped
+    const ResPlace q = res_place(g, p, (int)fastdiv((unsigned)p, g.div_ow), lane);
+    const int base[1] = {q.src};
+    v4i acc[1] = {*reinterpret_cast<const v4i*>(lds + (h.bias_at + ot * 64 + q.bias))};
+    res_products<1>(h, lds, lds + (h.w_at + ot * h.chunks * (RES_CHUNK * 1024) + lane * 16), lane, tap, base, acc);
+    if (pixel >= g.P) continue;
+    int32_t v[4] = {acc[0][0], acc[0][1], acc[0][2], acc[0][3]};
+    const bool chains = h.flags & (RES_CHAIN | RES_CHAIN2);
+    if (chains) {
+      res_chain(L->chain, v);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = res_clamp(v[e], h.lo, h.hi) >> h.shift;
+    }
+    if (h.residual) {
+      const uint32_t d = *reinterpret_cast<const uint32_t*>(lds + (q.res + oc));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = wadd(v[e], (int32_t)(int8_t)(d >> (8 * e)));
+      if (chains) {
+        res_chain(L->chain2, v);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = res_clamp(v[e], h.lo2, h.hi2) >> h.shift2;
+      }
+    }
+    res_store(h, g, L, lds, out_host, img, pixel, q.dst + oc, oc + (lane >> 4) * 4, v);
   }
 }
 
 __device__ __forceinline__ ResHead res_head(ResTable L) {
   ResHead h;
   typedef int v16i __attribute__((ext_vector_type(16)));
-  static_assert(sizeof(ResHead) == 192, "three lines of the scalar cache");
+  static_assert(sizeof(ResHead) == 128, "two lines of the scalar cache");
   const __attribute__((address_space(4))) v16i* w = (const __attribute__((address_space(4))) v16i*)L;
-  const v16i part[3] = {w[0], w[1], w[2]};
+  const v16i part[2] = {w[0], w[1]};
   __builtin_memcpy(&h, part, sizeof(h));
   return h;
 }
@@ -341,22 +337,7 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
   const int img = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   ResTable L = (ResTable)table;
-  if (img >= images) {
-    // Workgroups behind the images: they bring the filters into the L2 of their XCD (workgroups go to the eight XCDs in
-    // turn), which the images' workgroups would otherwise wait for layer by layer: every launch starts with an L2 that has
-    // to ask memory again, 0.8 us away.
-    const int part = (img - ((images + 7) & ~7)) >> 3, parts = ((int)gridDim.x - ((images + 7) & ~7)) >> 3;
-    if (img < ((images + 7) & ~7) || (img & 7) >= images) return;
-    for (int l = 0; l < nlayers; ++l, ++L) {
-      if (L->h.kind != RES_CONV) continue;
-      const int8_t* f = L->h.filter;
-      const int bytes = L->h.octiles * L->h.chunks * (RES_CHUNK * 1024) + L->h.chunks * (RES_CHUNK * 16);
-      int sum = 0;
-      for (int at = (part * RES_THREADS + tid) * 128; at < bytes; at += parts * RES_THREADS * 128) sum += res_load<int>(f + at);
-      asm volatile("" ::"v"(sum));
-    }
-    return;
-  }
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   // The table comes through the scalar cache, which is cold: every wavefront requests an eighth of its lines now, so that a
   // layer does not begin with dependent misses.
   {
@@ -368,47 +349,46 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
   }
   for (int l = 0; l < nlayers; ++l, ++L) {
     const ResHead h = res_head(L);
-    if (h.kind == RES_CONV) {
-      const bool plain = (h.flags & (RES_CHAIN | RES_CHAIN2 | RES_MASK | RES_OUT | RES_REGULAR)) == RES_REGULAR;
-      if (plain) {
-        if (h.tp == 1) res_conv<1, true>(h, L, lds, call.out_host, img, wave, lane);
-        else if (h.tp == 2) res_conv<2, true>(h, L, lds, call.out_host, img, wave, lane);
-        else res_conv<4, true>(h, L, lds, call.out_host, img, wave, lane);
-      } else {
-        if (h.tp == 1) res_conv<1, false>(h, L, lds, call.out_host, img, wave, lane);
-        else if (h.tp == 2) res_conv<2, false>(h, L, lds, call.out_host, img, wave, lane);
-        else res_conv<4, false>(h, L, lds, call.out_host, img, wave, lane);
-      }
+    res_barrier();
+    res_fetch_next(h, lds_base, wave, lane);
+    res_border(h, lds, tid);
+    if (h.flags & RES_PLAIN) {
+      if (h.tp == 1) res_plain_conv<1>(h, lds, wave, lane);
+      else if (h.tp == 2) res_plain_conv<2>(h, lds, wave, lane);
+      else res_plain_conv<4>(h, lds, wave, lane);
       continue;
     }
-    res_barrier();
-    res_border(h, L, lds, tid);
+    if (h.kind == RES_CONV) {
+      res_conv(h, L, lds, call.out_host, img, wave, lane);
+      continue;
+    }
+    const ResGeometry g = res_geometry(L);
     if (h.kind == RES_IMAGE) {
       const int C = L->C, range = L->range;
-      const int8_t* x = (call.image_host ? reinterpret_cast<const int8_t*>(call.image_host) : L->in) + (int64_t)img * C * h.P;
-      if (C <= 4 && (h.P & 3) == 0) {
+      const int8_t* x = (call.image_host ? reinterpret_cast<const int8_t*>(call.image_host) : L->in) + (int64_t)img * C * g.P;
+      if (C <= 4 && (g.P & 3) == 0) {
         // four pixels to a thread: all of an image's bytes are requested at once (host memory is 1.5 us away)
-        for (int p = tid * 4; p < h.P; p += RES_THREADS * 4) {
+        for (int p = tid * 4; p < g.P; p += RES_THREADS * 4) {
           uint32_t d[4];
 #pragma unroll
-          for (int c = 0; c < 4; ++c) d[c] = res_load<uint32_t>(x + (c < C ? c : C - 1) * h.P + p);
+          for (int c = 0; c < 4; ++c) d[c] = res_load<uint32_t>(x + (c < C ? c : C - 1) * g.P + p);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const int oy = (int)fastdiv((unsigned)(p + j), h.div_ow), at = h.dst + oy * h.dst_row + (p + j - oy * h.OW) * h.ocp;
+            const int oy = (int)fastdiv((unsigned)(p + j), g.div_ow), at = g.dst + oy * g.dst_row + (p + j - oy * g.OW) * g.ocp;
             int32_t v[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) v[c] = c < C ? res_clamp((int32_t)(int8_t)(d[c] >> (8 * j)), -range, range) : 0;
             *reinterpret_cast<uint4*>(lds + at) = make_uint4(res_pack(v), 0, 0, 0);
-            for (int c = 16; c < h.ocp; c += 16) *reinterpret_cast<uint4*>(lds + at + c) = make_uint4(0, 0, 0, 0);
+            for (int c = 16; c < g.ocp; c += 16) *reinterpret_cast<uint4*>(lds + at + c) = make_uint4(0, 0, 0, 0);
           }
         }
       } else {
-        for (int p = tid; p < h.P; p += RES_THREADS) {
-          const int oy = (int)fastdiv((unsigned)p, h.div_ow), at = h.dst + oy * h.dst_row + (p - oy * h.OW) * h.ocp;
-          for (int c0 = 0; c0 < h.ocp; c0 += 4) {
+        for (int p = tid; p < g.P; p += RES_THREADS) {
+          const int oy = (int)fastdiv((unsigned)p, g.div_ow), at = g.dst + oy * g.dst_row + (p - oy * g.OW) * g.ocp;
+          for (int c0 = 0; c0 < g.ocp; c0 += 4) {
             int32_t v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = c0 < C ? res_load<int8_t>(x + (int64_t)(c0 + e < C ? c0 + e : C - 1) * h.P + p) : 0;
+            for (int e = 0; e < 4; ++e) v[e] = c0 < C ? res_load<int8_t>(x + (int64_t)(c0 + e < C ? c0 + e : C - 1) * g.P + p) : 0;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = c0 + e < C ? res_clamp(v[e], -range, range) : 0;
             *reinterpret_cast<uint32_t*>(lds + at + c0) = res_pack(v);
@@ -417,37 +397,37 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
       }
     } else if (h.kind == RES_ACT) {
       // granules of 4 bytes: the tensor in memory may have 4 or 8 channels to a pixel
-      const int quads = h.ocp >> 2, gcp = L->gcp;
+      const int quads = g.ocp >> 2, gcp = L->gcp;
       const int8_t* x = L->in;
-      for (int i = tid; i < h.P * quads; i += RES_THREADS) {
+      for (int i = tid; i < g.P * quads; i += RES_THREADS) {
         const int p = i / quads, c = (i - p * quads) * 4;
-        const int oy = (int)fastdiv((unsigned)p, h.div_ow);
+        const int oy = (int)fastdiv((unsigned)p, g.div_ow);
         uint32_t d = 0;
-        if (c < gcp) d = res_load<uint32_t>(x + act_offset((int64_t)img * h.P + p, c, gcp));
-        *reinterpret_cast<uint32_t*>(lds + h.dst + oy * h.dst_row + (p - oy * h.OW) * h.ocp + c) = d;
+        if (c < gcp) d = res_load<uint32_t>(x + act_offset((int64_t)img * g.P + p, c, gcp));
+        *reinterpret_cast<uint32_t*>(lds + g.dst + oy * g.dst_row + (p - oy * g.OW) * g.ocp + c) = d;
       }
     } else if (h.kind == RES_SUM) {
       const int H = L->H, W = L->W, cp = L->cp, map = L->map, row = L->row;
+      const FastDiv div_w{L->div_w.m, L->div_w.l};
       for (int q = wave; q < (cp >> 2); q += RES_WAVES) {
         int32_t v[4] = {0, 0, 0, 0};
         for (int p = lane; p < H * W; p += 64) {
-          const int y = p / W;
+          const int y = (int)fastdiv((unsigned)p, div_w);
           const uint32_t d = *reinterpret_cast<const uint32_t*>(lds + map + y * row + (p - y * W) * cp + q * 4);
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] += (int32_t)(int8_t)(d >> (8 * e));
         }
-        for (int d = 32; d >= 1; d >>= 1)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += __shfl_xor(v[e], d, 64);
+        for (int e = 0; e < 4; ++e) v[e] = res_wave_sum(v[e]);
         res_chain(L->chain, v);
-        if (lane == 0) res_store(h, L, lds, call.out_host, img, 0, h.dst + q * 4, q * 4, v);
+        if (lane == 63) res_store(h, g, L, lds, call.out_host, img, 0, g.dst + q * 4, q * 4, v);
       }
     } else {
-      const int quads = h.ocp >> 2, H = L->H, W = L->W, cp = L->cp, map = L->map, row = L->row;
+      const int quads = g.ocp >> 2, H = L->H, W = L->W, cp = L->cp, map = L->map, row = L->row;
       const int KH = L->KH, KW = L->KW, SH = L->SH, SW = L->SW, PH = L->PH, PW = L->PW;
-      for (int i = tid; i < h.P * quads; i += RES_THREADS) {
+      for (int i = tid; i < g.P * quads; i += RES_THREADS) {
         const int p = i / quads, c = (i - p * quads) * 4;
-        const int oy = (int)fastdiv((unsigned)p, h.div_ow), ox = p - oy * h.OW;
+        const int oy = (int)fastdiv((unsigned)p, g.div_ow), ox = p - oy * g.OW;
         int32_t v[4] = {-128, -128, -128, -128};
         for (int r = 0; r < KH; ++r) {
           const int y = oy * SH - PH + r;
@@ -460,7 +440,7 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
             for (int e = 0; e < 4; ++e) v[e] = max(v[e], (int32_t)(int8_t)(d >> (8 * e)));
           }
         }
-        res_store(h, L, lds, call.out_host, img, p, h.dst + oy * h.dst_row + ox * h.ocp + c, c, v);
+        res_store(h, g, L, lds, call.out_host, img, p, g.dst + oy * g.dst_row + ox * g.ocp + c, c, v);
       }
     }
   }
@@ -477,8 +457,9 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
   }
 }
 
-// int32 OIHW -> fragments (a dword per thread), then the tap table for a map stored with `row` bytes to a row
-__global__ void __launch_bounds__(256) k_pack_resident(const int32_t* __restrict__ w, uint32_t* __restrict__ wp, int64_t dwords, int oc,
+// int32 OIHW -> fragments (a dword per thread), then the tap table for a map stored with `row` bytes to a row, then the bias
+__global__ void __launch_bounds__(256) k_pack_resident(const int32_t* __restrict__ w, const int32_t* __restrict__ bias, uint32_t* __restrict__ wp,
+                                                       int64_t dwords, int octiles, int oc,
                                                        int ic, int kh, int kw, int cp, int ksteps, int row, int dh, int dw) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int taps = kh * kw;
@@ -498,6 +479,9 @@ __global__ void __launch_bounds__(256) k_pack_resident(const int32_t* __restrict
     const int e = (int)(i - dwords), k = e * 16, tap = k / cp, c = k - tap * cp;
     // past the last tap the filter is zero: the window's first bytes will do
     wp[i] = tap < taps ? (uint32_t)((tap / kw) * dh * row + (tap % kw) * dw * cp + c) : 0u;
+  } else if (i < dwords + ksteps * 4 + octiles * 16) {
+    const int o = (int)(i - dwords - ksteps * 4);
+    wp[i] = bias && o < oc ? (uint32_t)bias[o] : 0u;
   }
 }
 
@@ -531,24 +515,34 @@ size_t cvmhip_resident_tensor_bytes(int c, int h, int w, int border_y, int borde
   return (size_t)res_cp(c) * (h + 2 * border_y) * (w + 2 * border_x);
 }
 
-size_t cvmhip_resident_filter_bytes(int oc, int c, int kh, int kw) {
-  if (oc < 1 || c < 1 || kh < 1 || kw < 1) return 0;
-  return ((size_t)(res_cp(oc) / 16) * 1024 + 16) * res_chunks(c, kh, kw) * RES_CHUNK;
+// as many pixel tiles per item (a filter fragment read once serves them all) as still leave every wavefront an item
+static int res_tiles(int ptiles, int octiles) { return ptiles * octiles >= 4 * RES_WAVES ? 4 : ptiles * octiles >= 2 * RES_WAVES ? 2 : 1; }
+static size_t res_places_at(int oc, int c, int kh, int kw) {
+  return ((size_t)(res_cp(oc) / 16) * 1024 + 16) * res_chunks(c, kh, kw) * RES_CHUNK + (size_t)res_cp(oc) * 4;
 }
 
-int cvmhip_resident_pack_filter(const int32_t* w, void* dst, int oc, int c, int kh, int kw, int dil_h, int dil_w, int stored_w, void* stream) {
+size_t cvmhip_resident_filter_bytes(int oc, int c, int kh, int kw, int oh, int ow) {
+  if (oc < 1 || c < 1 || kh < 1 || kw < 1 || oh < 1 || ow < 1) return 0;
+  const int ptiles = (oh * ow + 15) / 16, octiles = res_cp(oc) / 16, tp = res_tiles(ptiles, octiles);
+  return (res_places_at(oc, c, kh, kw) + 1024 + (size_t)octiles * ((ptiles + tp - 1) / tp) * sizeof(ResItem) + 1023) / 1024 * 1024;
+}
+
+int cvmhip_resident_pack_filter(const int32_t* w, const int32_t* bias, void* dst, int oc, int c, int kh, int kw, int dil_h, int dil_w,
+                                int stored_w, void* stream) {
   if (!w || !dst || ((uintptr_t)dst & 15) || oc < 1 || c < 1 || c > 4096 || kh < 1 || kw < 1 || dil_h < 1 || dil_w < 1 || stored_w < 1 ||
       stored_w > 255 || (kh - 1) * dil_h > 254 || (kw - 1) * dil_w > 254)
     return arg_error("resident_pack_filter");
   const int ksteps = res_chunks(c, kh, kw) * RES_CHUNK;
-  const int64_t dwords = (int64_t)(res_cp(oc) / 16) * ksteps * 256, all = dwords + ksteps * 4;
-  k_pack_resident<<<(unsigned)((all + 255) / 256), 256, 0, as_stream(stream)>>>(w, reinterpret_cast<uint32_t*>(dst), dwords, oc, c, kh, kw,
-                                                                               res_cp(c), ksteps, stored_w * res_cp(c), dil_h, dil_w);
+  const int64_t dwords = (int64_t)(res_cp(oc) / 16) * ksteps * 256, all = dwords + ksteps * 4 + res_cp(oc);
+  k_pack_resident<<<(unsigned)((all + 255) / 256), 256, 0, as_stream(stream)>>>(w, bias, reinterpret_cast<uint32_t*>(dst), dwords,
+                                                                               res_cp(oc) / 16, oc, c, kh, kw, res_cp(c), ksteps,
+                                                                               stored_w * res_cp(c), dil_h, dil_w);
   return check_launch("resident_pack_filter");
 }
 
-int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d) {
-  if (!table || index < 0 || !d) return arg_error("resident_layer");
+int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d, void* places, size_t* places_bytes, size_t* places_off) {
+  if (!table || index < 0 || !d || !places || !places_bytes || !places_off) return arg_error("resident_layer");
+  *places_bytes = *places_off = 0;
   auto bytes = [](const cvmhip_resident_map& m) { return cvmhip_resident_tensor_bytes(m.c, m.h, m.w, m.border_y, m.border_x); };
   auto inside = [&](const cvmhip_resident_map& m) {
     return m.at >= 0 && (m.at & 15) == 0 && bytes(m) > 0 && (size_t)m.at + bytes(m) <= RES_LDS_MOST;
@@ -564,27 +558,27 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d)
   ResHead& h = L.h;
   h.kind = d->kind;
   if (bytes(out) == 0) return arg_error("resident_layer: map too large");
-  h.P = out.h * out.w;
-  h.OW = out.w;
+  L.P = out.h * out.w;
+  L.OW = out.w;
   L.OC = out.c;
-  h.ocp = res_cp(out.c);
-  h.div_ow = make_fastdiv((uint32_t)out.w);
+  L.ocp = res_cp(out.c);
+  L.div_ow = make_fastdiv((uint32_t)out.w);
   L.gcp = pad_channels(out.c);
   L.out_mode = d->out_mode;
   L.out = d->out;
-  h.flags = (out.c == h.ocp ? 0 : RES_MASK) | (d->out_mode != 0 ? RES_OUT : 0) |
+  h.flags = (out.c == L.ocp ? 0 : RES_MASK) | (d->out_mode != 0 ? RES_OUT : 0) |
             (out.at >= 0 && (out.border_y > 0 || out.border_x > 0) && !d->border_clean ? RES_BORDER : 0);
-  h.dst = h.res = -1;
+  L.dst = L.res = -1;
   if (d->out_mode < 0 || d->out_mode > 2 || (d->out_mode != 0 && !d->out)) return arg_error("resident_layer output");
   if (out.at >= 0) {
     if (!inside(out)) return arg_error("resident_layer output");
-    h.dst = place(out, 0, 0);
-    h.dst_row = row(out);
-    L.border_at = out.at;
-    L.border_row = row(out);
-    L.border_side = 2 * out.border_x * h.ocp;
-    L.border_edge = out.border_y * row(out) + out.border_x * h.ocp;
-    L.border_rows = out.h;
+    L.dst = place(out, 0, 0);
+    L.dst_row = row(out);
+    h.border_at = out.at;
+    h.border_row = row(out);
+    h.border_side = 2 * out.border_x * L.ocp;
+    h.border_edge = out.border_y * row(out) + out.border_x * L.ocp;
+    h.border_rows = out.h;
   } else if (d->out_mode == 0) {
     return arg_error("resident_layer output");
   }
@@ -601,49 +595,72 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d)
       return arg_error("resident_layer operands");
     if (res.at >= 0) {
       if (!inside(res) || res.c != out.c || res.h != out.h || res.w != out.w || d->kind != RES_CONV) return arg_error("resident_layer residual");
-      h.res = place(res, 0, 0);
-      h.res_row = row(res);
+      L.res = place(res, 0, 0);
+      L.res_row = row(res);
+      h.residual = 1;
     }
     L.C = in.c; L.H = in.h; L.W = in.w; L.cp = res_cp(in.c);
     L.map = place(in, 0, 0);
     L.row = row(in);
     L.KH = d->kh; L.KW = d->kw; L.SH = d->sh; L.SW = d->sw; L.PH = d->ph; L.PW = d->pw;
     if (d->kind == RES_CONV) {
-      if (!d->filter || ((uintptr_t)d->filter & 15) || !d->bias || ((uintptr_t)d->bias & 15)) return arg_error("resident_layer filter");
+      const size_t blob = cvmhip_resident_filter_bytes(out.c, in.c, d->kh, d->kw, out.h, out.w);
+      if (!d->filter || ((uintptr_t)d->filter & 15) || d->filter_at < 0 || (d->filter_at & 15) || d->filter_at + blob > RES_LDS_MOST || index < 1)
+        return arg_error("resident_layer filter");
       // every tap of every window lies inside the stored map
       if (d->ph > in.border_y || d->pw > in.border_x || (out.h - 1) * d->sh - d->ph + (d->kh - 1) * d->dh > in.h - 1 + in.border_y ||
           (out.w - 1) * d->sw - d->pw + (d->kw - 1) * d->dw > in.w - 1 + in.border_x)
         return arg_error("resident_layer window");
-      // do all groups of tiles lie alike?
-      auto offsets = [&](int tile, int* src_at, int* dst_at, int* res_at) {
-        const int y = tile * 16 / out.w, x = tile * 16 % out.w;
-        *src_at = y * d->sh * row(in) + x * d->sw * res_cp(in.c);
-        *dst_at = y * h.dst_row + x * h.ocp;
-        *res_at = y * h.res_row + x * h.ocp;
-      };
-      h.src = place(in, -d->ph, -d->pw);
-      h.step_y = d->sh * row(in);
-      h.step_x = d->sw * res_cp(in.c);
+      L.src = place(in, -d->ph, -d->pw);
+      L.step_y = d->sh * row(in);
+      L.step_x = d->sw * res_cp(in.c);
+      L.octiles = L.ocp / 16;
+      L.div_oct = make_fastdiv((uint32_t)L.octiles);
       h.chunks = res_chunks(in.c, d->kh, d->kw);
-      h.octiles = h.ocp / 16;
-      const int ptiles = (h.P + 15) / 16;
-      // as many pixel tiles per item (a filter fragment read once serves them all) as still leave every wavefront an item
-      h.tp = ptiles * h.octiles >= 4 * RES_WAVES ? 4 : ptiles * h.octiles >= 2 * RES_WAVES ? 2 : 1;
-      h.items = h.octiles * ((ptiles + h.tp - 1) / h.tp);
-      bool regular = h.P % (16 * h.tp) == 0 && (out.w % 16 == 0 || 16 % out.w == 0);
-      for (int t = 0; regular && t < ptiles; ++t) {
-        int a[3], b[3];
-        offsets(t, &a[0], &a[1], &a[2]);
-        offsets(t - t % h.tp, &b[0], &b[1], &b[2]);
-        if (t < h.tp) { h.src_off[t] = a[0] - b[0]; h.dst_off[t] = a[1] - b[1]; h.res_off[t] = a[2] - b[2]; }
-        else regular = h.src_off[t % h.tp] == a[0] - b[0] && h.dst_off[t % h.tp] == a[1] - b[1] && h.res_off[t % h.tp] == a[2] - b[2];
+      h.w_at = d->filter_at;
+      h.taps_at = h.w_at + L.octiles * h.chunks * (RES_CHUNK * 1024);
+      h.bias_at = h.taps_at + h.chunks * (RES_CHUNK * 16);
+      // whole tiles, which all lie like the first one (part of a row, or whole rows), and a result for LDS only
+      const int ptiles = (L.P + 15) / 16, tp = res_tiles(ptiles, L.octiles);
+      if (!(h.flags & (RES_CHAIN | RES_CHAIN2 | RES_MASK | RES_OUT)) && L.P % (16 * tp) == 0 && (out.w % 16 == 0 || 16 % out.w == 0)) {
+        h.flags |= RES_PLAIN;
+        h.tp = tp;
+        h.items = L.octiles * (ptiles / tp);
+        const size_t at = res_places_at(out.c, in.c, d->kh, d->kw);
+        h.places_at = h.w_at + (int)at;
+        const ResGeometry g = {L.P, L.OW, L.div_ow, L.src, L.step_y, L.step_x, L.dst, L.dst_row, L.ocp, L.res, L.res_row};
+        ResPlace* own = reinterpret_cast<ResPlace*>(places);
+        ResItem* items = reinterpret_cast<ResItem*>(own + 64);
+        for (int l = 0; l < 64; ++l) own[l] = res_place(g, l & 15, (l & 15) / g.OW, l);
+        const ResPlace first = res_place(g, 0, 0, 0);
+        for (int i = 0; i < h.items; ++i) {
+          const int ot = i % L.octiles;
+          items[i] = ResItem{};
+          items[i].filter = h.w_at + ot * h.chunks * (RES_CHUNK * 1024);
+          items[i].bias = h.bias_at + ot * 64;
+          for (int t = 0; t < tp; ++t) {
+            const int p = (i / L.octiles * tp + t) * 16;
+            const ResPlace q = res_place(g, p, p / g.OW, 0);
+            items[i].src[t] = q.src - first.src;
+            items[i].dst[t] = q.dst - first.dst + ot * 16;
+            items[i].res[t] = q.res - first.res + ot * 16;
+          }
+        }
+        *places_off = at;
+        *places_bytes = 64 * sizeof(ResPlace) + h.items * sizeof(ResItem);
+      } else {
+        h.items = L.octiles * ptiles;
       }
-      if (regular) h.flags |= RES_REGULAR;
-      h.div_oct = make_fastdiv((uint32_t)h.octiles);
-      h.filter = reinterpret_cast<const int8_t*>(d->filter);
-      h.taps = reinterpret_cast<const int*>(h.filter + (size_t)h.octiles * h.chunks * (RES_CHUNK * 1024));
-      h.bias = d->bias;
+      // the layer in front of it fetches the filter
+      ResHead before;
+      char* at = reinterpret_cast<char*>(table) + (index - 1) * cvmhip_resident_layer_bytes();
+      memcpy(&before, at, sizeof(before));
+      before.next = reinterpret_cast<const int8_t*>(d->filter);
+      before.next_kb = (int)(blob / 1024);
+      before.next_at = d->filter_at;
+      memcpy(at, &before, sizeof(before));
     } else if (d->kind == RES_SUM) {
+      L.div_w = make_fastdiv((uint32_t)in.w);
       if (out.h != 1 || out.w != 1 || in.c != out.c) return arg_error("resident_layer sum");
     } else if (d->kind == RES_POOL) {
       if (in.c != out.c) return arg_error("resident_layer pool");
@@ -664,9 +681,8 @@ int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_
   char desc[64] = "";
   if (kernel_timing_enabled()) snprintf(desc, sizeof(desc), "%d layers in LDS, %d images", nlayers, images);
   KernelTimer timer("k_conv_resident", ops, as_stream(stream), bytes, desc);
-  const int grid = ((images + 7) & ~7) + 8 * RES_HELPERS;
-  k_conv_resident<<<(unsigned)grid, RES_THREADS, lds_bytes, as_stream(stream)>>>(reinterpret_cast<const ResLayer*>(dev_table), nlayers, images,
-                                                                                call ? *call : cvmhip_resident_call{});
+  k_conv_resident<<<(unsigned)images, RES_THREADS, lds_bytes, as_stream(stream)>>>(reinterpret_cast<const ResLayer*>(dev_table), nlayers, images,
+                                                                                  call ? *call : cvmhip_resident_call{});
   return check_launch("conv_resident");
 }
 

@@ -8,10 +8,10 @@
 //     the most that the per-layer kernels reach on maps of this size;
 //   * in LDS: per layer 1800 clocks from barrier to barrier without any work (the layer's head, the first filters, the first
 //     operands, the last result), and the largest of the filter's way through one compute unit (30 bytes a clock from the
-//     L2, and 64 where a further pixel group finds it in the L1), the instructions (4 clocks each, 4 per pixel tile and K
-//     step, 40 per tile for the result, over four SIMDs) and the latency of the K steps behind one another; rounds of
+//     L2, and 64 from LDS), the instructions (4 clocks each, 4 per pixel tile and K step, 40 per tile for the result, over
+//     four SIMDs) and the latency of the K steps behind one another; rounds of
 //     workgroups when there are more images than compute units.
-// Measured on ResNet-20: 38 us estimated, 41.5 us measured.  The tail of SSD-512 (10 x 10 maps and smaller, filters of
+// Measured on ResNet-20: 38 us estimated, 39 us measured.  The tail of SSD-512 (10 x 10 maps and smaller, filters of
 // 300 KB and more) was 32 us in one launch and the same as single ones: one compute unit reads a filter too slowly.
 // ResNet-50's 7 x 7 layers at batch 50 lost 300 us with the single launches estimated at 350 TOP/s.
 #include <algorithm>
@@ -295,6 +295,20 @@ HipGraphRuntime::ResidentDraft HipGraphRuntime::DraftResident(size_t first, size
     }
     l.d.border_clean = before && std::memcmp(&before->map, &x.map, sizeof(x.map)) == 0 ? 1 : 0;
   }
+  // behind the maps two places for filters, which the convolutions take in turn
+  size_t need[2] = {0, 0};
+  int convs = 0;
+  for (const ResidentDraft::Layer& l : r.layers) {
+    if (l.d.kind != 2) continue;
+    const PlanStep& st = plan_[l.step];
+    size_t& most = need[convs++ & 1];
+    most = std::max(most, cvmhip_resident_filter_bytes(st.oc, st.c, st.kh, st.kw, l.d.dst.h, l.d.dst.w));
+  }
+  const size_t filters = (r.lds + 15) & ~static_cast<size_t>(15);
+  convs = 0;
+  for (ResidentDraft::Layer& l : r.layers)
+    if (l.d.kind == 2) l.d.filter_at = static_cast<int>(filters + (convs++ & 1 ? need[0] : 0));
+  r.lds = filters + need[0] + need[1];
   r.ok = r.lds <= cvmhip_resident_lds_limit();
   return r;
 }
@@ -333,20 +347,19 @@ void HipGraphRuntime::BuildResident() {
     r.images = plan_[from].n;
     r.lds = d.lds;
     std::vector<char> table(d.layers.size() * cvmhip_resident_layer_bytes());
-    // filters, biases and table in one allocation: a layer's first touch of pages of its own is a trip to the page tables
+    // filters and table in one allocation: a layer's first touch of pages of its own is a trip to the page tables
     size_t total = AlignUp(table.size(), 256);
-    std::vector<size_t> filter_at(d.layers.size(), 0), bias_at(d.layers.size(), 0);
+    std::vector<size_t> filter_at(d.layers.size(), 0);
     for (size_t l = 0; l < d.layers.size(); ++l) {
       if (d.layers[l].d.kind != 2) continue;
       const PlanStep& st = plan_[d.layers[l].step];
       filter_at[l] = total;
-      total += AlignUp(cvmhip_resident_filter_bytes(st.oc, st.c, st.kh, st.kw), 256);
-      bias_at[l] = total;
-      total += AlignUp(static_cast<size_t>(Pad(st.oc)) * 4, 256);
+      total += cvmhip_resident_filter_bytes(st.oc, st.c, st.kh, st.kw, d.layers[l].d.dst.h, d.layers[l].d.dst.w);
     }
     auto buf = std::make_shared<DeviceBuffer>();
     Check(cvmhip_alloc(&buf->ptr, total), "resident run");
     char* base = static_cast<char*>(buf->ptr);
+    std::vector<char> places(total);
     for (size_t l = 0; l < d.layers.size(); ++l) {
       ResidentDraft::Layer& layer = d.layers[l];
       const PlanStep& st = plan_[layer.step];
@@ -354,18 +367,20 @@ void HipGraphRuntime::BuildResident() {
       if (layer.res >= 0) layer.d.res = d.tensors[layer.res].map;
       if (layer.dst >= 0) layer.d.dst = d.tensors[layer.dst].map;
       if (layer.d.kind == 2) {
-        void *filter = base + filter_at[l], *bias = base + bias_at[l];
-        Check(cvmhip_resident_pack_filter(entry_ptr_[st.wsrc], filter, st.oc, st.c, st.kh, st.kw, st.dh, st.dw,
+        void* filter = base + filter_at[l];
+        Check(cvmhip_resident_pack_filter(entry_ptr_[st.wsrc], st.bias, filter, st.oc, st.c, st.kh, st.kw, st.dh, st.dw,
                                           layer.d.src.w + 2 * layer.d.src.border_x, stream_), "resident filter");
-        Check(cvmhip_memset32(bias, 0, Pad(st.oc), stream_), "resident bias");
-        if (st.bias) Check(cvmhip_copy_d2d(bias, st.bias, static_cast<size_t>(st.oc) * 4, stream_), "resident bias");
         layer.d.filter = filter;
-        layer.d.bias = static_cast<const int32_t*>(bias);
         const double work = static_cast<double>(st.oc) * st.c * st.kh * st.kw;
         r.ops += 2.0 * r.images * layer.d.dst.h * layer.d.dst.w * work;
         r.bytes += work;
       }
-      Check(cvmhip_resident_layer(table.data(), static_cast<int>(l), &layer.d), "resident layer");
+      size_t bytes = 0, off = 0;
+      Check(cvmhip_resident_layer(table.data(), static_cast<int>(l), &layer.d, places.data(), &bytes, &off), "resident layer");
+      if (bytes > 0) {
+        Check(cvmhip_copy_h2d(base + filter_at[l] + off, places.data(), bytes, stream_), "resident places");
+        Check(cvmhip_stream_sync(stream_), "resident places");   // the buffer is used again
+      }
     }
     Check(cvmhip_copy_h2d(base, table.data(), table.size(), stream_), "resident table");
     Check(cvmhip_stream_sync(stream_), "resident table");   // the host copy goes away

@@ -446,8 +446,8 @@ int cvmhip_conv2d_stem_pool3_i8(const void* xs, const void* wp, const int32_t* b
                                 int pad_h, int pad_w, int pool_oh, int pool_ow, void* stream);
 /* A run of layers whose maps fit in LDS in one launch, a workgroup per image.  The table (nlayers entries of
  * cvmhip_resident_layer_bytes, filled on the host, read on the device at a 64-byte aligned address) holds the loads of what
- * the run reads (kind 0: int8 NCHW image clamped to +-range, 1: int8 act tensor), convolutions (2: filter from
- * cvmhip_resident_pack_filter, `bias` as many values as the output has channels in LDS: 16 or the next multiple of 32;
+ * the run reads (kind 0: int8 NCHW image clamped to +-range, 1: int8 act tensor), convolutions (2: filter and
+ * bias from cvmhip_resident_pack_filter;
  * v = chain(acc + bias), with a residual chain2(v + residual)), sums over the map (3, with chain) and max-pools (4).  A map
  * lies at byte `at` of LDS (a multiple of 16, below cvmhip_resident_lds_limit; -1: not in LDS) with a border of zeros as wide
  * as the padding of the convolutions that read it; maps that are alive together must not overlap.  out_mode: 0 the result
@@ -463,17 +463,18 @@ typedef struct cvmhip_resident_desc {
   int32_t border_clean;   /* the border of dst is zero already: the last map at this place had the same extent and border */
   const void* in;
   const void* filter;
-  const int32_t* bias;
+  int32_t filter_at;      /* where the filter lies in LDS during its layer and the one in front of it (which fetches it) */
   void* out;
   cvmhip_chain chain, chain2;
 } cvmhip_resident_desc;
 size_t cvmhip_resident_layer_bytes(void);
 size_t cvmhip_resident_lds_limit(void);
 size_t cvmhip_resident_tensor_bytes(int c, int h, int w, int border_y, int border_x);
-size_t cvmhip_resident_filter_bytes(int oc, int c, int kh, int kw);
-int cvmhip_resident_pack_filter(const int32_t* w, void* dst, int oc, int c, int kh, int kw, int dil_h, int dil_w,
+size_t cvmhip_resident_filter_bytes(int oc, int c, int kh, int kw, int oh, int ow);
+int cvmhip_resident_pack_filter(const int32_t* w, const int32_t* bias /* or NULL */, void* dst, int oc, int c, int kh, int kw, int dil_h, int dil_w,
                                 int stored_w /* row of the input map in LDS, with its border */, void* stream);
-int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* desc);
+/* `places`: host buffer of cvmhip_resident_filter_bytes; *places_bytes of it then belong *places_off behind desc->filter */
+int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* desc, void* places, size_t* places_bytes, size_t* places_off);
 /* A whole call in that launch: the image comes from pinned host memory instead of `in`, the int32 result also goes to
  * pinned memory, and `ticket` is stored to *flag_host behind it (cvmhip_export_wait; *counter is a zeroed device word). */
 typedef struct cvmhip_resident_call {

