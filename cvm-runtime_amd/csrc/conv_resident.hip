@@ -225,6 +225,11 @@ __device__ __forceinline__ void res_products(const ResHead& h, const char* lds, 
     }
     res_chunk<TP>(lds, w + c * (RES_CHUNK * 1024), now, base, acc);
   }
+  // A vector instruction may read an eight-pass product's registers 11 wait states behind it.  The compiler sees to that for
+  // instructions it knows, but res_clamp is inline assembly to it: the wait is part of the values' way there.
+  if constexpr (TP == 1) asm volatile("s_nop 15" : "+v"(acc[0]));
+  else if constexpr (TP == 2) asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]));
+  else asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
 }
 __device__ __forceinline__ void res_first_taps(const ResHead& h, const char* lds, int lane, int (&tap)[RES_CHUNK]) {
 #pragma unroll
