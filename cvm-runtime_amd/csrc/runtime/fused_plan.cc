@@ -734,6 +734,7 @@ void HipGraphRuntime::BuildPlan() {
   }
   if (hooks_.fold_bias) FoldRequant();
   BuildResident();
+  BuildSeparable();
   if (hooks_.seq) BuildSequences();
   BuildGroups();
 }
@@ -767,6 +768,40 @@ void HipGraphRuntime::FoldRequant() {
   }
 }
 
+// A depthwise 3x3 convolution whose only reader is the 1x1 convolution behind it becomes one launch with it, up to 512
+// channels (a workgroup goes through all of them one after the other: 1024 -> 1024 at 16 x 16 takes 9.7 us, as two launches
+// 8.1) and where the depthwise part is computed once or the layer is small: with more than 256 output channels several
+// workgroups repeat it, which up to 4096 pixels is hidden behind idle compute units.
+void HipGraphRuntime::BuildSeparable() {
+  if (!hooks_.separable) return;
+  for (size_t i = 0; i + 1 < plan_.size(); ++i) {
+    PlanStep& d = plan_[i];
+    const PlanStep& p = plan_[i + 1];
+    if (in_resident_[i] || in_resident_[i + 1] || d.kind != PlanStep::DWCONV || !d.out_i8 || d.kh != 3 || d.kw != 3 || d.dh != 1 || d.dw != 1 || d.wsrc == kNone)
+      continue;
+    if (p.kind != PlanStep::CONV || p.src != d.dst || p.src2 != kNone || !p.out_i8 || p.stem || p.nhwc || p.flat || p.ws || p.pool2 || p.pool3 ||
+        p.kh != 1 || p.kw != 1 || p.sh != 1 || p.sw != 1 || p.ph != 0 || p.pw != 0)
+      continue;
+    bool only = true;
+    for (size_t k = 0; k < plan_.size(); ++k)
+      only = only && (k == i || k == i + 1 || plan_[k].kind == PlanStep::NODE || (plan_[k].src != d.dst && plan_[k].src2 != d.dst));
+    if (!only || !cvmhip_separable_eligible(d.n, d.c, d.h, d.w, p.oc, d.sh, d.sw, d.ph, d.pw)) continue;
+    if (d.c > 512 || (p.oc > 256 && static_cast<int64_t>(p.n) * p.h * p.w > 4096)) continue;
+    if (((reinterpret_cast<uintptr_t>(d.bias) | reinterpret_cast<uintptr_t>(p.bias)) & 15) != 0) continue;
+    auto buf = std::make_shared<DeviceBuffer>();
+    Check(cvmhip_alloc(&buf->ptr, cvmhip_separable_filter_bytes(d.c)), "separable filter");
+    Check(cvmhip_pack_separable_filter(entry_ptr_[d.wsrc], buf->ptr, d.c, stream_), "separable filter");
+    d.separable = buf;
+  }
+}
+
+void HipGraphRuntime::RunSeparable(size_t step) {
+  const PlanStep &d = plan_[step], &p = plan_[step + 1];
+  Check(cvmhip_conv2d_separable_i8(i8_ptr_[d.src], static_cast<DeviceBuffer*>(d.separable.get())->ptr, d.bias, &d.chain,
+                                   static_cast<DeviceBuffer*>(p.weights.get())->ptr, p.bias, &p.chain, i8_ptr_[p.dst], d.n, d.c, d.h, d.w,
+                                   p.oc, d.sh, d.sw, d.ph, d.pw, stream_), "conv2d_separable_i8");
+}
+
 // Runs of at least three consecutive convolution steps that a layer-sequence launch can take (batch a multiple
 // of 8, int8 in and out, channels padded to 32, no K slices) become one launch each.  Consecutive plan steps
 // only depend on earlier ones, which is all a sequence needs.
@@ -780,7 +815,7 @@ void HipGraphRuntime::BuildSequences() {
     size_t j = i;
     for (; j < plan_.size(); ++j) {
       const PlanStep& st = plan_[j];
-      if (st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2) break;
+      if (InSeparable(j) || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2) break;
       table.resize((j - i + 1) * entry);
       const void* res = st.src2 == kNone ? nullptr : i8_ptr_[st.src2];
       const int rc = cvmhip_conv_seq_layer(table.data(), static_cast<int>(j - i), i8_ptr_[st.src],
@@ -844,7 +879,7 @@ void HipGraphRuntime::BuildGroups() {
     size_t j = i;
     for (; j < plan_.size(); ++j) {
       const PlanStep& st = plan_[j];
-      if (in_resident_[j] || st.kind != PlanStep::CONV || !st.nhwc || st.stem) break;
+      if (in_resident_[j] || InSeparable(j) || st.kind != PlanStep::CONV || !st.nhwc || st.stem) break;
       table.resize((j - i + 1) * entry);
       int nb = 0;
       const int32_t* bias = st.pair ? static_cast<const int32_t*>(static_cast<DeviceBuffer*>(st.pair_bias.get())->ptr) : st.bias;
@@ -895,7 +930,7 @@ void HipGraphRuntime::BuildGroups() {
     size_t j = i;
     for (; j < plan_.size(); ++j) {
       const PlanStep& st = plan_[j];
-      if (in_resident_[j] || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
+      if (in_resident_[j] || InSeparable(j) || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
       bool reads_member = false;
       for (uint32_t w : written) reads_member = reads_member || st.src == w || st.src2 == w;
       if (reads_member) break;

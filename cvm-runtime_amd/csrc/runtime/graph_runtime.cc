@@ -448,9 +448,12 @@ void HipGraphRuntime::ReadHooks() {
   auto env = [](const char* name) { const char* v = std::getenv(name); return std::string(v ? v : ""); };
   hooks_.fuse = env("CVM_HIP_FUSE") != "0";
   hooks_.resident = env("CVM_HIP_RESIDENT") != "0";
+  bool plain = true;
   for (const char* other : {"CVM_HIP_SEQ", "CVM_HIP_SEQCFG", "CVM_HIP_DW", "CVM_HIP_POOLFUSE", "CVM_HIP_HEADPAIR", "CVM_HIP_HEADGROUP",
                             "CVM_HIP_CONVGROUP", "CVM_HIP_FLATDENSE", "CVM_HIP_CONV", "CVM_HIP_WAVECFG", "CVM_HIP_TILE"})
-    hooks_.resident = hooks_.resident && env(other).empty();
+    plain = plain && env(other).empty();
+  hooks_.resident = hooks_.resident && plain;
+  hooks_.separable = plain && env("CVM_HIP_SEPARABLE") != "0";
   hooks_.fold_bias = env("CVM_HIP_FOLDBIAS") != "0";
   hooks_.graph = env("CVM_HIP_GRAPH") != "0";
   hooks_.graph_forced = !env("CVM_HIP_GRAPH").empty();
@@ -820,6 +823,9 @@ void HipGraphRuntime::Launch() {
         HipCheck(cvmhip_conv_seq_launch(r.table, r.nlayers, seq_sync_, r.ops, r.bytes, stream_), "layer-sequence launch");
         seq_ran_ = true;
         i = r.last + 1;
+      } else if (plan_[i].separable) {
+        RunSeparable(i);
+        i += 2;
       } else if (!group_at_.empty() && group_at_[i] >= 0) {
         const GroupRun& r = groups_[group_at_[i]];
         if (r.i8) HipCheck(cvmhip_conv_group_launch_i8(r.table, r.nlayers, r.blocks, r.ops, r.bytes, stream_), "grouped convolutions");

@@ -486,6 +486,15 @@ typedef struct cvmhip_resident_call {
 } cvmhip_resident_call;
 int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_t lds_bytes, const cvmhip_resident_call* call /* or NULL */,
                            double ops, double bytes, void* stream);
+/* Depthwise conv2d (3x3, dilation 1) and the 1x1 conv2d (stride 1, no padding) that reads it, in one launch; both channel
+ * counts multiples of 32, `wd` from cvmhip_pack_separable_filter (int32 [c][1][3][3]), `wp` from cvmhip_pack_weights, biases
+ * 16-byte aligned or NULL:  out = chain_p(conv1x1(chain_d(depthwise(x) + bias_d)) + bias_p), int8 act tensors. */
+size_t cvmhip_separable_filter_bytes(int c);
+int cvmhip_pack_separable_filter(const int32_t* w, void* wd, int c, void* stream);
+int cvmhip_separable_eligible(int n, int c, int h, int w, int oc, int stride_h, int stride_w, int pad_h, int pad_w);
+int cvmhip_conv2d_separable_i8(const void* xp, const void* wd, const int32_t* bias_d, const cvmhip_chain* chain_d, const void* wp,
+                               const int32_t* bias_p, const cvmhip_chain* chain_p, void* out, int n, int c, int h, int w, int oc,
+                               int stride_h, int stride_w, int pad_h, int pad_w, void* stream);
 /* depthwise conv2d (groups == channels == out channels) on int8 act tensors, filter packed by
  * cvmhip_pack_depthwise_weights into [kh*kw][cp] int8 */
 size_t cvmhip_packed_depthwise_bytes(int c, int kh, int kw);

@@ -1,0 +1,42 @@
+"""Depthwise and 1x1 convolution in one launch, against the oracle running the graph node by node."""
+import numpy as np
+import pytest
+
+import oracle.graph as og
+from cvm_runtime_amd import graphgen, runtime, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,stride,pad", [
+    (1, 32, 67, 61, 32, 1, 1),       # one channel tile: 256 pixels to a workgroup, ends inside one
+    (2, 64, 40, 40, 64, 2, 1),
+    (1, 96, 33, 50, 160, 1, 0),      # no padding; channel tiles that do not fill the last workgroup
+    (3, 128, 23, 30, 128, 1, 1),
+    (1, 512, 29, 31, 512, 1, 1),     # the depthwise tile computed by two workgroups
+    (1, 288, 30, 30, 320, 2, 2),     # padding wider than the filter needs, a second group of two channel tiles
+    (1, 512, 17, 18, 1024, 2, 1),    # filter requested in two rounds, four groups
+])
+@pytest.mark.parametrize("multiply", [False, True])
+def test_depthwise_and_pointwise_in_one_launch(n, c, h, w, oc, stride, pad, multiply, dev, monkeypatch):
+    g = graphgen.GraphBuilder("separable-%d-%d" % (c, oc))
+    x = g.var("data", (n, c, h, w), 8)
+    y, k = g.conv(x, c, 3, stride, pad, groups=c)
+    if multiply:   # a chain that is no clamp and shift
+        y = g.op("broadcast_mul", [y, g.param("m", (1,), 3, 3, 3)], {}, [g.shape(y)])[0]
+    y = g.rshift(g.relu(y), graphgen.shift_for(k) + 2 * multiply)
+    z, k = g.conv(y, oc, 1)
+    z = g.conv_relu_q(g.rshift(z, graphgen.shift_for(k)), 40, 1)   # reads it as int8
+    js, pb = g.build([z])
+    data = synth.tensor("separable", "data%d" % c, (n, c, h, w), -127, 127)
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "1")
+    m = runtime.HipModel(js, pb)
+    counts = [m.launch_counts()[0]]
+    got = np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int8 if m.output_length == int(np.prod(g.shape(z))) else np.int32)
+    m.close()
+    monkeypatch.setenv("CVM_HIP_SEPARABLE", "0")
+    m = runtime.HipModel(js, pb)
+    counts.append(m.launch_counts()[0])
+    m.close()
+    assert counts[0] == counts[1] - 1, counts
+    assert np.array_equal(got.astype(np.int32), og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))[0].ravel())
