@@ -450,13 +450,15 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
     }
   }
   if (call.flag_host) {
+    const uint32_t ticket = tid == 0 ? call.counter[1] + 1 : 0;
     __threadfence_system();
     __syncthreads();
     if (tid == 0) {
       const uint32_t before = __hip_atomic_fetch_add(call.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
       if (before == (uint32_t)images - 1) {
-        *call.counter = 0;
-        __hip_atomic_store(call.flag_host, call.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        call.counter[0] = 0;
+        call.counter[1] = ticket;
+        __hip_atomic_store(call.flag_host, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
   }

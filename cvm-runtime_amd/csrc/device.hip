@@ -170,7 +170,8 @@ struct ExportArgs {
 };
 
 __global__ void __launch_bounds__(256) k_export(ExportArgs a, const uint32_t* __restrict__ status, uint32_t* __restrict__ status_host,
-                                                uint32_t* __restrict__ counter, uint32_t* __restrict__ flag, uint32_t ticket) {
+                                                uint32_t* __restrict__ counter, uint32_t* __restrict__ flag) {
+  const uint32_t ticket = threadIdx.x == 0 ? counter[1] + 1 : 0;   // (written by the last workgroup of the export before)
   const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
   for (int k = 0; k < a.count; ++k) {
     const int64_t granules = a.words[k] / 4;
@@ -186,14 +187,15 @@ __global__ void __launch_bounds__(256) k_export(ExportArgs a, const uint32_t* __
   if (threadIdx.x == 0) {
     const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
     if (before == gridDim.x - 1) {
-      *counter = 0;
+      counter[0] = 0;
+      counter[1] = ticket;
       __hip_atomic_store(flag, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
 }
 
 int cvmhip_export_words(const void* const* src, void* const* dst_host, const int64_t* words, int count, const uint32_t* status,
-                        uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, uint32_t ticket, void* stream) {
+                        uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, void* stream) {
   if (!src || !dst_host || !words || count < 0 || count > CVMHIP_EXPORT_MAX || !counter || !flag_host || (status && !status_host))
     return arg_error("export_words");
   ExportArgs a{};
@@ -210,7 +212,7 @@ int cvmhip_export_words(const void* const* src, void* const* dst_host, const int
   int64_t blocks = (most / 4 + 255) / 256;
   if (blocks < 1) blocks = 1;
   if (blocks > 64) blocks = 64;
-  k_export<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(a, status, status_host, counter, flag_host, ticket);
+  k_export<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(a, status, status_host, counter, flag_host);
   return check_launch("export_words");
 }
 

@@ -499,7 +499,7 @@ void HipGraphRuntime::ApplyTuning() {
 
 void HipGraphRuntime::Release() {
   if (stream_) cvmhip_stream_sync(stream_);   // launches may still read the staging buffers
-  if (graph_exec_) { cvmhip_graph_destroy(graph_exec_); graph_exec_ = nullptr; }
+  DropGraphs();
   plan_.clear();
   if (seq_counted_) { CountSequenceModel(-1); seq_counted_ = false; }
   seqs_.clear();
@@ -729,12 +729,12 @@ void HipGraphRuntime::LoadParams(const std::string& blob) {
 }
 
 // A graph is one submission, and saves the host what it costs to issue every launch (2.8 to 4 us each); but it reaches the
-// device about 7 us later than a launch does, and what follows it waits as long (calls of CVMAPIInference: ResNet-20, one
-// launch between input and output, 61 us as a graph, 54 without; SSD-512, 35 launches, 312 and 293; VGG-16 at batch 16 484
-// and 475; ResNet-50 at batch 50 1020 and 999).  Where the host is hardly faster than the device, its every delay shows:
-// ResNet-50 at batch 1, 52 launches of 4.7 us, took 264 us without a graph in one process and 299 in the next, and 270 to 277
-// with one in all.  So a few calls are made when the model is loaded, and launches are issued one by one where a call has 6 us
-// or more for each of them (SSD at 300 x 300 6.6, SSD-512 8.4, ResNet-50 5.2 at batch 1 and 6.4 at batch 6).
+// device about 7 us later than a launch does, and is a little slower on it where launches are long.  With the ends of a call
+// in the graph (CaptureCall) calls of CVMAPIInference took, as a graph and launch by launch: SSD-512 (7 us a launch) 259 and
+// 258 us, ResNet-50 at batch 1 (4.7 us) 266 and, by the host of the process, 264 to 302, at batch 12 378 and 390, at batch
+// 50 (17 us) 1007 and 1000, VGG-16 at batch 16 475 and 478, ResNet-20 at batch 64 (one launch of 40 us) 67 and 60.  So a
+// few calls are made when the model is loaded, and launches are issued one by one where a call has 15 us or more for each
+// of them.
 // CVM_HIP_GRAPH=0 or 1 names a form (and with CVM_HIP_SEQ=1 nothing runs before the first call).
 void HipGraphRuntime::ChooseSubmission() {
   if (!fused_ || !hooks_.graph || hooks_.graph_forced || hooks_.seq_forced || GetInputPrecision() > 8) return;
@@ -751,7 +751,7 @@ void HipGraphRuntime::ChooseSubmission() {
   std::nth_element(us.begin(), us.begin() + 5, us.end());
   int launches = 0;
   LaunchCounts(&launches, nullptr, nullptr);
-  hooks_.graph = us[5] < 6.0 * launches;
+  hooks_.graph = us[5] < 15.0 * launches;
 }
 
 // Layer-sequence launches pay for layers that are bound by latency and cost a little where layers are large, and steps that
@@ -762,7 +762,7 @@ void HipGraphRuntime::CalibrateSequences() {
   float ms[2] = {0, 0};
   for (int with_seq = 0; with_seq < 2; ++with_seq) {
     use_seq_ = with_seq != 0;
-    if (graph_exec_) { cvmhip_graph_destroy(graph_exec_); graph_exec_ = nullptr; }
+    DropGraphs();
     graph_state_ = 0;
     for (int i = 0; i < 3; ++i) Run();   // eager, capture, first replay
     SyncStream();
@@ -779,7 +779,7 @@ void HipGraphRuntime::CalibrateSequences() {
   }
   use_seq_ = ms[1] < 0.98f * ms[0];   // a clear win only: within the noise of a few replays the plainer form stays
   if (!use_seq_) DropSequences();
-  if (graph_exec_) { cvmhip_graph_destroy(graph_exec_); graph_exec_ = nullptr; }
+  DropGraphs();
   graph_state_ = 0;
 }
 
@@ -858,7 +858,7 @@ void HipGraphRuntime::Run() {
   }
   const bool seq_now = SeqNow();
   if (seq_now != seq_mode_) {   // another model with sequence launches appeared or went away: the other form from here on
-    if (graph_exec_) { cvmhip_graph_destroy(graph_exec_); graph_exec_ = nullptr; }
+    DropGraphs();
     if (graph_state_ == 3) graph_state_ = 2;
     seq_mode_ = seq_now;
   }
@@ -971,7 +971,7 @@ void HipGraphRuntime::CheckSequences(bool requested) {
   std::cerr << "cvm hip: a layer-sequence launch could not keep all its workgroups resident; using one launch per layer\n";
   DropSequences();
   HipCheck(cvmhip_memset32(seq_sync_, 0, words, stream_), "sequence status");
-  if (graph_exec_) { cvmhip_graph_destroy(graph_exec_); graph_exec_ = nullptr; }
+  DropGraphs();
   graph_state_ = 0;
   Run();
   HipCheck(cvmhip_stream_sync(stream_), "repeat run");
@@ -983,8 +983,8 @@ void HipGraphRuntime::AllocOutputStage() {
   for (const NodeEntry& e : outputs_) total += AlignUp(static_cast<size_t>(shape_size(shape_[entry_id(e)])) * 4, 64);
   HipCheck(cvmhip_host_alloc(&out_stage_host_, total), "output staging buffer");
   std::memset(out_stage_host_, 0, 64);
-  HipCheck(cvmhip_alloc(&out_counter_, 4), "output counter");
-  HipCheck(cvmhip_memset32(out_counter_, 0, 1, stream_), "output counter");
+  HipCheck(cvmhip_alloc(&out_counter_, 8), "output counter");
+  HipCheck(cvmhip_memset32(out_counter_, 0, 2, stream_), "output counter");
   size_t off = 64;
   for (const NodeEntry& e : outputs_) {
     out_host_.push_back(reinterpret_cast<const int32_t*>(static_cast<char*>(out_stage_host_) + off));
@@ -1000,7 +1000,22 @@ const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, 
   const bool whole = fused_ && shape_size(InputShape()) <= (128 << 10) && residents_.size() == 1 && residents_[0].whole_call && !(residents_[0].under_seq && SeqNow()) &&
                      !seq_calibration_pending_ && !cvmhip_kernel_timing_active();
   if (!whole) {
-    SetDataI8(host, shape);
+    const bool as_call = graph_state_ == 3 && seq_mode_ == SeqNow() && !seq_calibration_pending_ && !cvmhip_kernel_timing_active() && CaptureCall();
+    if (as_call && call_imports_) {
+      CheckData(shape);
+      if (in_stage_busy_) HipCheck(cvmhip_stream_sync(stream_), "copy input to device");
+      in_stage_ahead_ = false;
+      in_stage_busy_ = true;
+      std::memcpy(in_stage_host_, host, static_cast<size_t>(shape_size(shape)));
+    } else {
+      SetDataI8(host, shape);
+    }
+    if (as_call) {
+      HipCheck(cvmhip_graph_launch(call_exec_, stream_), "graph launch");
+      ++ticket_;
+      if (seq_mode_) seq_ran_ = true;
+      return CollectOutputs(seq_mode_ && use_seq_ && seq_sync_);
+    }
     Run();
     return FetchOutputs();
   }
@@ -1012,8 +1027,9 @@ const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, 
   in_stage_ahead_ = true;
   const ResidentRun& r = residents_[0];
   uint32_t* head = static_cast<uint32_t*>(out_stage_host_);
-  const cvmhip_resident_call call = {in_stage_host_, const_cast<int32_t*>(out_host_[0]), static_cast<uint32_t*>(out_counter_), head, ++ticket_};
+  const cvmhip_resident_call call = {in_stage_host_, const_cast<int32_t*>(out_host_[0]), static_cast<uint32_t*>(out_counter_), head};
   HipCheck(cvmhip_resident_launch(r.table, r.nlayers, r.images, r.lds, &call, r.ops, r.bytes, stream_), "layers in LDS");
+  ++ticket_;
   AwaitTicket();
   return out_host_;
 }
@@ -1025,25 +1041,67 @@ void HipGraphRuntime::AwaitTicket() {
   in_stage_busy_ = false;
 }
 
+// One kernel behind the run writes every output, the sequence launches' status word and a ticket to pinned memory.
+void HipGraphRuntime::ExportOutputs(bool status) {
+  const void* src[CVMHIP_EXPORT_MAX];
+  void* dst[CVMHIP_EXPORT_MAX];
+  int64_t words[CVMHIP_EXPORT_MAX];
+  for (size_t k = 0; k < outputs_.size(); ++k) {
+    const uint32_t eid = entry_id(outputs_[k]);
+    src[k] = entry_ptr_[eid];
+    dst[k] = const_cast<int32_t*>(out_host_[k]);
+    words[k] = shape_size(shape_[eid]);
+  }
+  const uint32_t* word = status ? static_cast<uint32_t*>(seq_sync_) + (cvmhip_conv_seq_sync_bytes() / 4 - 64) : nullptr;
+  HipCheck(cvmhip_export_words(src, dst, words, static_cast<int>(outputs_.size()), word, word ? seq_error_host_ : nullptr,
+                               static_cast<uint32_t*>(out_counter_), static_cast<uint32_t*>(out_stage_host_), stream_), "copy output");
+}
+
+// The run, the export behind it and a small input in front of it as one graph: as a launch of its own the export waits 7 us for the graph in front of it
+// to be seen to have ended, and a graph behind an import waits for that (ResNet-50 at batch 1: 273.5 us a call with both
+// outside, 268.7 with the export in the graph, 266 with an input of one piece in it as well).
+bool HipGraphRuntime::CaptureCall() {
+  if (call_exec_) return true;
+  if (call_refused_ || outputs_.size() > CVMHIP_EXPORT_MAX) return false;
+  AllocOutputStage();
+  AllocInputStage();
+  call_refused_ = true;
+  HipCheck(cvmhip_stream_sync(stream_), "capture");
+  if (cvmhip_capture_begin(stream_) != CVMHIP_OK) return false;
+  bool ok = true;
+  try {
+    const size_t bytes = static_cast<size_t>(shape_size(InputShape()));
+    call_imports_ = data_stays_i8_ && bytes <= (256 << 10);
+    if (call_imports_) HipCheck(cvmhip_import_bytes(in_stage_dev_, in_stage_host_, bytes, stream_), "copy input to device");
+    Launch();
+    ExportOutputs(seq_mode_ && use_seq_ && seq_sync_);
+  } catch (...) {
+    ok = false;
+  }
+  void* exec = nullptr;
+  const bool ended = cvmhip_capture_end(stream_, &exec) == CVMHIP_OK;
+  if (!ended || !ok || !exec) {
+    if (exec) cvmhip_graph_destroy(exec);
+    return false;
+  }
+  call_exec_ = exec;
+  call_refused_ = false;
+  return true;
+}
+
+void HipGraphRuntime::DropGraphs() {
+  for (void** exec : {&graph_exec_, &call_exec_}) {
+    if (*exec) cvmhip_graph_destroy(*exec);
+    *exec = nullptr;
+  }
+}
+
 const std::vector<const int32_t*>& HipGraphRuntime::FetchOutputs() {
   AllocOutputStage();
-  // One kernel behind the run writes every output, the sequence launches' status word and a ticket to pinned memory.
   const bool status = seq_ran_ && use_seq_ && seq_sync_;
   if (outputs_.size() <= CVMHIP_EXPORT_MAX) {
-    const void* src[CVMHIP_EXPORT_MAX];
-    void* dst[CVMHIP_EXPORT_MAX];
-    int64_t words[CVMHIP_EXPORT_MAX];
-    for (size_t k = 0; k < outputs_.size(); ++k) {
-      const uint32_t eid = entry_id(outputs_[k]);
-      src[k] = entry_ptr_[eid];
-      dst[k] = const_cast<int32_t*>(out_host_[k]);
-      words[k] = shape_size(shape_[eid]);
-    }
-    uint32_t* head = static_cast<uint32_t*>(out_stage_host_);
-    const uint32_t* word = status ? static_cast<uint32_t*>(seq_sync_) + (cvmhip_conv_seq_sync_bytes() / 4 - 64) : nullptr;
-    HipCheck(cvmhip_export_words(src, dst, words, static_cast<int>(outputs_.size()), word, word ? seq_error_host_ : nullptr,
-                                 static_cast<uint32_t*>(out_counter_), head, ++ticket_, stream_), "copy output");
-    AwaitTicket();
+    ExportOutputs(status);
+    ++ticket_;
   } else {
     for (size_t k = 0; k < outputs_.size(); ++k) {
       const uint32_t eid = entry_id(outputs_[k]);
@@ -1051,8 +1109,13 @@ const std::vector<const int32_t*>& HipGraphRuntime::FetchOutputs() {
                                stream_), "copy output");
     }
     RequestSequenceStatus();
-    HipCheck(cvmhip_stream_sync(stream_), "copy output");
   }
+  return CollectOutputs(status);
+}
+
+const std::vector<const int32_t*>& HipGraphRuntime::CollectOutputs(bool status) {
+  if (outputs_.size() <= CVMHIP_EXPORT_MAX) AwaitTicket();
+  else HipCheck(cvmhip_stream_sync(stream_), "copy output");
   in_stage_busy_ = false;
   if (seq_ran_) {
     CheckSequences(status);

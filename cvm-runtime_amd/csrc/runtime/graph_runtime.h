@@ -228,6 +228,10 @@ class HipGraphRuntime {
   bool data_stays_i8_ = false;     // fused: nothing reads `data` as int32, the row-window packing takes in_stage_dev_
   int32_t data_range_ = 0;         // clamp of the input
   uint32_t CheckData(const Shape& shape) const;   // the shape `data` must have; its entry
+  void ExportOutputs(bool status);
+  bool CaptureCall();
+  void DropGraphs();
+  const std::vector<const int32_t*>& CollectOutputs(bool status);
   void AllocOutputStage();
   void AwaitTicket();
   void AllocInputStage();
@@ -240,6 +244,9 @@ class HipGraphRuntime {
   std::vector<Exec> execs_;
   bool params_loaded_ = false;
   void* graph_exec_ = nullptr;
+  void* call_exec_ = nullptr;    // the same launches and the export of the outputs
+  bool call_imports_ = false;    // and, in front of them, the import of the input
+  bool call_refused_ = false;    // that could not be captured
   int graph_state_ = 0;  // 0 undecided, -1 eager for good, 1 before the first run, 2 ready to capture, 3 captured
 
   // Test and tuning hooks, read from the environment once, when the model is constructed (never on the

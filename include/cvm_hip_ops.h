@@ -179,12 +179,13 @@ int cvmhip_widen_clamp_i8(const void* src, int32_t* dst, int64_t count, int32_t 
  * so no signal between an engine and the kernels around it.
  * import: `bytes` from pinned host memory to the device (both 16-byte aligned; the last granule may be partial).
  * export: up to CVMHIP_EXPORT_MAX device arrays of 32-bit words (sources and destinations 16-byte aligned), then `*status`
- * (may be NULL) to status_host, then `ticket` to *flag_host, which the host may poll: when it reads the ticket, everything
- * before it has arrived.  `counter` is one zeroed device word, left zero. */
+ * (may be NULL) to status_host, then a ticket to *flag_host, which the host may poll: when it reads the ticket, everything
+ * before it has arrived.  `counter` is two device words, zeroed once; the second one is the last ticket, and every export
+ * stores the next one (counted on the device, so that an export can be part of a captured graph). */
 #define CVMHIP_EXPORT_MAX 8
 int cvmhip_import_bytes(void* dst, const void* src_host, size_t bytes, void* stream);
 int cvmhip_export_words(const void* const* src, void* const* dst_host, const int64_t* words, int count, const uint32_t* status,
-                        uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, uint32_t ticket, void* stream);
+                        uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, void* stream);
 /* Waits until *flag_host is `ticket`, and returns an error if the stream comes to its end without that. */
 int cvmhip_export_wait(const uint32_t* flag_host, uint32_t ticket, void* stream);
 int cvmhip_copy_h2d(void* dst, const void* src, size_t bytes, void* stream);
@@ -476,13 +477,12 @@ int cvmhip_resident_pack_filter(const int32_t* w, const int32_t* bias /* or NULL
 /* `places`: host buffer of cvmhip_resident_filter_bytes; *places_bytes of it then belong *places_off behind desc->filter */
 int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* desc, void* places, size_t* places_bytes, size_t* places_off);
 /* A whole call in that launch: the image comes from pinned host memory instead of `in`, the int32 result also goes to
- * pinned memory, and `ticket` is stored to *flag_host behind it (cvmhip_export_wait; *counter is a zeroed device word). */
+ * pinned memory, and the next ticket to *flag_host behind it (`counter` and tickets as for cvmhip_export_words). */
 typedef struct cvmhip_resident_call {
   const void* image_host;
   int32_t* out_host;
   uint32_t* counter;
   uint32_t* flag_host;
-  uint32_t ticket;
 } cvmhip_resident_call;
 int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_t lds_bytes, const cvmhip_resident_call* call /* or NULL */,
                            double ops, double bytes, void* stream);
