@@ -1,7 +1,6 @@
 #include "graph_runtime.h"
 
 #include <algorithm>
-#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -456,7 +455,6 @@ void HipGraphRuntime::ReadHooks() {
   hooks_.separable = plain && env("CVM_HIP_SEPARABLE") != "0";
   hooks_.fold_bias = env("CVM_HIP_FOLDBIAS") != "0";
   hooks_.graph = env("CVM_HIP_GRAPH") != "0";
-  hooks_.graph_forced = !env("CVM_HIP_GRAPH").empty();
   hooks_.seq = env("CVM_HIP_SEQ") != "0" && env("CVM_HIP_RESIDENT") != "1";
   hooks_.seq_forced = env("CVM_HIP_SEQ") == "1";
   hooks_.seq_chains = env("CVM_HIP_SEQ_CHAIN") != "0";
@@ -725,33 +723,6 @@ void HipGraphRuntime::LoadParams(const std::string& blob) {
     if (SeqNow()) CalibrateSequences();
     else seq_calibration_pending_ = true;
   }
-  ChooseSubmission();
-}
-
-// A graph is one submission, and saves the host what it costs to issue every launch (2.8 to 4 us each); but it reaches the
-// device about 7 us later than a launch does, and is a little slower on it where launches are long.  With the ends of a call
-// in the graph (CaptureCall) calls of CVMAPIInference took, as a graph and launch by launch: SSD-512 (7 us a launch) 259 and
-// 258 us, ResNet-50 at batch 1 (4.7 us) 266 and, by the host of the process, 264 to 302, at batch 12 378 and 390, at batch
-// 50 (17 us) 1007 and 1000, VGG-16 at batch 16 475 and 478, ResNet-20 at batch 64 (one launch of 40 us) 67 and 60.  So a
-// few calls are made when the model is loaded, and launches are issued one by one where a call has 15 us or more for each
-// of them.
-// CVM_HIP_GRAPH=0 or 1 names a form (and with CVM_HIP_SEQ=1 nothing runs before the first call).
-void HipGraphRuntime::ChooseSubmission() {
-  if (!fused_ || !hooks_.graph || hooks_.graph_forced || hooks_.seq_forced || GetInputPrecision() > 8) return;
-  const std::vector<int8_t> input(static_cast<size_t>(shape_size(InputShape())), 0);
-  std::vector<double> us;
-  for (int i = 0; i < 11; ++i) {
-    const auto begin = std::chrono::steady_clock::now();
-    SetDataI8(input.data(), InputShape());
-    seq_mode_ = SeqNow();
-    Launch();
-    FetchOutputs();
-    us.push_back(1e6 * std::chrono::duration<double>(std::chrono::steady_clock::now() - begin).count());
-  }
-  std::nth_element(us.begin(), us.begin() + 5, us.end());
-  int launches = 0;
-  LaunchCounts(&launches, nullptr, nullptr);
-  hooks_.graph = us[5] < 15.0 * launches;
 }
 
 // Layer-sequence launches pay for layers that are bound by latency and cost a little where layers are large, and steps that
@@ -842,8 +813,7 @@ void HipGraphRuntime::Launch() {
 
 // The launches of a run never change (shapes, pointers and attributes are
 // fixed at load time), so after one eager run they are captured into an
-// executable graph and replayed with a single submission, unless issuing them one
-// by one measured faster (ChooseSubmission).  Per-kernel timing
+// executable graph and replayed with a single submission.  Per-kernel timing
 // needs the eager path (its event pairs must not end up inside a graph);
 // CVM_HIP_GRAPH=0 keeps it for good.
 void HipGraphRuntime::Run() {
@@ -1057,9 +1027,12 @@ void HipGraphRuntime::ExportOutputs(bool status) {
                                static_cast<uint32_t*>(out_counter_), static_cast<uint32_t*>(out_stage_host_), stream_), "copy output");
 }
 
-// The run, the export behind it and a small input in front of it as one graph: as a launch of its own the export waits 7 us for the graph in front of it
-// to be seen to have ended, and a graph behind an import waits for that (ResNet-50 at batch 1: 273.5 us a call with both
-// outside, 268.7 with the export in the graph, 266 with an input of one piece in it as well).
+// The run, the export behind it and a small input in front of it as one graph: as a launch of its own the export waits 7 us
+// for the graph in front of it to be seen to have ended, and a graph behind an import waits for that (ResNet-50 at batch 1:
+// 273.5 us a call with both outside, 268.7 with the export in the graph, 266 with an input of one piece in it as well).
+// Issued launch by launch instead, calls take the same time where launches are few or long (ResNet-20 at batch 64 59.5 us and
+// 59.3 as a graph, SSD-512 258 and 259, VGG-16 at batch 16 478 and 475, ResNet-50 at batch 50 1000 and 1007) and more where the
+// host is hardly faster than the device (ResNet-50 at batch 1 264 to 302, by the process; batch 12 at 180 x 180 390 and 378).
 bool HipGraphRuntime::CaptureCall() {
   if (call_exec_) return true;
   if (call_refused_ || outputs_.size() > CVMHIP_EXPORT_MAX) return false;

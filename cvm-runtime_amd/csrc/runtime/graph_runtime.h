@@ -255,7 +255,7 @@ class HipGraphRuntime {
   // depthwise layers on the vector kernel, CVM_HIP_CONV=lds|wave, CVM_HIP_WAVECFG=<i> and
   // CVM_HIP_TILE="wm,wn" force an implicit-GEMM kernel, a configuration or a tile.
   struct Hooks {
-    bool fold_bias = true, fuse = true, graph = true, graph_forced = false, dw_on_mfma = true, seq = true, seq_forced = false, pool_fuse = true, head_pair = true, head_group = true, conv_group = true;
+    bool fold_bias = true, fuse = true, graph = true, dw_on_mfma = true, seq = true, seq_forced = false, pool_fuse = true, head_pair = true, head_group = true, conv_group = true;
     int conv_kernel = 0, wave_cfg = -1, tile_wm = 0, tile_wn = 0;
     // layer-sequence launches: CVM_HIP_SEQ_SPIN=<polls> patience of a wait at a layer boundary (0: every wait gives up at once)
     int seq_spin = 2000000;
@@ -336,7 +336,6 @@ class HipGraphRuntime {
   std::vector<bool> in_resident_;       // per plan_ index: inside such a run
   std::vector<GroupRun> groups_;
   std::vector<int> group_at_;           // per plan_ index: the group that starts there, or -1
-  void ChooseSubmission();              // a run as a graph or launch by launch: measures both
   void CalibrateSequences();            // measures a run with and without sequence launches, keeps the faster
   static int CountSequenceModel(int delta);    // models with sequence launches alive in this process, after the change
   bool SeqNow() const;                  // does the next run use sequence launches?
