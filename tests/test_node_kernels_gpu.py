@@ -45,3 +45,15 @@ def test_depthwise_planes(n, c, mult, h, w, strides, padding, dilation, dev):
     b = synth.tensor("planes", "b%d" % c, (c * mult,), -32768, 32768)
     got = hipops.conv2d(T(x, dev), T(wt, dev), T(b, dev), strides, padding, dilation, groups=c).cpu().numpy()
     assert np.array_equal(got, oracle.conv2d(x, wt, b, strides, padding, dilation, groups=c))
+
+
+@pytest.mark.parametrize("widths,outer,inner", [
+    ((1, 1, 4), 24564, 1),                          # a detector's rows
+    ((3,), 5, 7),
+    ((1,) * 8, 3, 1), ((2,) * 9, 257, 3),           # a whole group, one more
+    ((5, 0, 1, 300, 2), 11, 2),
+])
+def test_concat_groups(widths, outer, inner, dev):
+    xs = [synth.tensor("concat", "x%d-%d" % (i, w), (outer, max(w, 1), inner), -2 ** 31, 2 ** 31 - 1)[:, :w] for i, w in enumerate(widths)]
+    got = hipops.concatenate([T(x, dev) for x in xs], 1).cpu().numpy()
+    assert np.array_equal(got, np.concatenate(xs, 1))
