@@ -768,6 +768,10 @@ void HipGraphRuntime::FoldRequant() {
   }
 }
 
+bool HipGraphRuntime::ReadsI8(const PlanStep& st, const void* tensor) const {
+  return i8_ptr_[st.src] == tensor || (st.src2 != kNone && i8_ptr_[st.src2] == tensor);
+}
+
 // A depthwise 3x3 convolution whose only reader is the 1x1 convolution behind it becomes one launch with it, up to 512
 // channels (a workgroup goes through all of them one after the other: 1024 -> 1024 at 16 x 16 takes 9.7 us, as two launches
 // 8.1) and where the depthwise part is computed once or the layer is small: with more than 256 output channels several
@@ -782,9 +786,11 @@ void HipGraphRuntime::BuildSeparable() {
     if (p.kind != PlanStep::CONV || p.src != d.dst || p.src2 != kNone || !p.out_i8 || p.stem || p.nhwc || p.flat || p.ws || p.pool2 || p.pool3 ||
         p.kh != 1 || p.kw != 1 || p.sh != 1 || p.sw != 1 || p.ph != 0 || p.pw != 0)
       continue;
+    // readers are told by memory, not by entry: a flatten of a 1x1 map in front of a dense layer is an entry of its own
+    // over the same bytes
     bool only = true;
     for (size_t k = 0; k < plan_.size(); ++k)
-      only = only && (k == i || k == i + 1 || plan_[k].kind == PlanStep::NODE || (plan_[k].src != d.dst && plan_[k].src2 != d.dst));
+      only = only && (k == i || k == i + 1 || plan_[k].kind == PlanStep::NODE || !ReadsI8(plan_[k], i8_ptr_[d.dst]));
     if (!only || !cvmhip_separable_eligible(d.n, d.c, d.h, d.w, p.oc, d.sh, d.sw, d.ph, d.pw)) continue;
     if (d.c > 512 || (p.oc > 256 && static_cast<int64_t>(p.n) * p.h * p.w > 4096)) continue;
     if (((reinterpret_cast<uintptr_t>(d.bias) | reinterpret_cast<uintptr_t>(p.bias)) & 15) != 0) continue;

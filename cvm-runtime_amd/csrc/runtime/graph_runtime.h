@@ -323,6 +323,7 @@ class HipGraphRuntime {
     bool under_seq = false;             // shares steps with a sequence launch, which runs instead where sequences are in use
     double ops = 0, bytes = 0;
   };
+  bool ReadsI8(const PlanStep& st, const void* tensor) const;   // is the int8 tensor an operand of a step other than a NODE?
   void BuildSeparable();
   void RunSeparable(size_t step);
   bool InSeparable(size_t step) const { return plan_[step].separable || (step > 0 && plan_[step - 1].separable); }

@@ -165,8 +165,7 @@ HipGraphRuntime::ResidentDraft HipGraphRuntime::DraftResident(size_t first, size
     for (size_t k = 0; k < plan_.size(); ++k) {
       const PlanStep& st = plan_[k];
       if (st.kind == PlanStep::NODE || st.kind == PlanStep::PACK || st.kind == PlanStep::STEMPACK || st.stem) continue;
-      const bool reads = i8_ptr_[st.src] == key || (st.src2 != kNone && i8_ptr_[st.src2] == key);
-      if (!reads) continue;
+      if (!ReadsI8(st, key)) continue;
       if (k < first || k > last) *outside = true;
       else if (k > producer) *inside = true;
     }

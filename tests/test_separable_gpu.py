@@ -40,3 +40,26 @@ def test_depthwise_and_pointwise_in_one_launch(n, c, h, w, oc, stride, pad, mult
     m.close()
     assert counts[0] == counts[1] - 1, counts
     assert np.array_equal(got.astype(np.int32), og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))[0].ravel())
+
+
+def test_a_depthwise_result_that_a_dense_layer_reads_too_is_written(dev, monkeypatch):
+    """flatten of a 1x1 map shares the map's memory under another entry: the 1x1 convolution is not its only reader."""
+    g = graphgen.GraphBuilder("separable-flatten")
+    x = g.var("data", (2, 512, 3, 3), 8)
+    y = g.conv_relu_q(x, 512, 3, 1, 0, groups=512)
+    z = g.conv_relu_q(g.conv_relu_q(y, 512, 1), 40, 1)
+    d, _ = g.dense(g.flatten(y), 24)
+    js, pb = g.build([g.reshape(z, (2, 1, 40)), g.reshape(g.rshift(d, 9), (2, 1, 24))])
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "0")    # the layers behind would do without the tensor's memory
+    counts = []
+    for separable in ("1", "0"):
+        monkeypatch.setenv("CVM_HIP_SEPARABLE", separable)
+        m = runtime.HipModel(js, pb)
+        counts.append(m.launch_counts()[0])
+        for i in range(3):
+            data = synth.tensor("separable-flatten", "data%d" % i, (2, 512, 3, 3), -127, 127)
+            want = og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))
+            got = np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32)
+            assert np.array_equal(got, np.concatenate([v.reshape(2, -1) for v in want], axis=1).ravel())
+        m.close()
+    assert counts[0] == counts[1], counts
