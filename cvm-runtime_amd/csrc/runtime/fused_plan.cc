@@ -938,7 +938,7 @@ void HipGraphRuntime::BuildGroups() {
       const PlanStep& st = plan_[j];
       if (in_resident_[j] || InSeparable(j) || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
       bool reads_member = false;
-      for (uint32_t w : written) reads_member = reads_member || st.src == w || st.src2 == w;
+      for (uint32_t w : written) reads_member = reads_member || ReadsI8(st, i8_ptr_[w]);
       if (reads_member) break;
       table.resize((j - i + 1) * entry);
       int nb = 0;

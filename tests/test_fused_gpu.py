@@ -1109,3 +1109,26 @@ def test_flatten_act_i8(dev):
     eq(got, x.reshape(n, c, hw).transpose(0, 2, 1), "flatten_act_i8")
     with pytest.raises(CvmHipError):
         hipops.flatten_act_i8(hipops.pack_act_i8(T(x[:, :40], dev)), n, 40, hw)   # channels not a multiple of 32
+
+
+def test_a_dense_layer_does_not_share_a_launch_with_the_convolution_it_reads(dev, monkeypatch):
+    """flatten of a 1x1 map shares the map's memory under another entry: the two layers are not independent."""
+    g = graphgen.GraphBuilder("group-flatten")
+    x = g.var("data", (2, 512, 3, 3), 8)
+    y = g.conv_relu_q(x, 512, 3, 1, 0)
+    z, k = g.dense(g.flatten(y), 96)
+    z = g.rshift(g.relu(z), graphgen.shift_for(k))
+    z, _ = g.dense(z, 10)                          # reads it as int8
+    js, pb = g.build([z])
+    monkeypatch.setenv("CVM_HIP_SEQ", "0")
+    counts, models = [], []
+    for group in ("1", "0"):
+        monkeypatch.setenv("CVM_HIP_CONVGROUP", group)
+        models.append(runtime.HipModel(js, pb))
+        counts.append(models[-1].launch_counts()[0])
+    assert counts[0] == counts[1], counts          # before anything runs
+    data = synth.tensor("group-flatten", "data", (2, 512, 3, 3), -127, 127)
+    want = og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))[0].ravel()
+    for m in models:
+        assert np.array_equal(np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int32), want)
+        m.close()
