@@ -717,7 +717,7 @@ void HipGraphRuntime::BuildPlan() {
   // An int8 input that only row-window convolutions read is packed for them from the caller's bytes.
   data_stays_i8_ = false;
   if (GetInputPrecision() <= 8) {
-    const uint32_t de = entry_id(input_nodes_[GetInputIndex("data")], 0);
+    const uint32_t de = DataEntry();
     bool only_stems = !is_head[de];
     for (const PlanStep& st : plan_) {
       if (st.kind == PlanStep::STEMPACK) {
@@ -995,7 +995,7 @@ void HipGraphRuntime::RunStep(PlanStep& st) {
       Check(cvmhip_unpack_nhwc_i8(i8_ptr_[st.src], entry_ptr_[st.dst], st.n, st.c, st.h, stream_), "unpack");
       break;
     case PlanStep::STEMPACK:
-      if (data_stays_i8_ && entry_ptr_[st.src] == DataDevicePtr()) {
+      if (PacksStagedInput(st)) {
         Check(cvmhip_pack_stem_input_i8(in_stage_dev_, data_range_, static_cast<DeviceBuffer*>(st.aux.get())->ptr, st.n, st.c, st.h, st.w,
                                         st.kh, st.kw, st.sh, st.sw, st.ph, st.pw, stream_), "pack_stem_input_i8");
         break;

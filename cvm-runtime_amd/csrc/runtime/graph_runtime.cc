@@ -1097,11 +1097,6 @@ const std::vector<const int32_t*>& HipGraphRuntime::CollectOutputs(bool status) 
   return out_host_;
 }
 
-int32_t* HipGraphRuntime::DataDevicePtr() {
-  const int idx = GetInputIndex("data");
-  return entry_ptr_[entry_id(input_nodes_[idx], 0)];
-}
-
 void HipGraphRuntime::SyncStream() {
   const bool status = RequestSequenceStatus();
   HipCheck(cvmhip_stream_sync(stream_), "synchronise");

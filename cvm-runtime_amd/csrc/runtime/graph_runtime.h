@@ -144,7 +144,6 @@ class HipGraphRuntime {
   const std::vector<const int32_t*>& InferI8(const int8_t* host, const Shape& shape);
 
   // device-resident variants used to time Run() alone
-  int32_t* DataDevicePtr();
   void SyncStream();
 
   int NumOutputs() const { return static_cast<int>(outputs_.size()); }
@@ -227,6 +226,9 @@ class HipGraphRuntime {
   bool in_stage_ahead_ = false;    // in_stage_host_ holds an input that in_stage_dev_ has not seen (InferI8)
   bool data_stays_i8_ = false;     // fused: nothing reads `data` as int32, the row-window packing takes in_stage_dev_
   int32_t data_range_ = 0;         // clamp of the input
+  uint32_t DataEntry() const { return entry_id(input_nodes_[GetInputIndex("data")], 0); }
+  // does a STEMPACK step take the caller's bytes?  Told by entry: the storage of `data` may be lent to a later tensor
+  bool PacksStagedInput(const PlanStep& st) const { return data_stays_i8_ && st.src == DataEntry(); }
   uint32_t CheckData(const Shape& shape) const;   // the shape `data` must have; its entry
   void ExportOutputs(bool status);
   bool CaptureCall();

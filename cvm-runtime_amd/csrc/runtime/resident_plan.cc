@@ -106,7 +106,7 @@ bool HipGraphRuntime::ResidentEligible(const PlanStep& st) const {
   if (st.n < 1) return false;
   switch (st.kind) {
     case PlanStep::STEMPACK:
-      return data_stays_i8_ && entry_ptr_[st.src] == entry_ptr_[entry_id(input_nodes_[GetInputIndex("data")], 0)] && fits(st.c, st.h, st.w);
+      return PacksStagedInput(st) && fits(st.c, st.h, st.w);
     case PlanStep::SUM:
       return fits(st.c, 1, 1);
     case PlanStep::POOL:

@@ -1,5 +1,7 @@
 """The two ends of CVMAPIInference: the caller's bytes through the pinned buffer (pieces, odd sizes, the clamp) into the
 row-window or the plain layout, and the outputs with their ticket back -- against the oracle's graph executor."""
+import json
+
 import numpy as np
 import pytest
 
@@ -47,4 +49,27 @@ def test_many_calls_in_a_row(dev):
     for i in range(140):
         got = np.frombuffer(model.inference(inputs[i % 3].astype(np.int8).tobytes()), np.int8).astype(np.int32)
         assert np.array_equal(got, want[i % 3]), i
+    model.close()
+
+
+@pytest.mark.parametrize("resident", ["0", "1"])
+def test_the_storage_of_the_input_lent_to_a_later_tensor(resident, dev, monkeypatch):
+    """A second row-window convolution over a tensor in the place that `data` had takes that tensor, not the input."""
+    g = graphgen.GraphBuilder("io-lent")
+    x = g.var("data", (2, 3, 12, 12), 8)
+    y = g.conv_relu_q(x, 3, 3, 1, 1, relu=False)
+    t = g.unary("abs", y)
+    z = g.conv_relu_q(t, 32, 3, 1, 1)
+    js, pb = g.build([z])
+    doc = json.loads(js)
+    sid = doc["attrs"]["storage_id"][1]
+    sid[g._eid(t)] = sid[g._eid(x)]
+    js = json.dumps(doc)
+    monkeypatch.setenv("CVM_HIP_RESIDENT", resident)
+    model = runtime.HipModel(js, pb)
+    for call in range(3):
+        data = synth.tensor("io-lent", "x%d" % call, (2, 3, 12, 12), -127, 127)
+        want = og.run_graph(js, graphgen.load_params(pb), data)[0].ravel()
+        got = np.frombuffer(model.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want), "call %d" % call
     model.close()
