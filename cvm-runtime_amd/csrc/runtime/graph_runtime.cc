@@ -1062,7 +1062,10 @@ bool HipGraphRuntime::CaptureCall() {
   return true;
 }
 
+// A call returns when its ticket is seen, which the last kernel of the graph writes before the graph has ended: the stream is
+// waited for first.  (An error of that wait shows again at the next call on the stream.)
 void HipGraphRuntime::DropGraphs() {
+  if (graph_exec_ || call_exec_) cvmhip_stream_sync(stream_);
   for (void** exec : {&graph_exec_, &call_exec_}) {
     if (*exec) cvmhip_graph_destroy(*exec);
     *exec = nullptr;

@@ -316,3 +316,25 @@ def test_while_two_models_with_sequences_are_alive_both_use_one_launch_per_layer
     finally:
         if first is not None:
             first.close()
+
+
+def test_graphs_are_dropped_behind_calls_that_returned_by_their_ticket(dev):
+    """A model whose calls replay a graph changes its launch form between two calls, with nothing waited for but tickets."""
+    g, heads = graphgen.resnet50(8, width=16, size=64, classes=50, config_id="seq-drop")
+    js, pb = g.build(heads)
+    x = synth.tensor("seq-drop", "data", (8, 3, 64, 64), -127, 127).astype(np.int8)
+    want = _run(js, pb, x, "0")
+    os.environ["CVM_HIP_SEQ"] = "1"
+    try:
+        first = runtime.HipModel(js, pb)
+        for _ in range(3):
+            for _ in range(4):                     # eager, capture, replays as a call
+                assert np.array_equal(np.frombuffer(first.inference(x.tobytes()), np.int32), want)
+            second = runtime.HipModel(js, pb)      # sequence launches are off from here ...
+            for _ in range(4):
+                assert np.array_equal(np.frombuffer(first.inference(x.tobytes()), np.int32), want)
+            second.close()                         # ... and on again
+        assert first.launch_counts()[1] >= 1
+        first.close()
+    finally:
+        os.environ.pop("CVM_HIP_SEQ", None)
