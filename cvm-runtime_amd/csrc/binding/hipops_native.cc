@@ -29,6 +29,17 @@ void Check(int rc) {
   throw Raised();
 }
 
+// The C ABI's part of a call, without the interpreter's lock: a launch can block (a full queue), and other threads go on
+// meanwhile.  Whatever can raise has been evaluated before.
+template <typename F>
+void Launch(F&& f) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = f();
+  Py_END_ALLOW_THREADS
+  Check(rc);
+}
+
 const at::Tensor& Any(PyObject* o) {
   if (!THPVariable_Check(o)) {
     PyErr_SetString(PyExc_AssertionError, "int32 contiguous CUDA tensor required");
@@ -126,25 +137,31 @@ PyObject* Unary(PyObject* const* a) {
   const int64_t n = x.numel();
   const int p = static_cast<int>(Int(a[3])), q = static_cast<int>(Int(a[4]));
   void* s = Stream();
-  int rc = CVMHIP_ERR_ARG;
-  switch (Int(a[0])) {
-    case 0: rc = cvmhip_relu(xp, yp, n, s); break;
-    case 1: rc = cvmhip_cvm_clip(xp, yp, n, p, s); break;
-    case 2: rc = cvmhip_cvm_right_shift(xp, yp, n, p, q, s); break;
-    case 3: rc = cvmhip_cvm_left_shift(xp, yp, n, p, q, s); break;
-    case 4: rc = cvmhip_clip(xp, yp, n, p, q, s); break;
-    case 5: rc = cvmhip_abs(xp, yp, n, s); break;
-    case 6: rc = cvmhip_negative(xp, yp, n, s); break;
-    case 7: rc = cvmhip_cvm_precision(xp, yp, n, s); break;
-  }
-  Check(rc);
+  const long long op = Int(a[0]);
+  Launch([&] {
+    switch (op) {
+      case 0: return cvmhip_relu(xp, yp, n, s);
+      case 1: return cvmhip_cvm_clip(xp, yp, n, p, s);
+      case 2: return cvmhip_cvm_right_shift(xp, yp, n, p, q, s);
+      case 3: return cvmhip_cvm_left_shift(xp, yp, n, p, q, s);
+      case 4: return cvmhip_clip(xp, yp, n, p, q, s);
+      case 5: return cvmhip_abs(xp, yp, n, s);
+      case 6: return cvmhip_negative(xp, yp, n, s);
+      case 7: return cvmhip_cvm_precision(xp, yp, n, s);
+    }
+    return static_cast<int>(CVMHIP_ERR_ARG);
+  });
   return THPVariable_Wrap(std::move(y));
 }
 
 PyObject* Elemwise(PyObject* const* a) {
   const at::Tensor &x = Any(a[1]), &y = Any(a[2]);
   at::Tensor z = a[3] == Py_None ? at::empty_like(x) : Any(a[3]);
-  Check(cvmhip_elemwise(static_cast<int>(Int(a[0])), Ptr(x), Ptr(y), Ptr(z), x.numel(), Stream()));
+  const int op = static_cast<int>(Int(a[0]));
+  const int32_t *xp = Ptr(x), *yp = Ptr(y);
+  int32_t* zp = Ptr(z);
+  void* s = Stream();
+  Launch([&] { return cvmhip_elemwise(op, xp, yp, zp, x.numel(), s); });
   return THPVariable_Wrap(std::move(z));
 }
 
@@ -157,8 +174,14 @@ PyObject* Broadcast(PyObject* const* a) {
     shape[i] = std::max<int64_t>(dx >= 0 ? x.size(dx) : 1, dy >= 0 ? y.size(dy) : 1);
   }
   at::Tensor z = New(shape, x);
-  Check(cvmhip_broadcast(static_cast<int>(Int(a[0])), Ptr(x), x.sizes().data(), static_cast<int>(x.dim()), Ptr(y), y.sizes().data(),
-                         static_cast<int>(y.dim()), Ptr(z), shape.data(), nd, Stream()));
+  const int op = static_cast<int>(Int(a[0]));
+  const int32_t *xp = Ptr(x), *yp = Ptr(y);
+  int32_t* zp = Ptr(z);
+  void* s = Stream();
+  Launch([&] {
+    return cvmhip_broadcast(op, xp, x.sizes().data(), static_cast<int>(x.dim()), yp, y.sizes().data(), static_cast<int>(y.dim()), zp,
+                            shape.data(), nd, s);
+  });
   return THPVariable_Wrap(std::move(z));
 }
 
@@ -175,9 +198,14 @@ PyObject* Conv2d(PyObject* const* a) {
   at::Tensor y = New({n, oc, oh, ow}, x);
   at::Tensor ws = Scratch(cvmhip_conv2d_workspace_bytes(n, ic, h, wd, oc, kh, kw, groups), x);
   ApplyConvTuning();
-  Check(cvmhip_conv2d(Ptr(x), Ptr(w), Ptr(a[2]), Ptr(y), n, ic, h, wd, oc, kh, kw, static_cast<int>(st[0]), static_cast<int>(st[1]),
-                      static_cast<int>(pd[0]), static_cast<int>(pd[1]), static_cast<int>(dl[0]), static_cast<int>(dl[1]), groups,
-                      ws.data_ptr(), static_cast<size_t>(ws.numel()), Stream()));
+  const int32_t *xp = Ptr(x), *wp = Ptr(w), *bp = Ptr(a[2]);
+  int32_t* yp = Ptr(y);
+  void* s = Stream();
+  Launch([&] {
+    return cvmhip_conv2d(xp, wp, bp, yp, n, ic, h, wd, oc, kh, kw, static_cast<int>(st[0]), static_cast<int>(st[1]),
+                         static_cast<int>(pd[0]), static_cast<int>(pd[1]), static_cast<int>(dl[0]), static_cast<int>(dl[1]), groups,
+                         ws.data_ptr(), static_cast<size_t>(ws.numel()), s);
+  });
   return THPVariable_Wrap(std::move(y));
 }
 
@@ -188,8 +216,11 @@ PyObject* Dense(PyObject* const* a) {
   at::Tensor y = New({m, n}, x);
   at::Tensor ws = Scratch(cvmhip_dense_workspace_bytes(m, k, n), x);
   ApplyConvTuning();
-  Check(cvmhip_dense(Ptr(x), Ptr(w), Ptr(a[2]), Ptr(y), m, k, n, static_cast<int>(Int(a[3])), ws.data_ptr(),
-                     static_cast<size_t>(ws.numel()), Stream()));
+  const int32_t *xp = Ptr(x), *wp = Ptr(w), *bp = Ptr(a[2]);
+  int32_t* yp = Ptr(y);
+  const int bits = static_cast<int>(Int(a[3]));
+  void* s = Stream();
+  Launch([&] { return cvmhip_dense(xp, wp, bp, yp, m, k, n, bits, ws.data_ptr(), static_cast<size_t>(ws.numel()), s); });
   return THPVariable_Wrap(std::move(y));
 }
 
@@ -206,8 +237,13 @@ PyObject* MaxPool2d(PyObject* const* a) {
   const int64_t ow = FloorDiv(w + 2 * pd[1] - k[1] + (ceil ? st[1] - 1 : 0), st[1]) + 1;
   at::Tensor y = New({x.size(0), x.size(1), oh, ow}, x);
   auto i = [](int64_t v) { return static_cast<int>(v); };
-  Check(cvmhip_max_pool2d(Ptr(x), Ptr(y), i(x.size(0)), i(x.size(1)), i(h), i(w), i(oh), i(ow), i(k[0]), i(k[1]), i(st[0]), i(st[1]),
-                          i(pd[0]), i(pd[1]), Stream()));
+  const int32_t* xp = Ptr(x);
+  int32_t* yp = Ptr(y);
+  void* s = Stream();
+  Launch([&] {
+    return cvmhip_max_pool2d(xp, yp, i(x.size(0)), i(x.size(1)), i(h), i(w), i(oh), i(ow), i(k[0]), i(k[1]), i(st[0]), i(st[1]),
+                             i(pd[0]), i(pd[1]), s);
+  });
   return THPVariable_Wrap(std::move(y));
 }
 
@@ -216,8 +252,14 @@ PyObject* Reduce(PyObject* const* a) {
   const at::Tensor& x = Any(a[1]);
   const auto ys = Ints(a[2]), ax = Ints(a[3]);
   at::Tensor y = New(ys, x);
-  Check(cvmhip_reduce(static_cast<int>(Int(a[0])), Ptr(x), x.sizes().data(), static_cast<int>(x.dim()), Ptr(y), y.numel(),
-                      ax.empty() ? nullptr : ax.data(), static_cast<int>(ax.size()), static_cast<int>(Int(a[4])), Stream()));
+  const int op = static_cast<int>(Int(a[0])), exclude = static_cast<int>(Int(a[4]));
+  const int32_t* xp = Ptr(x);
+  int32_t* yp = Ptr(y);
+  void* s = Stream();
+  Launch([&] {
+    return cvmhip_reduce(op, xp, x.sizes().data(), static_cast<int>(x.dim()), yp, y.numel(), ax.empty() ? nullptr : ax.data(),
+                         static_cast<int>(ax.size()), exclude, s);
+  });
   return THPVariable_Wrap(std::move(y));
 }
 
@@ -227,8 +269,11 @@ PyObject* GetValidCounts(PyObject* const* a) {
   const int b = static_cast<int>(x.size(0)), n = static_cast<int>(x.size(1)), k = static_cast<int>(x.size(2));
   at::Tensor vc = New({b}, x), y = at::empty_like(x);
   at::Tensor ws = Scratch(cvmhip_get_valid_counts_workspace_bytes(b, n), x);
-  Check(cvmhip_get_valid_counts(Ptr(x), Ptr(vc), Ptr(y), b, n, k, static_cast<int32_t>(Int(a[1])), ws.data_ptr(),
-                                static_cast<size_t>(ws.numel()), Stream()));
+  const int32_t* xp = Ptr(x);
+  int32_t *cp = Ptr(vc), *yp = Ptr(y);
+  const int32_t threshold = static_cast<int32_t>(Int(a[1]));
+  void* s = Stream();
+  Launch([&] { return cvmhip_get_valid_counts(xp, cp, yp, b, n, k, threshold, ws.data_ptr(), static_cast<size_t>(ws.numel()), s); });
   PyObject* v = THPVariable_Wrap(std::move(vc));
   PyObject* r = THPVariable_Wrap(std::move(y));
   PyObject* t = PyTuple_Pack(2, v, r);
@@ -245,8 +290,12 @@ PyObject* NonMaxSuppression(PyObject* const* a) {
   int v[7];
   for (int i = 0; i < 7; ++i) v[i] = i == 1 ? PyObject_IsTrue(a[4]) : static_cast<int>(Int(a[3 + i]));
   at::Tensor ws = Scratch(cvmhip_nms_workspace_bytes(b, n, k), x);
-  Check(cvmhip_non_max_suppression(Ptr(x), Ptr(a[1]), Ptr(a[2]), b, n, k, v[6], v[0], v[2], v[4], v[5], v[3], v[1], ws.data_ptr(),
-                                   static_cast<size_t>(ws.numel()), Stream()));
+  int32_t *xp = Ptr(x), *cp = Ptr(a[1]), *yp = Ptr(a[2]);
+  void* s = Stream();
+  Launch([&] {
+    return cvmhip_non_max_suppression(xp, cp, yp, b, n, k, v[6], v[0], v[2], v[4], v[5], v[3], v[1], ws.data_ptr(),
+                                      static_cast<size_t>(ws.numel()), s);
+  });
   Py_INCREF(a[2]);
   return a[2];
 }

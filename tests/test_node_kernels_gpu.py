@@ -1,5 +1,9 @@
 """Kernels of the int32 operator contract at the edges of their splits, against the oracle: long reductions, operand packing
 of a convolution, depthwise planes."""
+import sys
+import threading
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -57,3 +61,34 @@ def test_concat_groups(widths, outer, inner, dev):
     xs = [synth.tensor("concat", "x%d-%d" % (i, w), (outer, max(w, 1), inner), -2 ** 31, 2 ** 31 - 1)[:, :w] for i, w in enumerate(widths)]
     got = hipops.concatenate([T(x, dev) for x in xs], 1).cpu().numpy()
     assert np.array_equal(got, np.concatenate(xs, 1))
+
+
+def test_other_threads_run_during_an_operator_call(dev):
+    """The interpreter's lock is free while the library issues a launch: with switching by time all but off, another
+    thread gets on only if the calls let it."""
+    x = T(np.arange(64, dtype=np.int32), dev)
+    y = hipops.relu(x)   # written again by every call: an allocation or a release of its own could let go of the lock
+    seen, started, stop = [0], threading.Event(), threading.Event()
+
+    def other():
+        started.set()
+        while not stop.is_set():
+            seen[0] += 1
+            time.sleep(0)
+    t = threading.Thread(target=other)
+    interval = sys.getswitchinterval()
+    t.start()
+    started.wait()
+    sys.setswitchinterval(1000.0)
+    try:
+        before = seen[0]
+        for _ in range(5000):
+            hipops.relu(x, y)
+            if seen[0] >= before + 20:   # (a wait that began before the interval was set ends once more)
+                break
+        moved = seen[0] - before
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        t.join()
+    assert moved >= 20
