@@ -4,7 +4,8 @@ Every .hip / .cc file under csrc/ is compiled with hipcc for gfx950 and linked
 into cvm-runtime_amd/libcvm_runtime_hip.so, the one library that exports both
 the operator-level C ABI (include/cvm_hip_ops.h) and the model-level C ABI
 (include/cvm_c_api.h).  csrc/binding/ becomes _hipops_native.so, the native half of
-hipops.py; it is the only object that knows torch, and the library does not need it.
+hipops.py; it is the only object that knows torch, and the library does not need it: without
+torch's headers it is left out, and hipops goes through ctypes.
 """
 import glob
 import importlib.util
@@ -42,10 +43,20 @@ def _compile(src):
 
 
 def _build_binding():
-    torch = os.path.dirname(importlib.util.find_spec("torch").origin)
+    """The binding, where torch is installed with its headers; the library does without, and hipops then uses ctypes."""
+    if os.path.exists(BINDING):
+        os.remove(BINDING)   # never one that belongs to another build of the library
+    spec = importlib.util.find_spec("torch")
+    torch = os.path.dirname(spec.origin) if spec else ""
+    python = sysconfig.get_paths()["include"]
+    for need in (os.path.join(torch, "include", "torch", "csrc", "autograd", "python_variable.h"),
+                 os.path.join(torch, "include", "c10", "hip", "HIPStream.h"), os.path.join(python, "Python.h")):
+        if not os.path.exists(need):
+            sys.stderr.write("no %s: %s is left out\n" % (os.path.basename(need), os.path.basename(BINDING)))
+            return
     inc = [os.path.join(torch, "include"), os.path.join(torch, "include", "torch", "csrc", "api", "include"),
-           os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"), sysconfig.get_paths()["include"]]
-    cmd = (["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"] +
+           os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"), python]
+    cmd = ([HIPCC, "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-x", "c++"] +
            ["-I" + d for d in inc] + [os.path.join(CSRC, "binding", "hipops_native.cc"), "-o", BINDING, "-L" + HERE,
             "-l:" + os.path.basename(LIB), "-L" + os.path.join(torch, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
             "-lc10_hip", "-Wl,-rpath,$ORIGIN"])

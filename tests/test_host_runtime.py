@@ -101,3 +101,18 @@ def test_without_a_gpu_loading_a_model_fails_loudly(capfd):
     with pytest.raises(runtime.CVMError):
         runtime.HipModel(js, pb)
     capfd.readouterr()
+
+
+def test_the_build_does_without_torch(monkeypatch, tmp_path):
+    """No torch, no binding: the step is left out, and a binding of an earlier build does not stay behind."""
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("cvm_build_under_test", os.path.join(ROOT, "cvm-runtime_amd", "build.py"))
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+    stale = tmp_path / "_hipops_native.so"
+    stale.write_bytes(b"")
+    b.BINDING = str(stale)
+    b.subprocess = None                                   # nothing is compiled
+    monkeypatch.setattr(b.importlib.util, "find_spec", lambda name: None)
+    b._build_binding()
+    assert not stale.exists()

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+import cvm_runtime_amd
 import oracle
 from cvm_runtime_amd import hipops, synth
 
@@ -396,3 +397,32 @@ def test_argument_errors_are_reported_not_launched(dev):
     with pytest.raises(CvmHipError):
         hipops.non_max_suppression(big, T(np.ones((1,), np.int32), dev), torch.empty_like(big), iou_threshold=45)
     hipops.non_max_suppression(big, T(np.ones((1,), np.int32), dev), torch.empty_like(big), iou_threshold=45, top_k=100)
+
+
+def test_operators_without_the_native_binding(dev, monkeypatch, tmp_path):
+    """An installation that could not build the binding: the same calls through ctypes, announced by a warning."""
+    rng = np.random.default_rng(5)
+
+    def i32(*shape, lo=-127, hi=127):
+        return torch.from_numpy(rng.integers(lo, hi + 1, shape, dtype=np.int32)).to(dev)
+    x, w, b = i32(2, 8, 9, 7), i32(12, 8, 3, 3), i32(12, lo=-9999, hi=9999)
+    rows = i32(1, 40, 6, lo=0, hi=60)
+
+    def calls():
+        y = hipops.conv2d(x, w, b, (2, 1), (1, 1))
+        counts, kept = hipops.get_valid_counts(rows, 10)
+        out = torch.zeros_like(kept)
+        return [y, hipops.relu(y), hipops.cvm_clip(y, 8), hipops.cvm_right_shift(y, 8, 6), hipops.cvm_left_shift(x, 16, 3), hipops.clip(y, -5, 9),
+                hipops.abs_(x), hipops.negative(x), hipops.cvm_precision(x), hipops.elemwise("elemwise_sub", x, x), hipops.dense(w.view(12, 72), w.view(12, 72)),
+                hipops.broadcast("broadcast_max", x, x[:, :, :1, :].contiguous()), hipops.max_pool2d(x, (3, 2), (2, 2), (1,), True),
+                hipops.reduce("sum", x, (1, 3)), hipops.reduce("max", x, (), True), counts, kept,
+                hipops.non_max_suppression(kept, counts, out, 45, True, 30)]
+    want = calls()
+    monkeypatch.setattr(cvm_runtime_amd, "_native", None)
+    monkeypatch.setattr(cvm_runtime_amd, "NATIVE_PATH", str(tmp_path / "none.so"))
+    with pytest.warns(UserWarning, match="ctypes"):
+        got = calls()
+    for u, v in zip(want, got):
+        assert torch.equal(u, v)
+    with pytest.raises(cvm_runtime_amd.CvmHipError):
+        hipops.cvm_clip(x, 0)
