@@ -3090,6 +3090,8 @@ size_t conv_seq_layer_bytes() { return sizeof(SeqLayer); }
 int conv_seq_shares() { return SEQ_SHARES; }
 size_t conv_seq_sync_bytes() { return (SEQ_SHARES + 1) * SEQ_SYNC_WORDS * sizeof(unsigned); }
 
+constexpr int64_t SEQ_LEAVE_TILES = 400;   // tiles of 128 x 256: see conv_seq_layer
+
 // Fills entry `index` of a host copy of the table.  CVMHIP_ERR_ARG with "not eligible" when this convolution
 // cannot be one layer of a sequence (the caller then launches it on its own).
 int conv_seq_layer(void* table, int index, const int8_t* xp, const int8_t* wp, void* out, ConvGeom g, const Epilogue& ep_in) {
@@ -3108,9 +3110,13 @@ int conv_seq_layer(void* table, int index, const int8_t* xp, const int8_t* wp, v
       if (c->st[t].mul != 1) return arg_error("conv_seq_layer: not eligible (a requantisation chain that multiplies)");
   }
   const ConvTuning tune = t_conv_tuning;
-  // a layer that fills the chip several times over is faster as a launch of the large-tile kernel than as a layer of a
-  // sequence (whose tile is the wavefront kernel's); a run of layers ends there
-  if (tune.kernel == CONV_KERNEL_AUTO && tune.wave_cfg < 0 && choose_big_cfg(g) >= 0)
+  // A layer leaves a sequence only where it is large: choose_big_cfg compares the ring with a launch of the wavefront kernel,
+  // while here the ring launch also costs the cut (a second sequence launch, a join or a chain lost).  Measured on ResNet-50
+  // with layers leaving from 144, 200, 256 and 400 tiles on, in us a step: 16 images of 224 x 224 341, 331, 332, 331; 24 images
+  // 534, 511, 506, 506; 32 images 585, 554, 543, 543; 48 images 779, 783, 784, 780; 48 of 192 x 192 600, 569, 556, 556.  Only
+  // at 40 images did the cuts gain (609, 631, 617, 617), and there one launch per layer (620) is within what the load-time
+  // comparison asks for.  No layer of these has 400 tiles.
+  if (tune.kernel == CONV_KERNEL_AUTO && tune.wave_cfg < 0 && choose_big_cfg(g) >= 0 && big_cfg_blocks(kBigCfgs[1], g) >= SEQ_LEAVE_TILES)
     return arg_error("conv_seq_layer: not eligible (a layer for the large-tile kernel)");
   SeqLayer& L = reinterpret_cast<SeqLayer*>(table)[index];
   memset(&L, 0, sizeof(L));

@@ -137,3 +137,19 @@ def test_switched_off_and_forced_configurations(lib):
     finally:
         lib.cvmhip_set_seq_chains(1)
         lib.cvmhip_set_seq_layer_config(-1, -1)
+
+
+@pytest.mark.parametrize("n,ic,hw,oc,k,stride,stays", [
+    (16, 512, 28, 256, 1, 1, True),     # ResNet-50 at batch 16: 196 and 200 of the ring kernel's smaller tiles
+    (16, 512, 28, 1024, 1, 2, True),
+    (199, 512, 16, 256, 1, 1, True),    # 398 and 400 of its 128 x 256 tiles
+    (200, 512, 16, 256, 1, 1, False),
+    (200, 256, 16, 256, 1, 1, True),    # K below the ring kernel's range
+])
+def test_which_layers_are_left_to_the_ring_kernel(lib, n, ic, hw, oc, k, stride, stays):
+    buf = ctypes.create_string_buffer(lib.cvmhip_conv_seq_layer_bytes())
+    chain = hipops.Chain()
+    chain.count = 0
+    rc = lib.cvmhip_conv_seq_layer(buf, 0, X, W, None, ctypes.byref(chain), None, ctypes.byref(chain), 0x80000000, n, ic, hw, hw, oc,
+                                   k, k, stride, stride, 0, 0, 1, 1)
+    assert (rc == 0) == stays
