@@ -35,6 +35,21 @@ def test_conv_operand_packing(n, c, h, w, oc, k, dev):
     assert np.array_equal(got, oracle.conv2d(x, wt, None, (1, 1), (k // 2, k // 2)))
 
 
+@pytest.mark.parametrize("m,k,n", [
+    (1, 17, 5), (3, 31, 40),       # a granule that ends inside the channels, one that is all padding
+    (33, 64, 32), (70, 100, 7),
+    (5, 1023, 33),                 # rows that do not start on 16 bytes
+    (1, 16416, 4100),              # a filter of so many dwords that the workgroups that pack it go round
+])
+def test_dense_operand_packing(m, k, n, dev):
+    x = synth.tensor("rows", "x%d" % k, (m, k), -127, 127)
+    wt = synth.tensor("rows", "w%d" % k, (n, k), -127, 127)
+    got = hipops.dense(T(x, dev), T(wt, dev)).cpu().numpy()
+    assert np.array_equal(got, oracle.dense(x, wt, None))
+    packed = hipops.unpack_act_i8(hipops.pack_act_i8(T(x.reshape(m, k, 1, 1), dev)), m, k, 1, 1).cpu().numpy()
+    assert np.array_equal(packed.reshape(m, k), x)
+
+
 @pytest.mark.parametrize("n,c,mult,h,w,strides,padding,dilation", [
     (1, 2, 1, 3, 3, (1, 1), (0, 0), (1, 1)),       # one output
     (2, 3, 2, 5, 7, (1, 1), (1, 1), (1, 1)),       # a channel multiplier; rows that are not whole quads
