@@ -772,10 +772,33 @@ bool HipGraphRuntime::ReadsI8(const PlanStep& st, const void* tensor) const {
   return i8_ptr_[st.src] == tensor || (st.src2 != kNone && i8_ptr_[st.src2] == tensor);
 }
 
-// A depthwise 3x3 convolution whose only reader is the 1x1 convolution behind it becomes one launch with it, up to 512
-// channels (a workgroup goes through all of them one after the other: 1024 -> 1024 at 16 x 16 takes 9.7 us, as two launches
-// 8.1) and where the depthwise part is computed once or the layer is small: with more than 256 output channels several
-// workgroups repeat it, which up to 4096 pixels is hidden behind idle compute units.
+namespace {
+
+// Is the launch of both layers faster than the two, by its output pixels (all images)?  It saves a launch and the depthwise
+// tensor's way through memory; what it costs grows with the pixels once the chip is full:
+//   * more than 256 output channels: several workgroups repeat the depthwise part, hidden behind idle compute units up to 4096
+//     pixels; beyond 512 channels in, one workgroup goes through too many in a row (1024 -> 1024 at 16 x 16: 9.7 us against 8.1);
+//   * a number of channel tiles that is no power of two leaves wavefronts idle in the 1x1 part: 96 -> 96 at 49 K pixels 44.4 us
+//     as two launches and 41.0 as one, at 131 K 80.6 and 82.6, at 524 K 287 and 308; 160 -> 160 at 49 K 59.9 and 59.7;
+//   * more channels out than in make the results' stores, which a workgroup has nothing else to hide behind, most of it: 32 -> 64
+//     at 131 K pixels 54.1 and 53.9, at 1 M 310 and 334; 64 -> 128 at 131 K 83.9 and 83.8, at 524 K 310 and 325; 128 -> 256
+//     stride 2 at 131 K 225 and 218, at 262 K 455 and 474; 32 -> 128 at 65 K 47.9 and 48.2, at 131 K 71 and 78;
+//   * as many or fewer, at 1 M pixels: 128 -> 64 556 and 508, 32 -> 32 201 and 182, 64 -> 64 385 and 374, 128 -> 128 810 and 821
+//     (at 524 K 389 and 378).
+// (Each with the packing and the pool around it.)
+bool SeparableGains(int c, int oc, int64_t pixels) {
+  if (c > 512) return false;
+  if (oc > 256) return pixels <= 4096;
+  const int tiles = (oc + 31) / 32;
+  if ((tiles & (tiles - 1)) != 0 || oc > 2 * c) return pixels <= 49152;
+  return pixels <= (oc > c ? 131072 : 1048576);
+}
+
+}  // namespace
+
+// A depthwise 3x3 convolution whose only reader is the 1x1 convolution behind it becomes one launch with it where that gains.
+// The pair may cut a layer sequence that the 1x1 layer would begin: with 2 to 8 layers behind it, at 1 to 32 images of 14 x 14
+// to 56 x 56, the pair and what is left were 0.4 to 6 us ahead of the depthwise launch and the longer sequence.
 void HipGraphRuntime::BuildSeparable() {
   if (!hooks_.separable) return;
   for (size_t i = 0; i + 1 < plan_.size(); ++i) {
@@ -792,7 +815,7 @@ void HipGraphRuntime::BuildSeparable() {
     for (size_t k = 0; k < plan_.size(); ++k)
       only = only && (k == i || k == i + 1 || plan_[k].kind == PlanStep::NODE || !ReadsI8(plan_[k], i8_ptr_[d.dst]));
     if (!only || !cvmhip_separable_eligible(d.n, d.c, d.h, d.w, p.oc, d.sh, d.sw, d.ph, d.pw)) continue;
-    if (d.c > 512 || (p.oc > 256 && static_cast<int64_t>(p.n) * p.h * p.w > 4096)) continue;
+    if (!SeparableGains(d.c, p.oc, static_cast<int64_t>(p.n) * p.h * p.w)) continue;
     if (((reinterpret_cast<uintptr_t>(d.bias) | reinterpret_cast<uintptr_t>(p.bias)) & 15) != 0) continue;
     auto buf = std::make_shared<DeviceBuffer>();
     Check(cvmhip_alloc(&buf->ptr, cvmhip_separable_filter_bytes(d.c)), "separable filter");

@@ -63,3 +63,23 @@ def test_a_depthwise_result_that_a_dense_layer_reads_too_is_written(dev, monkeyp
             assert np.array_equal(got, np.concatenate([v.reshape(2, -1) for v in want], axis=1).ravel())
         m.close()
     assert counts[0] == counts[1], counts
+
+
+@pytest.mark.parametrize("n,c,hw,oc,fused", [
+    (3, 96, 128, 96, True), (4, 96, 128, 96, False),          # 48 K and 64 K pixels, three channel tiles
+    (1, 32, 128, 128, True), (4, 32, 128, 128, False),        # four times the channels
+    (8, 64, 128, 128, True), (9, 64, 128, 128, False),        # twice: 128 K pixels and more
+    (4, 32, 512, 32, True), (5, 32, 512, 32, False),          # as many: 1 M pixels and more
+])
+def test_pairs_of_many_pixels_stay_two_launches(n, c, hw, oc, fused, dev, monkeypatch):
+    g = graphgen.GraphBuilder("separable-rule-%d-%d" % (c, oc))
+    z = g.conv_relu_q(g.conv_relu_q(g.var("data", (n, c, hw, hw), 8), c, 3, 1, 1, groups=c), oc, 1)
+    js, pb = g.build([g.conv_relu_q(z, 40, 1)])
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "1")
+    counts = []
+    for separable in ("1", "0"):
+        monkeypatch.setenv("CVM_HIP_SEPARABLE", separable)
+        m = runtime.HipModel(js, pb)
+        counts.append(m.launch_counts()[0])
+        m.close()
+    assert counts[1] - counts[0] == fused, counts
