@@ -732,11 +732,11 @@ static int nms_check_args(const int32_t* x, const int32_t* valid_count, const in
   if (iou_threshold <= 0) return arg_error("non_max_suppression.iou_threshold must be positive");
   if (coord_start < 0 || coord_start + 4 > k || score_index < 0 || score_index >= k || id_index >= k)
     return arg_error("non_max_suppression indices");
-  // 2^24 is the largest dimension the reference's shape check accepts (src/runtime/infer_attr.cc).  Ranking is a sort, but
-  // the greedy walk over the candidate rows (the first top_k in sorted order, or all valid rows) compares every kept
-  // row with every later one, as the reference's does: one workgroup needs about 0.8 s for 100 000 candidate rows of
-  // which most are kept, and the time grows with the square.  More than 2^18 candidates (about 5 s at worst) are
-  // refused rather than launched as a kernel that runs for minutes.
+  // 2^24 is the largest dimension the reference's shape check accepts (src/runtime/infer_attr.cc).  The greedy walk compares
+  // every row with the kept rows of its class in front of it, and when all candidates (the first top_k in sorted order, or all
+  // valid rows) are of one class and stay, one workgroup does that: 5 000 rows take 3 ms, 25 000 0.13 s, 100 000 2.3 s (20
+  // classes: 0.2, 0.8 and about 1 ms), growing with the square.  More than 2^18 candidates (some 16 s at worst) are refused
+  // rather than launched as a kernel that runs for minutes.
   if (n > (1 << 24)) return arg_error("non_max_suppression: more than 2^24 anchors per batch");
   if (n > (1 << 18) && !(topk >= 0 && topk <= (1 << 18)))
     return arg_error("non_max_suppression: more than 2^18 candidate rows per batch (set top_k to bound the greedy walk)");

@@ -38,3 +38,25 @@ def test_tile_128_by_128(n, ic, h, w, oc, k, stride, residual, dev):
     got = hipops.unpack_act_i8(out, n, oc, oh, ow)
     torch.cuda.synchronize()
     assert np.array_equal(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("n,ic,h,w,oc", [
+    (9, 64, 32, 32, 256),     # whole tiles of pixels, the least that takes the tile
+    (11, 64, 30, 30, 200),    # pixels and channels that end inside a tile
+])
+@pytest.mark.parametrize("multiply", [False, True])
+def test_tile_128_by_128_with_a_fused_pool(n, ic, h, w, oc, multiply, dev):
+    cid = "tile128-pool-%d" % n
+    x = synth.tensor(cid, "x", (n, ic, h, w), -127, 127)
+    wt = synth.tensor(cid, "w", (oc, ic, 3, 3), -127, 127)
+    b = synth.tensor(cid, "b", (oc,), -32768, 32768)
+    v = oracle.conv2d(x, wt, b, (1, 1), (1, 1), (1, 1), 1)
+    chain = [("cvm_right_shift", 8, 9)]
+    if multiply:   # a chain that falls as its input grows: the maximum comes behind it
+        v, chain = -3 * v, [("mul", -3), ("cvm_right_shift", 8, 11)]
+    ref = oracle.max_pool2d(oracle.cvm_right_shift(v, *chain[-1][1:]), (2, 2), (2, 2), (0, 0), False)
+    out = hipops.conv2d_pool2_i8(hipops.pack_act_i8(T(x, dev)), n, ic, h, w, hipops.pack_weights(T(wt, dev)), oc, 3, 3, T(b, dev),
+                                 hipops.chain(*chain), padding=(1, 1))
+    got = hipops.unpack_act_i8(out, n, oc, h // 2, w // 2)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), ref)

@@ -60,7 +60,7 @@ def test_small_maps_stay_in_lds(case, batch, dev, monkeypatch):
 
 
 def test_images_in_rounds(dev):
-    """More images than compute units, and a partial last group of eight for the workgroups that fetch the filters."""
+    """More images than compute units: workgroups take a second image."""
     g, heads = _net(CASES[0], 261)
     js, pb = g.build(heads)
     x = synth.tensor("resident-rounds", "data", (261, 3, 16, 16), -127, 127).astype(np.int8)
