@@ -2762,8 +2762,7 @@ static int64_t big_cfg_blocks(const BigCfg& c, const ConvGeom& g) {
   const int bm = c.wgm * c.tm * 32, bn = c.wgn * c.tn * 32;
   return (int64_t)((g.OC + bm - 1) / bm) * ((g.P + bn - 1) / bn);
 }
-// The largest tile that does not reach past the layer's channels and still gives most compute units a tile; -1 when
-// the layer is too small for this kernel (fewer than 144 tiles of the smallest fitting shape, or a short K).
+// Which tile of the large-tile kernel a layer takes; -1 where the wavefront kernel is the faster.
 static int choose_big_cfg(const ConvGeom& g) {
   // K >= 512: with K = 256 (the 1x1 layers of a ResNet's second stage) the ring never fills and the wavefront
   // kernel is faster (7.5 us against 11.6 for 256 -> 128 channels over 16 x 56 x 56 pixels)
@@ -2772,12 +2771,20 @@ static int choose_big_cfg(const ConvGeom& g) {
   // 1.05-1.2 for the wavefront kernel); the 256 x 256 tile (one workgroup, 1.4) and the 64 x 512 one (0.65, below the
   // wavefront kernel's 0.96 on 64 -> 64 channels) are kept for forced use
   if (g.OC <= 64) return -1;
-  // From 144 tiles on, nine of sixteen compute units, the ring beats the wavefront kernel's own operand streams (ResNet-50 at
-  // batch 50, 154 tiles each: 20.7 -> 16.3 us for 128 -> 128 channels 3x3/2, 16.2 -> 12.7 for 1024 -> 512; batch 16, 100
-  // tiles: 7.4 -> 8.9 for the latter).  Where only the 128 x 128 tile has that many it takes the layer (14 x 14 pixels, 50
-  // images: 11.2 -> 9.5 us for 1024 -> 256, 19.4 -> 16.3 for 256 -> 256 3x3/2); with both the larger one is the faster
-  // (13.1 against 15.8 us for 512 -> 256 at 28 x 28).
-  return big_cfg_blocks(kBigCfgs[1], g) >= 144 ? 1 : big_cfg_blocks(kBigCfgs[3], g) >= 144 ? 3 : -1;
+  const int64_t large = big_cfg_blocks(kBigCfgs[1], g), small = big_cfg_blocks(kBigCfgs[3], g);
+  if (large >= 160) return 1;
+  // Fewer tiles than that leave the ring at a disadvantage of its own: a workgroup's start (the first stages of the ring) is
+  // paid once per tile, whatever K is, and there is no second workgroup to hide it.  It is worth it where K is long, or where
+  // the input comes from behind the L2, which the ring requests further ahead.  Ring against wavefront kernel, input from
+  // the L2, at 144 to 160 tiles of 128 x 256: K = 512 19 % slower, 1024 equal, 2048 19 % faster, 4608 27 %; at 144 to 290 tiles of
+  // 128 x 128: K = 512 25 % slower, 1024 (1x1) 15 % and 1152 12 % slower, 2304 equal, with stride 2 14 % faster, 4608 18 %.
+  // In models (one launch per layer, us a step with the tiles for every K >= 512, without them, and by this rule): ResNet-50
+  // with 12 images 387, 383, 383, with 24 528, 512, 512, with 50 798, 811, 799 (there 20 MB go into 512 -> 128 and 10 MB into
+  // 1024 -> 256); VGG-16 with 6 images 247, 264, 248, with 9 of 176 x 176 252, 259, 251.
+  const int64_t in_bytes = (int64_t)g.N * g.H * g.W * g.Cp;
+  if (large >= 144 && (g.K >= 1024 || in_bytes >= (16 << 20))) return 1;
+  if (small >= 144 && (g.K >= 2048 || (g.KH * g.KW == 1 && g.K >= 1024 && in_bytes >= (8 << 20)))) return 3;
+  return -1;
 }
 template <int OUT>
 static void launch_big_out(int cfg, unsigned grid, hipStream_t s, const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g,

@@ -30,7 +30,7 @@ def _ptr(t):
 
 def _apply_conv_tuning():
     """The library never reads the environment on a launch; this glue turns the test hooks CVM_HIP_CONV
-    (lds | wave | big), CVM_HIP_WAVECFG (index) and CVM_HIP_TILE ("wm,wn"; with big: "t,0" picks tile t = 1..3)
+    (lds | wave | big), CVM_HIP_WAVECFG (index) and CVM_HIP_TILE ("wm,wn"; with big: "t,0" picks tile t = 1..4)
     into the explicit per-thread setting."""
     kind = os.environ.get("CVM_HIP_CONV", "")
     cfg = os.environ.get("CVM_HIP_WAVECFG", "")

@@ -283,8 +283,8 @@ int cvmhip_fold_requant(const int32_t* bias, int oc, int64_t max_abs_acc, const 
 int cvmhip_pad_channels(int channels);
 /* Test and tuning hook: forces, for the calling thread's later convolution launches, the implicit-GEMM kernel
  * (0 automatic, 1 LDS-tiled, 2 wavefront-private, 3 large-tile wherever the layout allows it), a configuration of the
- * wavefront kernel (-1 automatic) and a tile of the tiled kernel (wm, wn in 1..2; 0 automatic; with kernel 3, wm = 1..3
- * picks the 256x256, 128x256 or 64x512 tile).  The library never reads the environment on a launch. */
+ * wavefront kernel (-1 automatic) and a tile of the tiled kernel (wm, wn in 1..2; 0 automatic; with kernel 3, wm = 1..4
+ * picks the 256x256, 128x256, 64x512 or 128x128 tile).  The library never reads the environment on a launch. */
 int cvmhip_set_conv_tuning(int kernel, int wave_cfg, int tile_wm, int tile_wn);
 /* The same for layer-sequence launches (cvmhip_conv_seq_*) of the calling thread: `spin_limit` = polls after which a wait
  * at a layer boundary gives up and raises the launch's error word (default 2 000 000; 0 makes every wait give up at

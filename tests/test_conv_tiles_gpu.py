@@ -1,11 +1,14 @@
 """Large-tile convolution kernel with the 128 x 128 tile, which the dispatch takes for layers of too few pixels for the
-128 x 256 one: edges of its range, against the oracle."""
+128 x 256 one: edges of the tile, against the oracle, and the lines of the dispatch."""
+import ctypes
+import json
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from cvm_runtime_amd import hipops, synth
+from cvm_runtime_amd import check, hipops, lib, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -14,12 +17,18 @@ def T(a, dev):
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).to(dev)
 
 
+@pytest.fixture
+def tile(monkeypatch):
+    monkeypatch.setenv("CVM_HIP_CONV", "big")
+    monkeypatch.setenv("CVM_HIP_TILE", "4,0")
+
+
 @pytest.mark.parametrize("n,ic,h,w,oc,k,stride,residual", [
-    (9, 64, 32, 32, 256, 3, 1, False),     # 144 tiles: the least that takes it
+    (9, 64, 32, 32, 256, 3, 1, False),     # whole tiles
     (11, 512, 29, 29, 200, 1, 1, True),    # pixels and channels that end inside a tile, shortest K, residual
     (47, 96, 28, 28, 130, 3, 2, False),    # two channels in the last tile, K of 864
 ])
-def test_tile_128_by_128(n, ic, h, w, oc, k, stride, residual, dev):
+def test_tile_128_by_128(n, ic, h, w, oc, k, stride, residual, dev, tile):
     cid = "tile128-%d-%d" % (n, ic)
     x = synth.tensor(cid, "x", (n, ic, h, w), -127, 127)
     wt = synth.tensor(cid, "w", (oc, ic, k, k), -127, 127)
@@ -41,11 +50,11 @@ def test_tile_128_by_128(n, ic, h, w, oc, k, stride, residual, dev):
 
 
 @pytest.mark.parametrize("n,ic,h,w,oc", [
-    (9, 64, 32, 32, 256),     # whole tiles of pixels, the least that takes the tile
+    (9, 64, 32, 32, 256),     # whole tiles of pixels
     (11, 64, 30, 30, 200),    # pixels and channels that end inside a tile
 ])
 @pytest.mark.parametrize("multiply", [False, True])
-def test_tile_128_by_128_with_a_fused_pool(n, ic, h, w, oc, multiply, dev):
+def test_tile_128_by_128_with_a_fused_pool(n, ic, h, w, oc, multiply, dev, tile):
     cid = "tile128-pool-%d" % n
     x = synth.tensor(cid, "x", (n, ic, h, w), -127, 127)
     wt = synth.tensor(cid, "w", (oc, ic, 3, 3), -127, 127)
@@ -60,3 +69,32 @@ def test_tile_128_by_128_with_a_fused_pool(n, ic, h, w, oc, multiply, dev):
     got = hipops.unpack_act_i8(out, n, oc, h // 2, w // 2)
     torch.cuda.synchronize()
     assert np.array_equal(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("n,ic,hw,oc,k,takes", [
+    (9, 256, 32, 256, 3, "big cfg 3"),      # 144 tiles of 128 x 128, K = 2304
+    (9, 224, 32, 256, 3, "wave"),           # K = 2016
+    (9, 256, 31, 256, 3, "wave"),           # 136 tiles
+    (9, 1024, 32, 256, 1, "big cfg 3"),     # K = 1024 and 9 MiB of input
+    (4, 1024, 32, 640, 1, "wave"),          # 160 tiles, 4 MiB
+    (18, 1024, 32, 256, 1, "big cfg 1"),    # 144 tiles of 128 x 256
+    (18, 512, 32, 256, 1, "wave"),          # K = 512 and 9 MiB
+    (36, 512, 32, 128, 1, "big cfg 1"),     # 18 MiB
+    (20, 512, 32, 256, 1, "big cfg 1"),     # 160 tiles
+])
+def test_which_layers_take_the_large_tiles(n, ic, hw, oc, k, takes, dev, monkeypatch):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(ic)
+    xp = hipops.pack_act_i8(torch.randint(-127, 128, (n, ic, hw, hw), dtype=torch.int32, device=dev, generator=gen))
+    wp = hipops.pack_weights(torch.randint(-127, 128, (oc, ic, k, k), dtype=torch.int32, device=dev, generator=gen))
+
+    def run():
+        return hipops.conv2d_i8(xp, n, ic, hw, hw, wp, oc, k, k, None, hipops.chain(("cvm_right_shift", 8, 10)), padding=(k // 2, k // 2))
+    lib().cvmhip_kernel_timing_begin()
+    out = run()
+    torch.cuda.synchronize()
+    buf = ctypes.create_string_buffer(1 << 16)
+    check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
+    assert takes in str(json.loads(buf.value.decode())[-1])
+    monkeypatch.setenv("CVM_HIP_CONV", "wave")
+    assert torch.equal(out, run())
