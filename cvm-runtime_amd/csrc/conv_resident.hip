@@ -16,12 +16,12 @@
 // the four 16-byte groups of every K step are a table behind the filter.
 // The filter of a layer, its tap offsets, biases and the places of its tiles lie in LDS as well, fetched while the layer in
 // front of it is computed.
-// What bounds it now (ResNet-20, one workgroup, 98 K clocks in all): 46 K of LDS transfers at 128 bytes a clock, 34 K of vector
-// instructions, 14 K of scalar ones and 17 K of products on each SIMD, which hardly overlap: behind a barrier all wavefronts
-// read at the same time and then compute at the same time.  On the way, same network at batch 1: all operand reads of a
-// chunk before its first product instead of a read and a wait each 62 -> 52 us; filters requested inside the loop that uses
-// them 54 -> 45; plain layers without the tests for other forms 45 -> 41.5; filters and places from LDS (no scalar register
-// is spilled any more) and a sum without LDS shuffles 41.5 -> 39.  No difference: 1024 threads, another priority for half of
+// What bounds it now (ResNet-20, one workgroup, 106 K clocks by the counters): 46 K of LDS transfers, 17 K of them bank
+// conflicts, 35 K of vector instructions, 14 K of scalar ones and 13 K of products on each SIMD, which hardly overlap: behind
+// a barrier all wavefronts read at the same time and then compute at the same time.  On the way, same network at batch 1:
+// all operand reads of a chunk before its first product instead of a read and a wait each 62 -> 52 us; filters requested
+// inside the loop that uses them 54 -> 45; plain layers without the tests for other forms 45 -> 41.5; filters and places
+// from LDS (no scalar register is spilled any more) and a sum without LDS shuffles 41.5 -> 39.  No difference: 1024 threads, another priority for half of
 // the wavefronts, pixels an odd number of granules apart.
 #include <string.h>
 
