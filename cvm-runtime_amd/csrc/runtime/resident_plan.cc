@@ -202,7 +202,9 @@ HipGraphRuntime::ResidentDraft HipGraphRuntime::DraftResident(size_t first, size
     const void* src = st.stem ? static_cast<const void*>(st.aux.get()) : i8_ptr_[st.src];
     if (!where.count(src)) {
       if (st.stem) return r;   // its packed image belongs to a step in front of the stretch
-      load(src, st.c, st.kind == PlanStep::SUM ? 1 : st.h, st.kind == PlanStep::SUM ? st.h : st.w, k);
+      // (a sum's own extent is its pixels in a row, but other layers may read the map as well)
+      const bool sum = st.kind == PlanStep::SUM;
+      load(src, st.c, sum ? static_cast<int>(shape_[st.src][2]) : st.h, sum ? static_cast<int>(shape_[st.src][3]) : st.w, k);
     }
     const void* res = st.kind == PlanStep::CONV && st.src2 != kNone ? i8_ptr_[st.src2] : nullptr;
     const int oh = st.kind == PlanStep::CONV ? ConvOut(st.h, st.kh, st.sh, st.ph, st.dh) : st.oh;

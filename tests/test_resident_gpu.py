@@ -71,3 +71,33 @@ def test_images_in_rounds(dev):
         one, heads1 = _net(CASES[0], 1)
         j1, p1 = one.build(heads1)
         assert np.array_equal(got[i], og.run_graph(j1, graphgen.load_params(p1), x[i:i + 1].astype(np.int32))[0].ravel())
+
+
+def _check_heads(g, heads, n, cid, monkeypatch):
+    js, pb = g.build([g.reshape(t, (n, 1, int(np.prod(g.shape(t)[1:])))) for t in heads])
+    params = graphgen.load_params(pb)
+    results = []
+    for resident in ("1", "0"):
+        monkeypatch.setenv("CVM_HIP_RESIDENT", resident)
+        m = runtime.HipModel(js, pb)
+        results.append(m.launch_counts()[0])
+        kind = np.int32 if runtime.CVMAPIGetOutputTypeSize(m.net) == 4 else np.int8
+        for i in range(3):
+            x = synth.tensor(cid, "data%d" % i, g.shape((0, 0)), -127, 127)
+            want = np.concatenate([v.reshape(n, -1) for v in og.run_graph(js, params, x)], axis=1).ravel()
+            got = np.frombuffer(m.inference(x.astype(np.int8).tobytes()), kind).astype(np.int32)
+            assert np.array_equal(got, want), "resident %s call %d" % (resident, i)
+        m.close()
+    return results
+
+
+def test_a_map_that_a_sum_reads_before_a_pool_does(dev, monkeypatch):
+    """The launch loads the map where the sum needs it, and the pool behind needs its rows."""
+    g = graphgen.GraphBuilder("resident-sum-first")
+    x = g.conv_relu_q(g.var("data", (4, 16, 17, 15), 8), 16, 3, 2, 1, groups=16)   # not a layer of such a launch
+    s, _ = g.global_sum(x)
+    d, k = g.dense(g.flatten(g.rshift(s, 7)), 128)
+    d, _ = g.dense(g.rshift(d, graphgen.shift_for(k)), 7)
+    y = g.conv_relu_q(g.conv_relu_q(g.max_pool(x, 3, 2, 1), 64, 1, 2), 32, 3, 1, 1)
+    launches = _check_heads(g, [y, g.rshift(d, 10)], 4, "resident-sum-first", monkeypatch)
+    assert launches[0] < launches[1], launches     # layers in LDS at all
