@@ -191,6 +191,12 @@ HipGraphRuntime::ResidentDraft HipGraphRuntime::DraftResident(size_t first, size
     ResidentDraft::Layer l;
     l.step = k;
     if (st.kind == PlanStep::STEMPACK) {
+      // the packed image exists in LDS only: its reader is part of the stretch (a second convolution over the input has a
+      // packing step of its own, which the stretch may end with)
+      bool inside = false, outside = false;
+      for (size_t q = 0; q < plan_.size(); ++q)
+        if (plan_[q].stem && plan_[q].aux == st.aux) (q > k && q <= last ? inside : outside) = true;
+      if (!inside || outside) return r;
       l.d.kind = 0;
       shape(&l.d, st.c, st.h, st.w);
       l.d.in = in_stage_dev_;

@@ -101,3 +101,13 @@ def test_a_map_that_a_sum_reads_before_a_pool_does(dev, monkeypatch):
     y = g.conv_relu_q(g.conv_relu_q(g.max_pool(x, 3, 2, 1), 64, 1, 2), 32, 3, 1, 1)
     launches = _check_heads(g, [y, g.rshift(d, 10)], 4, "resident-sum-first", monkeypatch)
     assert launches[0] < launches[1], launches     # layers in LDS at all
+
+
+def test_the_image_packed_for_a_convolution_outside_the_launch_is_written(dev, monkeypatch):
+    """Two convolutions over the input pack it for themselves; the launch may take the first one and not the second."""
+    g = graphgen.GraphBuilder("resident-two-stems")
+    x = g.var("data", (16, 1, 3, 3), 8)
+    a = g.conv_relu_q(x, 512, 3, 1, 1, relu=False)
+    b = g.conv_relu_q(g.conv_relu_q(x, 256, 3, 2, 1), 512, 1)      # 512 x 256: the filter does not fit beside the rest
+    b = g.conv_relu_q(g.conv_relu_q(b, 256, 1), 256, 3, 1, 1, groups=256)
+    _check_heads(g, [a, b], 16, "resident-two-stems", monkeypatch)
