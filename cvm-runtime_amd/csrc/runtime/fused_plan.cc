@@ -497,7 +497,7 @@ void HipGraphRuntime::BuildPlan() {
           const int ps = producer_step[x], pr = producer_step[r];
           if (ps < 0 || pr < 0 || pr >= ps || plan[ps].stem) continue;
           PlanStep& cs = plan[ps];
-          if (cs.kind != PlanStep::CONV || cs.dst != x || !cs.out_i8 || cs.src2 != kNone) continue;
+          if (cs.kind != PlanStep::CONV || cs.dst != x || !cs.out_i8 || cs.src2 != kNone || cs.pool2) continue;   // (no pooled form with a residual)
           if (uses[x].size() != 1 || is_head[x]) continue;
           cs.src2 = r;
           cs.chain2 = chain;

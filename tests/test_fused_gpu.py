@@ -1132,3 +1132,20 @@ def test_a_dense_layer_does_not_share_a_launch_with_the_convolution_it_reads(dev
     for m in models:
         assert np.array_equal(np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int32), want)
         m.close()
+
+
+def test_an_add_behind_a_pool_that_a_convolution_has_taken_keeps_its_launch(dev):
+    """conv -> max_pool2d(2x2) is one launch, which has no residual: the add of the pooled tensor is not folded into it."""
+    g = graphgen.GraphBuilder("pool-add")
+    x = g.var("data", (2, 32, 12, 12), 8)
+    y = g.max_pool(x, 2, 2)
+    other = g.conv_relu_q(y, 64, 1)
+    y = g.max_pool(g.conv_relu_q(x, 64, 3, 1, 1), 2, 2)
+    z = g.rshift(g.add(y, other), 1)
+    js, pb = g.build([g.conv_relu_q(z, 40, 1)])
+    m = runtime.HipModel(js, pb)
+    for i in range(3):
+        data = synth.tensor("pool-add", "x%d" % i, (2, 32, 12, 12), -127, 127)
+        want = og.run_graph(js, graphgen.load_params(pb), data)[0].ravel()
+        assert np.array_equal(np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32), want)
+    m.close()
