@@ -628,7 +628,8 @@ void HipGraphRuntime::BuildPlan() {
       }
     } else if (op == "flatten") {
       const uint32_t xe = entry_id(n.inputs[0]);
-      if (has_i8[xe] && !is_head[out0] && uses[out0].size() == 1) {
+      // (a dense layer takes the int8 form of values that are proven to fit it only, and the flattened tensor exists in no other)
+      if (has_i8[xe] && safe[xe] && !is_head[out0] && uses[out0].size() == 1) {
         const Node& c = nodes_[uses[out0][0]];
         const Shape& x = shape_[xe];
         bool to_dense = c.func_name == "dense" && entry_id(c.inputs[0]) == out0;

@@ -1052,6 +1052,23 @@ def test_dense_keeps_values_that_a_non_clipping_shift_leaves_outside_int8(four_d
         assert np.array_equal(got, want), "planner %s" % ("on" if mode == "1" else "off")
 
 
+@pytest.mark.parametrize("hw", [1, 2])
+def test_dense_over_a_map_whose_int8_form_only_a_convolution_may_take(hw, dev):
+    """The same values in a map that a convolution reads as well: it narrows them (ops.cc:430-432), dense does not."""
+    g = graphgen.GraphBuilder("dense-beside-conv-%d" % hw)
+    x = g.var("data", (3, 32, hw, hw), 32)
+    s = g.rshift(x, 24, 8)
+    c = g.conv_relu_q(s, 16, 1)
+    d, _ = g.dense(g.flatten(s), 24)
+    js, pb = g.build([g.reshape(c, (3, 1, 16 * hw * hw)), g.reshape(d, (3, 1, 24))])
+    xv = synth.tensor("dense-beside-conv", "data%d" % hw, (3, 32, hw, hw), -2 ** 31, 2 ** 31 - 1)
+    xv.flat[:5] = [2 ** 31 - 1, 2 ** 31 - 1, -2 ** 31, 2 ** 31 - 2 ** 23, 2 ** 31 - 2 ** 22]
+    want = np.concatenate([r.reshape(3, -1) for r in og.run_graph(js, graphgen.load_params(pb), xv)], axis=1).ravel()
+    m = runtime.HipModel(js, pb)
+    assert np.array_equal(np.frombuffer(m.inference(xv.astype(np.int32).tobytes()), np.int32), want)
+    m.close()
+
+
 def test_dense_int32_kernel_blocks_of_rows(dev):
     """The exact int32 dense kernel (operands wider than 8 bits) with row counts around its row block."""
     for m, k, n in ((1, 70, 5), (8, 64, 9), (9, 130, 33), (17, 257, 12)):
