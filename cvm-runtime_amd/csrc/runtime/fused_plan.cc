@@ -161,6 +161,10 @@ void HipGraphRuntime::BuildPlan() {
     if (sid_users[storage_id_[eid]] > 1) privatize(eid);
   };
 
+  // A run must leave its input as it is: one whose sequence launch gave up is repeated, and the comparison of launch forms may
+  // take place between an input and its run.
+  early_i32(DataEntry());
+
   std::vector<PlanStep> plan;
   auto need_i32 = [&](uint32_t eid) {
     if (has_i32[eid]) return;

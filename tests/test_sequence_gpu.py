@@ -2,6 +2,7 @@
 of the images; include/cvm_hip_ops.h: cvmhip_conv_seq_*) against the CPU oracle executing the same graph node
 by node, and against the same model with one launch per layer.  Bit-exact.  CVM_HIP_SEQ=1 forces the
 sequences (by default a model measures both ways when it is loaded and keeps the faster), =0 switches them off."""
+import json
 import os
 
 import numpy as np
@@ -338,3 +339,41 @@ def test_graphs_are_dropped_behind_calls_that_returned_by_their_ticket(dev):
         first.close()
     finally:
         os.environ.pop("CVM_HIP_SEQ", None)
+
+
+def _lent_input(cid):
+    """A run of convolutions behind a node that reads the input; the input's storage is lent to the node behind them."""
+    g = graphgen.GraphBuilder(cid)
+    x = g.var("data", (8, 32, 10, 10), 8)
+    y = g.unary("abs", x)
+    for oc in (64, 64, 64, 32):
+        y = g.conv_relu_q(y, oc, 3, 1, 1, relu=False)
+    z = g.unary("abs", y)
+    js, pb = g.build([z])
+    doc = json.loads(js)
+    sid = doc["attrs"]["storage_id"][1]
+    sid[g._eid(z)] = sid[g._eid(x)]
+    return json.dumps(doc), pb
+
+
+@pytest.mark.parametrize("how", ["gives up", "compares"])
+def test_a_run_that_is_repeated_finds_its_input(how, dev, monkeypatch):
+    js, pb = _lent_input("seq-lent")
+    inputs = [synth.tensor("seq-lent", "x%d" % i, (8, 32, 10, 10), -127, 127) for i in range(3)]
+    wants = [og.run_graph(js, graphgen.load_params(pb), x)[0].ravel() for x in inputs]
+    if how == "gives up":                       # every wait of the sequence launch does, and the run is repeated without it
+        monkeypatch.setenv("CVM_HIP_SEQ", "1")
+        monkeypatch.setenv("CVM_HIP_SEQ_SPIN", "0")
+        m = runtime.HipModel(js, pb)
+    else:                                       # loaded next to another such model: compares the launch forms at its first run alone
+        monkeypatch.setenv("CVM_HIP_SEQ", "1")
+        other = runtime.HipModel(js, pb)
+        monkeypatch.delenv("CVM_HIP_SEQ")
+        monkeypatch.setenv("CVM_HIP_RESIDENT", "0")
+        m = runtime.HipModel(js, pb)
+        other.close()
+    assert m.launch_counts()[1] == 1
+    for x, want in zip(inputs, wants):
+        got = np.frombuffer(m.inference(x.astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want)
+    m.close()
