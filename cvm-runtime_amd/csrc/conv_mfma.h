@@ -235,6 +235,9 @@ int pack_activations(const int32_t* x, int8_t* xp, int n, int c, int hw, hipStre
 int unpack_activations(const int8_t* xp, int32_t* x, int n, int c, int hw, hipStream_t s);
 int pack_weights(const int32_t* w, int8_t* wp, int oc, int ic, int kh, int kw, hipStream_t s);
 int conv_igemm(const int8_t* xp, const int8_t* wp, void* out, ConvGeom g, const Epilogue& ep, hipStream_t s);
+// groups > 1 on int32 tensors (conv_planes.hip)
+int conv_grouped_i32(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y, int n, int ic, int h, int wd, int oc, int oh, int ow,
+                     int kh, int kw, int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w, int groups, hipStream_t s);
 // The same with a workspace: a layer with at most 64 output pixels and K >= 8192 is then computed in K slices by
 // several workgroups per tile (partial sums in the workspace, a second kernel finishes).  Without a workspace, or for
 // any other layer, identical to conv_igemm.  conv_slices_workspace_bytes() gives the size (0 = not applicable).

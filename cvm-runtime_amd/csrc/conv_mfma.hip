@@ -2293,98 +2293,6 @@ __global__ void __launch_bounds__(256) k_unpack_act(const int8_t* __restrict__ x
 }
 
 // ---------------------------------------------------------------- exact int32 paths
-// groups > 1 (incl. depthwise): direct convolution on the int32 values, no
-// narrowing -- what the reference does for grouped filters (ops.cc:333-366).
-__global__ void __launch_bounds__(256)
-k_conv_grouped(const int32_t* __restrict__ x, const int32_t* __restrict__ w, const int32_t* __restrict__ bias,
-               int32_t* __restrict__ y, int64_t total, int ic, int h, int wd, int oc, int oh, int ow, int kh, int kw,
-               int sh, int sw, int ph, int pw, int dh, int dw, int icg, int ocg) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const int q = (int)(i % ow);
-    const int p = (int)((i / ow) % oh);
-    const int o = (int)((i / ((int64_t)ow * oh)) % oc);
-    const int64_t b = i / ((int64_t)ow * oh * oc);
-    const int cbase = (o / ocg) * icg;
-    int32_t acc = 0;
-    for (int c = 0; c < icg; ++c) {
-      const int32_t* xc = x + ((int64_t)b * ic + cbase + c) * h * wd;
-      const int32_t* wc = w + ((int64_t)o * icg + c) * kh * kw;
-      for (int r = 0; r < kh; ++r) {
-        const int ih = p * sh + r * dh - ph;
-        if (ih < 0 || ih >= h) continue;
-        for (int t = 0; t < kw; ++t) {
-          const int iw = q * sw + t * dw - pw;
-          if (iw < 0 || iw >= wd) continue;
-          acc = wadd(acc, wmul(xc[(int64_t)ih * wd + iw], wc[r * kw + t]));
-        }
-      }
-    }
-    y[i] = wadd(acc, bias ? bias[o] : 0);
-  }
-}
-
-// One input channel per group (depthwise, with or without a channel multiplier), filter rows of KW taps: four
-// neighbouring outputs of a row per thread, so a row of the window is read once for four outputs, and the filter, which is
-// the same for a whole workgroup (one output plane), comes through the scalar cache.  Same exact int32 products.
-// Bound by the 32-bit multiplies (a quarter of the rate of an add: 36 of them, 3.3 us of the chip for 4 x 96 x 75 x 75) and
-// by the masks of the border: 13.4 us there against 23 us for one output per thread.
-template <int KH, int KW, bool UNIT>
-__global__ void __launch_bounds__(256)
-k_conv_planes(const int32_t* __restrict__ x, const int32_t* __restrict__ w, const int32_t* __restrict__ bias, int32_t* __restrict__ y,
-              int planes, int ic, int h, int wd, int oc, int oh, int ow, int sh, int sw, int ph, int pw, int dh, int dw, int ocg,
-              FastDiv div_quads) {
-  const int quads = (ow + 3) >> 2;
-  for (int plane = blockIdx.y; plane < planes; plane += gridDim.y) {
-    const int b = plane / oc, o = plane - b * oc;
-    const int32_t* xc = x + ((int64_t)b * ic + o / ocg) * h * wd;
-    const int32_t* wc = w + (int64_t)o * KH * KW;
-    const int32_t b0 = bias ? bias[o] : 0;
-    const int lin = blockIdx.x * 256 + threadIdx.x;
-    if (lin >= oh * quads) continue;
-    const int p = (int)fastdiv((unsigned)lin, div_quads), q = (lin - p * quads) * 4;
-    // every load of the window is issued, from the nearest pixel inside, and masked afterwards; at stride 1 the windows
-    // of the four outputs share their columns
-    constexpr int COLS = UNIT ? KW + 3 : 4 * KW;
-    int32_t v[KH][COLS];
-#pragma unroll
-    for (int r = 0; r < KH; ++r) {
-      const int ih = p * sh + r * dh - ph;
-      const int32_t* xr = xc + (int64_t)(ih < 0 ? 0 : (ih < h ? ih : h - 1)) * wd;
-#pragma unroll
-      for (int e = 0; e < COLS; ++e) {
-        const int iw = UNIT ? q + e - pw : (q + e / KW) * sw + (e % KW) * dw - pw;
-        v[r][e] = xr[iw < 0 ? 0 : (iw < wd ? iw : wd - 1)];
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    int32_t acc[4] = {b0, b0, b0, b0};
-#pragma unroll
-    for (int r = 0; r < KH; ++r) {
-      const int ih = p * sh + r * dh - ph;
-      const bool row = ih >= 0 && ih < h;
-#pragma unroll
-      for (int e = 0; e < COLS; ++e) {
-        const int iw = UNIT ? q + e - pw : (q + e / KW) * sw + (e % KW) * dw - pw;
-        v[r][e] = row && iw >= 0 && iw < wd ? v[r][e] : 0;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int t = 0; t < KW; ++t) acc[u] = wadd(acc[u], wmul(v[r][UNIT ? u + t : u * KW + t], wc[r * KW + t]));
-    }
-    int32_t* yr = y + (int64_t)plane * oh * ow + (int64_t)p * ow + q;
-    typedef int v4i __attribute__((ext_vector_type(4), aligned(4)));   // rows need not start on 16 bytes
-    if (q + 3 < ow) {
-      *reinterpret_cast<v4i*>(yr) = v4i{acc[0], acc[1], acc[2], acc[3]};
-    } else {
-#pragma unroll
-      for (int u = 0; u < 3; ++u)
-        if (q + u < ow) yr[u] = acc[u];
-    }
-  }
-}
-
 // dense on int32 operands without narrowing (ops.cc:53-62 multiplies the full int32 values): one
 // wavefront per output column j and block of DENSE_MB rows, so a filter row is read once per block.
 constexpr int DENSE_MB = 8;
@@ -3412,25 +3320,8 @@ int cvmhip_conv2d(const int32_t* x, const int32_t* w, const int32_t* bias, int32
   const int ow = (wd + 2 * pad_w - (dil_w * (kw - 1) + 1)) / stride_w + 1;
   if (h + 2 * pad_h < dil_h * (kh - 1) + 1 || wd + 2 * pad_w < dil_w * (kw - 1) + 1) return arg_error("conv2d kernel exceeds input");
   hipStream_t s = as_stream(stream);
-  if (groups > 1) {
-    const int64_t total = (int64_t)n * oc * oh * ow;
-    const int64_t quads = (int64_t)oh * ((ow + 3) / 4), planes = (int64_t)n * oc;
-    if (ic == groups && kh == 3 && kw == 3 && planes < INT32_MAX && quads < INT32_MAX && (int64_t)h * wd < INT32_MAX) {
-      const dim3 grid((unsigned)((quads + 255) / 256), (unsigned)(planes < 65535 ? planes : 65535));
-      const FastDiv div_quads = make_fastdiv((uint32_t)((ow + 3) / 4));
-      if (stride_w == 1 && dil_w == 1)
-        k_conv_planes<3, 3, true><<<grid, 256, 0, s>>>(x, w, bias, y, (int)planes, ic, h, wd, oc, oh, ow, stride_h, stride_w, pad_h,
-                                                       pad_w, dil_h, dil_w, oc / groups, div_quads);
-      else
-        k_conv_planes<3, 3, false><<<grid, 256, 0, s>>>(x, w, bias, y, (int)planes, ic, h, wd, oc, oh, ow, stride_h, stride_w, pad_h,
-                                                        pad_w, dil_h, dil_w, oc / groups, div_quads);
-      return check_launch("conv_planes");
-    }
-    k_conv_grouped<<<grid_for(total, 256, 1 << 20), 256, 0, s>>>(x, w, bias, y, total, ic, h, wd, oc, oh, ow, kh, kw,
-                                                               stride_h, stride_w, pad_h, pad_w, dil_h, dil_w,
-                                                               ic / groups, oc / groups);
-    return check_launch("conv_grouped");
-  }
+  if (groups > 1)
+    return conv_grouped_i32(x, w, bias, y, n, ic, h, wd, oc, oh, ow, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, groups, s);
   const size_t need = cvmhip_conv2d_workspace_bytes(n, ic, h, wd, oc, kh, kw, 1);
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return arg_error("conv2d workspace");
   int8_t* xp = reinterpret_cast<int8_t*>(workspace);

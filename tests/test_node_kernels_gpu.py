@@ -66,6 +66,19 @@ def test_depthwise_planes(n, c, mult, h, w, strides, padding, dilation, dev):
     assert np.array_equal(got, oracle.conv2d(x, wt, b, strides, padding, dilation, groups=c))
 
 
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("n,c,h,w", [(1, 1, 1, 1), (1, 3, 2, 5), (2, 5, 7, 6), (1, 70, 19, 75), (4, 70, 64, 61)])   # the last: four rows a thread
+@pytest.mark.parametrize("last", [0, 2 ** 23])   # all values in 24 bits; one that is not, in the last wavefront
+def test_depthwise_planes_narrow(n, c, h, w, stride, last, dev):
+    x = synth.tensor("narrow", "x%d-%d" % (c, w), (n, c, h, w), -2 ** 23, 2 ** 23 - 1)
+    wt = synth.tensor("narrow", "w%d" % c, (c, 1, 3, 3), -2 ** 23, 2 ** 23 - 1)
+    if last:
+        x[-1, -1, -1, -1] = last
+    wt[0, 0, 1, 1], x[0, 0, 0, 0] = -2 ** 23, 2 ** 23 - 1
+    got = hipops.conv2d(T(x, dev), T(wt, dev), None, (stride, stride), (1, 1), groups=c).cpu().numpy()
+    assert np.array_equal(got, oracle.conv2d(x, wt, None, (stride, stride), (1, 1), (1, 1), groups=c))
+
+
 @pytest.mark.parametrize("widths,outer,inner", [
     ((1, 1, 4), 24564, 1),                          # a detector's rows
     ((3,), 5, 7),
