@@ -66,6 +66,20 @@ __device__ __forceinline__ int32_t wadd(int32_t a, int32_t b) { return (int32_t)
 __device__ __forceinline__ int32_t wsub(int32_t a, int32_t b) { return (int32_t)((uint32_t)a - (uint32_t)b); }
 __device__ __forceinline__ int32_t wmul(int32_t a, int32_t b) { return (int32_t)((uint32_t)a * (uint32_t)b); }
 
+// Inclusive sum over the lanes of a wavefront (lane 63 holds the total), all lanes active: 1, 2, 4 and 8 lanes to the right inside
+// rows of 16, then the rows' last lanes onward.  Six vector instructions; a shuffle step goes through LDS (100 clocks each).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int32_t wave_add_from(int32_t v) { return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false); }
+__device__ __forceinline__ int32_t wave_scan_add(int32_t v) {
+  v = wave_add_from<0x111, 0xf>(v);
+  v = wave_add_from<0x112, 0xf>(v);
+  v = wave_add_from<0x114, 0xf>(v);
+  v = wave_add_from<0x118, 0xf>(v);
+  v = wave_add_from<0x142, 0xa>(v);
+  return wave_add_from<0x143, 0xc>(v);
+}
+__device__ __forceinline__ int32_t wave_sum(int32_t v) { return __builtin_amdgcn_readlane(wave_scan_add(v), 63); }
+
 // Requantisation parameters prepared on the host once per launch.
 // mode 0: max==0 -> 0;  1: b>=31 -> a>>31;  2: p+b>=32 -> rounding shift, no clip;
 // 3: saturate on pre-shifted bounds, else rounding shift

@@ -44,3 +44,45 @@ def test_nms_splits(b, n, ids, extent, side, apart, force, top_k, keep, dev):
     tx, ty = T(x), T(init)
     hipops.non_max_suppression(tx, T(vc), ty, 45, force, top_k, max_output_size=keep)
     assert np.array_equal(ty.cpu().numpy(), y_ref) and np.array_equal(tx.cpu().numpy(), x_after)
+
+
+@pytest.mark.parametrize("b,n,ids,coords,force", [
+    (1, 128, 1, 100, True), (1, 129, 1, 100, True),            # the least number of rows for the masks, one below it
+    (1, 1024, 1, 400, True), (1, 1025, 1, 400, True),          # the most, one above it
+    (4, 961, 1, 400, True),
+    (1, 8200, 20, 2000, False), (2, 8192, 40, 2000, False),    # several workgroups to a class
+    (3, 600, 1, 200, True), (5, 400, 1, 200, True),
+    (1, 700, 2, 300, False),                                   # two ids that share a class
+    (1, 640, 1, 16384, True), (1, 640, 1, 16385, True),        # coordinates at the edge of 15 bits, one beyond it
+])
+def test_nms_pairs(b, n, ids, coords, force, dev):
+    """Classes of as many rows as the walk tests by masks, boxes with coordinates of both signs; with the caller's workspace and with
+    the static one, which has no room for masks."""
+    cid = "nms-pairs-%d-%d-%d" % (b, n, coords)
+    x = np.zeros((b, n, 6), np.int32)
+    x[:, :, 0] = synth.tensor(cid, "id", (b, n), 0, ids - 1) * (64 if ids == 2 else 1)
+    x[:, :, 1] = synth.tensor(cid, "score", (b, n), -127, 127)
+    x[:, :, 2:4] = synth.tensor(cid, "xy", (b, n, 2), -coords, coords - 1 - 64)
+    x[:, :, 4:6] = x[:, :, 2:4] + synth.tensor(cid, "wh", (b, n, 2), -2, 64)   # some empty
+    x[:, 0, 2:6] = (-coords, -coords, -coords + 70, -coords + 70)
+    x[:, 1, 2:6] = (coords - 71, coords - 71, coords - 1, coords - 1)
+    x[:, 2:40, 2:6] = x[:, :2, 2:6].repeat(19, 1) + synth.tensor(cid, "near", (b, 38, 4), 0, 1) * [1, 1, 0, 0]
+    vc = np.full((b,), n, np.int32)
+    init = np.full_like(x, 5)
+    y_ref, x_after = oracle.non_max_suppression(x, vc, 30, force, -1, max_output_size=-1, y_init=init)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    for call in (hipops.non_max_suppression, hipops.non_max_suppression_static):
+        tx, ty = T(x), T(init)
+        call(tx, T(vc), ty, 30, force, -1, max_output_size=-1)
+        assert np.array_equal(ty.cpu().numpy(), y_ref) and np.array_equal(tx.cpu().numpy(), x_after)
+
+
+@pytest.mark.parametrize("n,k", [(1, 6), (255, 6), (257, 2), (8192, 6), (8193, 6), (300, 8), (300, 9)])   # one launch up to 8192; rows in registers up to 8
+def test_valid_counts_splits(n, k, dev):
+    x = synth.tensor("gvc", "%d-%d" % (n, k), (2, n, k), -127, 127)
+    vc, y = hipops.get_valid_counts(torch.from_numpy(x).to(dev), 20)
+    for b in range(2):
+        rows = x[b][x[b][:, 1] > 20]
+        assert int(vc[b]) == len(rows)
+        got = y[b].cpu().numpy()
+        assert np.array_equal(got[:len(rows)], rows) and (got[len(rows):] == -1).all()
