@@ -235,6 +235,10 @@ int pack_activations(const int32_t* x, int8_t* xp, int n, int c, int hw, hipStre
 int unpack_activations(const int8_t* xp, int32_t* x, int n, int c, int hw, hipStream_t s);
 int pack_weights(const int32_t* w, int8_t* wp, int oc, int ic, int kh, int kw, hipStream_t s);
 int conv_igemm(const int8_t* xp, const int8_t* wp, void* out, ConvGeom g, const Epilogue& ep, hipStream_t s);
+// groups == 1 on int32 tensors through packed operands: workspace of cvmhip_conv2d_workspace_bytes()
+int conv2d_two_launches(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y, int n, int ic, int h, int wd, int oc, int oh, int ow,
+                        int kh, int kw, int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w, void* workspace, hipStream_t s);
+bool conv_kernel_forced();   // cvmhip_set_conv_tuning has named a kernel, configuration or tile for this thread
 // groups > 1 on int32 tensors (conv_planes.hip)
 int conv_grouped_i32(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y, int n, int ic, int h, int wd, int oc, int oh, int ow,
                      int kh, int kw, int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w, int groups, hipStream_t s);

@@ -3253,6 +3253,24 @@ int conv_seq_launch(const void* dev_table, int nlayers, void* sync, double ops, 
   return check_launch("conv_seq");
 }
 
+int conv2d_two_launches(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y, int n, int ic, int h, int wd, int oc, int oh, int ow,
+                        int kh, int kw, int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w, void* workspace, hipStream_t s) {
+  int8_t* xp = reinterpret_cast<int8_t*>(workspace);
+  int8_t* wp = xp + packed_act_bytes((int64_t)n * h * wd, ic);
+  const int rc = pack_operands(x, xp, n, ic, h * wd, w, wp, oc, kh, kw, s);
+  if (rc) return rc;
+  ConvGeom g = {};
+  g.N = n; g.H = h; g.W = wd; g.Cp = pad_channels(ic); g.C = ic;
+  g.OC = oc; g.OH = oh; g.OW = ow;
+  g.KH = kh; g.KW = kw; g.SH = stride_h; g.SW = stride_w; g.PH = pad_h; g.PW = pad_w; g.DH = dil_h; g.DW = dil_w;
+  Epilogue ep = {};
+  ep.bias = bias;
+  ep.out_mode = OUT_I32_NCHW;
+  return conv_igemm(xp, wp, y, g, ep, s);
+}
+
+bool conv_kernel_forced() { return t_conv_tuning.kernel != CONV_KERNEL_AUTO || t_conv_tuning.wave_cfg >= 0 || t_conv_tuning.tile_wm > 0; }
+
 }  // namespace cvmhip
 
 using namespace cvmhip;
@@ -3306,36 +3324,6 @@ int cvmhip_set_seq_chains(int on) {
 size_t cvmhip_conv2d_workspace_bytes(int n, int ic, int h, int w, int oc, int kh, int kw, int groups) {
   if (groups != 1) return 0;
   return packed_act_bytes((int64_t)n * h * w, ic) + packed_weight_bytes(oc, ic, kh, kw);
-}
-
-int cvmhip_conv2d(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y,
-                  int n, int ic, int h, int wd, int oc, int kh, int kw,
-                  int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w,
-                  int groups, void* workspace, size_t workspace_bytes, void* stream) {
-  if (!x || !w || !y) return arg_error("conv2d null tensor");
-  if (n < 1 || ic < 1 || h < 1 || wd < 1 || oc < 1 || kh < 1 || kw < 1 || stride_h < 1 || stride_w < 1 ||
-      pad_h < 0 || pad_w < 0 || dil_h < 1 || dil_w < 1 || groups < 1 || ic % groups || oc % groups)
-    return arg_error("conv2d attributes");
-  const int oh = (h + 2 * pad_h - (dil_h * (kh - 1) + 1)) / stride_h + 1;
-  const int ow = (wd + 2 * pad_w - (dil_w * (kw - 1) + 1)) / stride_w + 1;
-  if (h + 2 * pad_h < dil_h * (kh - 1) + 1 || wd + 2 * pad_w < dil_w * (kw - 1) + 1) return arg_error("conv2d kernel exceeds input");
-  hipStream_t s = as_stream(stream);
-  if (groups > 1)
-    return conv_grouped_i32(x, w, bias, y, n, ic, h, wd, oc, oh, ow, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, groups, s);
-  const size_t need = cvmhip_conv2d_workspace_bytes(n, ic, h, wd, oc, kh, kw, 1);
-  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return arg_error("conv2d workspace");
-  int8_t* xp = reinterpret_cast<int8_t*>(workspace);
-  int8_t* wp = xp + packed_act_bytes((int64_t)n * h * wd, ic);
-  const int rc = pack_operands(x, xp, n, ic, h * wd, w, wp, oc, kh, kw, s);
-  if (rc) return rc;
-  ConvGeom g = {};
-  g.N = n; g.H = h; g.W = wd; g.Cp = pad_channels(ic); g.C = ic;
-  g.OC = oc; g.OH = oh; g.OW = ow;
-  g.KH = kh; g.KW = kw; g.SH = stride_h; g.SW = stride_w; g.PH = pad_h; g.PW = pad_w; g.DH = dil_h; g.DW = dil_w;
-  Epilogue ep = {};
-  ep.bias = bias;
-  ep.out_mode = OUT_I32_NCHW;
-  return conv_igemm(xp, wp, y, g, ep, s);
 }
 
 size_t cvmhip_dense_workspace_bytes(int m, int k, int n) {

@@ -35,6 +35,27 @@ def test_conv_operand_packing(n, c, h, w, oc, k, dev):
     assert np.array_equal(got, oracle.conv2d(x, wt, None, (1, 1), (k // 2, k // 2)))
 
 
+@pytest.mark.parametrize("n,c,h,w,oc,k,strides,padding,dilation", [
+    # one launch, K split over a workgroup: halves of the channels of 1 and 0, 1 and 1, 2 and 1; ends of K inside a chunk
+    (1, 1, 1, 4, 1, 1, (1, 1), (0, 0), (1, 1)), (1, 2, 3, 5, 33, 1, (1, 1), (0, 0), (1, 1)), (2, 3, 9, 7, 32, 3, (1, 1), (1, 1), (1, 1)),
+    (1, 31, 6, 6, 31, 1, (1, 1), (1, 1), (1, 1)), (3, 33, 5, 13, 65, 1, (2, 2), (0, 0), (1, 1)), (1, 640, 8, 4, 34, 1, (1, 1), (0, 0), (1, 1)),
+    (1, 71, 11, 9, 40, 3, (1, 2), (2, 1), (2, 1)), (2, 64, 12, 12, 64, 3, (2, 2), (0, 0), (1, 1)), (1, 17, 40, 3, 5, 3, (1, 1), (3, 4), (1, 3)),
+    # beyond the tiles of that: filters in LDS, one and two rounds of pixel groups, a last group of few pixels
+    (5, 20, 41, 37, 80, 1, (1, 1), (0, 0), (1, 1)), (1, 255, 50, 51, 200, 1, (1, 1), (0, 0), (1, 1)), (16, 33, 57, 57, 130, 1, (1, 1), (0, 0), (1, 1)),
+    (4, 256, 33, 32, 129, 1, (2, 1), (1, 0), (1, 1)),
+    # the first sizes of the general path: K of 641 and 257, tiles
+    (1, 641, 8, 4, 34, 1, (1, 1), (0, 0), (1, 1)), (1, 257, 60, 64, 128, 1, (1, 1), (0, 0), (1, 1)), (2, 64, 56, 57, 64, 3, (1, 1), (1, 1), (1, 1)),
+])
+def test_conv_direct(n, c, h, w, oc, k, strides, padding, dilation, dev):
+    cid = "direct-%d-%d-%d-%d" % (c, h, w, oc)
+    x = synth.tensor(cid, "x", (n, c, h, w), -300, 300)   # narrowed like the reference narrows
+    wt = synth.tensor(cid, "w", (oc, c, k, k), -300, 300)
+    b = synth.tensor(cid, "b", (oc,), -2 ** 31, 2 ** 31 - 1)
+    for bias in (None, b):
+        got = hipops.conv2d(T(x, dev), T(wt, dev), None if bias is None else T(b, dev), strides, padding, dilation).cpu().numpy()
+        assert np.array_equal(got, oracle.conv2d(x, wt, bias, strides, padding, dilation))
+
+
 @pytest.mark.parametrize("m,k,n", [
     (1, 17, 5), (3, 31, 40),       # a granule that ends inside the channels, one that is all padding
     (33, 64, 32), (70, 100, 7),
