@@ -21,8 +21,10 @@
 // a barrier all wavefronts read at the same time and then compute at the same time.  On the way, same network at batch 1:
 // all operand reads of a chunk before its first product instead of a read and a wait each 62 -> 52 us; filters requested
 // inside the loop that uses them 54 -> 45; plain layers without the tests for other forms 45 -> 41.5; filters and places
-// from LDS (no scalar register is spilled any more) and a sum without LDS shuffles 41.5 -> 39.  No difference: 1024 threads, another priority for half of
-// the wavefronts, pixels an odd number of granules apart.
+// from LDS (no scalar register is spilled any more) and a sum without LDS shuffles 41.5 -> 39; a wavefront beside the others that fetches filters and
+// clears borders 39 -> 37, two by two tiles for layers of 32 channels -> 36.5.  No difference: 1024 threads, another priority for half of
+// the wavefronts, pixels an odd number of granules apart.  Slower: all operands of a 16-channel item requested at once, or of a 64-channel one (the
+// launch is bound by LDS transfers and vector instructions in turn, not by the latency of either); the next layer's head in scalar registers (spills).
 #include <string.h>
 
 #include "conv_mfma.h"
@@ -31,7 +33,7 @@ namespace cvmhip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-constexpr int RES_THREADS = 512, RES_WAVES = RES_THREADS / 64;
+constexpr int RES_THREADS = 512, RES_WAVES = RES_THREADS / 64;   // the wavefronts that compute; one more prepares the next layer
 constexpr int RES_CHUNK = 3;        // K steps computed together (a 3 x 3 filter over 16, 64, 128, ... channels is whole chunks)
 constexpr int RES_LDS_MOST = 150 * 1024;
 
@@ -51,9 +53,9 @@ struct ResHead {
   // border of the output map: start, bytes of a stored row, of the gap between two rows, in front of the first pixel; rows
   int border_at, border_row, border_side, border_edge, border_rows;
   // filter of the next convolution, to be fetched during this layer: KiB, where to, where from
-  int next_kb, next_at, unused;
+  int next_kb, next_at, form;           // form: RES_PLAIN: res_form()
   const int8_t* next;
-  int unused2[6];
+  int unused[6];
 };
 // Byte offsets of a lane's pixel of a tile, in LDS, without what the tile adds: first tap of the window, result, residual; and
 // the lane's bytes of a channel tile's biases.
@@ -189,24 +191,33 @@ __host__ __device__ inline ResPlace res_place(const ResGeometry& g, int p, int y
 // compiler, which could not tell them from the operands it waits for.)
 __device__ __forceinline__ void res_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-__device__ __forceinline__ void res_fetch_next(const ResHead& h, uint32_t lds_base, int wave, int lane) {
-  for (int k = wave; k < h.next_kb; k += RES_WAVES) {
-    const int8_t* from = h.next + (unsigned)k * 1024u + (unsigned)lane * 16u;
-    // (the s_nop is the wait state between a scalar write to M0 and its use)
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_base + (uint32_t)(h.next_at + k * 1024)) : "memory");
-  }
+__device__ __forceinline__ void res_fetch_next(const ResHead& h, uint32_t lds_base, int lane) {
+  const uint32_t own = (uint32_t)lane * 16u;
+  uint32_t to = lds_base + (uint32_t)h.next_at;
+  const int8_t* from = h.next;
+  int left = h.next_kb;
+  // (the s_nop is the wait state between a scalar write to M0 and its use)
+  for (; left >= 4; left -= 4, from += 4096, to += 4096)
+    asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\t"
+                 "s_add_u32 m0, %5, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\t"
+                 "s_add_u32 m0, %5, 0x800\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4\n\t"
+                 "s_add_u32 m0, %5, 0xc00\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %4" ::"v"(own), "v"(own + 1024u), "v"(own + 2048u), "v"(own + 3072u),
+                 "s"(from), "s"(to)
+                 : "memory", "scc");
+  for (; left > 0; --left, from += 1024, to += 1024)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(own), "s"(from), "s"(to) : "memory");
 }
 
-__device__ __forceinline__ void res_border(const ResHead& h, char* lds, int tid) {
+__device__ __forceinline__ void res_border(const ResHead& h, char* lds, int lane) {
   if (h.flags & RES_BORDER) {
     // the border is three runs: in front of the first pixel, behind the last one, and between the rows
     const int row = h.border_row, side = h.border_side, edge = h.border_edge, rows = h.border_rows, at = h.border_at;
     const uint4 zero = make_uint4(0, 0, 0, 0);
-    for (int i = tid * 16; i < edge; i += RES_THREADS * 16) {
+    for (int i = lane * 16; i < edge; i += 64 * 16) {
       *reinterpret_cast<uint4*>(lds + at + i) = zero;
       *reinterpret_cast<uint4*>(lds + at + edge + rows * row - side + i) = zero;
     }
-    for (int y = tid; y < rows - 1; y += RES_THREADS)
+    for (int y = lane; y < rows - 1; y += 64)
       for (int i = 0; i < side; i += 16) *reinterpret_cast<uint4*>(lds + at + edge + (y + 1) * row - side + i) = zero;
   }
 }
@@ -288,6 +299,102 @@ __device__ __forceinline__ void res_plain_conv(const ResHead& h, char* lds, int 
   }
 }
 
+// The same for layers of an even number of channel tiles and STEPS of K known here: TM channel tiles share the operands of TP pixel
+// tiles, all of an item's operands are requested at once, and the next item's behind its products.  Two by two tiles take a
+// 16 x 16 x 32 layer from 2 600 to 2 330 clocks (3 050 to 2 660 with a residual) against one by four.
+template <int TM, int TP, int STEPS>
+__device__ __forceinline__ void res_item_conv(const ResHead& h, char* lds, int wave, int lane) {
+  if (wave >= h.items) return;
+  const ResPlace own = *reinterpret_cast<const ResPlace*>(lds + (h.places_at + lane * 16));
+  const char* rec = lds + (h.places_at + 1024 + wave * 64);
+  int tap[STEPS];
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) tap[u] = *reinterpret_cast<const int*>(lds + (h.taps_at + (lane >> 4) * 4 + u * 16));
+  const int next_channels = h.chunks * (RES_CHUNK * 1024);   // from a channel tile's filter to the next one's
+  v4i a[STEPS][TM], x[STEPS][TP], acc[TM][TP], bias[TM], src, dst, res;
+  uint32_t residual[TM][TP];
+  int filter, bias_at;
+  auto record = [&]() {
+    src = *reinterpret_cast<const v4i*>(rec);
+    filter = *reinterpret_cast<const int*>(rec + 48);
+    bias_at = *reinterpret_cast<const int*>(rec + 52);
+    dst = *reinterpret_cast<const v4i*>(rec + 16);
+    if (h.residual) res = *reinterpret_cast<const v4i*>(rec + 32);
+  };
+  auto request = [&]() {
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m) a[u][m] = *reinterpret_cast<const v4i*>(lds + (filter + lane * 16) + m * next_channels + u * 1024);
+#pragma unroll
+      for (int j = 0; j < TP; ++j) x[u][j] = *reinterpret_cast<const v4i*>(lds + (own.src + src[j] + tap[u]));
+    }
+  };
+  record();
+  request();
+  for (int item = wave;;) {
+    const v4i to = dst, beside = res;
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      bias[m] = *reinterpret_cast<const v4i*>(lds + (bias_at + own.bias + m * 64));
+      if (h.residual) {
+#pragma unroll
+        for (int j = 0; j < TP; ++j) residual[m][j] = *reinterpret_cast<const uint32_t*>(lds + (own.res + beside[j] + m * 16));
+      }
+    }
+    item += RES_WAVES;
+    const bool more = item < h.items;
+    if (more) {
+      rec += RES_WAVES * 64;
+      record();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int j = 0; j < TP; ++j) acc[m][j] = bias[m];
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u)
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int j = 0; j < TP; ++j) acc[m][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u][m], x[u][j], acc[m][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) request();
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int j = 0; j < TP; ++j) asm volatile("s_nop 15" : "+v"(acc[m][j]));   // as in res_products
+    if (h.residual) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int j = 0; j < TP; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[m][j][e] = res_clamp(wadd(res_clamp(acc[m][j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[m][j] >> (8 * e))), h.lo2, h.hi2) >> h.shift2;
+    } else {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int j = 0; j < TP; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[m][j][e] = res_clamp(acc[m][j][e], h.lo, h.hi) >> h.shift;
+    }
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int j = 0; j < TP; ++j) {
+        const int32_t v[4] = {acc[m][j][0], acc[m][j][1], acc[m][j][2], acc[m][j][3]};
+        *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j] + m * 16)) = res_pack(v);
+      }
+    if (!more) return;
+  }
+}
+// (TM, TP, STEPS) of res_item_conv in one number; 0: res_plain_conv
+__host__ __device__ constexpr int res_form(int tm, int tp, int steps) { return steps * 16 + tm * 8 - 8 + tp; }
+#define RES_FORMS(F) F(2, 2, 3) F(2, 2, 5)
+
 // any convolution, one pixel tile at a time
 __device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds, int32_t* out_host, int img, int wave, int lane) {
   const ResGeometry g = res_geometry(L);
@@ -336,7 +443,7 @@ __device__ __forceinline__ ResHead res_head(ResTable L) {
   return h;
 }
 
-__global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* table, int nlayers, int images,
+__global__ void __launch_bounds__(RES_THREADS + 64) k_conv_resident(const ResLayer* table, int nlayers, int images,
                                                                const cvmhip_resident_call call) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int img = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
@@ -349,15 +456,29 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
     const int lines = nlayers * (int)sizeof(ResLayer) / 64;
     typedef const __attribute__((address_space(4))) int* Word;
     int sum = 0;
-    for (int i = wave; i < lines; i += RES_WAVES) sum += *(Word)((uintptr_t)table + 64 * i);
+    for (int i = wave; i < lines; i += RES_WAVES + 1) sum += *(Word)((uintptr_t)table + 64 * i);
     asm volatile("" ::"s"(sum));
   }
+  // The last wavefront fetches the next layer's filter and clears the border of this layer's map while the others compute: as
+  // the first thing all of them did behind the barrier it was 300 to 1 600 of a layer's 4 000 clocks.
+  if (wave == RES_WAVES) {
+    for (int l = 0; l < nlayers; ++l, ++L) {
+      const ResHead h = res_head(L);
+      res_barrier();
+      res_fetch_next(h, lds_base, lane);
+      res_border(h, lds, lane);
+    }
+  } else {
   for (int l = 0; l < nlayers; ++l, ++L) {
     const ResHead h = res_head(L);
     res_barrier();
-    res_fetch_next(h, lds_base, wave, lane);
-    res_border(h, lds, tid);
     if (h.flags & RES_PLAIN) {
+#define RES_CASE(TM, TP, STEPS) case res_form(TM, TP, STEPS): res_item_conv<TM, TP, STEPS>(h, lds, wave, lane); continue;
+      switch (h.form) {
+        RES_FORMS(RES_CASE)
+        default: break;
+      }
+#undef RES_CASE
       if (h.tp == 1) res_plain_conv<1>(h, lds, wave, lane);
       else if (h.tp == 2) res_plain_conv<2>(h, lds, wave, lane);
       else res_plain_conv<4>(h, lds, wave, lane);
@@ -449,6 +570,7 @@ __global__ void __launch_bounds__(RES_THREADS) k_conv_resident(const ResLayer* t
       }
     }
   }
+  }
   if (call.flag_host) {
     const uint32_t ticket = tid == 0 ? call.counter[1] + 1 : 0;
     __threadfence_system();
@@ -522,16 +644,32 @@ size_t cvmhip_resident_tensor_bytes(int c, int h, int w, int border_y, int borde
   return (size_t)res_cp(c) * (h + 2 * border_y) * (w + 2 * border_x);
 }
 
-// as many pixel tiles per item (a filter fragment read once serves them all) as still leave every wavefront an item
-static int res_tiles(int ptiles, int octiles) { return ptiles * octiles >= 4 * RES_WAVES ? 4 : ptiles * octiles >= 2 * RES_WAVES ? 2 : 1; }
+// Tiles of an item, as many as still leave every wavefront one: a filter fragment read once serves all pixel tiles, an activation
+// operand all channel tiles.  Two by two reads 8 operands for 8 products of two steps where one by four reads 10.
+struct ResTiling {
+  int tm, tp, form;
+};
+static ResTiling res_tiling(int ptiles, int octiles, int steps) {
+  const int tp = ptiles * octiles >= 4 * RES_WAVES ? 4 : ptiles * octiles >= 2 * RES_WAVES ? 2 : 1;
+  auto known = [&](int tm, int t) {
+#define RES_KNOWN(TM, TP, STEPS) if (tm == TM && t == TP && steps == STEPS) return true;
+    RES_FORMS(RES_KNOWN)
+#undef RES_KNOWN
+    return false;
+  };
+  if (tp == 4 && octiles % 2 == 0 && ptiles % 2 == 0 && known(2, 2)) return {2, 2, res_form(2, 2, steps)};
+  return {1, tp, 0};
+}
+static int res_steps(int c, int kh, int kw) { return (kh * kw * res_cp(c) + 63) / 64; }
 static size_t res_places_at(int oc, int c, int kh, int kw) {
   return ((size_t)(res_cp(oc) / 16) * 1024 + 16) * res_chunks(c, kh, kw) * RES_CHUNK + (size_t)res_cp(oc) * 4;
 }
 
 size_t cvmhip_resident_filter_bytes(int oc, int c, int kh, int kw, int oh, int ow) {
   if (oc < 1 || c < 1 || kh < 1 || kw < 1 || oh < 1 || ow < 1) return 0;
-  const int ptiles = (oh * ow + 15) / 16, octiles = res_cp(oc) / 16, tp = res_tiles(ptiles, octiles);
-  return (res_places_at(oc, c, kh, kw) + 1024 + (size_t)octiles * ((ptiles + tp - 1) / tp) * sizeof(ResItem) + 1023) / 1024 * 1024;
+  const int ptiles = (oh * ow + 15) / 16, octiles = res_cp(oc) / 16;
+  const ResTiling t = res_tiling(ptiles, octiles, res_steps(c, kh, kw));
+  return (res_places_at(oc, c, kh, kw) + 1024 + (size_t)(octiles / t.tm) * ((ptiles + t.tp - 1) / t.tp) * sizeof(ResItem) + 1023) / 1024 * 1024;
 }
 
 int cvmhip_resident_pack_filter(const int32_t* w, const int32_t* bias, void* dst, int oc, int c, int kh, int kw, int dil_h, int dil_w,
@@ -628,11 +766,14 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d,
       h.taps_at = h.w_at + L.octiles * h.chunks * (RES_CHUNK * 1024);
       h.bias_at = h.taps_at + h.chunks * (RES_CHUNK * 16);
       // whole tiles, which all lie like the first one (part of a row, or whole rows), and a result for LDS only
-      const int ptiles = (L.P + 15) / 16, tp = res_tiles(ptiles, L.octiles);
+      const int ptiles = (L.P + 15) / 16;
+      const ResTiling tiling = res_tiling(ptiles, L.octiles, res_steps(in.c, d->kh, d->kw));
+      const int tp = tiling.tp, groups = L.octiles / tiling.tm;
       if (!(h.flags & (RES_CHAIN | RES_CHAIN2 | RES_MASK | RES_OUT)) && L.P % (16 * tp) == 0 && (out.w % 16 == 0 || 16 % out.w == 0)) {
         h.flags |= RES_PLAIN;
         h.tp = tp;
-        h.items = L.octiles * (ptiles / tp);
+        h.form = tiling.form;
+        h.items = groups * (ptiles / tp);
         const size_t at = res_places_at(out.c, in.c, d->kh, d->kw);
         h.places_at = h.w_at + (int)at;
         const ResGeometry g = {L.P, L.OW, L.div_ow, L.src, L.step_y, L.step_x, L.dst, L.dst_row, L.ocp, L.res, L.res_row};
@@ -641,12 +782,12 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d,
         for (int l = 0; l < 64; ++l) own[l] = res_place(g, l & 15, (l & 15) / g.OW, l);
         const ResPlace first = res_place(g, 0, 0, 0);
         for (int i = 0; i < h.items; ++i) {
-          const int ot = i % L.octiles;
+          const int ot = i % groups * tiling.tm;
           items[i] = ResItem{};
           items[i].filter = h.w_at + ot * h.chunks * (RES_CHUNK * 1024);
           items[i].bias = h.bias_at + ot * 64;
           for (int t = 0; t < tp; ++t) {
-            const int p = (i / L.octiles * tp + t) * 16;
+            const int p = (i / groups * tp + t) * 16;
             const ResPlace q = res_place(g, p, p / g.OW, 0);
             items[i].src[t] = q.src - first.src;
             items[i].dst[t] = q.dst - first.dst + ot * 16;
@@ -688,7 +829,7 @@ int cvmhip_resident_launch(const void* dev_table, int nlayers, int images, size_
   char desc[64] = "";
   if (kernel_timing_enabled()) snprintf(desc, sizeof(desc), "%d layers in LDS, %d images", nlayers, images);
   KernelTimer timer("k_conv_resident", ops, as_stream(stream), bytes, desc);
-  k_conv_resident<<<(unsigned)images, RES_THREADS, lds_bytes, as_stream(stream)>>>(reinterpret_cast<const ResLayer*>(dev_table), nlayers, images,
+  k_conv_resident<<<(unsigned)images, RES_THREADS + 64, lds_bytes, as_stream(stream)>>>(reinterpret_cast<const ResLayer*>(dev_table), nlayers, images,
                                                                                   call ? *call : cvmhip_resident_call{});
   return check_launch("conv_resident");
 }
