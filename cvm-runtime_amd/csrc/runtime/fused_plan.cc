@@ -1009,6 +1009,8 @@ void HipGraphRuntime::BuildGroups() {
   }
 }
 
+void* HipGraphRuntime::PackedImage(const PlanStep& st) { return static_cast<DeviceBuffer*>(st.aux.get())->ptr; }
+
 void HipGraphRuntime::RunStep(PlanStep& st) {
   switch (st.kind) {
     case PlanStep::NODE: {

@@ -136,7 +136,7 @@ class HipGraphRuntime {
   void SetData(const int32_t* host, const Shape& shape);
   void SetDataI8(const int8_t* host, const Shape& shape);   // the same for an input given as int8 bytes
   void Run();      // replays the captured graph once it exists
-  void Launch();   // issues every launch of a run on the stream, one by one
+  void Launch(size_t first = 0);   // issues every launch of a run on the stream, one by one
   void CopyOutputTo(int index, int32_t* host);  // synchronises the stream
   // every output copied into pinned host memory owned by the runtime (valid until the next call); one synchronisation
   const std::vector<const int32_t*>& FetchOutputs();
@@ -249,6 +249,16 @@ class HipGraphRuntime {
   void* call_exec_ = nullptr;    // the same launches and the export of the outputs
   bool call_imports_ = false;    // and, in front of them, the import of the input
   bool call_refused_ = false;    // that could not be captured
+  // The input packed by a launch in front of the call's graph while the host copies it (cvmhip_import_stem_i8)
+  bool call_packs_ = false;      // call_exec_ begins behind that packing
+  bool gate_refused_ = false;    // such a launch has given up: not again with this model
+  bool GateEligible() const;
+  void GateInput(const int8_t* host);
+  bool GateGaveUp();
+  static void* PackedImage(const PlanStep& st);
+  void* gate_host_ = nullptr;    // pinned: progress (8 bytes), error word
+  void* gate_dev_ = nullptr;     // the launch's copy of the progress
+  uint32_t gate_ticket_ = 0;
   int graph_state_ = 0;  // 0 undecided, -1 eager for good, 1 before the first run, 2 ready to capture, 3 captured
 
   // Test and tuning hooks, read from the environment once, when the model is constructed (never on the
@@ -259,6 +269,8 @@ class HipGraphRuntime {
   struct Hooks {
     bool fold_bias = true, fuse = true, graph = true, dw_on_mfma = true, seq = true, seq_forced = false, pool_fuse = true, head_pair = true, head_group = true, conv_group = true;
     int conv_kernel = 0, wave_cfg = -1, tile_wm = 0, tile_wn = 0;
+    // CVM_HIP_GATE_US=<us> patience of the packing launch with the host's copy (0: gives up at once; default half a second)
+    uint32_t gate_us = 500000;
     // layer-sequence launches: CVM_HIP_SEQ_SPIN=<polls> patience of a wait at a layer boundary (0: every wait gives up at once)
     int seq_spin = 2000000;
     // CVM_HIP_RESIDENT=0: no launches with the maps in LDS; =1: no layer sequences, which a measurement at load may

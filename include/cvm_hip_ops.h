@@ -151,8 +151,8 @@ int cvmhip_non_max_suppression(int32_t* x, const int32_t* valid_count, int32_t* 
 /* The same operator for callers that cannot allocate device memory or bring a workspace (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The scratch is
  * a fixed array inside the library's code object, cvmhip_nms_static_capacity_bytes() bytes (2 MiB) per GPU,
- * held until the process ends; a call whose cvmhip_nms_workspace_bytes(batches, n, k) exceeds it returns
- * CVMHIP_ERR_ARG.  The call allocates and frees nothing.  All calls on one GPU share the array: calls that
+ * held until the process ends; a call whose rows (cvmhip_nms_workspace_bytes(batches, n, k) without what it holds for the overlap
+ * masks of the walk, 80 bytes a row, which this entry does without) exceed it returns CVMHIP_ERR_ARG.  The call allocates and frees nothing.  All calls on one GPU share the array: calls that
  * overlap in time on one GPU (two streams, two threads) race and must be serialised by the caller.  The
  * first call on a device looks the array's address up (hipGetSymbolAddress); make it outside stream capture. */
 size_t cvmhip_nms_static_capacity_bytes(void);
@@ -186,6 +186,15 @@ int cvmhip_widen_clamp_i8(const void* src, int32_t* dst, int64_t count, int32_t 
 int cvmhip_import_bytes(void* dst, const void* src_host, size_t bytes, void* stream);
 int cvmhip_export_words(const void* const* src, void* const* dst_host, const int64_t* words, int count, const uint32_t* status,
                         uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, void* stream);
+/* An int8 image batch in pinned host memory (16-byte aligned, 16 readable bytes behind it) into the layout of cvmhip_pack_stem_input_i8, by a launch that may be
+ * issued before the bytes are there: the host copies chunks of cvmhip_import_stem_rows image rows (0: not available for these sizes), all channels
+ * of them, image by image, and stores `ticket << 32 | chunks copied` to *progress_host (pinned) behind each.  Waits are bounded by patience_us: a
+ * launch that gives up sets *error_host (pinned), and what it was to write is undefined.  `progress_dev`: a device word of the caller's,
+ * zeroed once; `ticket` differs from the one before it. */
+int cvmhip_import_stem_rows(int n, int c, int h, int w);
+int cvmhip_import_stem_i8(const void* src_host, int32_t range, void* xs, int n, int c, int h, int w, int kh, int kw, int stride_h, int stride_w,
+                          int pad_h, int pad_w, const uint64_t* progress_host, uint64_t* progress_dev, uint32_t* error_host, uint32_t ticket,
+                          uint32_t patience_us, void* stream);
 /* Waits until *flag_host is `ticket`, and returns an error if the stream comes to its end without that. */
 int cvmhip_export_wait(const uint32_t* flag_host, uint32_t ticket, void* stream);
 int cvmhip_copy_h2d(void* dst, const void* src, size_t bytes, void* stream);

@@ -38,6 +38,35 @@ def test_inference_ends(n, c, h, w, k, stride, precision, second_reader, dev):
     model.close()
 
 
+@pytest.mark.parametrize("patience", ["", "0"])   # the packing launch follows the host's copy; it gives up at once and the call is run again
+@pytest.mark.parametrize("n,c,h,w,k,stride,precision", [
+    (3, 3, 224, 225, 3, 2, 6),        # rows that begin anywhere in a granule, several chunks to an image, the clamp
+    (1, 3, 511, 513, 7, 1, 8),        # one image
+    (300, 1, 31, 33, 5, 2, 8),        # many images to a chunk's worth of bytes
+    (2, 4, 5, 9001, 3, 1, 8),         # a band of one row
+    (5, 3, 260, 90, 3, 1, 8),
+])
+def test_packing_follows_the_copy(n, c, h, w, k, stride, precision, patience, dev, monkeypatch):
+    if patience:
+        monkeypatch.setenv("CVM_HIP_GATE_US", patience)
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "0")
+    g = graphgen.GraphBuilder("io-gate-%d-%d-%d" % (n, c, w))
+    x = g.var("data", (n, c, h, w), precision)
+    js, pb = g.build([g.conv_relu_q(x, 8, k, stride, k // 2)])
+    model = runtime.HipModel(js, pb)
+    params = graphgen.load_params(pb)
+    top = (1 << (precision - 1)) - 1
+    for call in range(5):   # eager, capture, replays; each on another input
+        data = synth.tensor("io-gate", "x%d" % call, (n, c, h, w), -128, 127)
+        want = og.run_graph(js, params, np.clip(data, -top, top))[0].ravel()
+        got = np.frombuffer(model.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want), "call %d" % call
+        if call == 3:   # the same input again, as a run of its own
+            model.run()
+            assert np.array_equal(np.frombuffer(model.get_output(), np.int8).astype(np.int32), want)
+    model.close()
+
+
 def test_many_calls_in_a_row(dev):
     """Past the 64 calls after which the stream itself is waited for; outputs of several kilobytes."""
     g, heads = graphgen.conv_op_graph(n=1, c=32, h=9, w=9, oc=40)
