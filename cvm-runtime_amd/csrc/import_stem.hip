@@ -9,14 +9,16 @@
 // The host counts chunks of rows in a word of pinned memory.  Only the first workgroup reads that word (a trip over the bus); it
 // repeats the count in device memory, where the others look.  Every wait is bounded: a launch that gives up writes nothing
 // more, sets *error_host and ends.
-// Bound by the bus (46 GB/s in reads of 64 bytes; 2.4 MB 58 us, 7.5 MB 173 us) with 6 KiB in flight from each of 256 workgroups.
+// Bound by the bus, or by the host's copy where its source is not in the CPU's caches (44 GB/s).  64 workgroups with 6 KiB in flight each:
+// the bus carries 52 to 55 GB/s for 256 KiB in flight and 42 to 46 for a megabyte (256 workgroups: ResNet-50 at batch 50 1 016 us a call,
+// 64 982, 32 1 037).
 #include <algorithm>
 
 #include "conv_mfma.h"
 
 namespace cvmhip {
 
-constexpr int IMPORT_THREADS = 256, IMPORT_GROUPS = 256, IMPORT_BAND = 6144, IMPORT_CHUNK = 65536, IMPORT_LDS_MOST = 48 * 1024;
+constexpr int IMPORT_THREADS = 256, IMPORT_GROUPS = 64, IMPORT_BAND = 6144, IMPORT_CHUNK = 65536, IMPORT_LDS_MOST = 48 * 1024;
 constexpr uint32_t IMPORT_GIVEN_UP = 0xffffffffu;
 
 struct ImportStem {
