@@ -573,9 +573,9 @@ __global__ void __launch_bounds__(RES_THREADS + 64) k_conv_resident(const ResLay
   }
   if (call.flag_host) {
     const uint32_t ticket = tid == 0 ? call.counter[1] + 1 : 0;
-    __threadfence_system();
-    __syncthreads();
+    stores_done_barrier();
     if (tid == 0) {
+      __threadfence_system();
       const uint32_t before = __hip_atomic_fetch_add(call.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
       if (before == (uint32_t)images - 1) {
         call.counter[0] = 0;

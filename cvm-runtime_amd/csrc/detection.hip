@@ -771,8 +771,7 @@ k_nms_walk(const int32_t* __restrict__ valid_count, const int32_t* __restrict__ 
       uint32_t* own = masks + b * mask_words * 2 + (int64_t)base * (NMS_PAIRS_WORDS * 2);
       __syncthreads();
       nms_pairs(s_row, total, iou_threshold, own, part * NMS_WAVES + wave, parts * NMS_WAVES, lane);
-      // one fence for the workgroup: a wavefront's own is a write-back of the L2, which takes them one at a time
-      __syncthreads();
+      stores_done_barrier();
       if (parts > 1) {
         if (tid == 0) s_k = __hip_atomic_fetch_add(&tl[NMS_ARRIVED + cls], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();

@@ -159,7 +159,7 @@ int cvmhip_import_bytes(void* dst, const void* src_host, size_t bytes, void* str
   return check_launch("import_bytes");
 }
 
-// Device -> pinned host memory, and a word that says so.  Every workgroup makes its stores visible to the host before it
+// Device -> pinned host memory, and a word that says so.  Every workgroup makes its stores visible to the host, by one fence, before it
 // counts itself out; the last one to count stores the ticket.  The host polls that word instead of waiting for the
 // stream (7.5 us from launch to seen, against 11.7 us for a launch and a stream synchronisation, and no copy calls).
 struct ExportArgs {
@@ -182,9 +182,9 @@ __global__ void __launch_bounds__(256) k_export(ExportArgs a, const uint32_t* __
     if (at < a.words[k]) a.dst[k][at] = a.src[k][at];
   }
   if (status && blockIdx.x == 0 && threadIdx.x == 0) *status_host = *status;
-  __threadfence_system();
-  __syncthreads();
+  stores_done_barrier();
   if (threadIdx.x == 0) {
+    __threadfence_system();
     const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
     if (before == gridDim.x - 1) {
       counter[0] = 0;

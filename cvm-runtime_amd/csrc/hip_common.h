@@ -80,6 +80,14 @@ __device__ __forceinline__ int32_t wave_scan_add(int32_t v) {
 }
 __device__ __forceinline__ int32_t wave_sum(int32_t v) { return __builtin_amdgcn_readlane(wave_scan_add(v), 63); }
 
+// In front of what one thread of a workgroup tells others about the stores of all: every wavefront's stores are performed, then the
+// thread fences.  (A fence of every wavefront's own is a write-back of the L2 each, which
+// takes them one at a time: 256 workgroups of nine wavefronts that end so add 32 us, with one fence each hardly anything.)
+__device__ __forceinline__ void stores_done_barrier() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 // Requantisation parameters prepared on the host once per launch.
 // mode 0: max==0 -> 0;  1: b>=31 -> a>>31;  2: p+b>=32 -> rounding shift, no clip;
 // 3: saturate on pre-shifted bounds, else rounding shift

@@ -966,12 +966,12 @@ void HipGraphRuntime::AllocOutputStage() {
   }
 }
 
-// A call of a model that is one launch with the maps in LDS: that launch fetches the image from pinned memory itself, and
-// writes the result and the ticket there (ResNet-20 at batch 1: 55 -> 52 us).  Up to 128 KiB of input: the launch's reads are
-// short ones, at 196 KB (batch 64) they already take as long as the launches they save, and a larger input is copied to the
-// pinned buffer in pieces behind which the device already reads.
+// A call of a model that is one launch with the maps in LDS: that launch fetches the images from pinned memory itself, and
+// writes the result and the ticket there (ResNet-20, us a call with an import in front of the launch and without: batch 1 50 and 47, 64
+// 57 and 53, 128 68 and 61, 256 84 and 78).  Larger inputs than measured are copied to the pinned buffer in pieces behind which the device already reads.
 const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, const Shape& shape) {
-  const bool whole = fused_ && shape_size(InputShape()) <= (128 << 10) && residents_.size() == 1 && residents_[0].whole_call && !(residents_[0].under_seq && SeqNow()) &&
+  const size_t size = static_cast<size_t>(shape_size(InputShape()));
+  const bool whole = fused_ && residents_.size() == 1 && residents_[0].whole_call && !(residents_[0].under_seq && SeqNow()) &&
                      !seq_calibration_pending_ && !cvmhip_kernel_timing_active();
   if (!whole) {
     const bool as_call = graph_state_ == 3 && seq_mode_ == SeqNow() && !seq_calibration_pending_ && !cvmhip_kernel_timing_active() && CaptureCall();
@@ -1000,15 +1000,20 @@ const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, 
     Run();
     return FetchOutputs();
   }
-  CheckData(shape);
-  AllocInputStage();
+  const bool direct = size <= (1 << 20);
   AllocOutputStage();
-  if (in_stage_busy_) HipCheck(cvmhip_stream_sync(stream_), "copy input to device");
-  std::memcpy(in_stage_host_, host, static_cast<size_t>(shape_size(shape)));
-  in_stage_ahead_ = true;
+  if (direct) {
+    CheckData(shape);
+    AllocInputStage();
+    if (in_stage_busy_) HipCheck(cvmhip_stream_sync(stream_), "copy input to device");
+    std::memcpy(in_stage_host_, host, size);
+    in_stage_ahead_ = true;
+  } else {
+    SetDataI8(host, shape);
+  }
   const ResidentRun& r = residents_[0];
   uint32_t* head = static_cast<uint32_t*>(out_stage_host_);
-  const cvmhip_resident_call call = {in_stage_host_, const_cast<int32_t*>(out_host_[0]), static_cast<uint32_t*>(out_counter_), head};
+  const cvmhip_resident_call call = {direct ? in_stage_host_ : in_stage_dev_, const_cast<int32_t*>(out_host_[0]), static_cast<uint32_t*>(out_counter_), head};
   HipCheck(cvmhip_resident_launch(r.table, r.nlayers, r.images, r.lds, &call, r.ops, r.bytes, stream_), "layers in LDS");
   ++ticket_;
   AwaitTicket();
