@@ -4,7 +4,7 @@
 // prologue, first operands, reduction and drain inside it another 2-3 us, while the arithmetic of a 32 x 32 x 16 layer is a
 // few hundred clocks of one compute unit.  Here the activations of an image never leave the compute unit: a layer boundary
 // is a workgroup barrier, and the batch spreads over the chip by images.  ResNet-20: 96 us in 23 launches at
-// batch 1, 39 us in one; 114 us at batch 64, 39.5 us.
+// batch 1, 34.4 us in one; 114 us at batch 64, 36 us.
 //
 // Arithmetic: v_mfma_i32_16x16x64_i8 with the filter as the first operand and 16 pixels as the second.  Lane l supplies
 // filter row l & 15 and pixel l & 15, both with the 16 bytes (l >> 4) of the 64 bytes of K, and receives channels
@@ -16,14 +16,14 @@
 // the four 16-byte groups of every K step are a table behind the filter.
 // The filter of a layer, its tap offsets, biases and the places of its tiles lie in LDS as well, fetched while the layer in
 // front of it is computed.
-// What bounds it now (ResNet-20, one workgroup, 106 K clocks by the counters): 46 K of LDS transfers, 17 K of them bank
+// What bounds it (ResNet-20, one workgroup; 106 K clocks by the counters when a launch was 39 us): 46 K of LDS transfers, 17 K of them bank
 // conflicts, 35 K of vector instructions, 14 K of scalar ones and 13 K of products on each SIMD, which hardly overlap: behind
 // a barrier all wavefronts read at the same time and then compute at the same time.  On the way, same network at batch 1:
 // all operand reads of a chunk before its first product instead of a read and a wait each 62 -> 52 us; filters requested
 // inside the loop that uses them 54 -> 45; plain layers without the tests for other forms 45 -> 41.5; filters and places
 // from LDS (no scalar register is spilled any more) and a sum without LDS shuffles 41.5 -> 39; a wavefront beside the others that fetches filters and
-// clears borders 39 -> 37, two by two tiles for layers of 32 channels -> 36.5.  No difference: 1024 threads, another priority for half of
-// the wavefronts, pixels an odd number of granules apart.  Slower: all operands of a 16-channel item requested at once, or of a 64-channel one (the
+// clears borders 39 -> 37, two by two tiles for layers of 32 channels -> 36.5; rows that share operands in layers of 16 -> 34.4.  No difference: 1024 threads, another priority for half of
+// the wavefronts, pixels an odd number of granules apart.  Slower: all operands of a 16-channel item of four tiles on their own requested at once, or of a 64-channel one (the
 // launch is bound by LDS transfers and vector instructions in turn, not by the latency of either); the next layer's head in scalar registers (spills).
 #include <string.h>
 
@@ -32,6 +32,7 @@
 namespace cvmhip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
 
 constexpr int RES_THREADS = 512, RES_WAVES = RES_THREADS / 64;   // the wavefronts that compute; one more prepares the next layer
 constexpr int RES_CHUNK = 3;        // K steps computed together (a 3 x 3 filter over 16, 64, 128, ... channels is whole chunks)
@@ -125,6 +126,14 @@ __device__ __forceinline__ void res_chain(const L& c, int32_t (&v)[4]) {
 __device__ __forceinline__ uint32_t res_pack(const int32_t (&v)[4]) {
   const uint32_t lo2 = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x0c0c0400u);
   const uint32_t hi2 = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x0c0c0400u);
+  return __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
+}
+
+// four values that are inside int8 once shifted -> one dword: three instructions where a shift each and res_pack are seven
+__device__ __forceinline__ uint32_t res_shift_pack(const int32_t (&v)[4], int shift) {
+  uint32_t lo2, hi2;   // (the builtin's 16 bits would be masked once more)
+  asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(lo2) : "v"(v[0]), "v"(v[1]), "s"(shift));
+  asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(hi2) : "v"(v[2]), "v"(v[3]), "s"(shift));
   return __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
 }
 
@@ -253,6 +262,7 @@ __device__ __forceinline__ void res_first_taps(const ResHead& h, const char* lds
 template <int TP>
 __device__ __forceinline__ void res_plain_conv(const ResHead& h, char* lds, int wave, int lane) {
   if (wave >= h.items) return;
+  const int last = h.residual ? h.shift2 : h.shift;
   const ResPlace own = *reinterpret_cast<const ResPlace*>(lds + (h.places_at + lane * 16));
   const char* rec = lds + (h.places_at + 1024 + wave * 64);
   int tap[RES_CHUNK];
@@ -280,18 +290,18 @@ __device__ __forceinline__ void res_plain_conv(const ResHead& h, char* lds, int 
       for (int j = 0; j < TP; ++j) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          acc[j][e] = res_clamp(wadd(res_clamp(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2) >> h.shift2;
+          acc[j][e] = res_clamp(wadd(res_clamp(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2);
       }
     } else {
 #pragma unroll
       for (int j = 0; j < TP; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[j][e] = res_clamp(acc[j][e], h.lo, h.hi) >> h.shift;
+        for (int e = 0; e < 4; ++e) acc[j][e] = res_clamp(acc[j][e], h.lo, h.hi);
     }
 #pragma unroll
     for (int j = 0; j < TP; ++j) {
       const int32_t v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
-      *reinterpret_cast<uint32_t*>(lds + (own.dst + dst[j])) = res_pack(v);
+      *reinterpret_cast<uint32_t*>(lds + (own.dst + dst[j])) = res_shift_pack(v, last);
     }
     item += RES_WAVES;
     if (item >= h.items) return;
@@ -305,6 +315,7 @@ __device__ __forceinline__ void res_plain_conv(const ResHead& h, char* lds, int 
 template <int TM, int TP, int STEPS>
 __device__ __forceinline__ void res_item_conv(const ResHead& h, char* lds, int wave, int lane) {
   if (wave >= h.items) return;
+  const int last = h.residual ? h.shift2 : h.shift;
   const ResPlace own = *reinterpret_cast<const ResPlace*>(lds + (h.places_at + lane * 16));
   const char* rec = lds + (h.places_at + 1024 + wave * 64);
   int tap[STEPS];
@@ -372,25 +383,128 @@ __device__ __forceinline__ void res_item_conv(const ResHead& h, char* lds, int w
         for (int j = 0; j < TP; ++j)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            acc[m][j][e] = res_clamp(wadd(res_clamp(acc[m][j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[m][j] >> (8 * e))), h.lo2, h.hi2) >> h.shift2;
+            acc[m][j][e] = res_clamp(wadd(res_clamp(acc[m][j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[m][j] >> (8 * e))), h.lo2, h.hi2);
     } else {
 #pragma unroll
       for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int j = 0; j < TP; ++j)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[m][j][e] = res_clamp(acc[m][j][e], h.lo, h.hi) >> h.shift;
+          for (int e = 0; e < 4; ++e) acc[m][j][e] = res_clamp(acc[m][j][e], h.lo, h.hi);
     }
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
       for (int j = 0; j < TP; ++j) {
         const int32_t v[4] = {acc[m][j][0], acc[m][j][1], acc[m][j][2], acc[m][j][3]};
-        *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j] + m * 16)) = res_pack(v);
+        *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j] + m * 16)) = res_shift_pack(v, last);
       }
     if (!more) return;
   }
 }
+// 3 x 3 over 16 channels, stride 1: K is ordered (column of the window, row), four rows to a step with a filter of zeros for the fourth
+// (res_pair_order), so the operand that one output row reads holds the rows of the output row below it as well: the same
+// operand times the filter moved on by one row of the window.  Six operands serve four tiles where res_plain_conv reads
+// twelve, the filter stays in registers, and an item's operands are requested behind the products of the one in front of it;
+// tiles 2 and 3 of an item lie below tiles 0 and 1.  A 32 x 32 x 16 layer: 3 550 -> 2 970 clocks, 4 300 -> 3 560 with a residual
+// (of these 770 products, and 1 000 or 1 800 vector instructions of each SIMD's four items).
+__device__ __forceinline__ void res_pair_conv(const ResHead& h, char* lds, int wave, int lane) {
+  if (wave >= h.items) return;
+  const int last = h.residual ? h.shift2 : h.shift;
+  const int group = lane >> 4;
+  const char* rec = lds + (h.places_at + 1024 + wave * 64);
+  struct Record {   // of an ResItem
+    v2i src, at;    // at: filter, bias
+    v4i dst, res;
+  } now, next;
+  auto record = [&](Record& r) {
+    r.src = *reinterpret_cast<const v2i*>(rec);
+    r.at = *reinterpret_cast<const v2i*>(rec + 48);
+    r.dst = *reinterpret_cast<const v4i*>(rec + 16);
+    r.res = *reinterpret_cast<const v4i*>(rec + 32);
+    rec += RES_WAVES * 64;
+  };
+  // all that has a known place, then all that these say, so that a layer begins with two waits for LDS
+  const ResPlace own = *reinterpret_cast<const ResPlace*>(lds + (h.places_at + lane * 16));
+  record(now);
+  int tap[3];
+#pragma unroll
+  for (int u = 0; u < 3; ++u) tap[u] = *reinterpret_cast<const int*>(lds + (h.taps_at + u * 16 + min(group, 2) * 4));
+  const int row1 = *reinterpret_cast<const int*>(lds + (h.taps_at + 4)), row2 = *reinterpret_cast<const int*>(lds + (h.taps_at + 8));
+  int item = wave + RES_WAVES;
+  if (item < h.items) record(next);
+  __builtin_amdgcn_sched_barrier(0);
+  const int below = group == 3 ? row2 - row1 : 0;   // (the table's fourth row is no row)
+#pragma unroll
+  for (int u = 0; u < 3; ++u) tap[u] += own.src + below;
+  v4i a[2][3], x[3][2], bias;
+  uint32_t residual[4];
+  int loaded = -1;
+  auto request = [&](const Record& r) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) x[u][j] = *reinterpret_cast<const v4i*>(lds + (r.src[j] + tap[u]));
+    const int at = __builtin_amdgcn_readfirstlane(r.at[0]);
+    if (at != loaded) {
+      loaded = at;
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        a[0][u] = *reinterpret_cast<const v4i*>(lds + (at + u * 1024 + lane * 16));
+        a[1][u] = *reinterpret_cast<const v4i*>(lds + (at + u * 1024 + (group ? lane - 16 : 48 + lane) * 16));   // (a step's last 16 lanes hold zeros)
+      }
+    }
+    bias = *reinterpret_cast<const v4i*>(lds + (r.at[1] + own.bias));
+  };
+  auto beside = [&](const Record& r) {
+    if (h.residual) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) residual[j] = *reinterpret_cast<const uint32_t*>(lds + (own.res + r.res[j]));
+    }
+  };
+  request(now);
+  beside(now);
+  for (;;) {
+    const bool more = item < h.items;
+    const v4i to = now.dst;
+    __builtin_amdgcn_sched_barrier(0);
+    v4i acc[4] = {bias, bias, bias, bias};
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j >> 1][u], x[u][j & 1], acc[j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) request(next);
+    asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));   // as in res_products
+    if (h.residual) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[j][e] = res_clamp(wadd(res_clamp(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[j][e] = res_clamp(acc[j][e], h.lo, h.hi);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int32_t v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
+      *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j])) = res_shift_pack(v, last);
+    }
+    if (!more) return;
+    beside(next);
+    now = next;
+    item += RES_WAVES;
+    if (item < h.items) record(next);
+  }
+}
+constexpr int RES_PAIR = 1;   // ResHead::form
+// does the filter of a layer have the order (column, row) of res_pair_conv?  (All layers that could have it do: the places of its
+// groups come from a table, any kernel takes them.)
+__host__ __device__ constexpr bool res_pair_order(int kh, int kw, int cp) { return kh == 3 && kw == 3 && cp == 16; }
+
 // (TM, TP, STEPS) of res_item_conv in one number; 0: res_plain_conv
 __host__ __device__ constexpr int res_form(int tm, int tp, int steps) { return steps * 16 + tm * 8 - 8 + tp; }
 #define RES_FORMS(F) F(2, 2, 3) F(2, 2, 5)
@@ -476,6 +590,7 @@ __global__ void __launch_bounds__(RES_THREADS + 64) k_conv_resident(const ResLay
 #define RES_CASE(TM, TP, STEPS) case res_form(TM, TP, STEPS): res_item_conv<TM, TP, STEPS>(h, lds, wave, lane); continue;
       switch (h.form) {
         RES_FORMS(RES_CASE)
+        case RES_PAIR: res_pair_conv(h, lds, wave, lane); continue;
         default: break;
       }
 #undef RES_CASE
@@ -597,7 +712,9 @@ __global__ void __launch_bounds__(256) k_pack_resident(const int32_t* __restrict
     const int64_t t = i >> 8;
     const int s = (int)(t % ksteps);
     const int64_t o = t / ksteps * 16 + (lane & 15);
-    const int k = s * 64 + (lane >> 4) * 16 + d * 4, tap = k / cp, c = k - tap * cp;
+    const bool pair = res_pair_order(kh, kw, cp);
+    const int k = s * 64 + (lane >> 4) * 16 + d * 4;
+    const int tap = pair ? (lane >> 4 < 3 && s < 3 ? (lane >> 4) * 3 + s : taps) : k / cp, c = pair ? d * 4 : k - tap * cp;
     uint32_t pack = 0;
     if (o < oc && tap < taps) {
 #pragma unroll
@@ -605,7 +722,9 @@ __global__ void __launch_bounds__(256) k_pack_resident(const int32_t* __restrict
     }
     wp[i] = pack;
   } else if (i < dwords + ksteps * 4) {
-    const int e = (int)(i - dwords), k = e * 16, tap = k / cp, c = k - tap * cp;
+    const int e = (int)(i - dwords), k = e * 16;
+    const bool pair = res_pair_order(kh, kw, cp);
+    const int tap = pair ? (e % 4 < 3 && e < 12 ? e % 4 * 3 + e / 4 : taps) : k / cp, c = pair ? 0 : k - tap * cp;
     // past the last tap the filter is zero: the window's first bytes will do
     wp[i] = tap < taps ? (uint32_t)((tap / kw) * dh * row + (tap % kw) * dw * cp + c) : 0u;
   } else if (i < dwords + ksteps * 4 + octiles * 16) {
@@ -628,6 +747,8 @@ static bool res_plain(const DevChain& c, int* lo, int* hi, int* shift) {
   *shift = c.st[0].s1 + c.st[0].s2;
   return true;
 }
+// are its results int8 whatever it is given?  (res_shift_pack saturates where the other forms take the low byte.)
+static bool res_narrow(int lo, int hi, int shift) { return lo >> shift >= -128 && hi >> shift <= 127; }
 
 }  // namespace cvmhip
 
@@ -769,11 +890,16 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d,
       const int ptiles = (L.P + 15) / 16;
       const ResTiling tiling = res_tiling(ptiles, L.octiles, res_steps(in.c, d->kh, d->kw));
       const int tp = tiling.tp, groups = L.octiles / tiling.tm;
-      if (!(h.flags & (RES_CHAIN | RES_CHAIN2 | RES_MASK | RES_OUT)) && L.P % (16 * tp) == 0 && (out.w % 16 == 0 || 16 % out.w == 0)) {
+      const bool narrow = h.residual ? res_narrow(h.lo2, h.hi2, h.shift2) : res_narrow(h.lo, h.hi, h.shift);
+      if (narrow && !(h.flags & (RES_CHAIN | RES_CHAIN2 | RES_MASK | RES_OUT)) && L.P % (16 * tp) == 0 && (out.w % 16 == 0 || 16 % out.w == 0)) {
         h.flags |= RES_PLAIN;
         h.tp = tp;
         h.form = tiling.form;
         h.items = groups * (ptiles / tp);
+        // tiles one above the other: two of a row and the two below them, or four of a map one tile wide
+        const bool pair = res_pair_order(d->kh, d->kw, res_cp(in.c)) && d->sh == 1 && d->sw == 1 && d->dh == 1 && d->dw == 1 && tp == 4 && tiling.tm == 1 &&
+                          (out.w % 32 == 0 ? out.h % 2 == 0 : out.w == 16 && out.h % 4 == 0);
+        if (pair) h.form = RES_PAIR;
         const size_t at = res_places_at(out.c, in.c, d->kh, d->kw);
         h.places_at = h.w_at + (int)at;
         const ResGeometry g = {L.P, L.OW, L.div_ow, L.src, L.step_y, L.step_x, L.dst, L.dst_row, L.ocp, L.res, L.res_row};
@@ -787,7 +913,13 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d,
           items[i].filter = h.w_at + ot * h.chunks * (RES_CHUNK * 1024);
           items[i].bias = h.bias_at + ot * 64;
           for (int t = 0; t < tp; ++t) {
-            const int p = (i / groups * tp + t) * 16;
+            int p = (i / groups * tp + t) * 16;
+            if (pair && out.w == 16) {
+              p = i / groups * 64 + ((t & 1) * 2 + (t >> 1)) * 16;
+            } else if (pair) {
+              const int across = out.w / 32, g2 = i / groups, y = g2 / across * 2 + (t >> 1), x = (g2 % across) * 32 + (t & 1) * 16;
+              p = y * out.w + x;
+            }
             const ResPlace q = res_place(g, p, p / g.OW, 0);
             items[i].src[t] = q.src - first.src;
             items[i].dst[t] = q.dst - first.dst + ot * 16;

@@ -111,3 +111,40 @@ def test_the_image_packed_for_a_convolution_outside_the_launch_is_written(dev, m
     b = g.conv_relu_q(g.conv_relu_q(x, 256, 3, 2, 1), 512, 1)      # 512 x 256: the filter does not fit beside the rest
     b = g.conv_relu_q(g.conv_relu_q(b, 256, 1), 256, 3, 1, 1, groups=256)
     _check_heads(g, [a, b], 16, "resident-two-stems", monkeypatch)
+
+
+@pytest.mark.parametrize("h,w,channels,pad,batch", [
+    (16, 32, (16, 16), 1, 2),        # two tiles of a row and the two below
+    (18, 64, (12, 16), 1, 1),        # several of these in a row; channels past the last
+    (6, 96, (16, 9), 1, 1),
+    (32, 16, (16, 16), 1, 2),        # four rows of a map one tile wide
+    (34, 16, (16, 16), 1, 1),        # not a multiple of four: tiles on their own
+    (18, 34, (16, 16), 0, 1),        # a window that begins inside the map
+    (16, 32, (16, 32, 16), 1, 1),
+    (64, 64, (16, 16, 16), 1, 100),  # images past 1 MiB: the kernel reads the copy on the device
+])
+def test_rows_that_share_operands(h, w, channels, pad, batch, dev, monkeypatch):
+    def net(n):
+        g = graphgen.GraphBuilder("resident-rows")
+        x = g.conv_relu_q(g.var("data", (n, 3, h, w), 8), channels[0], 3, 1 + h // 64, 1)
+        for oc in channels[1:]:
+            y = g.conv_relu_q(x, oc, 3, 1, pad)
+            z = g.conv_relu_q(y, oc, 3, 1, 1, relu=False)
+            x = g.rshift(g.relu(g.add(z, y)), 1)
+        s, _ = g.global_sum(x)
+        y, _ = g.dense(g.flatten(g.rshift(s, 6)), 5)
+        return g.build([y])
+
+    js, pb = net(batch)
+    x = synth.tensor("resident-rows", "data", (batch, 3, h, w), -127, 127).astype(np.int8)
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "1")
+    m = runtime.HipModel(js, pb)
+    assert m.launch_counts()[0] <= 3
+    got = [np.frombuffer(m.inference(x.tobytes()), np.int32).reshape(batch, -1) for _ in range(2)]
+    m.close()
+    j1, p1 = net(1)
+    p1 = graphgen.load_params(p1)
+    for i in {0, 1 % batch, batch // 2, batch - 1}:
+        want = og.run_graph(j1, p1, x[i:i + 1].astype(np.int32))[0].ravel()
+        for v in got:
+            assert np.array_equal(v[i], want), i
