@@ -1,0 +1,258 @@
+// 3 x 3 convolution, stride 1, padding 1, over 64 channels of a pixel-blocked tensor, int8 out, with or without the 2 x 2
+// max_pool2d behind it: the filter and the input pixels under a patch of 512 output pixels lie in LDS.
+//
+// K is short (18 chunks of 32 bytes), so that a wavefront that streams its operands from memory waits for most of them: each input
+// byte is asked for nine times, through an L1 that holds less than the rows under the workgroups of a compute unit, and the filter by every
+// wavefront.  Here a workgroup requests each byte of a patch once, memory -> LDS, a border of one pixel included, and the filter
+// once for all its patches; the K loop reads LDS with offsets known when it is compiled.  Two workgroups share a compute unit: one fetches or stores
+// while the other multiplies.
+// In LDS the 16 bytes that a lane feeds to a product are a granule, granules of the same channels lie pixel by pixel: the 32 pixels
+// of a block are 512 contiguous bytes.  With the pool a block is one corner of 32 windows, and the columns are sorted into
+// even and odd ones for that.
+// Measured (us; in front of it k_conv_wave): 64 -> 64 at 16 x 224 x 224 with the pool 46 -> 30, without 51 -> 33; 64 -> 128 at 16 x 112 x 112 29 -> 22; 64 -> 64
+// at 50 x 56 x 56 16.6 -> 13.  Bound by the requests: a patch takes a workgroup 700 clocks of waiting, 5 400 of products (4 608 at the rate of the
+// matrix pipe), 3 400 to 3 900 in which its wavefronts are held until their requests are taken, and 1 400 (pool) to 3 500 of
+// requantisation and stores.  No difference: operands requested a step ahead or left to the compiler; slower: a workgroup a patch, each with a
+// filter of its own (36 instead of 30).
+#include <algorithm>
+
+#include "conv_mfma.h"
+
+namespace cvmhip {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+constexpr int HALO_CHUNKS = 18, HALO_FILTER = 2 * HALO_CHUNKS * 1024, HALO_PIXELS = 512;
+
+__device__ const int g_halo_zero[4] = {0, 0, 0, 0};
+
+struct HaloGeom {
+  const int8_t* x;
+  const int8_t* wf;
+  int8_t* out;
+  const int32_t* bias;
+  int H, W, OC, tile_bytes;            // tile_bytes: from 32 filter rows to the next 32
+  int lo, hi, shift;
+  FastDiv div_oc, div_x, div_y;        // channel groups, patches of a row, rows of patches
+  int ocs, across, down, patches;
+};
+
+__device__ __forceinline__ void halo_request(const void* from, uint32_t lds_at) {
+  // (M0 is written for the instruction behind it: a wait state.  The compiler does not count these requests: stores_done_barrier waits)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_at) : "memory");
+}
+
+// (lo <= hi)
+__device__ __forceinline__ int halo_clamp(int v, int lo, int hi) {
+  int r;
+  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(lo), "v"(hi));
+  return r;
+}
+
+template <bool POOL, int PW>
+__global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
+  constexpr int PH = HALO_PIXELS / PW, ROW = PW + 2, PLANE = (PH + 2) * ROW, HALF = ROW / 2;
+  constexpr int REQUESTS = (4 * PLANE + 63) / 64;
+  __shared__ __attribute__((aligned(16))) int8_t smem[HALO_FILTER + REQUESTS * 1024];
+  __shared__ __attribute__((aligned(16))) int s_bias[64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, lgrp = lane >> 5;
+  // A workgroup keeps the filter of its channels and takes patches in turn; an eighth of the patches to each XCD, where neighbours share
+  // the pixels between them in one L2.
+  int slot = blockIdx.x, slots = gridDim.x, begin = 0, end = a.patches;
+  if (gridDim.x % (8 * a.ocs) == 0) {
+    const int xcd = slot & 7, per = a.patches >> 3, extra = a.patches & 7;
+    slot >>= 3;
+    slots >>= 3;
+    begin = xcd * per + (xcd < extra ? xcd : extra);
+    end = begin + per + (xcd < extra ? 1 : 0);
+  }
+  const int first_patch = (int)fastdiv((unsigned)slot, a.div_oc), oc0 = (slot - first_patch * a.ocs) * 64, stride = (int)fastdiv((unsigned)slots, a.div_oc);
+  int patch = begin + first_patch;
+  if (patch >= end) return;
+  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)smem;
+
+  const int8_t* filter = a.wf + (int64_t)(oc0 >> 5) * a.tile_bytes + lane * 16;
+#pragma unroll
+  for (int k = 0; k < 2 * HALO_CHUNKS / 4; ++k) {
+    const int c = wave + 4 * k;
+    halo_request(filter + (c >= HALO_CHUNKS ? a.tile_bytes + (c - HALO_CHUNKS) * 1024 : c * 1024), lds + (uint32_t)c * 1024u);
+  }
+  // the places of a patch's granules, the same for all patches: row, column, granule of the pixel
+  constexpr int MINE = (REQUESTS + 3) / 4;
+  int place[MINE];
+#pragma unroll
+  for (int k = 0; k < MINE; ++k) {
+    const int t = (wave + 4 * k) * 64 + lane, g = t / PLANE, q = t - g * PLANE, r = q / ROW, m = q - r * ROW;
+    place[k] = g >= 4 ? -1 : r | (POOL ? (m >= HALF ? 2 * (m - HALF) + 1 : 2 * m) : m) << 8 | g << 16;
+  }
+  int n, x0, y0;
+  auto fetch = [&](int which) __attribute__((always_inline)) {
+    const int line = (int)fastdiv((unsigned)which, a.div_x);
+    n = (int)fastdiv((unsigned)line, a.div_y);
+    x0 = (which - line * a.across) * PW;
+    y0 = (line - n * a.down) * PH;
+    const int corner = (n * a.H + y0 - 1) * a.W + x0 - 1;
+#pragma unroll
+    for (int k = 0; k < MINE; ++k) {
+      if (wave + 4 * k < REQUESTS) {
+        const int r = place[k] & 255, c = place[k] >> 8 & 255, g = place[k] >> 16;
+        const bool ok = g >= 0 && (unsigned)(y0 - 1 + r) < (unsigned)a.H && (unsigned)(x0 - 1 + c) < (unsigned)a.W;
+        const int p = corner + r * a.W + c;
+        const uint64_t inside = (uint64_t)(uintptr_t)a.x + (uint32_t)((p >> 5) * 2048 + g * 512 + (p & 31) * 16), outside = (uint64_t)(uintptr_t)g_halo_zero;
+        halo_request(reinterpret_cast<const void*>(ok ? inside : outside), lds + HALO_FILTER + (uint32_t)(wave + 4 * k) * 1024u);
+      }
+    }
+  };
+  fetch(patch);
+  if (tid < 64) s_bias[tid] = a.bias ? a.bias[oc0 + tid] : 0;
+  v16i acc[2][4];
+  // this lane's pixel of block 0 at the window's first tap
+  const int wy = PW == 64 ? wave : wave * 2 + (lrow >> 4), wx = PW == 64 ? lrow : lrow & 15;   // POOL: its window
+  const int origin = POOL ? 2 * wy * ROW + wx : wave * (PW == 32 ? 4 : 2) * ROW + lrow;
+  const int8_t* px = smem + HALO_FILTER + (origin + lgrp * PLANE) * 16;
+  const int8_t* fl = smem + lane * 16;
+  // K by column of the window and half of the channels, and in these by row: the operand of a row of blocks serves three products, the rows below it
+  // included.  A step requests what the next one needs and multiplies what the step before requested.
+  constexpr int COLS = POOL || PW == 64 ? 2 : 1, ROWS = 4 / COLS;   // blocks of a wavefront
+  v4i f[2][2], b[2][ROWS + 2][COLS];
+  auto request = [&](const int t) __attribute__((always_inline)) {
+    const int s = t / 6, half = t / 3 % 2, r = t % 3;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) f[t & 1][i] = *reinterpret_cast<const v4i*>(fl + (i * HALO_CHUNKS + (r * 3 + s) * 2 + half) * 1024);
+#pragma unroll
+    for (int y = r == 0 ? 0 : ROWS + r - 1; y < ROWS + r; ++y)
+#pragma unroll
+      for (int x = 0; x < COLS; ++x) {
+        const int at = y * ROW + (POOL ? ((x + s) & 1) * HALF + ((x + s) >> 1) : x * 32 + s);
+        b[t / 3 & 1][y][x] = *reinterpret_cast<const v4i*>(px + (half * 2 * PLANE + at) * 16);
+      }
+  };
+  for (;;) {
+    stores_done_barrier();   // the requests have landed
+    request(0);
+    // the sums start from the bias: element e of a lane is channel (e / 4) * 8 + lgrp * 4 + e % 4 of 32
+    v16i first[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v4i v = *reinterpret_cast<const v4i*>(s_bias + i * 32 + q * 8 + lgrp * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) first[i][q * 4 + e] = v[e];
+      }
+#pragma unroll
+    for (int t = 0; t < HALO_CHUNKS; ++t) {
+      if (t + 1 < HALO_CHUNKS) request(t + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[t & 1][i], b[t / 3 & 1][j / COLS + t % 3][j % COLS], t == 0 ? first[i] : acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+
+    const int now_n = n, now_x = x0, now_y = y0;
+    patch += stride;
+    const bool more = patch < end;
+    __syncthreads();   // the patch has been read
+    if (more) fetch(patch);
+    // A vector instruction may read a product's registers 19 wait states behind it.  The compiler sees to that for instructions it knows; halo_clamp
+    // is inline assembly to it.
+    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[1][2]),
+                 "+v"(acc[1][3]));
+    const int OW = POOL ? a.W >> 1 : a.W, OH = POOL ? a.H >> 1 : a.H;
+    const int cblocks = a.OC >> 5;
+#pragma unroll
+    for (int j = 0; j < (POOL ? 1 : 4); ++j) {
+      const int y = POOL ? (now_y >> 1) + wy : PW == 32 ? now_y + wave * 4 + j : now_y + wave * 2 + (j >> 1);
+      const int x = POOL ? (now_x >> 1) + wx : PW == 32 ? now_x + lrow : now_x + (j & 1) * 32 + lrow;
+      const int p = (now_n * OH + y) * OW + x;
+      const bool ok = y < OH && x < OW;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        uint32_t d[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          int v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            int m = acc[i][j][q * 4 + e];
+            if (POOL) m = max(max(m, acc[i][1][q * 4 + e]), max(acc[i][2][q * 4 + e], acc[i][3][q * 4 + e]));
+            v[e] = halo_clamp(m, a.lo, a.hi);
+          }
+          // (results are int8 whatever they come from: the saturation never acts)
+          const uint32_t lo2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[0], (uint32_t)v[1], (uint32_t)a.shift);
+          const uint32_t hi2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[2], (uint32_t)v[3], (uint32_t)a.shift);
+          d[q] = __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
+        }
+        // lower half of the wavefront: channels 0 .. 15 of the 32, upper: 16 .. 31
+        typedef unsigned v2u __attribute__((ext_vector_type(2)));
+        const v2u s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+        if (ok) {
+          const v4i w = {(int)s0.x, (int)s0.y, (int)s1.x, (int)s1.y};
+          const int64_t at = ((int64_t)(p >> 5) * cblocks + (oc0 >> 5) + i) * 1024 + lgrp * 512 + (p & 31) * 16;
+          __builtin_nontemporal_store(w, reinterpret_cast<v4i*>(a.out + at));
+        }
+      }
+    }
+    if (!more) break;
+  }
+}
+
+// the patch that covers the image with fewer pixels outside it
+static int halo_width(int h, int w) {
+  const int64_t a = (int64_t)((w + 31) / 32) * ((h + 15) / 16), b = (int64_t)((w + 63) / 64) * ((h + 7) / 8);
+  return a <= b ? 32 : 64;
+}
+static int64_t halo_patches(const ConvGeom& g) {
+  return halo_width(g.H, g.W) == 32 ? (int64_t)g.N * ((g.W + 31) / 32) * ((g.H + 15) / 16) : (int64_t)g.N * ((g.W + 63) / 64) * ((g.H + 7) / 8);
+}
+
+// (g and ep as conv_prepare leaves them)
+// From 150 workgroups on (us here / k_conv_wave, 64 channels at 56 x 56: 112 workgroups 9.6 / 9.2, 140 9.9 / 9.6, 168 10.2 / 11.4, 224 10.5 / 12.7), and
+// where the patches have at most half as many pixels again as the image (64 x 100 x 75, 1.43 times: 26.7 / 29.9; 128 x 33 x 48, 1.62: 16.9 / 15.8).
+int64_t conv_halo_blocks(const ConvGeom& g, const Epilogue& ep) {
+  if (g.dw || g.row_bytes || g.Cp != 64 || g.OC % 64 != 0 || g.KH != 3 || g.KW != 3 || g.SH != 1 || g.SW != 1 || g.PH != 1 || g.PW != 1 || g.DH != 1 ||
+      g.DW != 1 || ep.out_mode != OUT_I8_ACT || ep.out_cp != g.OC || ep.residual || ep.split)
+    return 0;
+  if ((int64_t)g.N * g.H * g.W * 64 > INT32_MAX) return 0;
+  const DevStage& q = ep.chain.st[0];   // one clamp and one shift to int8
+  if (ep.chain.count != 1 || q.mul != 1 || q.add != 0 || (q.s1 && q.s2) || q.lo > q.hi || q.lo >> (q.s1 + q.s2) < -128 || q.hi >> (q.s1 + q.s2) > 127) return 0;
+  const int64_t patches = halo_patches(g), blocks = patches * (g.OC / 64);
+  if (blocks < 150 || blocks > INT32_MAX || patches * HALO_PIXELS * 2 > (int64_t)g.N * g.H * g.W * 3) return 0;
+  return blocks;
+}
+
+int conv_halo(const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g, const Epilogue& ep, hipStream_t s) {
+  const int width = halo_width(g.H, g.W);
+  HaloGeom a = {};
+  a.x = xp;
+  a.wf = wp;
+  a.out = reinterpret_cast<int8_t*>(out);
+  a.bias = ep.bias;
+  a.H = g.H; a.W = g.W; a.OC = g.OC;
+  a.tile_bytes = (HALO_CHUNKS + 1) * 1024;
+  a.lo = ep.chain.st[0].lo;
+  a.hi = ep.chain.st[0].hi;
+  a.shift = ep.chain.st[0].s1 + ep.chain.st[0].s2;
+  a.ocs = g.OC / 64;
+  a.patches = (int)halo_patches(g);
+  a.across = (g.W + width - 1) / width;
+  a.down = (g.H + HALO_PIXELS / width - 1) / (HALO_PIXELS / width);
+  a.div_oc = make_fastdiv((uint32_t)a.ocs);
+  a.div_x = make_fastdiv((uint32_t)a.across);
+  a.div_y = make_fastdiv((uint32_t)a.down);
+  const int at_once = std::max(1, 512 / a.ocs);   // patches: two workgroups a compute unit
+  const unsigned grid = (unsigned)(a.ocs * std::min(a.patches, at_once));
+  if (ep.pool && width == 32) k_conv_halo<true, 32><<<grid, 256, 0, s>>>(a);
+  else if (ep.pool) k_conv_halo<true, 64><<<grid, 256, 0, s>>>(a);
+  else if (width == 32) k_conv_halo<false, 32><<<grid, 256, 0, s>>>(a);
+  else k_conv_halo<false, 64><<<grid, 256, 0, s>>>(a);
+  return check_launch("conv_halo");
+}
+
+}  // namespace cvmhip

@@ -2858,6 +2858,13 @@ int conv_igemm_ws(const int8_t* xp, const int8_t* wp, void* out, ConvGeom g, con
   // them or a configuration of the wavefront kernel; nothing is read from the environment here.
   const bool force_lds = tune.kernel == CONV_KERNEL_LDS, force_wave = tune.kernel == CONV_KERNEL_WAVE;
   const int wave_forced = tune.wave_cfg;
+  if (tune.kernel == CONV_KERNEL_AUTO && wave_forced < 0) {
+    if (const int64_t nhalo = conv_halo_blocks(g, ep)) {
+      const ConvDesc desc(g, ep, "halo", 0, 0, (long)nhalo);
+      KernelTimer timer("k_conv_halo", 2.0 * (double)g.P * g.OC * (double)g.taps * (double)(g.C ? g.C : g.Cp), s, conv_bytes(g, ep), desc.text);
+      return conv_halo(xp, wp, out, g, ep, s);
+    }
+  }
   const bool nopad = g.PH == 0 && g.PW == 0;
   const bool rows = g.row_bytes != 0;
   const bool wave_ok = rows || ((g.Cp % 32) == 0 && (nopad || (g.KH <= 32 && g.KW <= 32)));

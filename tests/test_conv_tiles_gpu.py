@@ -98,3 +98,51 @@ def test_which_layers_take_the_large_tiles(n, ic, hw, oc, k, takes, dev, monkeyp
     assert takes in str(json.loads(buf.value.decode())[-1])
     monkeypatch.setenv("CVM_HIP_CONV", "wave")
     assert torch.equal(out, run())
+
+
+@pytest.mark.parametrize("n,h,w,oc,pool,lo,hi,shift,takes", [
+    (16, 16, 32, 640, False, -508, 508, 2, True),     # whole patches
+    (16, 16, 32, 640, True, -508, 508, 2, True),
+    (4, 50, 96, 256, False, 0, 127, 0, True),         # the last row of patches ends inside; 16 rows of 32
+    (4, 50, 96, 256, True, 0, 127, 0, True),
+    (6, 40, 59, 320, False, -128, 127, 0, True),      # 8 rows of 64, a column of pixels past the image
+    (6, 40, 58, 320, True, -2048, 2047, 4, True),
+    (11, 127, 161, 128, False, -127, 127, 0, True),   # several patches to a workgroup, odd extents
+    (11, 126, 162, 128, True, -127, 127, 0, True),
+    (37, 16, 32, 256, False, -127, 127, 0, False),    # 148 workgroups
+    (64, 33, 48, 128, False, -127, 127, 0, False),    # patches of 1.6 times the image
+    (16, 16, 32, 640, False, -512, 512, 2, False),    # 128 after the shift: its low byte
+    (16, 16, 32, 608, False, -127, 127, 0, False),    # channels that are no multiple of 64
+])
+def test_filter_and_patch_in_lds(n, h, w, oc, pool, lo, hi, shift, takes, dev, monkeypatch):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(h * w)
+    x = torch.randint(-4, 5, (n, 64, h, w), dtype=torch.int32, device=dev, generator=gen)
+    wt = torch.randint(-9, 10, (oc, 64, 3, 3), dtype=torch.int32, device=dev, generator=gen)
+    xp, wp = hipops.pack_act_i8(x), hipops.pack_weights(wt)
+    b = torch.randint(-300, 300, (oc,), dtype=torch.int32, device=dev, generator=gen)
+    chain = hipops.Chain()
+    chain.count = 1
+    chain.stage[0] = hipops.Stage(5, 0, shift, lo, hi)
+    op = hipops.conv2d_pool2_i8 if pool else hipops.conv2d_i8
+
+    def run():
+        lib().cvmhip_kernel_timing_begin()
+        out = op(xp, n, 64, h, w, wp, oc, 3, 3, b, chain, padding=(1, 1))
+        torch.cuda.synchronize()
+        buf = ctypes.create_string_buffer(1 << 16)
+        check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
+        size = (h // 2, w // 2) if pool else (h, w)
+        return hipops.unpack_act_i8(out, n, oc, *size), "k_conv_halo" in str(json.loads(buf.value.decode())[-1])
+
+    got, halo = run()
+    assert halo == takes
+    monkeypatch.setenv("CVM_HIP_CONV", "wave")
+    want, halo = run()
+    assert not halo and torch.equal(got, want)
+    if h * w * oc < 400000:   # the last image against the oracle as well
+        v = oracle.conv2d(x[n - 1:].cpu().numpy(), wt.cpu().numpy(), b.cpu().numpy(), (1, 1), (1, 1), (1, 1), 1)
+        v = (np.clip(v, lo, hi) >> shift).astype(np.int8).astype(np.int32)
+        if pool:
+            v = oracle.max_pool2d(v, (2, 2), (2, 2), (0, 0), False)
+        assert np.array_equal(got[n - 1:].cpu().numpy(), v)
