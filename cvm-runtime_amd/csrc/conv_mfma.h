@@ -227,6 +227,10 @@ int pack_stem_weights(const int32_t* w, int8_t* wp, int oc, int c, int kh, int k
 bool stem_pool_eligible(int c, int oc, int kh, int kw, int oh, int ow, int qh, int qw);
 int stem_pool(const int8_t* xs, const int8_t* wp, const int32_t* bias, const DevChain& chain, int8_t* out, int n, int c, int h,
               int w, int oc, int kh, int kw, int sh, int sw, int ph, int pw, int qh, int qw, hipStream_t s);
+// the same for larger batches (conv_stem_pool.hip), where conv_stem_pool_takes says so
+bool conv_stem_pool_takes(int n, int oc, int kh, int kw, int sh, int sw, int qh, int qw);
+int conv_stem_pool(const int8_t* xs, const int8_t* wp, const int32_t* bias, const DevChain& chain, int8_t* out, const StemGeom& sg, int n, int oh, int ow, int qh,
+                   int qw, hipStream_t s);
 void weight_dims(int oc, int ic, int kh, int kw, int* ocp, int* kp);
 size_t packed_weight_bytes(int oc, int ic, int kh, int kw);
 // Two filters over the same input packed as one: the first one's 32-row tiles, then the second one's.

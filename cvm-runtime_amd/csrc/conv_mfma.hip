@@ -1612,7 +1612,7 @@ k_conv_big(const int8_t* __restrict__ xp, const int8_t* __restrict__ wf, void* _
 // A workgroup's chain of steps is long (0.6 us of addresses, 2 us of requests and MFMAs, 1.8 us of requantisation
 // into LDS, 0.6 us of maxima at one workgroup per CU), so this pays while the grid is a single round of workgroups
 // (a ResNet's head at batch 1: 8.0 against 4.0 + 4.7 us and a launch gap); at batch 16 its three rounds take 22 us
-// against 17 us for the two launches, and the caller keeps those.
+// against 17 us for the two launches; conv_stem_pool.hip has the form for that, 10 us.
 struct StemPool {
   int N, Hs, Ws;         // stored (zero padded) input extent in pixels of 4 bytes
   int OH, OW, QH, QW;    // extent of the convolution's and of the pool's output
@@ -2999,12 +2999,14 @@ int stem_pool(const int8_t* xs, const int8_t* wp, const int32_t* bias, const Dev
   a.tiles_y = (qh + SP_PH - 1) / SP_PH;
   a.chain = chain;
   a.bias = bias;
-  if (n > 65535 || a.tiles_y > 65535 || sg.bytes > INT32_MAX) return arg_error("conv2d_stem_pool3_i8: tensor too large");
+  const bool large = conv_stem_pool_takes(n, oc, kh, kw, sh, sw, qh, qw);
+  if ((!large && (n > 65535 || a.tiles_y > 65535)) || sg.bytes > INT32_MAX) return arg_error("conv2d_stem_pool3_i8: tensor too large");
   char desc[128] = "";
   if (kernel_timing_enabled())
     snprintf(desc, sizeof(desc), "%dx%d/%d %d->%d in %dx%dx%d out %dx%d + 3x3/2 max-pool -> %dx%d", kh, kw, sh, c, oc, n, h, w, oh, ow, qh, qw);
-  KernelTimer timer("k_stem_pool", 2.0 * n * (double)oh * ow * oc * c * kh * kw, s,
+  KernelTimer timer(large ? "k_conv_stem_pool" : "k_stem_pool", 2.0 * n * (double)oh * ow * oc * c * kh * kw, s,
                     4.0 * n * sg.hp * sg.wp + (double)oc * c * kh * kw + (double)n * qh * qw * oc, desc);
+  if (large) return conv_stem_pool(xs, wp, bias, chain, out, sg, n, oh, ow, qh, qw, s);
   k_stem_pool<<<dim3((unsigned)a.tiles_x, (unsigned)a.tiles_y, (unsigned)n), 256, 0, s>>>(xs, wp, out, a);
   return check_launch("conv2d_stem_pool3_i8");
 }

@@ -558,12 +558,12 @@ void HipGraphRuntime::BuildPlan() {
         // the convolution takes the maximum itself and writes the pooled tensor (the full-resolution one is never stored).
         const int ps = producer_step[xe];
         // The head of a ResNet: a 3x3 window with stride 2 and padding 1 behind a row-window convolution with 32 or 64
-        // output channels that nobody else reads becomes part of that convolution's launch (at small batches).
+        // output channels that nobody else reads becomes part of that convolution's launch, where that is the faster form.
         if (st.out_i8 && hooks_.pool_fuse && ps >= 0 && plan[ps].kind == PlanStep::CONV && plan[ps].dst == xe &&
             plan[ps].out_i8 && plan[ps].stem && !plan[ps].pool3 && uses[xe].size() == 1 && !is_head[xe] && st.kh == 3 &&
             st.kw == 3 && st.sh == 2 && st.sw == 2 && st.ph == 1 && st.pw == 1 &&
-            // one workgroup per 4 x 8 pooled pixels: worth it while they all run at once (small batches)
-            (int64_t)plan[ps].n * ((st.oh + 3) / 4) * ((st.ow + 7) / 8) <= 512 &&
+            cvmhip_conv2d_stem_pool3_i8_pays(plan[ps].n, plan[ps].h, plan[ps].w, plan[ps].oc, plan[ps].kh, plan[ps].kw, plan[ps].sh,
+                                             plan[ps].sw, plan[ps].ph, plan[ps].pw, st.oh, st.ow) &&
             cvmhip_conv2d_stem_pool3_i8_eligible(plan[ps].n, plan[ps].c, plan[ps].h, plan[ps].w, plan[ps].oc, plan[ps].kh,
                                                  plan[ps].kw, plan[ps].sh, plan[ps].sw, plan[ps].ph, plan[ps].pw, st.oh, st.ow)) {
           PlanStep& cs = plan[ps];

@@ -448,9 +448,11 @@ int cvmhip_conv2d_stem_i8(const void* xs, const void* wp, const int32_t* bias, c
  * (requantised to int8; pixels outside the convolution's output count as the smallest value, like the reference's
  * INT32_MIN padding) and takes the maxima there.  out: the pooled int8 act tensor (n, oc, pool_oh, pool_ow), with
  * pool_oh, pool_ow as the graph's shape inference gives them.  Eligible: the convolution is (cvmhip_stem_eligible),
- * oc is 32 or 64, and every window touches the convolution's output. */
+ * oc is 32 or 64, and every window touches the convolution's output.  _pays: one launch is the faster form as well (few patches, or a
+ * 7 x 7 convolution with stride 2 to 64 channels, which has a kernel for many). */
 int cvmhip_conv2d_stem_pool3_i8_eligible(int n, int c, int h, int wd, int oc, int kh, int kw, int stride_h, int stride_w,
                                          int pad_h, int pad_w, int pool_oh, int pool_ow);
+int cvmhip_conv2d_stem_pool3_i8_pays(int n, int h, int wd, int oc, int kh, int kw, int stride_h, int stride_w, int pad_h, int pad_w, int pool_oh, int pool_ow);
 int cvmhip_conv2d_stem_pool3_i8(const void* xs, const void* wp, const int32_t* bias, const cvmhip_chain* chain, void* out,
                                 int n, int c, int h, int wd, int oc, int kh, int kw, int stride_h, int stride_w,
                                 int pad_h, int pad_w, int pool_oh, int pool_ow, void* stream);

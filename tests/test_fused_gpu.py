@@ -1,6 +1,8 @@
 """GPU parity of the fused int8 entry points (include/cvm_hip_ops.h, "fused int8
 path") against the CPU oracle running the same nodes one by one, and of the
 fused graph executor against the node-by-node executor.  Bit-exact."""
+import ctypes
+import json
 import os
 
 import numpy as np
@@ -9,7 +11,7 @@ import torch
 
 import oracle
 import oracle.graph as og
-from cvm_runtime_amd import CvmHipError, graphgen, hipops, runtime, synth
+from cvm_runtime_amd import CvmHipError, check, graphgen, hipops, lib, runtime, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -478,6 +480,37 @@ def test_conv2d_stem_with_fused_3x3_max_pool(case, dev):
     out = hipops.conv2d_stem_pool3_i8(T(x, dev), T(wt, dev), T(b, dev), hipops.chain(*stages), (st, st), (pd, pd), qh, qw)
     torch.cuda.synchronize()
     eq(act_to_nchw(out, n, oc, qh, qw), ref, "stem + 3x3 max-pool")
+
+
+@pytest.mark.parametrize("n,c,h,w,kw,pad,stages,kernel", [
+    (5, 3, 224, 224, 7, 3, [("relu",), ("cvm_right_shift", 8, 9)], "k_conv_stem_pool"),   # whole patches of 8 x 14 pooled pixels; a chain with a rounding term
+    (5, 3, 224, 224, 7, 3, [("clip", -90, 127)], "k_conv_stem_pool"),                    # one clamp and no shift
+    (40, 4, 61, 93, 8, 3, [("clip", -128, 127)], "k_conv_stem_pool"),                    # patches past the pool's last row and column, the widest window
+    (80, 1, 23, 19, 5, 0, [("relu",), ("cvm_right_shift", 8, 6)], "k_conv_stem_pool"),   # no padding, a patch an image
+    (900, 3, 17, 60, 7, 3, [("cvm_right_shift", 8, 8)], "k_conv_stem_pool"),             # several patches to a workgroup
+    (79, 1, 23, 19, 5, 0, [("relu",), ("cvm_right_shift", 8, 6)], "k_stem_pool"),        # too few patches
+])
+def test_stem_and_pool_of_many_images(n, c, h, w, kw, pad, stages, kernel, dev):
+    """The form for larger batches against the oracle, image by image at both ends of the batch."""
+    cid = "stempool-many-%d-%d" % (n, w)
+    x = synth.tensor(cid, "x", (n, c, h, w), -127, 127)
+    wt = synth.tensor(cid, "w", (64, c, 7, kw), -31, 31)
+    b = synth.tensor(cid, "b", (64,), -3000, 3000)
+    if stages[0][0] == "clip":
+        x, wt, b = x // 32, wt // 8, b // 30
+    oh, ow = (h + 2 * pad - 7) // 2 + 1, (w + 2 * pad - kw) // 2 + 1
+    qh, qw = (oh + 2 - 3) // 2 + 1, (ow + 2 - 3) // 2 + 1
+    lib().cvmhip_kernel_timing_begin()
+    out = hipops.conv2d_stem_pool3_i8(T(x, dev), T(wt, dev), T(b, dev), hipops.chain(*stages), (2, 2), (pad, pad), qh, qw)
+    torch.cuda.synchronize()
+    buf = ctypes.create_string_buffer(1 << 16)
+    check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
+    assert json.loads(buf.value.decode())[-1]["kernel"] == kernel
+    got = act_to_nchw(out, n, 64, qh, qw)
+    got = got.cpu().numpy() if hasattr(got, "cpu") else np.asarray(got)
+    for i in sorted({0, 1, n // 2, n - 1}):
+        conv = run_chain(oracle.conv2d(x[i:i + 1], wt, b, (2, 2), (pad, pad), (1, 1), 1), stages)
+        assert np.array_equal(got[i:i + 1], oracle.max_pool2d(conv, (3, 3), (2, 2), (1, 1), False)), i
 
 
 def test_conv2d_stem_pool_eligibility(dev):
