@@ -13,7 +13,10 @@
 // at 50 x 56 x 56 16.6 -> 13.  Bound by the requests: a patch takes a workgroup 700 clocks of waiting, 5 400 of products (4 608 at the rate of the
 // matrix pipe), 3 400 to 3 900 in which its wavefronts are held until their requests are taken, and 1 400 (pool) to 3 500 of
 // requantisation and stores.  No difference: operands requested a step ahead or left to the compiler; slower: a workgroup a patch, each with a
-// filter of its own (36 instead of 30).
+// filter of its own (36 instead of 30); half of the next patch's requests in the middle of the products (32).
+// The two layers at the head of a VGG are one launch (STEM): the pixels under a patch, a fifth more than are asked for, are computed from the image by the
+// first layer's products where they would be fetched, and the largest tensor of the network is neither written nor read:
+// 16 x 224 x 224 with the pool 21 + 30 -> 40 us.
 #include <algorithm>
 
 #include "conv_mfma.h"
@@ -36,6 +39,10 @@ struct HaloGeom {
   int lo, hi, shift;
   FastDiv div_oc, div_x, div_y;        // channel groups, patches of a row, rows of patches
   int ocs, across, down, patches;
+  // STEM: the convolution over a few channels in front of it (row-window form, conv_mfma.h: StemGeom), whose result is the input
+  const int8_t* stem_wf;
+  const int32_t* stem_bias;
+  int hp, wp, stem_lo, stem_hi, stem_shift;
 };
 
 __device__ __forceinline__ void halo_request(const void* from, uint32_t lds_at) {
@@ -50,12 +57,39 @@ __device__ __forceinline__ int halo_clamp(int v, int lo, int hi) {
   return r;
 }
 
-template <bool POOL, int PW>
+// shift and saturate sixteen results of a lane to int8, 16 consecutive channels of its pixel: lower half of the wavefront channels 0 .. 15 of the 32, upper 16 .. 31
+// (results are int8 whatever they come from: the saturation never acts)
+__device__ __forceinline__ v4i halo_pack(const int (&v)[16], int shift) {
+  uint32_t d[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t lo2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[q * 4], (uint32_t)v[q * 4 + 1], (uint32_t)shift);
+    const uint32_t hi2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[q * 4 + 2], (uint32_t)v[q * 4 + 3], (uint32_t)shift);
+    d[q] = __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
+  }
+  typedef unsigned v2u __attribute__((ext_vector_type(2)));
+  const v2u s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+  return v4i{(int)s0.x, (int)s0.y, (int)s1.x, (int)s1.y};
+}
+
+// 16 sums of a lane as they start, from 32 biases in LDS: element e is channel (e / 4) * 8 + lgrp * 4 + e % 4
+__device__ __forceinline__ v16i halo_first(const int* bias, int lgrp) {
+  v16i first;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const v4i v = *reinterpret_cast<const v4i*>(bias + q * 8 + lgrp * 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) first[q * 4 + e] = v[e];
+  }
+  return first;
+}
+
+template <bool POOL, int PW, bool STEM>
 __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
   constexpr int PH = HALO_PIXELS / PW, ROW = PW + 2, PLANE = (PH + 2) * ROW, HALF = ROW / 2;
   constexpr int REQUESTS = (4 * PLANE + 63) / 64;
   __shared__ __attribute__((aligned(16))) int8_t smem[HALO_FILTER + REQUESTS * 1024];
-  __shared__ __attribute__((aligned(16))) int s_bias[64];
+  __shared__ __attribute__((aligned(16))) int s_bias[STEM ? 128 : 64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lgrp = lane >> 5;
@@ -80,6 +114,13 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
     const int c = wave + 4 * k;
     halo_request(filter + (c >= HALO_CHUNKS ? a.tile_bytes + (c - HALO_CHUNKS) * 1024 : c * 1024), lds + (uint32_t)c * 1024u);
   }
+  int n, x0, y0;
+  auto corner_of = [&](int which) __attribute__((always_inline)) {
+    const int line = (int)fastdiv((unsigned)which, a.div_x);
+    n = (int)fastdiv((unsigned)line, a.div_y);
+    x0 = (which - line * a.across) * PW;
+    y0 = (line - n * a.down) * PH;
+  };
   // the places of a patch's granules, the same for all patches: row, column, granule of the pixel
   constexpr int MINE = (REQUESTS + 3) / 4;
   int place[MINE];
@@ -88,12 +129,7 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
     const int t = (wave + 4 * k) * 64 + lane, g = t / PLANE, q = t - g * PLANE, r = q / ROW, m = q - r * ROW;
     place[k] = g >= 4 ? -1 : r | (POOL ? (m >= HALF ? 2 * (m - HALF) + 1 : 2 * m) : m) << 8 | g << 16;
   }
-  int n, x0, y0;
-  auto fetch = [&](int which) __attribute__((always_inline)) {
-    const int line = (int)fastdiv((unsigned)which, a.div_x);
-    n = (int)fastdiv((unsigned)line, a.div_y);
-    x0 = (which - line * a.across) * PW;
-    y0 = (line - n * a.down) * PH;
+  auto fetch = [&]() __attribute__((always_inline)) {
     const int corner = (n * a.H + y0 - 1) * a.W + x0 - 1;
 #pragma unroll
     for (int k = 0; k < MINE; ++k) {
@@ -106,8 +142,62 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
       }
     }
   };
-  fetch(patch);
-  if (tid < 64) s_bias[tid] = a.bias ? a.bias[oc0 + tid] : 0;
+  // STEM: the patch's pixels are computed, a block of 32 places after the other to the wavefronts.
+  constexpr int STEM_BLOCKS = (PLANE + 127) / 128;
+  v4i window[STEM ? STEM_BLOCKS : 1][2], stem_f[2][2];
+  int column;   // of this lane, out of the compiler's sight: what it could work out once for all patches would cost registers that the products need
+  auto stem_pixel = [&](int k, int& y, int& x) __attribute__((always_inline)) {
+    const int q = (wave + 4 * k) * 32 + column, r = q / ROW, m = q - r * ROW;
+    y = y0 - 1 + r;
+    x = x0 - 1 + (POOL ? (m >= HALF ? 2 * (m - HALF) + 1 : 2 * m) : m);
+    return q < PLANE && y >= 0 && y < a.H && x >= 0 && x < a.W;
+  };
+  auto stem_request = [&]() __attribute__((always_inline)) {
+    typedef int v4w __attribute__((ext_vector_type(4), aligned(4)));
+    column = lrow;
+    asm volatile("" : "+v"(column));
+    const int8_t* filter_at = a.stem_wf + column * 16 + lgrp * 512;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) stem_f[i][c] = *reinterpret_cast<const v4i*>(filter_at + (i * 3 + c) * 1024);
+#pragma unroll
+    for (int k = 0; k < STEM_BLOCKS; ++k) {
+      int y, x;
+      const bool ok = stem_pixel(k, y, x);
+      const int at = ok ? ((n * a.hp + y) * a.wp + x) * 4 : 0;   // the first of three rows of 16 bytes
+      window[k][0] = *reinterpret_cast<const v4w*>(a.x + (at + lgrp * a.wp * 4));
+      window[k][1] = *reinterpret_cast<const v4w*>(a.x + (at + 2 * a.wp * 4));   // (times a filter of zeros in the upper half)
+    }
+  };
+  auto stem_compute = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < STEM_BLOCKS; ++k) {
+      int y, x;
+      const bool ok = stem_pixel(k, y, x);
+      const int q = (wave + 4 * k) * 32 + column;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        v16i sum = halo_first(s_bias + 64 + i * 32, lgrp);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(stem_f[i][c], window[k][c], sum, 0, 0, 0);
+        asm volatile("s_nop 15\n\ts_nop 7" : "+v"(sum));   // as below
+        int v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = halo_clamp(sum[e], a.stem_lo, a.stem_hi);
+        const v4i w = halo_pack(v, a.stem_shift);
+        if (q < PLANE) *reinterpret_cast<v4i*>(smem + HALO_FILTER + ((i * 2 + lgrp) * PLANE + q) * 16) = ok ? w : v4i{0, 0, 0, 0};
+      }
+    }
+  };
+  corner_of(patch);
+  if constexpr (STEM) stem_request();
+  else fetch();
+  if (tid < 64) {
+    s_bias[tid] = a.bias ? a.bias[oc0 + tid] : 0;
+    if (STEM) s_bias[64 + tid] = a.stem_bias ? a.stem_bias[tid] : 0;
+  }
+  if (STEM) __syncthreads();
   v16i acc[2][4];
   // this lane's pixel of block 0 at the window's first tap
   const int wy = PW == 64 ? wave : wave * 2 + (lrow >> 4), wx = PW == 64 ? lrow : lrow & 15;   // POOL: its window
@@ -131,18 +221,10 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
       }
   };
   for (;;) {
+    if constexpr (STEM) stem_compute();
     stores_done_barrier();   // the requests have landed
     request(0);
-    // the sums start from the bias: element e of a lane is channel (e / 4) * 8 + lgrp * 4 + e % 4 of 32
-    v16i first[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const v4i v = *reinterpret_cast<const v4i*>(s_bias + i * 32 + q * 8 + lgrp * 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) first[i][q * 4 + e] = v[e];
-      }
+    const v16i first[2] = {halo_first(s_bias, lgrp), halo_first(s_bias + 32, lgrp)};
 #pragma unroll
     for (int t = 0; t < HALO_CHUNKS; ++t) {
       if (t + 1 < HALO_CHUNKS) request(t + 1);
@@ -159,7 +241,10 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
     patch += stride;
     const bool more = patch < end;
     __syncthreads();   // the patch has been read
-    if (more) fetch(patch);
+    if (more) {
+      corner_of(patch);
+      if constexpr (!STEM) fetch();
+    }
     // A vector instruction may read a product's registers 19 wait states behind it.  The compiler sees to that for instructions it knows; halo_clamp
     // is inline assembly to it.
     asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[1][2]),
@@ -174,32 +259,22 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
       const bool ok = y < OH && x < OW;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        uint32_t d[4];
+        int v[16];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          int v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            int m = acc[i][j][q * 4 + e];
-            if (POOL) m = max(max(m, acc[i][1][q * 4 + e]), max(acc[i][2][q * 4 + e], acc[i][3][q * 4 + e]));
-            v[e] = halo_clamp(m, a.lo, a.hi);
-          }
-          // (results are int8 whatever they come from: the saturation never acts)
-          const uint32_t lo2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[0], (uint32_t)v[1], (uint32_t)a.shift);
-          const uint32_t hi2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[2], (uint32_t)v[3], (uint32_t)a.shift);
-          d[q] = __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
+        for (int e = 0; e < 16; ++e) {
+          int m = acc[i][j][e];
+          if (POOL) m = max(max(m, acc[i][1][e]), max(acc[i][2][e], acc[i][3][e]));
+          v[e] = halo_clamp(m, a.lo, a.hi);
         }
-        // lower half of the wavefront: channels 0 .. 15 of the 32, upper: 16 .. 31
-        typedef unsigned v2u __attribute__((ext_vector_type(2)));
-        const v2u s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+        const v4i w = halo_pack(v, a.shift);
         if (ok) {
-          const v4i w = {(int)s0.x, (int)s0.y, (int)s1.x, (int)s1.y};
           const int64_t at = ((int64_t)(p >> 5) * cblocks + (oc0 >> 5) + i) * 1024 + lgrp * 512 + (p & 31) * 16;
           __builtin_nontemporal_store(w, reinterpret_cast<v4i*>(a.out + at));
         }
       }
     }
     if (!more) break;
+    if constexpr (STEM) stem_request();   // (in front of the requantisation the registers do not suffice)
   }
 }
 
@@ -212,6 +287,15 @@ static int64_t halo_patches(const ConvGeom& g) {
   return halo_width(g.H, g.W) == 32 ? (int64_t)g.N * ((g.W + 31) / 32) * ((g.H + 15) / 16) : (int64_t)g.N * ((g.W + 63) / 64) * ((g.H + 7) / 8);
 }
 
+// one clamp and one shift to int8
+static bool halo_chain(const DevChain& c, int* lo, int* hi, int* shift) {
+  const DevStage& q = c.st[0];
+  *lo = q.lo;
+  *hi = q.hi;
+  *shift = q.s1 + q.s2;
+  return c.count == 1 && q.mul == 1 && q.add == 0 && !(q.s1 && q.s2) && q.lo <= q.hi && q.lo >> *shift >= -128 && q.hi >> *shift <= 127;
+}
+
 // (g and ep as conv_prepare leaves them)
 // From 150 workgroups on (us here / k_conv_wave, 64 channels at 56 x 56: 112 workgroups 9.6 / 9.2, 140 9.9 / 9.6, 168 10.2 / 11.4, 224 10.5 / 12.7), and
 // where the patches have at most half as many pixels again as the image (64 x 100 x 75, 1.43 times: 26.7 / 29.9; 128 x 33 x 48, 1.62: 16.9 / 15.8).
@@ -220,39 +304,99 @@ int64_t conv_halo_blocks(const ConvGeom& g, const Epilogue& ep) {
       g.DW != 1 || ep.out_mode != OUT_I8_ACT || ep.out_cp != g.OC || ep.residual || ep.split)
     return 0;
   if ((int64_t)g.N * g.H * g.W * 64 > INT32_MAX) return 0;
-  const DevStage& q = ep.chain.st[0];   // one clamp and one shift to int8
-  if (ep.chain.count != 1 || q.mul != 1 || q.add != 0 || (q.s1 && q.s2) || q.lo > q.hi || q.lo >> (q.s1 + q.s2) < -128 || q.hi >> (q.s1 + q.s2) > 127) return 0;
+  int lo, hi, shift;
+  if (!halo_chain(ep.chain, &lo, &hi, &shift)) return 0;
   const int64_t patches = halo_patches(g), blocks = patches * (g.OC / 64);
   if (blocks < 150 || blocks > INT32_MAX || patches * HALO_PIXELS * 2 > (int64_t)g.N * g.H * g.W * 3) return 0;
   return blocks;
+}
+
+static void halo_geom(HaloGeom* a, const int8_t* wp, void* out, const ConvGeom& g, const Epilogue& ep, int width) {
+  a->wf = wp;
+  a->out = reinterpret_cast<int8_t*>(out);
+  a->bias = ep.bias;
+  a->H = g.H; a->W = g.W; a->OC = g.OC;
+  a->tile_bytes = (HALO_CHUNKS + 1) * 1024;
+  halo_chain(ep.chain, &a->lo, &a->hi, &a->shift);
+  a->ocs = g.OC / 64;
+  a->patches = (int)halo_patches(g);
+  a->across = (g.W + width - 1) / width;
+  a->down = (g.H + HALO_PIXELS / width - 1) / (HALO_PIXELS / width);
+  a->div_oc = make_fastdiv((uint32_t)a->ocs);
+  a->div_x = make_fastdiv((uint32_t)a->across);
+  a->div_y = make_fastdiv((uint32_t)a->down);
+}
+
+template <bool STEM>
+static int halo_launch(const HaloGeom& a, bool pool, int width, hipStream_t s) {
+  const int at_once = std::max(1, 512 / a.ocs);   // patches: two workgroups a compute unit
+  const unsigned grid = (unsigned)(a.ocs * std::min(a.patches, at_once));
+  if (pool && width == 32) k_conv_halo<true, 32, STEM><<<grid, 256, 0, s>>>(a);
+  else if (pool) k_conv_halo<true, 64, STEM><<<grid, 256, 0, s>>>(a);
+  else if (width == 32) k_conv_halo<false, 32, STEM><<<grid, 256, 0, s>>>(a);
+  else k_conv_halo<false, 64, STEM><<<grid, 256, 0, s>>>(a);
+  return check_launch("conv_halo");
 }
 
 int conv_halo(const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g, const Epilogue& ep, hipStream_t s) {
   const int width = halo_width(g.H, g.W);
   HaloGeom a = {};
   a.x = xp;
-  a.wf = wp;
-  a.out = reinterpret_cast<int8_t*>(out);
-  a.bias = ep.bias;
-  a.H = g.H; a.W = g.W; a.OC = g.OC;
-  a.tile_bytes = (HALO_CHUNKS + 1) * 1024;
-  a.lo = ep.chain.st[0].lo;
-  a.hi = ep.chain.st[0].hi;
-  a.shift = ep.chain.st[0].s1 + ep.chain.st[0].s2;
-  a.ocs = g.OC / 64;
-  a.patches = (int)halo_patches(g);
-  a.across = (g.W + width - 1) / width;
-  a.down = (g.H + HALO_PIXELS / width - 1) / (HALO_PIXELS / width);
-  a.div_oc = make_fastdiv((uint32_t)a.ocs);
-  a.div_x = make_fastdiv((uint32_t)a.across);
-  a.div_y = make_fastdiv((uint32_t)a.down);
-  const int at_once = std::max(1, 512 / a.ocs);   // patches: two workgroups a compute unit
-  const unsigned grid = (unsigned)(a.ocs * std::min(a.patches, at_once));
-  if (ep.pool && width == 32) k_conv_halo<true, 32><<<grid, 256, 0, s>>>(a);
-  else if (ep.pool) k_conv_halo<true, 64><<<grid, 256, 0, s>>>(a);
-  else if (width == 32) k_conv_halo<false, 32><<<grid, 256, 0, s>>>(a);
-  else k_conv_halo<false, 64><<<grid, 256, 0, s>>>(a);
-  return check_launch("conv_halo");
+  halo_geom(&a, wp, out, g, ep, width);
+  return halo_launch<false>(a, ep.pool != 0, width, s);
+}
+
+// The first two layers of a VGG
+static bool halo_stem_prepare(const cvmhip_chain* stem_chain, const cvmhip_chain* chain, int n, int c, int h, int w, int pool, ConvGeom* g, Epilogue* ep,
+                              HaloGeom* a, StemGeom* sg) {
+  if (n < 1 || c < 1 || c > 4 || h < 1 || w < 1 || (pool && (h % 2 || w % 2)) || cvmhip_stem_input_bytes(n, h, w, 3, 3, 1, 1, 1, 1) == 0) return false;
+  *sg = stem_geom(n, h, w, 3, 3, 1, 1, 1, 1);
+  if (sg->bytes > INT32_MAX || sg->row_bytes != 16) return false;
+  DevChain first;
+  if (!make_chain(stem_chain, &first) || !halo_chain(first, &a->stem_lo, &a->stem_hi, &a->stem_shift) || !make_chain(chain, &ep->chain)) return false;
+  g->N = n; g->H = g->OH = h; g->W = g->OW = w; g->Cp = g->OC = 64;
+  g->KH = g->KW = 3; g->SH = g->SW = g->PH = g->PW = g->DH = g->DW = 1;
+  ep->out_mode = OUT_I8_ACT;
+  ep->out_cp = 64;
+  ep->pool = pool;
+  return conv_halo_blocks(*g, *ep) > 0;
 }
 
 }  // namespace cvmhip
+
+using namespace cvmhip;
+
+extern "C" {
+
+int cvmhip_conv2d_stem_conv_i8_eligible(const cvmhip_chain* stem_chain, const cvmhip_chain* chain, int n, int c, int h, int w, int pool) {
+  ConvGeom g = {};
+  Epilogue ep = {};
+  HaloGeom a = {};
+  StemGeom sg;
+  return stem_chain && chain && halo_stem_prepare(stem_chain, chain, n, c, h, w, pool, &g, &ep, &a, &sg) ? 1 : 0;
+}
+
+int cvmhip_conv2d_stem_conv_i8(const void* xs, const void* stem_wp, const int32_t* stem_bias, const cvmhip_chain* stem_chain, const void* wp, const int32_t* bias,
+                               const cvmhip_chain* chain, void* out, int n, int c, int h, int w, int pool, void* stream) {
+  ConvGeom g = {};
+  Epilogue ep = {};
+  HaloGeom a = {};
+  StemGeom sg;
+  if (!xs || !stem_wp || !stem_chain || !wp || !chain || !out || (((uintptr_t)xs | (uintptr_t)stem_wp | (uintptr_t)wp | (uintptr_t)out) & 15) ||
+      !halo_stem_prepare(stem_chain, chain, n, c, h, w, pool, &g, &ep, &a, &sg))
+    return arg_error("conv2d_stem_conv_i8: not eligible");
+  ep.bias = bias;
+  const int width = halo_width(h, w);
+  a.x = reinterpret_cast<const int8_t*>(xs);
+  halo_geom(&a, reinterpret_cast<const int8_t*>(wp), out, g, ep, width);
+  a.stem_wf = reinterpret_cast<const int8_t*>(stem_wp);
+  a.stem_bias = stem_bias;
+  a.hp = sg.hp; a.wp = sg.wp;
+  char desc[128] = "";
+  if (kernel_timing_enabled()) snprintf(desc, sizeof(desc), "3x3/1 %d->64 and 3x3/1 64->64 in %dx%dx%d%s", c, n, h, w, pool ? " +pool" : "");
+  KernelTimer timer("k_conv_halo", 2.0 * n * h * w * 64 * 9 * (64.0 + c), as_stream(stream),
+                    4.0 * n * sg.hp * sg.wp + 64.0 * 9 * (64 + c) + (double)n * h * w * 64 / (pool ? 4 : 1), desc);
+  return halo_launch<true>(a, pool != 0, width, as_stream(stream));
+}
+
+}  // extern "C"

@@ -740,6 +740,7 @@ void HipGraphRuntime::BuildPlan() {
   if (hooks_.fold_bias) FoldRequant();
   BuildResident();
   BuildSeparable();
+  BuildStemConv();
   if (hooks_.seq) BuildSequences();
   BuildGroups();
 }
@@ -827,6 +828,33 @@ void HipGraphRuntime::BuildSeparable() {
     Check(cvmhip_pack_separable_filter(entry_ptr_[d.wsrc], buf->ptr, d.c, stream_), "separable filter");
     d.separable = buf;
   }
+}
+
+// The two 3x3 layers at the head of a VGG, the second the only reader of the first, become one launch.
+void HipGraphRuntime::BuildStemConv() {
+  if (!hooks_.separable) return;
+  for (size_t i = 0; i + 1 < plan_.size(); ++i) {
+    PlanStep& d = plan_[i];
+    const PlanStep& p = plan_[i + 1];
+    auto free = [&](size_t k) { return !in_resident_[k] && resident_at_[k] < 0 && !InSeparable(k); };
+    if (!free(i) || !free(i + 1) || d.kind != PlanStep::CONV || !d.stem || d.pool3 || !d.out_i8 || d.oc != 64 || d.kh != 3 || d.kw != 3 || d.sh != 1 || d.sw != 1 ||
+        d.ph != 1 || d.pw != 1)
+      continue;
+    if (p.kind != PlanStep::CONV || p.src != d.dst || p.src2 != kNone || !p.out_i8 || p.stem || p.nhwc || p.flat || p.ws || p.pool3 || p.c != 64 || p.oc != 64 ||
+        p.kh != 3 || p.kw != 3 || p.sh != 1 || p.sw != 1 || p.ph != 1 || p.pw != 1 || p.dh != 1 || p.dw != 1)
+      continue;
+    bool only = true;
+    for (size_t k = 0; k < plan_.size(); ++k)
+      only = only && (k == i || k == i + 1 || plan_[k].kind == PlanStep::NODE || !ReadsI8(plan_[k], i8_ptr_[d.dst]));
+    d.stem_conv = only && cvmhip_conv2d_stem_conv_i8_eligible(&d.chain, &p.chain, d.n, d.c, d.h, d.w, p.pool2 ? 1 : 0);
+  }
+}
+
+void HipGraphRuntime::RunStemConv(size_t step) {
+  const PlanStep &d = plan_[step], &p = plan_[step + 1];
+  Check(cvmhip_conv2d_stem_conv_i8(PackedImage(d), static_cast<DeviceBuffer*>(d.weights.get())->ptr, d.bias, &d.chain,
+                                   static_cast<DeviceBuffer*>(p.weights.get())->ptr, p.bias, &p.chain, i8_ptr_[p.dst], d.n, d.c, d.h, d.w, p.pool2 ? 1 : 0,
+                                   stream_), "conv2d_stem_conv_i8");
 }
 
 void HipGraphRuntime::RunSeparable(size_t step) {

@@ -118,6 +118,7 @@ struct PlanStep {
   int oc2 = 0;
   std::shared_ptr<void> pair_bias;
   std::shared_ptr<void> folded_bias;   // CONV, DWCONV: the bias with the chains' rounding terms added (device); `bias` then points here
+  bool stem_conv = false;         // CONV (stem): one launch with the convolution behind it (the next step, cvmhip_conv2d_stem_conv_i8)
   std::shared_ptr<void> separable;   // DWCONV: its filter for one launch with the 1x1 convolution behind it (the next step)
   uint32_t wsrc = UINT32_MAX, bsrc = UINT32_MAX;   // CONV: entries of the filter and the bias (UINT32_MAX: none)
   int n = 0, c = 0, h = 0, w = 0, oc = 0, kh = 1, kw = 1, sh = 1, sw = 1, ph = 0, pw = 0, dh = 1, dw = 1, oh = 0, ow = 0;
@@ -178,7 +179,7 @@ class HipGraphRuntime {
     int extra = 0;   // steps of two launches: a dense layer over a whole map behind the copy that flattens the map
     if (fused_)
       for (const PlanStep& st : plan_) extra += st.flat ? 1 : 0;
-    for (const PlanStep& st : plan_) grouped += st.separable ? 1 : 0;
+    for (const PlanStep& st : plan_) grouped += st.separable || st.stem_conv ? 1 : 0;
     for (const ResidentRun& r : residents_)
       if (!(r.under_seq && SeqNow())) grouped += static_cast<int>(r.last - r.first);
     if (launches) *launches = static_cast<int>(NumSteps()) - lay + seq - (fused_ ? grouped : 0) + extra;
@@ -277,7 +278,7 @@ class HipGraphRuntime {
     // prefer to them.  Off as well when another launch form is asked for by name
     // (any of the switches of the planner or of the kernel choice is set): those name forms of single layers.
     bool resident = true;
-    bool separable = true;    // CVM_HIP_SEPARABLE=0, or a switch as above: depthwise and 1x1 convolutions stay two launches
+    bool separable = true;    // CVM_HIP_SEPARABLE=0, or a switch as above: depthwise and 1x1 convolutions, and the first two of a VGG, stay two launches
     bool flat_dense = true;   // CVM_HIP_FLATDENSE=0: a dense layer over a whole map gathers its operand from the map as it lies
     bool seq_chains = true;   // CVM_HIP_SEQ_CHAIN=0: no 1x1 layers chained behind the layer that feeds them (cvmhip_conv_seq_link)
     std::vector<std::pair<int, int>> seq_layer_cfg;   // CVM_HIP_SEQCFG: (layer of a sequence, configuration)
@@ -340,7 +341,10 @@ class HipGraphRuntime {
   bool ReadsI8(const PlanStep& st, const void* tensor) const;   // is the int8 tensor an operand of a step other than a NODE?
   void BuildSeparable();
   void RunSeparable(size_t step);
-  bool InSeparable(size_t step) const { return plan_[step].separable || (step > 0 && plan_[step - 1].separable); }
+  bool InSeparable(size_t step) const { return InPair(step) || (step > 0 && InPair(step - 1)); }
+  bool InPair(size_t first) const { return plan_[first].separable || plan_[first].stem_conv; }
+  void BuildStemConv();
+  void RunStemConv(size_t step);
   struct ResidentDraft;
   void BuildResident();
   bool ResidentEligible(const PlanStep& st) const;

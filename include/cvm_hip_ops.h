@@ -443,6 +443,12 @@ int cvmhip_pack_stem_weights(const int32_t* w, void* wp, int oc, int c, int kh, 
 int cvmhip_conv2d_stem_i8(const void* xs, const void* wp, const int32_t* bias, const cvmhip_chain* chain,
                           void* out, int out_is_i8, int n, int c, int h, int wd, int oc, int kh, int kw,
                           int stride_h, int stride_w, int pad_h, int pad_w, void* stream);
+/* The first two layers of a VGG in one launch: a 3x3 convolution with stride 1 and padding 1 over at most four channels (xs, stem_wp as above) to 64
+ * channels, and one of 64 to 64 channels behind it (wp from cvmhip_pack_weights), with max_pool2d(2x2, stride 2) behind that if `pool`; the tensor
+ * between the two is never stored.  Eligible: both chains are one clamp and one shift to int8, and there are pixels enough for the chip. */
+int cvmhip_conv2d_stem_conv_i8_eligible(const cvmhip_chain* stem_chain, const cvmhip_chain* chain, int n, int c, int h, int w, int pool);
+int cvmhip_conv2d_stem_conv_i8(const void* xs, const void* stem_wp, const int32_t* stem_bias, const cvmhip_chain* stem_chain, const void* wp, const int32_t* bias,
+                               const cvmhip_chain* chain, void* out, int n, int c, int h, int w, int pool, void* stream);
 /* The same convolution followed by max_pool2d with a 3x3 window, stride 2 and padding 1 (ops.cc:466-523; the head of a
  * ResNet) in ONE launch: a workgroup computes the convolution pixels under a patch of 4 x 8 pooled pixels into LDS
  * (requantised to int8; pixels outside the convolution's output count as the smallest value, like the reference's

@@ -83,3 +83,41 @@ def test_pairs_of_many_pixels_stay_two_launches(n, c, hw, oc, fused, dev, monkey
         counts.append(m.launch_counts()[0])
         m.close()
     assert counts[1] - counts[0] == fused, counts
+
+
+@pytest.mark.parametrize("n,c,h,w,pool", [
+    (10, 3, 64, 128, True),       # whole patches of 32 x 16
+    (9, 1, 62, 130, True),        # patches that end outside
+    (9, 3, 61, 131, False),
+    (8, 4, 40, 250, True),        # patches of 64 x 8
+    (8, 3, 39, 250, False),
+    (600, 3, 16, 30, False),      # several patches to a workgroup
+    (7, 3, 64, 128, True),        # too few
+])
+def test_first_two_layers_of_a_vgg(n, c, h, w, pool, dev, monkeypatch):
+    def net(k):
+        g = graphgen.GraphBuilder("stem-conv-%d-%d" % (c, w))
+        x = g.conv_relu_q(g.var("data", (k, c, h, w), 8), 64, 3, 1, 1)
+        y = g.conv_relu_q(x, 64, 3, 1, 1)
+        return g.build([g.conv_relu_q(g.max_pool(y, 2, 2) if pool else y, 8, 1)])
+
+    js, pb = net(n)
+    x = synth.tensor("stem-conv", "x%d" % w, (n, c, h, w), -128, 127)
+    out, launches = [], []
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "0")
+    for pair in ("1", "0"):
+        monkeypatch.setenv("CVM_HIP_SEPARABLE", pair)
+        m = runtime.HipModel(js, pb)
+        launches.append(m.launch_counts()[0])
+        for _ in range(4):   # eager, capture, replays
+            out.append(np.frombuffer(m.inference(x.astype(np.int8).tobytes()), np.int8).reshape(n, -1))
+        m.close()
+    assert launches[1] - launches[0] == (0 if n == 7 else 1), launches
+    j1, p1 = net(1)
+    p1 = graphgen.load_params(p1)
+    for i in (0, n - 1):
+        want = og.run_graph(j1, p1, np.clip(x[i:i + 1], -127, 127))[0].ravel()
+        for v in out:
+            assert np.array_equal(v[i], want), i
+    for v in out[1:]:
+        assert np.array_equal(v, out[0])
