@@ -26,8 +26,8 @@ PEAK_I8_TOPS = 5000.0   # MI355X dense int8 MFMA peak, TOP/s
 # The third field is the first 16 hex digits of the SHA-256 of the kernels' source file as it was when the counters were
 # read: a figure is only reported while that file is unchanged, otherwise `traffic` is null (measured figures go stale).
 TRAFFIC_BYTES_PER_LAUNCH = {
-    ("resnet50", "k_conv_seq", 16): (530.8e6, "profiles/k_conv_seq_resnet50_b16_traffic.txt", "cc05fcc94e3978d9"),
-    ("vgg16", "k_conv_big", 16): (28.7e6, "profiles/k_conv_big_vgg16_b16_traffic.txt", "cc05fcc94e3978d9"),
+    ("resnet50", "k_conv_seq", 16): (531.0e6, "profiles/k_conv_seq_resnet50_b16_traffic.txt", "36f3cb30d3ec1daa"),
+    ("vgg16", "k_conv_big", 16): (27.1e6, "profiles/k_conv_big_vgg16_b16_traffic.txt", "36f3cb30d3ec1daa"),
 }
 KERNEL_SOURCE = os.path.join(ROOT, "cvm-runtime_amd", "csrc", "conv_mfma.hip")
 
@@ -45,7 +45,7 @@ def dominant_conv(kt, wall_s, steps):
     average launch duration with the cost of an event pair taken off, and the figures derived from it."""
     n_timed = sum(v["launches"] for v in kt.values())
     pair_cost_us = max(0.0, (sum(v["ms"] for v in kt.values()) * 1e3 - wall_s * 1e6) / max(n_timed, 1))
-    convs = {k: v for k, v in kt.items() if k in ("k_conv_wave", "k_conv_igemm", "k_conv_seq", "k_conv_big", "k_conv_group", "k_stem_pool", "k_conv_resident")}
+    convs = {k: v for k, v in kt.items() if k in ("k_conv_wave", "k_conv_igemm", "k_conv_seq", "k_conv_big", "k_conv_group", "k_conv_halo", "k_stem_pool", "k_conv_stem_pool", "k_conv_resident")}
     dom = max(convs, key=lambda k: convs[k]["ms"]) if convs else "k_conv_wave"
     conv = convs.get(dom, {"launches": 0, "ms": 0.0, "work": 0.0})
     launches = max(conv["launches"], 1)
