@@ -296,6 +296,10 @@ static bool conv_direct(const int32_t* x, const int32_t* w, const int32_t* bias,
       const int c = one ? j : (p + j) / 9, t = one ? 0 : (p + j) % 9;
       a.tab[p][j] = (c * a.HW + (t / 3) * dil_h * wd + (t % 3) * dil_w) * 4;
     }
+  char desc[128] = "";
+  if (kernel_timing_enabled())
+    snprintf(desc, sizeof(desc), "%dx%d/%d %d->%d in %dx%dx%d out %dx%d i32 operands, i32 out", kh, kw, stride_h, ic, oc, n, h, wd, oh, ow);
+  KernelTimer timer(few ? "k_conv_direct" : "k_conv_slab", 2.0 * (double)pixels * oc * K, s, (double)bytes + 4.0 * (double)filter + 4.0 * (double)pixels * oc, desc);
   if (few) {
     a.octiles = (oc + 31) / 32;
     const unsigned blocks = (unsigned)tiles;

@@ -2472,6 +2472,7 @@ static int pack_operands(const int32_t* x, int8_t* xp, int n, int ic, int hw, co
     const int64_t act_blocks = (plan.total + 255) / 256, all_blocks = (w_total + 255) / 256;
     const int64_t w_blocks = kh * kw == 1 && all_blocks > 65536 ? grid_for(w_total, 256) : all_blocks;
     if (act_blocks + w_blocks <= INT32_MAX) {
+      KernelTimer timer("k_pack_both", ((double)npix * ic + (double)oc * ic * kh * kw) * 5.0, s);  // bytes: 4 read + 1 written per element
       k_pack_both<<<(unsigned)(act_blocks + w_blocks), 256, 0, s>>>(x, xp, plan, (unsigned)act_blocks, w, wp, w_total, oc, kh * kw, nch);
       return check_launch("pack_operands");
     }

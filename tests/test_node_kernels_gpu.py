@@ -1,5 +1,7 @@
 """Kernels of the int32 operator contract at the edges of their splits, against the oracle: long reductions, operand packing
 of a convolution, depthwise planes."""
+import ctypes
+import json
 import sys
 import threading
 import time
@@ -8,8 +10,9 @@ import numpy as np
 import pytest
 import torch
 
+import bench
 import oracle
-from cvm_runtime_amd import hipops, synth
+from cvm_runtime_amd import check, hipops, lib, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -69,6 +72,35 @@ def test_dense_operand_packing(m, k, n, dev):
     assert np.array_equal(got, oracle.dense(x, wt, None))
     packed = hipops.unpack_act_i8(hipops.pack_act_i8(T(x.reshape(m, k, 1, 1), dev)), m, k, 1, 1).cpu().numpy()
     assert np.array_equal(packed.reshape(m, k), x)
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,k,kernels", [
+    (1, 256, 14, 15, 65, 1, {"k_conv_direct"}),
+    (1, 64, 14, 15, 65, 3, {"k_conv_direct"}),
+    (4, 96, 61, 75, 160, 1, {"k_conv_slab"}),
+    (1, 128, 28, 28, 64, 3, {"k_pack_both", "k_conv_wave"}),
+    (1, 16, 28, 28, 64, 5, {"k_pack_act", "k_conv_igemm"}),   # few channels
+])
+def test_every_form_of_conv2d_is_timed(n, c, h, w, oc, k, kernels, dev):
+    """The launches between cvmhip_kernel_timing_begin and _end, with the work and the bytes of the layer."""
+    x, wt = T(synth.tensor("timed", "x%d" % c, (n, c, h, w), -127, 127), dev), T(synth.tensor("timed", "w%d" % c, (oc, c, k, k), -127, 127), dev)
+    ends = {}
+    for name in ("cvmhip_kernel_timing_end", "cvmhip_kernel_timing_end_launches"):
+        check(lib().cvmhip_kernel_timing_begin())
+        for _ in range(3):
+            y = hipops.conv2d(x, wt, None, (1, 1), (k // 2, k // 2))
+        buf = ctypes.create_string_buffer(1 << 16)
+        check(getattr(lib(), name)(buf, len(buf)))
+        ends[name] = json.loads(buf.value.decode())
+    kt, launches = ends.values()
+    assert set(kt) == kernels == {e["kernel"] for e in launches}
+    dominant = bench.dominant_conv(kt, 0.0, 3)
+    assert dominant["kernel"] in kernels and dominant["kernel"].startswith("k_conv")
+    assert dominant["conv"]["launches"] == 3 and dominant["conv"]["ms"] > 0 and dominant["ops_per_launch"] == pytest.approx(2 * y.numel() * c * k * k, rel=1e-5)
+    one = [e for e in launches if e["kernel"] == dominant["kernel"]][0]
+    assert "%dx%d/1 %d->%d in %dx%dx%d out %dx%d" % (k, k, c, oc, n, h, w, h, w) in one["desc"] and one["ms"] > 0
+    if len(kernels) == 1:
+        assert one["bytes"] == pytest.approx(4 * (x.numel() + wt.numel() + y.numel()), rel=1e-5)   # (written with seven digits)
 
 
 @pytest.mark.parametrize("n,c,mult,h,w,strides,padding,dilation", [
