@@ -296,19 +296,33 @@ static bool halo_chain(const DevChain& c, int* lo, int* hi, int* shift) {
   return c.count == 1 && q.mul == 1 && q.add == 0 && !(q.s1 && q.s2) && q.lo <= q.hi && q.lo >> *shift >= -128 && q.hi >> *shift <= 127;
 }
 
-// (g and ep as conv_prepare leaves them)
-// From 150 workgroups on (us here / k_conv_wave, 64 channels at 56 x 56: 112 workgroups 9.6 / 9.2, 140 9.9 / 9.6, 168 10.2 / 11.4, 224 10.5 / 12.7), and
-// where the patches have at most half as many pixels again as the image (64 x 100 x 75, 1.43 times: 26.7 / 29.9; 128 x 33 x 48, 1.62: 16.9 / 15.8).
-int64_t conv_halo_blocks(const ConvGeom& g, const Epilogue& ep) {
+// Is it such a layer?  (g and ep as conv_prepare leaves them)
+static bool halo_layer(const ConvGeom& g, const Epilogue& ep) {
   if (g.dw || g.row_bytes || g.Cp != 64 || g.OC % 64 != 0 || g.KH != 3 || g.KW != 3 || g.SH != 1 || g.SW != 1 || g.PH != 1 || g.PW != 1 || g.DH != 1 ||
       g.DW != 1 || ep.out_mode != OUT_I8_ACT || ep.out_cp != g.OC || ep.residual || ep.split)
-    return 0;
-  if ((int64_t)g.N * g.H * g.W * 64 > INT32_MAX) return 0;
+    return false;
   int lo, hi, shift;
-  if (!halo_chain(ep.chain, &lo, &hi, &shift)) return 0;
-  const int64_t patches = halo_patches(g), blocks = patches * (g.OC / 64);
-  if (blocks < 150 || blocks > INT32_MAX || patches * HALO_PIXELS * 2 > (int64_t)g.N * g.H * g.W * 3) return 0;
-  return blocks;
+  return (int64_t)g.N * g.H * g.W * 64 <= INT32_MAX && halo_patches(g) * (g.OC / 64) <= INT32_MAX && halo_chain(ep.chain, &lo, &hi, &shift);
+}
+// From 150 workgroups on (us here / k_conv_wave, 64 channels at 56 x 56: 112 workgroups 9.4 / 9.0, 140 9.9 / 9.6, 168 10.2 / 11.4, 224 10.8 / 13.4), and
+// where the patches have at most half as many pixels again as the image (64 x 100 x 75, 1.43 times: 26.7 / 29.9; 128 x 33 x 48, 1.62: 16.9 / 15.8).
+static bool halo_fills(const ConvGeom& g) {
+  const int64_t patches = halo_patches(g);
+  return patches * (g.OC / 64) >= 150 && patches * HALO_PIXELS * 2 <= (int64_t)g.N * g.H * g.W * 3;
+}
+
+// Without the pool also only past the 512 tiles of 64 channels x 128 pixels up to which k_conv_wave splits K over its wavefronts and is through in one
+// round.  Layers of 150 to 200 workgroups here (their patches 1.14 to 1.49 times the image), us here / there: with up to 512 such tiles 9.3-9.8 / 8.8-9.3
+// whatever the channels (64 to 384), with more 9.5-10.2 / 10.6-12.9; with the pool 8.3-8.5 / 8.9-10.5 on the near side of the line as well.
+// 192 channels are a tile and a half of k_conv_big, which would have such a layer from 160 tiles on: 9.4-9.7 / 12.4-12.6 between the two lines.
+// More channels (before it k_conv_big): 8 x 56 x 56 to 192 10.0 / 12.9, 16 x 28 x 28 to 512 10.3 / 13.2, 32 x 56 x 56 to 320 28.8 / 39.0 (with the pool
+// 22.6 / 30.7), 16 x 112 x 112 to 256 37.2 / 50.4; the least, 16 x 75 x 75 to 512, 40.5 / 44.0.
+int64_t conv_halo_blocks(const ConvGeom& g, const Epilogue& ep) {
+  if (!halo_layer(g, ep) || !halo_fills(g)) return 0;
+  const int64_t pixels = (int64_t)g.N * g.H * g.W;
+  const bool one_round = (pixels + 127) / 128 * (g.OC / 64) <= 512, large = g.OC > 64 && (pixels + 255) / 256 * ((g.OC + 127) / 128) >= 160;
+  if (!ep.pool && one_round && !large) return 0;
+  return halo_patches(g) * (g.OC / 64);
 }
 
 static void halo_geom(HaloGeom* a, const int8_t* wp, void* out, const ConvGeom& g, const Epilogue& ep, int width) {
@@ -359,7 +373,7 @@ static bool halo_stem_prepare(const cvmhip_chain* stem_chain, const cvmhip_chain
   ep->out_mode = OUT_I8_ACT;
   ep->out_cp = 64;
   ep->pool = pool;
-  return conv_halo_blocks(*g, *ep) > 0;
+  return halo_layer(*g, *ep) && halo_fills(*g);
 }
 
 }  // namespace cvmhip

@@ -109,6 +109,12 @@ def test_which_layers_take_the_large_tiles(n, ic, hw, oc, k, takes, dev, monkeyp
     (6, 40, 58, 320, True, -2048, 2047, 4, True),
     (11, 127, 161, 128, False, -127, 127, 0, True),   # several patches to a workgroup, odd extents
     (11, 126, 162, 128, True, -127, 127, 0, True),
+    (16, 28, 28, 320, False, -127, 127, 0, False),    # 160 workgroups, 490 tiles of 64 x 128
+    (16, 28, 28, 320, True, -127, 127, 0, True),      # with the pool
+    (25, 28, 28, 192, False, -127, 127, 0, False),    # 150 workgroups, 462 tiles of 64 x 128, 154 of 128 x 256
+    (26, 28, 28, 192, False, -127, 127, 0, True),     # 160 of 128 x 256
+    (84, 28, 28, 64, False, -127, 127, 0, True),      # 515 tiles of 64 x 128
+    (83, 28, 28, 64, False, -127, 127, 0, False),     # 509
     (37, 16, 32, 256, False, -127, 127, 0, False),    # 148 workgroups
     (64, 33, 48, 128, False, -127, 127, 0, False),    # patches of 1.6 times the image
     (16, 16, 32, 640, False, -512, 512, 2, False),    # 128 after the shift: its low byte
