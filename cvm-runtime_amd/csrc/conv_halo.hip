@@ -283,9 +283,10 @@ static int halo_width(int h, int w) {
   const int64_t a = (int64_t)((w + 31) / 32) * ((h + 15) / 16), b = (int64_t)((w + 63) / 64) * ((h + 7) / 8);
   return a <= b ? 32 : 64;
 }
-static int64_t halo_patches(const ConvGeom& g) {
-  return halo_width(g.H, g.W) == 32 ? (int64_t)g.N * ((g.W + 31) / 32) * ((g.H + 15) / 16) : (int64_t)g.N * ((g.W + 63) / 64) * ((g.H + 7) / 8);
+static int64_t halo_patches(const ConvGeom& g, int width) {
+  return (int64_t)g.N * ((g.W + width - 1) / width) * ((g.H + HALO_PIXELS / width - 1) / (HALO_PIXELS / width));
 }
+static int64_t halo_patches(const ConvGeom& g) { return halo_patches(g, halo_width(g.H, g.W)); }
 
 // one clamp and one shift to int8
 static bool halo_chain(const DevChain& c, int* lo, int* hi, int* shift) {
@@ -333,7 +334,7 @@ static void halo_geom(HaloGeom* a, const int8_t* wp, void* out, const ConvGeom& 
   a->tile_bytes = (HALO_CHUNKS + 1) * 1024;
   halo_chain(ep.chain, &a->lo, &a->hi, &a->shift);
   a->ocs = g.OC / 64;
-  a->patches = (int)halo_patches(g);
+  a->patches = (int)halo_patches(g, width);
   a->across = (g.W + width - 1) / width;
   a->down = (g.H + HALO_PIXELS / width - 1) / (HALO_PIXELS / width);
   a->div_oc = make_fastdiv((uint32_t)a->ocs);
@@ -360,7 +361,16 @@ int conv_halo(const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g, 
   return halo_launch<false>(a, ep.pool != 0, width, s);
 }
 
-// The first two layers of a VGG
+// The first two layers of a VGG in one launch: where halo_fills.  206 cases of 150 to 1 568 patches, up to 1.49 times the image, with the pool and without it, against
+// the faster of the two launches with k_conv_halo and with k_conv_wave for the second layer: 0.95 to 1.45 times as fast, 1.19 in the middle (us here / there:
+// 2 x 224 x 224 12.4 / 16.3, 4 x 224 x 224 17.2 / 20.3, 2 x 300 x 300 16.8 / 23.6, 43 x 46 x 46 15.4 / 16.0, 58 x 38 x 90 22.0 / 23.4, 300 x 24 x 30 22.4 / 23.9).
+// Patches of 64 x 8 need six blocks of the first layer for each wavefront instead of five, 1.14 times the time: 35 x 36 x 180 25.7 / 24.8, where 32 x 16
+// takes 22.6.  Time goes by rounds of 256 patches, one to a compute unit, so the wide ones stay where they save a round: 14 x 66 x 128 14.4 instead of 15.5,
+// 133 x 24 x 44 18.1 instead of 20.8.  (Slower than two launches: 233 x 24 x 44 and the like, 700 wide patches of 1.45 times the image, 26.2 / 25.2.)
+static int halo_stem_width(const ConvGeom& g) {
+  const int64_t narrow = (halo_patches(g, 32) + 255) / 256, wide = (halo_patches(g, 64) + 255) / 256;
+  return wide * 8 < narrow * 7 ? 64 : 32;
+}
 static bool halo_stem_prepare(const cvmhip_chain* stem_chain, const cvmhip_chain* chain, int n, int c, int h, int w, int pool, ConvGeom* g, Epilogue* ep,
                               HaloGeom* a, StemGeom* sg) {
   if (n < 1 || c < 1 || c > 4 || h < 1 || w < 1 || (pool && (h % 2 || w % 2)) || cvmhip_stem_input_bytes(n, h, w, 3, 3, 1, 1, 1, 1) == 0) return false;
@@ -373,7 +383,7 @@ static bool halo_stem_prepare(const cvmhip_chain* stem_chain, const cvmhip_chain
   ep->out_mode = OUT_I8_ACT;
   ep->out_cp = 64;
   ep->pool = pool;
-  return halo_layer(*g, *ep) && halo_fills(*g);
+  return halo_layer(*g, *ep) && halo_fills(*g) && halo_patches(*g, halo_stem_width(*g)) <= INT32_MAX;
 }
 
 }  // namespace cvmhip
@@ -400,14 +410,15 @@ int cvmhip_conv2d_stem_conv_i8(const void* xs, const void* stem_wp, const int32_
       !halo_stem_prepare(stem_chain, chain, n, c, h, w, pool, &g, &ep, &a, &sg))
     return arg_error("conv2d_stem_conv_i8: not eligible");
   ep.bias = bias;
-  const int width = halo_width(h, w);
+  const int width = halo_stem_width(g);
   a.x = reinterpret_cast<const int8_t*>(xs);
   halo_geom(&a, reinterpret_cast<const int8_t*>(wp), out, g, ep, width);
   a.stem_wf = reinterpret_cast<const int8_t*>(stem_wp);
   a.stem_bias = stem_bias;
   a.hp = sg.hp; a.wp = sg.wp;
   char desc[128] = "";
-  if (kernel_timing_enabled()) snprintf(desc, sizeof(desc), "3x3/1 %d->64 and 3x3/1 64->64 in %dx%dx%d%s", c, n, h, w, pool ? " +pool" : "");
+  if (kernel_timing_enabled()) snprintf(desc, sizeof(desc), "3x3/1 %d->64 and 3x3/1 64->64 in %dx%dx%d%s, patches of %d x %d", c, n, h, w, pool ? " +pool" : "", width,
+                                        HALO_PIXELS / width);
   KernelTimer timer("k_conv_halo", 2.0 * n * h * w * 64 * 9 * (64.0 + c), as_stream(stream),
                     4.0 * n * sg.hp * sg.wp + 64.0 * 9 * (64 + c) + (double)n * h * w * 64 / (pool ? 4 : 1), desc);
   return halo_launch<true>(a, pool != 0, width, as_stream(stream));

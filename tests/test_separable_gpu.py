@@ -1,9 +1,12 @@
 """Depthwise and 1x1 convolution in one launch, against the oracle running the graph node by node."""
+import ctypes
+import json
+
 import numpy as np
 import pytest
 
 import oracle.graph as og
-from cvm_runtime_amd import graphgen, runtime, synth
+from cvm_runtime_amd import check, graphgen, lib, runtime, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -89,7 +92,7 @@ def test_pairs_of_many_pixels_stay_two_launches(n, c, hw, oc, fused, dev, monkey
     (10, 3, 64, 128, True),       # whole patches of 32 x 16
     (9, 1, 62, 130, True),        # patches that end outside
     (9, 3, 61, 131, False),
-    (8, 4, 40, 250, True),        # patches of 64 x 8
+    (8, 4, 40, 250, True),        # outside on both sides
     (8, 3, 39, 250, False),
     (600, 3, 16, 30, False),      # several patches to a workgroup
     (7, 3, 64, 128, True),        # too few
@@ -121,3 +124,37 @@ def test_first_two_layers_of_a_vgg(n, c, h, w, pool, dev, monkeypatch):
             assert np.array_equal(v[i], want), i
     for v in out[1:]:
         assert np.array_equal(v, out[0])
+
+
+@pytest.mark.parametrize("n,h,w,pool,patches", [
+    (5, 130, 170, True, "64 x 8"),      # 270 patches of 32 x 16, 255 of 64 x 8: one round of workgroups instead of two
+    (5, 130, 170, False, "64 x 8"),
+    (14, 66, 122, True, "64 x 8"),      # 280 and 252; patches that end outside on both sides
+    (8, 130, 170, True, "32 x 16"),     # 432 and 408: two rounds either way
+    (35, 36, 180, False, "32 x 16"),    # 630 and 525: three
+    (29, 66, 128, True, "32 x 16"),
+])
+def test_patches_of_the_first_two_layers(n, h, w, pool, patches, dev, monkeypatch):
+    def net(k):
+        g = graphgen.GraphBuilder("stem-patch-%d" % w)
+        y = g.conv_relu_q(g.conv_relu_q(g.var("data", (k, 3, h, w), 8), 64, 3, 1, 1), 64, 3, 1, 1)
+        return g.build([g.conv_relu_q(g.max_pool(y, 2, 2) if pool else y, 8, 1)])
+
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "0")
+    js, pb = net(n)
+    x = synth.tensor("stem-patch", "x%d" % w, (n, 3, h, w), -127, 127)
+    out = []
+    for pair in ("1", "0"):
+        monkeypatch.setenv("CVM_HIP_SEPARABLE", pair)
+        m = runtime.HipModel(js, pb)
+        check(lib().cvmhip_kernel_timing_begin())
+        out.append(np.frombuffer(m.inference(x.astype(np.int8).tobytes()), np.int8).reshape(n, -1))
+        buf = ctypes.create_string_buffer(1 << 16)
+        check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
+        launches = [e["desc"] for e in json.loads(buf.value.decode()) if e["desc"].startswith("3x3/1 3->64 and")]
+        assert [d.split("patches of ")[1] for d in launches] == ([patches] if pair == "1" else [])
+        m.close()
+    assert np.array_equal(out[0], out[1])
+    j1, p1 = net(1)
+    for i in (0, n - 1):
+        assert np.array_equal(out[0][i], og.run_graph(j1, graphgen.load_params(p1), x[i:i + 1])[0].ravel()), i
