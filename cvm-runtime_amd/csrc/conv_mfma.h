@@ -227,6 +227,9 @@ int pack_stem_weights(const int32_t* w, int8_t* wp, int oc, int c, int kh, int k
 bool stem_pool_eligible(int c, int oc, int kh, int kw, int oh, int ow, int qh, int qw);
 int stem_pool(const int8_t* xs, const int8_t* wp, const int32_t* bias, const DevChain& chain, int8_t* out, int n, int c, int h,
               int w, int oc, int kh, int kw, int sh, int sw, int ph, int pw, int qh, int qw, hipStream_t s);
+// its tiles of 4 x 8 pooled pixels, and how many of them the chip runs at once
+constexpr int STEM_POOL_AT_ONCE = 512;
+inline int64_t stem_pool_tiles(int n, int qh, int qw) { return (int64_t)n * ((qh + 3) / 4) * ((qw + 7) / 8); }
 // the same for larger batches (conv_stem_pool.hip), where conv_stem_pool_takes says so
 bool conv_stem_pool_takes(int n, int oc, int kh, int kw, int sh, int sw, int qh, int qw);
 int conv_stem_pool(const int8_t* xs, const int8_t* wp, const int32_t* bias, const DevChain& chain, int8_t* out, const StemGeom& sg, int n, int oh, int ow, int qh,

@@ -195,9 +195,17 @@ __global__ void __launch_bounds__(256, 2) k_conv_stem_pool(const HeadGeom a) {
 
 static int64_t head_patches(int n, int qh, int qw) { return (int64_t)n * ((qh + HEAD_QH - 1) / HEAD_QH) * ((qw + HEAD_QW - 1) / HEAD_QW); }
 
-// From 80 patches on (us here / k_stem_pool at 224 x 224: batch 2, 56 patches, 9.2 / 8.3, batch 3, 84, 9.3 / 9.4, batch 5 9.4 / 9.9, 8 9.4 / 15.0, 16 11.7 / 23.2).
+// us here / k_stem_pool / two launches.  Up to 512 tiles of 4 x 8 pooled pixels k_stem_pool runs them all at once; it is the faster one while no compute unit has two
+// (3 x 224 x 224, 294 tiles, 8.4 / 8.9; 2 x 224 x 224, 196, 8.4 / 7.5; 27 x 64 x 64, 216, 8.3 / 7.6; 256 tiles 8.1 / 7.5), and where the patches, which are larger, come to a
+// second one (36 x 100 x 60, 504 tiles and 288 patches, 11.5 / 9.1).  With 257 to 330 tiles the gain depends on the map: 16 x 96 x 96 8.1 / 9.0, 5 x 171 x 171 9.2 / 8.9.
+// Past 512 tiles the alternative is two launches, and what counts is how much of the patches lies outside the map: 16 x 224 x 224, nothing, 11.5 / 22.7 / 20.5;
+// 50 x 171 x 171, 1.45 times the map, 19.5 / 37.7 / 29.0; 100 x 68 x 116, 2.04, 15.8 / 24.1 / 19.9; 200 x 100 x 60, 2.39, 25.1 / 32.4 / 26.9; 900 x 17 x 60, 2.99, 25.2 / 40.7 /
+// 24.4; 640 x 36 x 60, 3.32, 32.5 / 42.1 / 28.7; 800 x 20 x 20, 4.5, 14.9 / 22.0 / 13.7.
 bool conv_stem_pool_takes(int n, int oc, int kh, int kw, int sh, int sw, int qh, int qw) {
-  return oc == 64 && kh == HEAD_K && kw > 4 && kw <= 8 && sh == 2 && sw == 2 && head_patches(n, qh, qw) >= 80 && head_patches(n, qh, qw) <= INT32_MAX;
+  if (oc != 64 || kh != HEAD_K || kw <= 4 || kw > 8 || sh != 2 || sw != 2) return false;
+  const int64_t patches = head_patches(n, qh, qw), tiles = stem_pool_tiles(n, qh, qw);
+  if (tiles <= STEM_POOL_AT_ONCE) return patches >= 80 && tiles > 256 && patches <= 256;
+  return (patches * (HEAD_QH * HEAD_QW) <= 3 * (int64_t)n * qh * qw || n > 65535) && patches <= INT32_MAX;   // (k_stem_pool's grid ends at 65 535 images)
 }
 
 int conv_stem_pool(const int8_t* xs, const int8_t* wp, const int32_t* bias, const DevChain& chain, int8_t* out, const StemGeom& sg, int n, int oh, int ow, int qh,

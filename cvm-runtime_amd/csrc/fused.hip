@@ -582,7 +582,7 @@ int cvmhip_conv2d_stem_pool3_i8_eligible(int n, int c, int h, int wd, int oc, in
 
 int cvmhip_conv2d_stem_pool3_i8_pays(int n, int h, int wd, int oc, int kh, int kw, int stride_h, int stride_w, int pad_h, int pad_w, int pool_oh, int pool_ow) {
   // k_stem_pool has a workgroup for every 4 x 8 pooled pixels: worth it while they all run at once
-  if ((int64_t)n * ((pool_oh + 3) / 4) * ((pool_ow + 7) / 8) <= 512) return 1;
+  if (stem_pool_tiles(n, pool_oh, pool_ow) <= STEM_POOL_AT_ONCE) return 1;
   return conv_stem_pool_takes(n, oc, kh, kw, stride_h, stride_w, pool_oh, pool_ow) &&
          cvmhip_stem_input_bytes(n, h, wd, kh, kw, stride_h, stride_w, pad_h, pad_w) <= INT32_MAX;
 }

@@ -486,8 +486,12 @@ def test_conv2d_stem_with_fused_3x3_max_pool(case, dev):
     (5, 3, 224, 224, 7, 3, [("relu",), ("cvm_right_shift", 8, 9)], "k_conv_stem_pool"),   # whole patches of 8 x 14 pooled pixels; a chain with a rounding term
     (5, 3, 224, 224, 7, 3, [("clip", -90, 127)], "k_conv_stem_pool"),                    # one clamp and no shift
     (40, 4, 61, 93, 8, 3, [("clip", -128, 127)], "k_conv_stem_pool"),                    # patches past the pool's last row and column, the widest window
-    (80, 1, 23, 19, 5, 0, [("relu",), ("cvm_right_shift", 8, 6)], "k_conv_stem_pool"),   # no padding, a patch an image
-    (900, 3, 17, 60, 7, 3, [("cvm_right_shift", 8, 8)], "k_conv_stem_pool"),             # several patches to a workgroup
+    (80, 1, 37, 59, 5, 0, [("relu",), ("cvm_right_shift", 8, 6)], "k_conv_stem_pool"),   # no padding, a patch an image
+    (80, 1, 23, 19, 5, 0, [("relu",), ("cvm_right_shift", 8, 6)], "k_stem_pool"),        # 160 tiles of k_stem_pool: one for a compute unit
+    (33, 1, 69, 61, 5, 0, [("relu",), ("cvm_right_shift", 8, 6)], "k_conv_stem_pool"),   # 264 tiles, 132 patches that end outside
+    (36, 3, 100, 60, 7, 3, [("cvm_right_shift", 8, 8)], "k_stem_pool"),                  # 504 tiles, 288 patches: a second one for some compute units
+    (900, 3, 17, 60, 7, 3, [("cvm_right_shift", 8, 8)], "k_conv_stem_pool"),             # several patches to a workgroup, 2.99 times the map
+    (320, 3, 36, 60, 7, 3, [("cvm_right_shift", 8, 8)], "k_stem_pool"),                  # 3.3 times the map
     (79, 1, 23, 19, 5, 0, [("relu",), ("cvm_right_shift", 8, 6)], "k_stem_pool"),        # too few patches
 ])
 def test_stem_and_pool_of_many_images(n, c, h, w, kw, pad, stages, kernel, dev):

@@ -116,3 +116,16 @@ def test_the_build_does_without_torch(monkeypatch, tmp_path):
     monkeypatch.setattr(b.importlib.util, "find_spec", lambda name: None)
     b._build_binding()
     assert not stale.exists()
+
+
+@pytest.mark.parametrize("n,h,w,pays", [
+    (2, 224, 224, 1), (5, 224, 224, 1),     # up to 512 tiles of 4 x 8 pooled pixels
+    (50, 224, 224, 1), (50, 171, 171, 1),   # patches of 8 x 14 that cover the map, and 1.45 times it
+    (900, 17, 60, 1),                       # 2.99 times
+    (320, 36, 60, 0), (800, 20, 20, 0),     # 3.3 and 4.5 times
+    (80, 36, 60, 1),                        # 480 tiles
+    (70000, 20, 20, 1),                     # past the other kernel's grid
+])
+def test_where_a_resnet_head_is_one_launch(n, h, w, pays):
+    q = lambda v: ((v - 1) // 2) // 2 + 1
+    assert cvm_runtime_amd.lib().cvmhip_conv2d_stem_pool3_i8_pays(n, h, w, 64, 7, 7, 2, 2, 3, 3, q(h), q(w)) == pays
