@@ -289,7 +289,7 @@ PyObject* NonMaxSuppression(PyObject* const* a) {
   const int b = static_cast<int>(x.size(0)), n = static_cast<int>(x.size(1)), k = static_cast<int>(x.size(2));
   int v[7];
   for (int i = 0; i < 7; ++i) v[i] = i == 1 ? PyObject_IsTrue(a[4]) : static_cast<int>(Int(a[3 + i]));
-  at::Tensor ws = Scratch(cvmhip_nms_workspace_bytes(b, n, k), x);
+  at::Tensor ws = Scratch(cvmhip_nms_topk_workspace_bytes(b, n, k, v[2]), x);
   int32_t *xp = Ptr(x), *cp = Ptr(a[1]), *yp = Ptr(a[2]);
   void* s = Stream();
   Launch([&] {

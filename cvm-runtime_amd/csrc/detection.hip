@@ -998,8 +998,13 @@ static size_t nms_rows_bytes(int batches, int n, int k) {
   else per += (size_t)BIN_COUNT * ((n + BIN_CHUNK - 1) / BIN_CHUNK) + BIN_COUNT + 1;
   return (size_t)batches * per * sizeof(int32_t);
 }
+// rows of a batch that the walk may see
+static int nms_candidates(int n, int topk) { return topk >= 0 && topk < n ? topk : n; }
 // overlap masks of a batch's candidates (at most 2^18: nms_check_args)
-static int64_t nms_mask_words(int n) { return n < NMS_PAIRS_LEAST ? 0 : (int64_t)(n < (1 << 18) ? n : 1 << 18) * NMS_PAIRS_WORDS; }
+static int64_t nms_mask_words(int n, int topk) {
+  const int most = nms_candidates(n, topk);
+  return most < NMS_PAIRS_LEAST ? 0 : (int64_t)(most < (1 << 18) ? most : 1 << 18) * NMS_PAIRS_WORDS;
+}
 
 // Validation and launches shared by the two entry points.  `workspace`: nms_rows_bytes(), behind it the tally of every batch and, where
 // the caller has room for them, the overlap masks.
@@ -1053,7 +1058,7 @@ static int nms_launch(int32_t* x, const int32_t* valid_count, int32_t* y,
   // the ranks, or positions, have been read: their words hold the keep flags of the sorted positions from here on
   uint8_t* flags = reinterpret_cast<uint8_t*>(rank);
   const int by_class = force_suppress || id_index < 0 ? 0 : 1;
-  const int most = topk > 0 && topk < n ? topk : n;
+  const int most = nms_candidates(n, topk);
   const int classes = by_class ? NMS_CLASSES : 1;
   if (most < NMS_PAIRS_LEAST) masks = nullptr;
   // A workgroup has a compute unit to itself (100 KiB of LDS): what goes past one round of them is paid by classes that have no pairs
@@ -1064,7 +1069,7 @@ static int nms_launch(int32_t* x, const int32_t* valid_count, int32_t* y,
     const int most_groups = most >= 8192 ? 512 : 256;
     while (parts < 4 && classes * batches * parts * 2 <= most_groups) parts *= 2;
   }
-  k_nms_walk<<<dim3(classes * parts, batches), NMS_THREADS, 0, s>>>(valid_count, sorted, code, list, kept, flags, tally, masks, nms_mask_words(n), n, k,
+  k_nms_walk<<<dim3(classes * parts, batches), NMS_THREADS, 0, s>>>(valid_count, sorted, code, list, kept, flags, tally, masks, nms_mask_words(n, topk), n, k,
                                                                    iou_threshold, topk, coord_start, id_index, by_class, parts);
   rc = check_launch("nms.walk");
   if (rc) return rc;
@@ -1105,9 +1110,10 @@ int cvmhip_get_valid_counts(const int32_t* x, int32_t* valid_count, int32_t* y,
   return check_launch("get_valid_counts.scatter");
 }
 
-size_t cvmhip_nms_workspace_bytes(int batches, int n, int k) {
-  return nms_rows_bytes(batches, n, k) + (size_t)batches * (NMS_TALLY * 4 + (size_t)nms_mask_words(n) * 8);
+size_t cvmhip_nms_topk_workspace_bytes(int batches, int n, int k, int topk) {
+  return nms_rows_bytes(batches, n, k) + (size_t)batches * (NMS_TALLY * 4 + (size_t)nms_mask_words(n, topk) * 8);
 }
+size_t cvmhip_nms_workspace_bytes(int batches, int n, int k) { return cvmhip_nms_topk_workspace_bytes(batches, n, k, -1); }
 
 int cvmhip_non_max_suppression(int32_t* x, const int32_t* valid_count, int32_t* y,
                                int batches, int n, int k, int max_output_size,
@@ -1116,7 +1122,7 @@ int cvmhip_non_max_suppression(int32_t* x, const int32_t* valid_count, int32_t* 
                                void* workspace, size_t workspace_bytes, void* stream) {
   const int rc = nms_check_args(x, valid_count, y, batches, n, k, iou_threshold, coord_start, score_index, id_index, topk);
   if (rc) return rc;
-  if (!workspace || workspace_bytes < cvmhip_nms_workspace_bytes(batches, n, k)) return arg_error("non_max_suppression workspace");
+  if (!workspace || workspace_bytes < cvmhip_nms_topk_workspace_bytes(batches, n, k, topk)) return arg_error("non_max_suppression workspace");
   return nms_launch(x, valid_count, y, batches, n, k, max_output_size, iou_threshold, topk, coord_start, score_index,
                     id_index, force_suppress, workspace, true, as_stream(stream));
 }

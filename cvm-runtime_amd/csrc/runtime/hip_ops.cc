@@ -226,7 +226,7 @@ void RegisterAll() {
   {
     OpKernel k;
     k.workspace_bytes = [](const OpCall& c) {
-      return cvmhip_nms_workspace_bytes((int)c.in[0].shape[0], (int)c.in[0].shape[1], (int)c.in[0].shape[2]);
+      return cvmhip_nms_topk_workspace_bytes((int)c.in[0].shape[0], (int)c.in[0].shape[1], (int)c.in[0].shape[2], (int)c.attrs->i("top_k"));
     };
     k.run = [](OpCall& c) {
       const Shape& x = c.in[0].shape;

@@ -88,7 +88,7 @@ def get_valid_counts(x, score_threshold):
 
 def non_max_suppression(x, valid_count, y, iou_threshold, force_suppress, top_k, id_index, coord_start, score_index, max_output_size):
     b, n, k = x.shape
-    ws = _workspace(lib().cvmhip_nms_workspace_bytes(b, n, k), x.device)
+    ws = _workspace(lib().cvmhip_nms_topk_workspace_bytes(b, n, k, top_k), x.device)
     check(lib().cvmhip_non_max_suppression(_ptr(x), _ptr(valid_count), _ptr(y), b, n, k, max_output_size, iou_threshold, top_k,
                                            coord_start, score_index, id_index, int(bool(force_suppress)), _scratch(ws), _size(ws),
                                            _stream()))

@@ -307,8 +307,8 @@ int64_t HIPOpExtraSpace(const cvm::NodeAttrs& attrs, const std::vector<TShape>& 
   } else if (op == "get_valid_counts" && in_shapes.size() >= 1 && in_shapes[0].ndim() == 3) {
     bytes = cvmhip_get_valid_counts_workspace_bytes(static_cast<int>(in_shapes[0][0]), static_cast<int>(in_shapes[0][1]));
   } else if (op == "non_max_suppression" && in_shapes.size() >= 1 && in_shapes[0].ndim() == 3) {
-    bytes = cvmhip_nms_workspace_bytes(static_cast<int>(in_shapes[0][0]), static_cast<int>(in_shapes[0][1]),
-                                       static_cast<int>(in_shapes[0][2]));
+    bytes = cvmhip_nms_topk_workspace_bytes(static_cast<int>(in_shapes[0][0]), static_cast<int>(in_shapes[0][1]), static_cast<int>(in_shapes[0][2]),
+                                            cvm::get<cvm::top::NonMaximumSuppressionParam>(attrs.parsed).top_k);
   }
   return static_cast<int64_t>((bytes + 3) / 4);
 }

@@ -141,7 +141,9 @@ int cvmhip_get_valid_counts(const int32_t* x, int32_t* valid_count, int32_t* y,
  * batch with no valid rows, its stop at the first negative id and its in-place
  * overwrite of x rows past top_k (x is therefore written, and must not alias y).
  * No host synchronisation: valid_count is read on the device.
- * `workspace`: cvmhip_nms_workspace_bytes() bytes of scratch. */
+ * `workspace`: cvmhip_nms_topk_workspace_bytes() bytes of scratch for the topk of the call, which is what the overlap masks of the
+ * walk are sized by; cvmhip_nms_workspace_bytes() bytes do for any topk. */
+size_t cvmhip_nms_topk_workspace_bytes(int batches, int n, int k, int topk);
 size_t cvmhip_nms_workspace_bytes(int batches, int n, int k);
 int cvmhip_non_max_suppression(int32_t* x, const int32_t* valid_count, int32_t* y,
                                int batches, int n, int k, int max_output_size,
@@ -151,10 +153,10 @@ int cvmhip_non_max_suppression(int32_t* x, const int32_t* valid_count, int32_t* 
 /* The same operator for callers that cannot allocate device memory or bring a workspace (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The scratch is
  * a fixed array inside the library's code object, cvmhip_nms_static_capacity_bytes() bytes (2 MiB) per GPU,
- * held until the process ends; a call whose rows (cvmhip_nms_workspace_bytes(batches, n, k) without what it holds for the overlap
- * masks of the walk, 80 bytes a row, which this entry does without) exceed it returns CVMHIP_ERR_ARG.  The call allocates and frees nothing.  All calls on one GPU share the array: calls that
- * overlap in time on one GPU (two streams, two threads) race and must be serialised by the caller.  The
- * first call on a device looks the array's address up (hipGetSymbolAddress); make it outside stream capture. */
+ * held until the process ends.  This entry walks without overlap masks: a call for whose rows alone the array is too small
+ * (cvmhip_nms_topk_workspace_bytes(batches, n, k, 0) less 516 bytes a batch) returns CVMHIP_ERR_ARG.  The call allocates and frees nothing.
+ * All calls on one GPU share the array: calls that overlap in time on one GPU (two streams, two threads) race and must be
+ * serialised by the caller.  The first call on a device looks the array's address up (hipGetSymbolAddress); make it outside stream capture. */
 size_t cvmhip_nms_static_capacity_bytes(void);
 int cvmhip_non_max_suppression_static(int32_t* x, const int32_t* valid_count, int32_t* y,
                                       int batches, int n, int k, int max_output_size,

@@ -1,11 +1,13 @@
 """Non-maximum suppression at the edges of its split: windows of rows, kept rows beyond the LDS list, classes sharing a
 workgroup, the ranking's slices and chunks -- against the oracle, output and mutated input."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from cvm_runtime_amd import hipops, synth
+from cvm_runtime_amd import check, hipops, lib, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +88,29 @@ def test_valid_counts_splits(n, k, dev):
         assert int(vc[b]) == len(rows)
         got = y[b].cpu().numpy()
         assert np.array_equal(got[:len(rows)], rows) and (got[len(rows):] == -1).all()
+
+
+@pytest.mark.parametrize("b,n,ids,force,top_k", [
+    (2, 5000, 20, False, 128), (2, 5000, 1, False, 129),      # the masks begin at 129 candidates
+    (2, 5000, 1, True, 400), (3, 1100, 1, False, 1024), (2, 8200, 8, False, 1000), (2, 1100, 1, False, -1), (2, 300, 2, False, 0),
+])
+def test_nms_workspace_of_a_top_k(b, n, ids, force, top_k, dev):
+    """The walk stays inside a workspace that holds masks for top_k rows, and one byte less is refused."""
+    x = _rows("nms-ws-%d-%d" % (n, top_k), b, n, (0, ids - 1), 512, 48, False)
+    vc = np.full((b,), n, np.int32)
+    init = np.full_like(x, 5)
+    y_ref, x_after = oracle.non_max_suppression(x, vc, 45, force, top_k, max_output_size=-1, y_init=init)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    tx, tv, ty = T(x), T(vc), T(init)
+    need = lib().cvmhip_nms_topk_workspace_bytes(b, n, 6, top_k)
+    ws = torch.full((need + 65536,), 0x5a, dtype=torch.uint8, device=dev)
+
+    def call(size):
+        return lib().cvmhip_non_max_suppression(ctypes.c_void_p(tx.data_ptr()), ctypes.c_void_p(tv.data_ptr()), ctypes.c_void_p(ty.data_ptr()), b, n, 6, -1, 45,
+                                                top_k, 2, 1, 0, int(force), ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(size), None)
+    assert call(need - 1) == 10
+    torch.cuda.synchronize()
+    check(call(need))
+    torch.cuda.synchronize()
+    assert np.array_equal(ty.cpu().numpy(), y_ref) and np.array_equal(tx.cpu().numpy(), x_after)
+    assert bool((ws[need:] == 0x5a).all())

@@ -129,3 +129,15 @@ def test_the_build_does_without_torch(monkeypatch, tmp_path):
 def test_where_a_resnet_head_is_one_launch(n, h, w, pays):
     q = lambda v: ((v - 1) // 2) // 2 + 1
     assert cvm_runtime_amd.lib().cvmhip_conv2d_stem_pool3_i8_pays(n, h, w, 64, 7, 7, 2, 2, 3, 3, q(h), q(w)) == pays
+
+
+def test_nms_workspace_by_its_candidates():
+    L = cvm_runtime_amd.lib()
+    rows = L.cvmhip_nms_topk_workspace_bytes(1, 24564, 6, 0)
+    assert rows < 2 << 20
+    assert L.cvmhip_nms_topk_workspace_bytes(1, 24564, 6, 400) == rows + 400 * 80
+    assert L.cvmhip_nms_topk_workspace_bytes(2, 24564, 6, 128) == 2 * rows              # too few for masks
+    assert L.cvmhip_nms_topk_workspace_bytes(1, 24564, 6, -1) == rows + 24564 * 80
+    assert L.cvmhip_nms_topk_workspace_bytes(1, 24564, 6, 30000) == L.cvmhip_nms_workspace_bytes(1, 24564, 6) == rows + 24564 * 80
+    # the static entry takes what fits without masks
+    assert L.cvmhip_nms_topk_workspace_bytes(1, 37000, 6, 0) - 516 <= L.cvmhip_nms_static_capacity_bytes() < L.cvmhip_nms_workspace_bytes(1, 37000, 6)
