@@ -67,12 +67,12 @@ __global__ void __launch_bounds__(IMPORT_THREADS) k_import_stem(const ImportStem
     if (tid != 0) return;
     const uint32_t total = (uint32_t)(a.n * a.chunks);
     const uint64_t began = wall_clock64();
-    for (uint32_t seen = 0; seen < total;) {
+    for (uint32_t seen = 0; seen < total;) {   // (no patience at all gives up whatever the host has copied)
       const uint64_t v = __hip_atomic_load(a.progress_host, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      if ((uint32_t)(v >> 32) == a.ticket && (uint32_t)v > seen) {
+      if ((uint32_t)(v >> 32) == a.ticket && (uint32_t)v > seen && a.patience != 0) {
         seen = (uint32_t)v;
         __hip_atomic_store(a.progress_dev, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      } else if (wall_clock64() - began > a.patience) {
+      } else if (wall_clock64() - began >= a.patience) {
         __hip_atomic_store(a.error_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         __hip_atomic_store(a.progress_dev, (uint64_t)a.ticket << 32 | IMPORT_GIVEN_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         break;

@@ -474,7 +474,11 @@ void HipGraphRuntime::ReadHooks() {
   const std::string spin = env("CVM_HIP_SEQ_SPIN");
   if (!spin.empty() && spin[0] >= '0' && spin[0] <= '9') hooks_.seq_spin = std::atoi(spin.c_str());
   const std::string gate = env("CVM_HIP_GATE_US");
-  if (!gate.empty() && gate[0] >= '0' && gate[0] <= '9') hooks_.gate_us = static_cast<uint32_t>(std::atoi(gate.c_str()));
+  if (!gate.empty() && gate[0] >= '0' && gate[0] <= '9') {
+    hooks_.gate_us = hooks_.gate_us_later = static_cast<uint32_t>(std::atoi(gate.c_str()));
+    const size_t comma = gate.find(',');
+    if (comma != std::string::npos) hooks_.gate_us_later = static_cast<uint32_t>(std::atoi(gate.c_str() + comma + 1));
+  }
   // CVM_HIP_SEQCFG="index:config,index:config,...": the tile configuration of single layers of a sequence launch
   const std::string per_layer = env("CVM_HIP_SEQCFG");
   for (size_t at = 0; at < per_layer.size();) {
@@ -977,6 +981,7 @@ const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, 
   const bool whole = fused_ && residents_.size() == 1 && residents_[0].whole_call && !(residents_[0].under_seq && SeqNow()) &&
                      !seq_calibration_pending_ && !cvmhip_kernel_timing_active();
   if (!whole) {
+    if (gate_rest_ > 0 && --gate_rest_ == 0) DropCallGraph();   // the packing launch is tried again
     const bool as_call = graph_state_ == 3 && seq_mode_ == SeqNow() && !seq_calibration_pending_ && !cvmhip_kernel_timing_active() && CaptureCall();
     if (as_call && call_packs_) {
       CheckData(shape);
@@ -1027,7 +1032,7 @@ const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, 
 // before the host copies the caller's bytes and follows the copy (a call of ResNet-50 at batch 16 418 -> 401 us, VGG-16 490 -> 472, SSD-512
 // 255 -> 243; ResNet-50 at batch 50 1 050 -> 1 044: there the host's copy from memory, 44 GB/s, is as long as the bus).
 bool HipGraphRuntime::GateEligible() const {
-  if (gate_refused_ || !fused_ || !data_stays_i8_ || shape_size(InputShape()) <= (256 << 10) || plan_.empty()) return false;
+  if (gate_rest_ > 0 || !fused_ || !data_stays_i8_ || shape_size(InputShape()) <= (256 << 10) || plan_.empty()) return false;
   const PlanStep& st = plan_[0];
   if (st.kind != PlanStep::STEMPACK || !PacksStagedInput(st) || in_resident_[0] || resident_at_[0] >= 0) return false;
   for (size_t i = 1; i < plan_.size(); ++i)
@@ -1069,12 +1074,20 @@ void HipGraphRuntime::GateInput(const int8_t* host) {
 }
 
 // The packing launch has waited in vain (the host was kept from copying for its patience): what ran behind it is void, and the
-// call is run again on the bytes in the pinned buffer, by the launches that the model started with.
+// call is run again on the bytes in the pinned buffer, by the launches that the model started with.  So are the next GATE_REST calls: one
+// stall (the first touch of a mapped file, a host thread that was not scheduled) must not cost the form for good, and a source that stalls every
+// time must not cost its patience every time.
 bool HipGraphRuntime::GateGaveUp() {
   uint32_t* error = reinterpret_cast<uint32_t*>(static_cast<uint64_t*>(gate_host_) + 1);
-  if (__atomic_load_n(error, __ATOMIC_ACQUIRE) == 0) return false;
+  if (__atomic_load_n(error, __ATOMIC_ACQUIRE) == 0) {
+    gate_rest_next_ = GATE_REST;
+    return false;
+  }
   *error = 0;
-  gate_refused_ = true;
+  std::cerr << "cvm hip: the host was kept from copying an input while the device waited for it; the next " << gate_rest_next_ << " calls copy it first\n";
+  gate_rest_ = gate_rest_next_ + 1;
+  gate_rest_next_ = std::min(2 * gate_rest_next_, GATE_REST_MOST);
+  hooks_.gate_us = hooks_.gate_us_later;
   DropGraphs();
   if (graph_state_ == 3) graph_state_ = 2;
   return true;
@@ -1153,6 +1166,13 @@ void HipGraphRuntime::DropGraphs() {
     if (*exec) cvmhip_graph_destroy(*exec);
     *exec = nullptr;
   }
+}
+
+void HipGraphRuntime::DropCallGraph() {
+  if (!call_exec_) return;
+  cvmhip_stream_sync(stream_);
+  cvmhip_graph_destroy(call_exec_);
+  call_exec_ = nullptr;
 }
 
 const std::vector<const int32_t*>& HipGraphRuntime::FetchOutputs() {

@@ -234,6 +234,7 @@ class HipGraphRuntime {
   void ExportOutputs(bool status);
   bool CaptureCall();
   void DropGraphs();
+  void DropCallGraph();
   const std::vector<const int32_t*>& CollectOutputs(bool status);
   void AllocOutputStage();
   void AwaitTicket();
@@ -252,7 +253,9 @@ class HipGraphRuntime {
   bool call_refused_ = false;    // that could not be captured
   // The input packed by a launch in front of the call's graph while the host copies it (cvmhip_import_stem_i8)
   bool call_packs_ = false;      // call_exec_ begins behind that packing
-  bool gate_refused_ = false;    // such a launch has given up: not again with this model
+  // After one that has given up the input is copied first for GATE_REST calls, for twice as many after each further one in a row
+  static constexpr uint32_t GATE_REST = 64, GATE_REST_MOST = 65536;
+  uint32_t gate_rest_ = 0, gate_rest_next_ = GATE_REST;
   bool GateEligible() const;
   void GateInput(const int8_t* host);
   bool GateGaveUp();
@@ -270,8 +273,9 @@ class HipGraphRuntime {
   struct Hooks {
     bool fold_bias = true, fuse = true, graph = true, dw_on_mfma = true, seq = true, seq_forced = false, pool_fuse = true, head_pair = true, head_group = true, conv_group = true;
     int conv_kernel = 0, wave_cfg = -1, tile_wm = 0, tile_wn = 0;
-    // CVM_HIP_GATE_US=<us> patience of the packing launch with the host's copy (0: gives up at once; default half a second)
-    uint32_t gate_us = 500000;
+    // CVM_HIP_GATE_US=<us>[,<us>] patience of the packing launch with the host's copy (0: gives up at once; default half a second), and of
+    // those behind the first one that gives up
+    uint32_t gate_us = 500000, gate_us_later = 500000;
     // layer-sequence launches: CVM_HIP_SEQ_SPIN=<polls> patience of a wait at a layer boundary (0: every wait gives up at once)
     int seq_spin = 2000000;
     // CVM_HIP_RESIDENT=0: no launches with the maps in LDS; =1: no layer sequences, which a measurement at load may

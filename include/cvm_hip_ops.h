@@ -190,7 +190,7 @@ int cvmhip_export_words(const void* const* src, void* const* dst_host, const int
                         uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, void* stream);
 /* An int8 image batch in pinned host memory (16-byte aligned, 16 readable bytes behind it) into the layout of cvmhip_pack_stem_input_i8, by a launch that may be
  * issued before the bytes are there: the host copies chunks of cvmhip_import_stem_rows image rows (0: not available for these sizes), all channels
- * of them, image by image, and stores `ticket << 32 | chunks copied` to *progress_host (pinned) behind each.  Waits are bounded by patience_us: a
+ * of them, image by image, and stores `ticket << 32 | chunks copied` to *progress_host (pinned) behind each.  Waits are bounded by patience_us (0: gives up at once): a
  * launch that gives up sets *error_host (pinned), and what it was to write is undefined.  `progress_dev`: a device word of the caller's,
  * zeroed once; `ticket` differs from the one before it. */
 int cvmhip_import_stem_rows(int n, int c, int h, int w);

@@ -67,6 +67,24 @@ def test_packing_follows_the_copy(n, c, h, w, k, stride, precision, patience, de
     model.close()
 
 
+@pytest.mark.parametrize("patience,calls,told", [("0", 67, 1), ("0", 68, 2), ("0,500000", 200, 1)])
+def test_packing_is_tried_again(patience, calls, told, dev, monkeypatch, capfd):
+    """A packing launch that gives up says so; 64 calls later the form is taken again, and stays if that one does not."""
+    monkeypatch.setenv("CVM_HIP_GATE_US", patience)
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "0")
+    g = graphgen.GraphBuilder("io-again")
+    js, pb = g.build([g.conv_relu_q(g.var("data", (1, 3, 300, 300), 8), 8, 3, 2, 1)])
+    model = runtime.HipModel(js, pb)
+    params = graphgen.load_params(pb)
+    inputs = [synth.tensor("io-again", str(i), (1, 3, 300, 300), -127, 127) for i in range(3)]
+    want = [og.run_graph(js, params, v)[0].ravel() for v in inputs]
+    for i in range(calls):   # the third is the first with a packing launch
+        got = np.frombuffer(model.inference(inputs[i % 3].astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want[i % 3]), i
+    model.close()
+    assert capfd.readouterr().err.count("the host was kept from copying") == told
+
+
 def test_many_calls_in_a_row(dev):
     """Past the 64 calls after which the stream itself is waited for; outputs of several kilobytes."""
     g, heads = graphgen.conv_op_graph(n=1, c=32, h=9, w=9, oc=40)
