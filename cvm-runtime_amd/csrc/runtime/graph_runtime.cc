@@ -475,9 +475,9 @@ void HipGraphRuntime::ReadHooks() {
   if (!spin.empty() && spin[0] >= '0' && spin[0] <= '9') hooks_.seq_spin = std::atoi(spin.c_str());
   const std::string gate = env("CVM_HIP_GATE_US");
   if (!gate.empty() && gate[0] >= '0' && gate[0] <= '9') {
-    hooks_.gate_us = hooks_.gate_us_later = static_cast<uint32_t>(std::atoi(gate.c_str()));
+    hooks_.gate_us = hooks_.gate_us_later = std::atoi(gate.c_str());
     const size_t comma = gate.find(',');
-    if (comma != std::string::npos) hooks_.gate_us_later = static_cast<uint32_t>(std::atoi(gate.c_str() + comma + 1));
+    if (comma != std::string::npos) hooks_.gate_us_later = std::atoi(gate.c_str() + comma + 1);
   }
   // CVM_HIP_SEQCFG="index:config,index:config,...": the tile configuration of single layers of a sequence launch
   const std::string per_layer = env("CVM_HIP_SEQCFG");
@@ -1044,9 +1044,12 @@ void HipGraphRuntime::GateInput(const int8_t* host) {
   const PlanStep& st = plan_[0];
   uint64_t* progress = static_cast<uint64_t*>(gate_host_);
   const uint64_t call = static_cast<uint64_t>(++gate_ticket_) << 32;
+  // Patience: 0.1 s and the copy at 1 GB/s.  While the launch waits it holds up to 65 compute units that a layer-sequence launch of another model needs all at
+  // once; that one gives up after 0.27 s (seq_spin polls) and is then off for good, so a host thread that stalls here must not keep it as long.
+  const uint32_t patience = static_cast<uint32_t>(hooks_.gate_us >= 0 ? hooks_.gate_us : 100000 + shape_size(InputShape()) / 1000);
   HipCheck(cvmhip_import_stem_i8(in_stage_host_, data_range_, PackedImage(st), st.n, st.c, st.h, st.w, st.kh, st.kw,
                                  st.sh, st.sw, st.ph, st.pw, progress, static_cast<uint64_t*>(gate_dev_), reinterpret_cast<uint32_t*>(progress + 1),
-                                 gate_ticket_, hooks_.gate_us, stream_), "import_stem_i8");
+                                 gate_ticket_, patience, stream_), "import_stem_i8");
   const size_t plane = static_cast<size_t>(st.h) * st.w, rows = static_cast<size_t>(cvmhip_import_stem_rows(st.n, st.c, st.h, st.w));
   char* to = static_cast<char*>(in_stage_host_);
   const char* from = reinterpret_cast<const char*>(host);

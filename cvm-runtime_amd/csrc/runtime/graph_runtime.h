@@ -273,9 +273,9 @@ class HipGraphRuntime {
   struct Hooks {
     bool fold_bias = true, fuse = true, graph = true, dw_on_mfma = true, seq = true, seq_forced = false, pool_fuse = true, head_pair = true, head_group = true, conv_group = true;
     int conv_kernel = 0, wave_cfg = -1, tile_wm = 0, tile_wn = 0;
-    // CVM_HIP_GATE_US=<us>[,<us>] patience of the packing launch with the host's copy (0: gives up at once; default half a second), and of
+    // CVM_HIP_GATE_US=<us>[,<us>] patience of the packing launch with the host's copy (0: gives up at once; default GateInput's own), and of
     // those behind the first one that gives up
-    uint32_t gate_us = 500000, gate_us_later = 500000;
+    int64_t gate_us = -1, gate_us_later = -1;
     // layer-sequence launches: CVM_HIP_SEQ_SPIN=<polls> patience of a wait at a layer boundary (0: every wait gives up at once)
     int seq_spin = 2000000;
     // CVM_HIP_RESIDENT=0: no launches with the maps in LDS; =1: no layer sequences, which a measurement at load may

@@ -2,14 +2,16 @@
 of the images; include/cvm_hip_ops.h: cvmhip_conv_seq_*) against the CPU oracle executing the same graph node
 by node, and against the same model with one launch per layer.  Bit-exact.  CVM_HIP_SEQ=1 forces the
 sequences (by default a model measures both ways when it is loaded and keeps the faster), =0 switches them off."""
+import ctypes
 import json
 import os
 
 import numpy as np
 import pytest
+import torch
 
 import oracle.graph as og
-from cvm_runtime_amd import graphgen, runtime, synth
+from cvm_runtime_amd import check, graphgen, lib, runtime, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -377,3 +379,47 @@ def test_a_run_that_is_repeated_finds_its_input(how, dev, monkeypatch):
         got = np.frombuffer(m.inference(x.astype(np.int8).tobytes()), np.int8).astype(np.int32)
         assert np.array_equal(got, want)
     m.close()
+
+
+@pytest.mark.parametrize("spin", ["", "200"])   # patience of the sequence's waits: its own, or some 100 us, which may run out meanwhile
+def test_a_sequence_beside_a_packing_launch_whose_host_does_not_copy(spin, dev, monkeypatch):
+    """Another model's packing launch (cvmhip_import_stem_i8) holds up to 65 workgroups while its host copies, and a sequence launch
+    needs every compute unit.  Here nobody copies: the packing launch gives up after 20 ms, the sequence waits for the compute units or
+    gives up as well, and the model's results are the right ones either way."""
+    g, heads = graphgen.resnet50(8, width=16, size=64, classes=50, config_id="seq-beside")
+    js, pb = g.build(heads)
+    x = synth.tensor("seq-beside", "data", (8, 3, 64, 64), -127, 127).astype(np.int8)
+    want = _run(js, pb, x, "0")
+    monkeypatch.setenv("CVM_HIP_SEQ", "1")
+    if spin:
+        monkeypatch.setenv("CVM_HIP_SEQ_SPIN", spin)
+    m = runtime.HipModel(js, pb)
+    L = lib()
+    n, c, h, w = 16, 3, 224, 224
+    assert L.cvmhip_import_stem_rows(n, c, h, w) > 0
+    L.cvmhip_stem_input_bytes.restype = ctypes.c_size_t
+    host, word, stream = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    check(L.cvmhip_host_alloc(ctypes.byref(host), ctypes.c_size_t(n * c * h * w + 16)))
+    check(L.cvmhip_host_alloc(ctypes.byref(word), ctypes.c_size_t(64)))
+    ctypes.memset(word, 0, 64)
+    check(L.cvmhip_stream_create(ctypes.byref(stream)))
+    xs = torch.zeros(L.cvmhip_stem_input_bytes(n, h, w, 7, 7, 2, 2, 3, 3), dtype=torch.uint8, device=dev)
+    seen = torch.zeros(1, dtype=torch.int64, device=dev)
+    gave_up = ctypes.c_uint32.from_address(word.value + 8)
+    outs = [m.inference(x.tobytes()) for _ in range(3)]   # eager, capture, replay
+    torch.cuda.synchronize()
+    for ticket in (1, 2, 3):
+        check(L.cvmhip_import_stem_i8(host, 127, ctypes.c_void_p(xs.data_ptr()), n, c, h, w, 7, 7, 2, 2, 3, 3, word, ctypes.c_void_p(seen.data_ptr()),
+                                      ctypes.c_void_p(word.value + 8), ticket, 20000, stream))
+        outs += [m.inference(x.tobytes()) for _ in range(3)]
+        check(L.cvmhip_stream_sync(stream))
+        assert gave_up.value == 1
+        gave_up.value = 0
+    after = m.launch_counts()
+    m.close()
+    check(L.cvmhip_stream_destroy(stream))
+    check(L.cvmhip_host_free(host))
+    check(L.cvmhip_host_free(word))
+    for o in outs:
+        assert np.array_equal(np.frombuffer(o, np.int32), want)
+    assert spin or after[1] >= 1, "20 ms are within the sequence's own patience"
