@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "conv_mfma.h"
+#include "requant.h"
 
 namespace cvmhip {
 
@@ -50,26 +51,12 @@ __device__ __forceinline__ void halo_request(const void* from, uint32_t lds_at) 
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_at) : "memory");
 }
 
-// (lo <= hi)
-__device__ __forceinline__ int halo_clamp(int v, int lo, int hi) {
-  int r;
-  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(lo), "v"(hi));
-  return r;
-}
-
-// shift and saturate sixteen results of a lane to int8, 16 consecutive channels of its pixel: lower half of the wavefront channels 0 .. 15 of the 32, upper 16 .. 31
-// (results are int8 whatever they come from: the saturation never acts)
+// shift sixteen results of a lane to int8 (results are int8 whatever they come from: the saturation never acts)
 __device__ __forceinline__ v4i halo_pack(const int (&v)[16], int shift) {
   uint32_t d[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const uint32_t lo2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[q * 4], (uint32_t)v[q * 4 + 1], (uint32_t)shift);
-    const uint32_t hi2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[q * 4 + 2], (uint32_t)v[q * 4 + 3], (uint32_t)shift);
-    d[q] = __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
-  }
-  typedef unsigned v2u __attribute__((ext_vector_type(2)));
-  const v2u s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
-  return v4i{(int)s0.x, (int)s0.y, (int)s1.x, (int)s1.y};
+  for (int q = 0; q < 4; ++q) d[q] = shift_to_bytes(v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3], shift);
+  return sixteen_channels(d);
 }
 
 // 16 sums of a lane as they start, from 32 biases in LDS: element e is channel (e / 4) * 8 + lgrp * 4 + e % 4
@@ -181,10 +168,10 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
         v16i sum = halo_first(s_bias + 64 + i * 32, lgrp);
 #pragma unroll
         for (int c = 0; c < 2; ++c) sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(stem_f[i][c], window[k][c], sum, 0, 0, 0);
-        asm volatile("s_nop 15\n\ts_nop 7" : "+v"(sum));   // as below
+        asm volatile(WAIT_16_PASSES : "+v"(sum));
         int v[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = halo_clamp(sum[e], a.stem_lo, a.stem_hi);
+        for (int e = 0; e < 16; ++e) v[e] = clamp_uniform(sum[e], a.stem_lo, a.stem_hi);
         const v4i w = halo_pack(v, a.stem_shift);
         if (q < PLANE) *reinterpret_cast<v4i*>(smem + HALO_FILTER + ((i * 2 + lgrp) * PLANE + q) * 16) = ok ? w : v4i{0, 0, 0, 0};
       }
@@ -245,9 +232,7 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
       corner_of(patch);
       if constexpr (!STEM) fetch();
     }
-    // A vector instruction may read a product's registers 19 wait states behind it.  The compiler sees to that for instructions it knows; halo_clamp
-    // is inline assembly to it.
-    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[1][2]),
+    asm volatile(WAIT_16_PASSES : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[1][2]),
                  "+v"(acc[1][3]));
     const int OW = POOL ? a.W >> 1 : a.W, OH = POOL ? a.H >> 1 : a.H;
     const int cblocks = a.OC >> 5;
@@ -264,7 +249,7 @@ __global__ void __launch_bounds__(256, 2) k_conv_halo(const HaloGeom a) {
         for (int e = 0; e < 16; ++e) {
           int m = acc[i][j][e];
           if (POOL) m = max(max(m, acc[i][1][e]), max(acc[i][2][e], acc[i][3][e]));
-          v[e] = halo_clamp(m, a.lo, a.hi);
+          v[e] = clamp_uniform(m, a.lo, a.hi);
         }
         const v4i w = halo_pack(v, a.shift);
         if (ok) {
@@ -289,13 +274,7 @@ static int64_t halo_patches(const ConvGeom& g, int width) {
 static int64_t halo_patches(const ConvGeom& g) { return halo_patches(g, halo_width(g.H, g.W)); }
 
 // one clamp and one shift to int8
-static bool halo_chain(const DevChain& c, int* lo, int* hi, int* shift) {
-  const DevStage& q = c.st[0];
-  *lo = q.lo;
-  *hi = q.hi;
-  *shift = q.s1 + q.s2;
-  return c.count == 1 && q.mul == 1 && q.add == 0 && !(q.s1 && q.s2) && q.lo <= q.hi && q.lo >> *shift >= -128 && q.hi >> *shift <= 127;
-}
+static bool halo_chain(const DevChain& c, int* lo, int* hi, int* shift) { return clamp_shift_of(c, lo, hi, shift) && clamp_shift_narrow(*lo, *hi, *shift); }
 
 // Is it such a layer?  (g and ep as conv_prepare leaves them)
 static bool halo_layer(const ConvGeom& g, const Epilogue& ep) {

@@ -28,6 +28,7 @@
 #include <string.h>
 
 #include "conv_mfma.h"
+#include "requant.h"
 
 namespace cvmhip {
 
@@ -40,7 +41,7 @@ constexpr int RES_LDS_MOST = 150 * 1024;
 
 enum { RES_IMAGE = 0, RES_ACT = 1, RES_CONV = 2, RES_SUM = 3, RES_POOL = 4 };
 // flags: a chain that is not one clamp and shift; channels past OC exist; the result goes to memory; its map has a border;
-// none of these, and the pixels of every item exist: the places are in LDS (res_plain)
+// none of these, and the pixels of every item exist: the places are in LDS (res_plain_conv)
 enum { RES_CHAIN = 1, RES_CHAIN2 = 2, RES_MASK = 4, RES_OUT = 8, RES_BORDER = 16, RES_PLAIN = 32 };
 
 // What the common path of a layer needs, in scalar registers from the layer's first instruction on: read field by field
@@ -105,13 +106,6 @@ __device__ __forceinline__ int32_t res_wave_sum(int32_t v) {
   return res_add_from<0x143, 0xc>(v);
 }
 
-// (lo <= hi)
-__device__ __forceinline__ int res_clamp(int v, int lo, int hi) {
-  int r;
-  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(lo), "v"(hi));
-  return r;
-}
-
 template <typename L>
 __device__ __forceinline__ void res_chain(const L& c, int32_t (&v)[4]) {
   const int count = c.count;
@@ -119,22 +113,8 @@ __device__ __forceinline__ void res_chain(const L& c, int32_t (&v)[4]) {
   for (int t = 0; t < count; ++t) {
     const int lo = c.st[t].lo, hi = c.st[t].hi, s1 = c.st[t].s1, add = c.st[t].add, s2 = c.st[t].s2, mul = c.st[t].mul;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = wadd(wmul(res_clamp(v[e], lo, hi), mul) >> s1, add) >> s2;
+    for (int e = 0; e < 4; ++e) v[e] = wadd(wmul(clamp_uniform(v[e], lo, hi), mul) >> s1, add) >> s2;
   }
-}
-
-__device__ __forceinline__ uint32_t res_pack(const int32_t (&v)[4]) {
-  const uint32_t lo2 = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x0c0c0400u);
-  const uint32_t hi2 = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x0c0c0400u);
-  return __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
-}
-
-// four values that are inside int8 once shifted -> one dword: three instructions where a shift each and res_pack are seven
-__device__ __forceinline__ uint32_t res_shift_pack(const int32_t (&v)[4], int shift) {
-  uint32_t lo2, hi2;   // (the builtin's 16 bits would be masked once more)
-  asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(lo2) : "v"(v[0]), "v"(v[1]), "s"(shift));
-  asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(hi2) : "v"(v[2]), "v"(v[3]), "s"(shift));
-  return __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
 }
 
 // where the pixels of a layer lie, for the forms that are not RES_PLAIN
@@ -150,7 +130,7 @@ __device__ __forceinline__ ResGeometry res_geometry(ResTable L) {
 // four channels of pixel p of this image, to LDS byte `at` and wherever else the layer wants them
 __device__ __forceinline__ void res_store(const ResHead& h, const ResGeometry& q, ResTable L, char* lds, int32_t* out_host, int img, int p, int at, int oc,
                                           const int32_t (&v)[4]) {
-  uint32_t d = res_pack(v);
+  uint32_t d = low_bytes(v[0], v[1], v[2], v[3]);
   if (h.flags & RES_MASK) {
     const int left = L->OC - oc;
     d = left >= 4 ? d : left <= 0 ? 0u : d & ((1u << (8 * left)) - 1u);
@@ -245,11 +225,9 @@ __device__ __forceinline__ void res_products(const ResHead& h, const char* lds, 
     }
     res_chunk<TP>(lds, w + c * (RES_CHUNK * 1024), now, base, acc);
   }
-  // A vector instruction may read an eight-pass product's registers 11 wait states behind it.  The compiler sees to that for
-  // instructions it knows, but res_clamp is inline assembly to it: the wait is part of the values' way there.
-  if constexpr (TP == 1) asm volatile("s_nop 15" : "+v"(acc[0]));
-  else if constexpr (TP == 2) asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]));
-  else asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+  if constexpr (TP == 1) asm volatile(WAIT_8_PASSES : "+v"(acc[0]));
+  else if constexpr (TP == 2) asm volatile(WAIT_8_PASSES : "+v"(acc[0]), "+v"(acc[1]));
+  else asm volatile(WAIT_8_PASSES : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
 }
 __device__ __forceinline__ void res_first_taps(const ResHead& h, const char* lds, int lane, int (&tap)[RES_CHUNK]) {
 #pragma unroll
@@ -290,18 +268,18 @@ __device__ __forceinline__ void res_plain_conv(const ResHead& h, char* lds, int 
       for (int j = 0; j < TP; ++j) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          acc[j][e] = res_clamp(wadd(res_clamp(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2);
+          acc[j][e] = clamp_uniform(wadd(clamp_uniform(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2);
       }
     } else {
 #pragma unroll
       for (int j = 0; j < TP; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[j][e] = res_clamp(acc[j][e], h.lo, h.hi);
+        for (int e = 0; e < 4; ++e) acc[j][e] = clamp_uniform(acc[j][e], h.lo, h.hi);
     }
 #pragma unroll
     for (int j = 0; j < TP; ++j) {
       const int32_t v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
-      *reinterpret_cast<uint32_t*>(lds + (own.dst + dst[j])) = res_shift_pack(v, last);
+      *reinterpret_cast<uint32_t*>(lds + (own.dst + dst[j])) = shift_to_bytes(v[0], v[1], v[2], v[3], last);
     }
     item += RES_WAVES;
     if (item >= h.items) return;
@@ -375,7 +353,7 @@ __device__ __forceinline__ void res_item_conv(const ResHead& h, char* lds, int w
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
-      for (int j = 0; j < TP; ++j) asm volatile("s_nop 15" : "+v"(acc[m][j]));   // as in res_products
+      for (int j = 0; j < TP; ++j) asm volatile(WAIT_8_PASSES : "+v"(acc[m][j]));
     if (h.residual) {
 #pragma unroll
       for (int m = 0; m < TM; ++m)
@@ -383,21 +361,21 @@ __device__ __forceinline__ void res_item_conv(const ResHead& h, char* lds, int w
         for (int j = 0; j < TP; ++j)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            acc[m][j][e] = res_clamp(wadd(res_clamp(acc[m][j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[m][j] >> (8 * e))), h.lo2, h.hi2);
+            acc[m][j][e] = clamp_uniform(wadd(clamp_uniform(acc[m][j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[m][j] >> (8 * e))), h.lo2, h.hi2);
     } else {
 #pragma unroll
       for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int j = 0; j < TP; ++j)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[m][j][e] = res_clamp(acc[m][j][e], h.lo, h.hi);
+          for (int e = 0; e < 4; ++e) acc[m][j][e] = clamp_uniform(acc[m][j][e], h.lo, h.hi);
     }
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
       for (int j = 0; j < TP; ++j) {
         const int32_t v[4] = {acc[m][j][0], acc[m][j][1], acc[m][j][2], acc[m][j][3]};
-        *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j] + m * 16)) = res_shift_pack(v, last);
+        *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j] + m * 16)) = shift_to_bytes(v[0], v[1], v[2], v[3], last);
       }
     if (!more) return;
   }
@@ -475,23 +453,23 @@ __device__ __forceinline__ void res_pair_conv(const ResHead& h, char* lds, int w
       for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j >> 1][u], x[u][j & 1], acc[j], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
     if (more) request(next);
-    asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));   // as in res_products
+    asm volatile(WAIT_8_PASSES : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
     if (h.residual) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          acc[j][e] = res_clamp(wadd(res_clamp(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2);
+          acc[j][e] = clamp_uniform(wadd(clamp_uniform(acc[j][e], h.lo, h.hi) >> h.shift, (int32_t)(int8_t)(residual[j] >> (8 * e))), h.lo2, h.hi2);
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[j][e] = res_clamp(acc[j][e], h.lo, h.hi);
+        for (int e = 0; e < 4; ++e) acc[j][e] = clamp_uniform(acc[j][e], h.lo, h.hi);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int32_t v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
-      *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j])) = res_shift_pack(v, last);
+      *reinterpret_cast<uint32_t*>(lds + (own.dst + to[j])) = shift_to_bytes(v[0], v[1], v[2], v[3], last);
     }
     if (!more) return;
     beside(next);
@@ -530,7 +508,7 @@ __device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds
       res_chain(L->chain, v);
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = res_clamp(v[e], h.lo, h.hi) >> h.shift;
+      for (int e = 0; e < 4; ++e) v[e] = clamp_uniform(v[e], h.lo, h.hi) >> h.shift;
     }
     if (h.residual) {
       const uint32_t d = *reinterpret_cast<const uint32_t*>(lds + (q.res + oc));
@@ -540,7 +518,7 @@ __device__ __forceinline__ void res_conv(const ResHead& h, ResTable L, char* lds
         res_chain(L->chain2, v);
       } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = res_clamp(v[e], h.lo2, h.hi2) >> h.shift2;
+        for (int e = 0; e < 4; ++e) v[e] = clamp_uniform(v[e], h.lo2, h.hi2) >> h.shift2;
       }
     }
     res_store(h, g, L, lds, out_host, img, pixel, q.dst + oc, oc + (lane >> 4) * 4, v);
@@ -618,8 +596,8 @@ __global__ void __launch_bounds__(RES_THREADS + 64) k_conv_resident(const ResLay
             const int oy = (int)fastdiv((unsigned)(p + j), g.div_ow), at = g.dst + oy * g.dst_row + (p + j - oy * g.OW) * g.ocp;
             int32_t v[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] = c < C ? res_clamp((int32_t)(int8_t)(d[c] >> (8 * j)), -range, range) : 0;
-            *reinterpret_cast<uint4*>(lds + at) = make_uint4(res_pack(v), 0, 0, 0);
+            for (int c = 0; c < 4; ++c) v[c] = c < C ? clamp_uniform((int32_t)(int8_t)(d[c] >> (8 * j)), -range, range) : 0;
+            *reinterpret_cast<uint4*>(lds + at) = make_uint4(low_bytes(v[0], v[1], v[2], v[3]), 0, 0, 0);
             for (int c = 16; c < g.ocp; c += 16) *reinterpret_cast<uint4*>(lds + at + c) = make_uint4(0, 0, 0, 0);
           }
         }
@@ -631,8 +609,8 @@ __global__ void __launch_bounds__(RES_THREADS + 64) k_conv_resident(const ResLay
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = c0 < C ? res_load<int8_t>(x + (int64_t)(c0 + e < C ? c0 + e : C - 1) * g.P + p) : 0;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = c0 + e < C ? res_clamp(v[e], -range, range) : 0;
-            *reinterpret_cast<uint32_t*>(lds + at + c0) = res_pack(v);
+            for (int e = 0; e < 4; ++e) v[e] = c0 + e < C ? clamp_uniform(v[e], -range, range) : 0;
+            *reinterpret_cast<uint32_t*>(lds + at + c0) = low_bytes(v[0], v[1], v[2], v[3]);
           }
         }
       }
@@ -735,20 +713,6 @@ __global__ void __launch_bounds__(256) k_pack_resident(const int32_t* __restrict
 
 static int res_cp(int c) { return c <= 16 ? 16 : pad_channels(c); }
 static int res_chunks(int c, int kh, int kw) { return (kh * kw * res_cp(c) + RES_CHUNK * 64 - 1) / (RES_CHUNK * 64); }
-// one clamp and one shift?
-static bool res_plain(const DevChain& c, int* lo, int* hi, int* shift) {
-  *lo = INT32_MIN;
-  *hi = INT32_MAX;
-  *shift = 0;
-  if (c.count == 0) return true;
-  if (c.count > 1 || c.st[0].mul != 1 || c.st[0].add != 0 || (c.st[0].s1 != 0 && c.st[0].s2 != 0)) return false;
-  *lo = c.st[0].lo;
-  *hi = c.st[0].hi;
-  *shift = c.st[0].s1 + c.st[0].s2;
-  return true;
-}
-// are its results int8 whatever it is given?  (res_shift_pack saturates where the other forms take the low byte.)
-static bool res_narrow(int lo, int hi, int shift) { return lo >> shift >= -128 && hi >> shift <= 127; }
 
 }  // namespace cvmhip
 
@@ -849,8 +813,8 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d,
     return arg_error("resident_layer output");
   }
   if (!make_chain(&d->chain, &L.chain) || !make_chain(&d->chain2, &L.chain2)) return arg_error("resident_layer chain");
-  if (!res_plain(L.chain, &h.lo, &h.hi, &h.shift)) h.flags |= RES_CHAIN;
-  if (!res_plain(L.chain2, &h.lo2, &h.hi2, &h.shift2)) h.flags |= RES_CHAIN2;
+  if (!clamp_shift_of(L.chain, &h.lo, &h.hi, &h.shift)) h.flags |= RES_CHAIN;
+  if (!clamp_shift_of(L.chain2, &h.lo2, &h.hi2, &h.shift2)) h.flags |= RES_CHAIN2;
   L.range = d->range;
   if (load) {
     if (!d->in || out.at < 0 || d->out_mode != 0) return arg_error("resident_layer input");
@@ -890,7 +854,7 @@ int cvmhip_resident_layer(void* table, int index, const cvmhip_resident_desc* d,
       const int ptiles = (L.P + 15) / 16;
       const ResTiling tiling = res_tiling(ptiles, L.octiles, res_steps(in.c, d->kh, d->kw));
       const int tp = tiling.tp, groups = L.octiles / tiling.tm;
-      const bool narrow = h.residual ? res_narrow(h.lo2, h.hi2, h.shift2) : res_narrow(h.lo, h.hi, h.shift);
+      const bool narrow = h.residual ? clamp_shift_narrow(h.lo2, h.hi2, h.shift2) : clamp_shift_narrow(h.lo, h.hi, h.shift);
       if (narrow && !(h.flags & (RES_CHAIN | RES_CHAIN2 | RES_MASK | RES_OUT)) && L.P % (16 * tp) == 0 && (out.w % 16 == 0 || 16 % out.w == 0)) {
         h.flags |= RES_PLAIN;
         h.tp = tp;

@@ -19,6 +19,7 @@
 #include <string.h>
 
 #include "conv_mfma.h"
+#include "requant.h"
 
 namespace cvmhip {
 
@@ -26,7 +27,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v3i __attribute__((ext_vector_type(3)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
 
 // a chain, and its values if it is one clamp and shift
 struct SepChain {
@@ -54,11 +54,7 @@ constexpr size_t SEP_LDS_MOST = 64 * 1024;   // of the depthwise tile
 __device__ __forceinline__ void sep_chain(const SepChain& c, int32_t (&v)[16]) {
   if (c.plain) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      int r;
-      asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v[e]), "s"(c.lo), "v"(c.hi));
-      v[e] = r >> c.shift;
-    }
+    for (int e = 0; e < 16; ++e) v[e] = clamp_uniform(v[e], c.lo, c.hi) >> c.shift;
     return;
   }
 #pragma unroll
@@ -69,19 +65,11 @@ __device__ __forceinline__ void sep_chain(const SepChain& c, int32_t (&v)[16]) {
     for (int e = 0; e < 16; ++e) v[e] = apply_stage(s, v[e]);
   }
 }
-__device__ __forceinline__ uint32_t sep_pack(int32_t a, int32_t b, int32_t c, int32_t d) {
-  const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u), hi = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x0c0c0400u);
-  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-}
 // the 16 values of a lane are channels 8q + 4 (lane >> 5) .. + 3, q = 0 .. 3
 __device__ __forceinline__ void sep_bias(const int32_t* bias, int c0, int lgrp, v4i (&v)[4]) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) v[q] = bias ? *reinterpret_cast<const v4i*>(bias + c0 + q * 8 + lgrp * 4) : v4i{0, 0, 0, 0};
 }
-
-// A vector instruction may read a sixteen-pass product's registers 19 wait states behind it.  The compiler sees to that for
-// instructions it knows, but the clamp is inline assembly to it: the wait is part of the values' way there.
-__device__ __forceinline__ void sep_settle(v16i& acc) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc)); }
 
 template <int WO>
 __global__ void __launch_bounds__(512) k_conv_separable(const SepArgs a) {
@@ -141,7 +129,7 @@ __global__ void __launch_bounds__(512) k_conv_separable(const SepArgs a) {
         const v4i diag = {all & mask[0], all & mask[1], all & mask[2], all & mask[3]};
         acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(diag, x[t], acc, 0, 0, 0);
       }
-      sep_settle(acc);
+      asm volatile(WAIT_16_PASSES : "+v"(acc));
       int32_t v[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) v[e] = acc[e];
@@ -149,7 +137,7 @@ __global__ void __launch_bounds__(512) k_conv_separable(const SepArgs a) {
       int8_t* f = sep_lds + (kt * WP + pb) * 1024 + lrow * 16 + lgrp * 4;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<uint32_t*>(f + (q >> 1) * 512 + (q & 1) * 8) = sep_pack(v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]);
+        *reinterpret_cast<uint32_t*>(f + (q >> 1) * 512 + (q & 1) * 8) = low_bytes(v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]);
     }
   }
   __syncthreads();
@@ -181,11 +169,10 @@ __global__ void __launch_bounds__(512) k_conv_separable(const SepArgs a) {
   sep_chain(a.second, v);
   uint32_t d[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) d[q] = sep_pack(v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]);
-  const v2u s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+  for (int q = 0; q < 4; ++q) d[q] = low_bytes(v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]);
+  const v4i w = sixteen_channels(d);
   const int p = px0 + wp * 32 + lrow;
-  if (p < a.P)
-    *reinterpret_cast<v4i*>(a.out + ((int64_t)(p >> 5) * a.octiles + ot) * 1024 + lane * 16) = v4i{(int)s0.x, (int)s0.y, (int)s1.x, (int)s1.y};
+  if (p < a.P) *reinterpret_cast<v4i*>(a.out + ((int64_t)(p >> 5) * a.octiles + ot) * 1024 + lane * 16) = w;
 }
 
 __global__ void __launch_bounds__(256) k_pack_separable(const int32_t* __restrict__ w, uint32_t* __restrict__ wd, int channels) {
@@ -197,10 +184,8 @@ __global__ void __launch_bounds__(256) k_pack_separable(const int32_t* __restric
 }
 
 static SepChain sep_chain_of(const DevChain& c) {
-  SepChain s = {c, 0, INT32_MIN, INT32_MAX, 0};
-  if (c.count == 0) s.plain = 1;
-  if (c.count == 1 && c.st[0].mul == 1 && c.st[0].add == 0 && (c.st[0].s1 == 0 || c.st[0].s2 == 0) && c.st[0].lo <= c.st[0].hi)
-    s = {c, 1, c.st[0].lo, c.st[0].hi, c.st[0].s1 + c.st[0].s2};
+  SepChain s = {c, 0, 0, 0, 0};
+  s.plain = clamp_shift_of(c, &s.lo, &s.hi, &s.shift);
   return s;
 }
 

@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "conv_mfma.h"
+#include "requant.h"
 
 namespace cvmhip {
 
@@ -36,13 +37,6 @@ struct HeadGeom {
   int plain, lo, hi, shift;      // the chain is one clamp and one shift to int8
   DevChain chain;
 };
-
-// (lo <= hi)
-__device__ __forceinline__ int head_clamp(int v, int lo, int hi) {
-  int r;
-  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(lo), "v"(hi));
-  return r;
-}
 
 __global__ void __launch_bounds__(256, 2) k_conv_stem_pool(const HeadGeom a) {
   __shared__ __attribute__((aligned(16))) int8_t s_tile[4 * HEAD_PIXELS * 16];   // [16 channels][convolution pixel of the patch]
@@ -134,9 +128,7 @@ __global__ void __launch_bounds__(256, 2) k_conv_stem_pool(const HeadGeom a) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[i][r], b, acc[i], 0, 0, 0);
       }
-      // A vector instruction may read a product's registers 19 wait states behind it.  The compiler sees to that for instructions it knows; head_clamp
-      // is inline assembly to it.
-      asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1]));
+      asm volatile(WAIT_16_PASSES : "+v"(acc[0]), "+v"(acc[1]));
       const int cy = now_y + ry[j], cx = now_x + rx[j];
       const bool inside = cy >= 0 && cy < a.OH && cx >= 0 && cx < a.OW;
       const int u = (wave * 4 + j) * 32 + lrow;
@@ -148,11 +140,8 @@ __global__ void __launch_bounds__(256, 2) k_conv_stem_pool(const HeadGeom a) {
           for (int q = 0; q < 4; ++q) {
             int v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = head_clamp(acc[i][q * 4 + e], a.lo, a.hi);
-            // (results are int8 whatever they come from: the saturation never acts)
-            const uint32_t lo2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[0], (uint32_t)v[1], (uint32_t)a.shift);
-            const uint32_t hi2 = __builtin_amdgcn_ashr_pk_i8_i32((uint32_t)v[2], (uint32_t)v[3], (uint32_t)a.shift);
-            d[q] = __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
+            for (int e = 0; e < 4; ++e) v[e] = clamp_uniform(acc[i][q * 4 + e], a.lo, a.hi);
+            d[q] = shift_to_bytes(v[0], v[1], v[2], v[3], a.shift);   // (results are int8 whatever they come from: the saturation never acts)
           }
         } else {
 #pragma unroll
@@ -160,16 +149,11 @@ __global__ void __launch_bounds__(256, 2) k_conv_stem_pool(const HeadGeom a) {
             int v[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = apply_chain(a.chain, acc[i][q * 4 + e]);
-            const uint32_t lo2 = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x0c0c0400u);
-            const uint32_t hi2 = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x0c0c0400u);
-            d[q] = __builtin_amdgcn_perm(hi2, lo2, 0x05040100u);
+            d[q] = low_bytes(v[0], v[1], v[2], v[3]);
           }
         }
-        // lower half of the wavefront: channels 0 .. 15 of the 32, upper: 16 .. 31
-        typedef unsigned v2u __attribute__((ext_vector_type(2)));
-        const v2u s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
         const int none = (int)0x80808080u;   // outside the convolution's output: less than any value (a window holds at least one)
-        const v4i w = inside ? v4i{(int)s0.x, (int)s0.y, (int)s1.x, (int)s1.y} : v4i{none, none, none, none};
+        const v4i channels = sixteen_channels(d), w = inside ? channels : v4i{none, none, none, none};
         *reinterpret_cast<v4i*>(s_tile + (i * 2 + lgrp) * HEAD_PIXELS * 16 + u * 16) = w;
       }
     }
@@ -225,11 +209,7 @@ int conv_stem_pool(const int8_t* xs, const int8_t* wp, const int32_t* bias, cons
   a.div_x = make_fastdiv((uint32_t)a.across);
   a.div_y = make_fastdiv((uint32_t)a.down);
   a.chain = chain;
-  const DevStage& q = chain.st[0];
-  a.plain = chain.count == 1 && q.mul == 1 && q.add == 0 && !(q.s1 && q.s2) && q.lo <= q.hi && q.lo >> (q.s1 + q.s2) >= -128 && q.hi >> (q.s1 + q.s2) <= 127;
-  a.lo = q.lo;
-  a.hi = q.hi;
-  a.shift = q.s1 + q.s2;
+  a.plain = clamp_shift_of(chain, &a.lo, &a.hi, &a.shift) && clamp_shift_narrow(a.lo, a.hi, a.shift);
   k_conv_stem_pool<<<(unsigned)std::min(a.patches, 768), 256, 0, s>>>(a);
   return check_launch("conv2d_stem_pool3_i8");
 }
