@@ -26,8 +26,8 @@ PEAK_I8_TOPS = 5000.0   # MI355X dense int8 MFMA peak, TOP/s
 # The third field is the first 16 hex digits of the SHA-256 of the kernels' source file as it was when the counters were
 # read: a figure is only reported while that file is unchanged, otherwise `traffic` is null (measured figures go stale).
 TRAFFIC_BYTES_PER_LAUNCH = {
-    ("resnet50", "k_conv_seq", 16): (531.0e6, "profiles/k_conv_seq_resnet50_b16_traffic.txt", "36f3cb30d3ec1daa"),
-    ("vgg16", "k_conv_big", 16): (27.1e6, "profiles/k_conv_big_vgg16_b16_traffic.txt", "36f3cb30d3ec1daa"),
+    ("resnet50", "k_conv_seq", 16): (531.0e6, "profiles/k_conv_seq_resnet50_b16_traffic.txt", "38f4298682774f68"),
+    ("vgg16", "k_conv_big", 16): (27.2e6, "profiles/k_conv_big_vgg16_b16_traffic.txt", "38f4298682774f68"),
 }
 KERNEL_SOURCE = os.path.join(ROOT, "cvm-runtime_amd", "csrc", "conv_mfma.hip")
 

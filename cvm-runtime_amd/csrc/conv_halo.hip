@@ -9,14 +9,15 @@
 // In LDS the 16 bytes that a lane feeds to a product are a granule, granules of the same channels lie pixel by pixel: the 32 pixels
 // of a block are 512 contiguous bytes.  With the pool a block is one corner of 32 windows, and the columns are sorted into
 // even and odd ones for that.
-// Measured (us; in front of it k_conv_wave): 64 -> 64 at 16 x 224 x 224 with the pool 46 -> 30, without 51 -> 33; 64 -> 128 at 16 x 112 x 112 29 -> 22; 64 -> 64
-// at 50 x 56 x 56 16.6 -> 13.  Bound by the requests: a patch takes a workgroup 700 clocks of waiting, 5 400 of products (4 608 at the rate of the
-// matrix pipe), 3 400 to 3 900 in which its wavefronts are held until their requests are taken, and 1 400 (pool) to 3 500 of
-// requantisation and stores.  No difference: operands requested a step ahead or left to the compiler; slower: a workgroup a patch, each with a
-// filter of its own (36 instead of 30); half of the next patch's requests in the middle of the products (32).
+// Measured (us between event pairs): against k_conv_wave 64 -> 64 at 16 x 224 x 224 with the pool 46 -> 30, without 51 -> 33, at 50 x 56 x 56 16.6 -> 13; against
+// k_conv_big 64 -> 128 at 16 x 112 x 112 29 -> 22 (more channels: conv_halo_blocks).
+// Bound by the requests: a patch takes a workgroup 700 clocks of waiting, 5 400 of products (4 608 at the rate of the matrix pipe), 3 400 to 3 900 in
+// which its wavefronts are held until their requests are taken, and 1 400 (pool) to 3 500 of requantisation and stores.  No difference: operands requested
+// a step ahead or left to the compiler; slower: a workgroup a patch, each with a filter of its own (36 instead of 30); half of the next patch's requests in
+// the middle of the products (32).
 // The two layers at the head of a VGG are one launch (STEM): the pixels under a patch, a fifth more than are asked for, are computed from the image by the
 // first layer's products where they would be fetched, and the largest tensor of the network is neither written nor read:
-// 16 x 224 x 224 with the pool 21 + 30 -> 40 us.
+// 16 x 224 x 224 with the pool 21 + 28 -> 36 us (trace; other sizes: halo_stem_width).
 #include <algorithm>
 
 #include "conv_mfma.h"
