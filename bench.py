@@ -45,7 +45,7 @@ def dominant_conv(kt, wall_s, steps):
     average launch duration with the cost of an event pair taken off, and the figures derived from it."""
     n_timed = sum(v["launches"] for v in kt.values())
     pair_cost_us = max(0.0, (sum(v["ms"] for v in kt.values()) * 1e3 - wall_s * 1e6) / max(n_timed, 1))
-    convs = {k: v for k, v in kt.items() if k in ("k_conv_wave", "k_conv_igemm", "k_conv_seq", "k_conv_big", "k_conv_group", "k_conv_halo",
+    convs = {k: v for k, v in kt.items() if k in ("k_conv_wave", "k_conv_igemm", "k_conv_seq", "k_conv_big", "k_conv_block", "k_conv_group", "k_conv_halo",
                                               "k_conv_direct", "k_conv_slab", "k_stem_pool", "k_conv_stem_pool", "k_conv_resident")}
     dom = max(convs, key=lambda k: convs[k]["ms"]) if convs else "k_conv_wave"
     conv = convs.get(dom, {"launches": 0, "ms": 0.0, "work": 0.0})

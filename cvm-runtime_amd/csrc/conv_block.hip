@@ -1,0 +1,426 @@
+// The tail of a ResNet bottleneck and the head of the next one, one launch for three layers:
+//   A  3 x 3, padding 1, stride 1 or 2, M -> M channels
+//   B  1 x 1, M -> 4 M, the residual added
+//   C  1 x 1, 4 M -> M or 2 M (the first layer of the next block)
+// with M = 64, 128 or 256; B's result is stored (the next block's residual), A's never leaves the compute unit and C reads B's where it was made.
+//
+// As launches of their own the three are bound by what surrounds their products: a launch, the first operands' way, a partial last round and a
+// tensor of 4 M channels written and fetched again.  Here a workgroup of eight wavefronts computes all channels of all three layers for a tile of
+// 16 * NT consecutive output pixels.  The pixels under the 3 x 3 windows, a run of the input's pixels, are fetched into LDS once, and the residual
+// to where B's result will lie; A's and B's results stay in LDS, pixel by pixel, as the operand of the layer behind.  The filters are not shared inside a
+// workgroup (each wavefront has channels of its own), so they go from memory to registers: a wavefront's fragments of all three layers are one stream,
+// requested RING fragments ahead across the layers.
+// v_mfma_i32_16x16x64_i8 with the filter as first operand: a lane's four results are four consecutive channels of one pixel, a dword of the operand.
+#include <algorithm>
+
+#include "conv_mfma.h"
+#include "requant.h"
+
+namespace cvmhip {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+__device__ const int g_block_zero[4] = {0, 0, 0, 0};
+
+struct BlockRequant { int lo, hi, shift; };
+struct BlockArgs {
+  const int8_t *x, *wa, *wb, *wc, *res;
+  const int32_t *ba, *bb, *bc;
+  int8_t *out, *next;
+  int H, W, S, P, in_pixels;          // input extent, stride of A, output pixels and input pixels of all images
+  int patch, tiles;                   // pixels of a tile's run of the input, tiles
+  FastDiv div_ohw, div_ow, div_patch;
+  int OHW, OW;
+  BlockRequant qa, qb, qr, qc;        // qb in front of the residual, qr behind it
+};
+
+// Where things lie in LDS: sixteen zeros for windows that leave the image, biases, A's result, B's result, the run of the input.  Granules of 16 channels
+// lie pixel by pixel, channel group after channel group: a quarter of a wavefront requests, reads and writes 16 neighbouring pixels, and these are
+// neighbours in memory too.
+template <int M, int NT, int UC>
+struct BlockLds {
+  static constexpr int P = 16 * NT, GROUP = P * 16;   // bytes of a channel group of A's and B's results
+  static constexpr int bias_requests = ((5 + UC) * M * 4 + 1023) / 1024;
+  static constexpr int zero = 0, bias = 64, mid = bias + bias_requests * 1024, wide = mid + M / 16 * GROUP, patch = wide + M / 4 * GROUP;
+  static size_t bytes(int patch_pixels) { return (size_t)patch + (size_t)((patch_pixels * (M / 16) + 63) / 64) * 1024; }
+};
+
+__device__ __forceinline__ void block_request(const void* from, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_at) : "memory");
+}
+// all but the last N requests of this wavefront have landed (they do so in order)
+template <int N>
+__device__ __forceinline__ void block_landed() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory"); }
+// LDS written before is read behind it; requests of memory stay in flight
+__device__ __forceinline__ void block_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// (the wait is part of the values' way, see WAIT_8_PASSES)
+template <int N, int I = 0>
+__device__ __forceinline__ void block_settle(v4i (&acc)[N]) {
+  if constexpr (N - I >= 8) {
+    asm volatile(WAIT_8_PASSES : "+v"(acc[I]), "+v"(acc[I + 1]), "+v"(acc[I + 2]), "+v"(acc[I + 3]), "+v"(acc[I + 4]), "+v"(acc[I + 5]), "+v"(acc[I + 6]), "+v"(acc[I + 7]));
+    block_settle<N, I + 8>(acc);
+  } else if constexpr (N - I >= 4) {
+    asm volatile(WAIT_8_PASSES : "+v"(acc[I]), "+v"(acc[I + 1]), "+v"(acc[I + 2]), "+v"(acc[I + 3]));
+    block_settle<N, I + 4>(acc);
+  } else if constexpr (N - I >= 2) {
+    asm volatile(WAIT_8_PASSES : "+v"(acc[I]), "+v"(acc[I + 1]));
+    block_settle<N, I + 2>(acc);
+  } else if constexpr (N - I == 1) {
+    asm volatile(WAIT_8_PASSES : "+v"(acc[I]));
+  }
+}
+
+template <int M, int NT, int UC, int RING, int OCC>
+__global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) {
+  typedef BlockLds<M, NT, UC> L;
+  constexpr int CTA = M == 256 ? 2 : 1, PGA = M == 64 ? 2 : 1, NTA = NT / PGA;   // A and C: 16-channel tiles of a wavefront at a time, groups of pixels
+  constexpr int KA = M / 64, UB = M / 64, KC = M / 16;                           // 64-byte steps of K: of a tap, of B (units of 32 channels likewise), of C
+  constexpr int FA = 9 * KA * CTA, FB = UB * KA * 2, FC = UC * KC * CTA, F = FA + FB + FC;
+  constexpr int TILE_A = (9 * M / 32 + 1) * 1024, TILE_B = (M / 32 + 1) * 1024, TILE_C = (M / 8 + 1) * 1024;   // from 32 filter rows to the next
+  static_assert(NT % PGA == 0, "pixels are split between wavefronts by 16");
+  extern __shared__ __attribute__((aligned(16))) int8_t block_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)block_lds;
+
+  // an eighth of the tiles to each XCD, where neighbours share the pixels between them
+  int tile;
+  {
+    const int xcd = blockIdx.x & 7, per = a.tiles >> 3, extra = a.tiles & 7;
+    tile = xcd * per + (xcd < extra ? xcd : extra) + ((int)blockIdx.x >> 3);
+  }
+  const int p0 = tile * L::P;
+  auto corner = [&](int p, int& row, int& column, int& n) __attribute__((always_inline)) {   // of a pixel's window, in the input
+    n = (int)fastdiv((unsigned)p, a.div_ohw);
+    const int rem = p - n * a.OHW, oh = (int)fastdiv((unsigned)rem, a.div_ow);
+    row = oh * a.S - 1;
+    column = (rem - oh * a.OW) * a.S - 1;
+  };
+  int first;   // pixel of the input at the start of the run
+  {
+    int r, c, n;
+    corner(p0, r, c, n);
+    first = (n * a.H + r) * a.W + c;
+  }
+
+  // ---- biases, then the run of the input
+  if (wave < L::bias_requests) {
+    const int i = (wave * 64 + lane) * 4;
+    const int32_t* b = i < M ? a.ba : i < 5 * M ? a.bb : a.bc;
+    const int at = i < M ? i : i < 5 * M ? i - M : i - 5 * M;
+    block_request(b && i < (5 + UC) * M ? b + at : g_block_zero, lds + L::bias + (uint32_t)wave * 1024u);
+  }
+  const int run_requests = (a.patch * (M / 16) + 63) >> 6;
+  for (int k = wave; k < run_requests; k += 8) {
+    const int t = k * 64 + lane;
+    int g = (int)fastdiv((unsigned)t, a.div_patch), p = first + t - g * a.patch;
+    p = p < 0 ? 0 : p > a.in_pixels - 1 ? a.in_pixels - 1 : p;   // (what such pixels hold is not used)
+    g = g < M / 16 ? g : M / 16 - 1;
+    block_request(a.x + ((int64_t)(p >> 5) * (M / 32) + (g >> 1)) * 1024 + (g & 1) * 512 + (p & 31) * 16, lds + L::patch + (uint32_t)k * 1024u);
+  }
+
+  // ---- the stream of filter fragments of this wavefront: 16 channels x 64 bytes of K each
+  const int ca = M == 64 ? (wave & 3) : wave * CTA, pg = M == 64 ? wave >> 2 : 0;   // first channel tile (16) in A and C, group of pixels
+  const int8_t* fa = a.wa + (ca >> 1) * TILE_A + (ca & 1) * 256;
+  const int8_t* fb = a.wb + wave * UB * TILE_B;
+  const int8_t* fc = a.wc + (ca >> 1) * TILE_C + (ca & 1) * 256;
+  const unsigned flane = (unsigned)((kg >> 1) * 1024 + (kg & 1) * 512 + col * 16);
+  v4i ring[RING];
+  auto fragment = [&](const int f) __attribute__((always_inline)) {
+    if (f >= F) return;
+    const int8_t* p;
+    if (f < FA) p = fa + (f / CTA) * 2048 + (f % CTA) * 256;
+    else if (f < FA + FB) p = fb + ((f - FA) / (KA * 2)) * TILE_B + (f - FA) % KA * 2048 + ((f - FA) / KA & 1) * 256;
+    else p = fc + (f - FA - FB) / (KC * CTA) * (M / 32) * TILE_C + (f - FA - FB) / CTA % KC * 2048 + (f - FA - FB) % CTA * 256;
+    ring[f % RING] = *reinterpret_cast<const v4i*>(p + flane);
+  };
+#pragma unroll
+  for (int f = 0; f < RING; ++f) fragment(f);
+
+  // ---- the residual: behind the first fragments, which need not wait for it
+  constexpr int RES = NT * M / 128;
+#pragma unroll
+  for (int k = 0; k < RES; ++k) {
+    const int part = (k * 8 + wave) * 4 + kg, g = part / NT;
+    int p = p0 + (part - g * NT) * 16 + col;
+    p = p > a.P - 1 ? a.P - 1 : p;
+    block_request(a.res + ((int64_t)(p >> 5) * (M / 8) + (g >> 1)) * 1024 + (g & 1) * 512 + (p & 31) * 16, lds + L::wide + (uint32_t)(k * 8 + wave) * 1024u);
+  }
+  if (tid < 4) *reinterpret_cast<v4i*>(block_lds + L::zero + tid * 16) = v4i{0, 0, 0, 0};
+
+  // ---- windows of this lane's pixels: the byte of the first tap, and which of three rows and columns are inside
+  int base[NTA], inside[NTA];
+#pragma unroll
+  for (int j = 0; j < NTA; ++j) {
+    int p = p0 + (pg * NTA + j) * 16 + col, r, c, n;
+    p = p > a.P - 1 ? a.P - 1 : p;
+    corner(p, r, c, n);
+    base[j] = L::patch + ((n * a.H + r) * a.W + c - first + kg * a.patch) * 16;
+    inside[j] = 0;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+      inside[j] |= ((unsigned)(r + t / 3) < (unsigned)a.H && (unsigned)(c + t % 3) < (unsigned)a.W ? 1 : 0) << t;
+  }
+  block_landed<(RING < F ? RING : F) + RES>();   // biases and run
+  block_barrier();
+
+  // ---- A
+  {
+    v4i acc[CTA * NTA], b[2][NTA];
+    auto operand = [&](const int step) __attribute__((always_inline)) {
+      const int t = step / KA, k = step % KA, shift = ((t / 3) * a.W + t % 3 + k * 4 * a.patch) * 16;
+#pragma unroll
+      for (int j = 0; j < NTA; ++j) b[step & 1][j] = *reinterpret_cast<const v4i*>(block_lds + (inside[j] >> t & 1 ? base[j] + shift : L::zero));
+    };
+    operand(0);
+#pragma unroll
+    for (int i = 0; i < CTA; ++i)
+#pragma unroll
+      for (int j = 0; j < NTA; ++j) acc[i * NTA + j] = *reinterpret_cast<const v4i*>(block_lds + L::bias + ((ca + i) * 16 + kg * 4) * 4);
+#pragma unroll
+    for (int step = 0; step < 9 * KA; ++step) {
+      if (step + 1 < 9 * KA) operand(step + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < CTA; ++i) {
+#pragma unroll
+        for (int j = 0; j < NTA; ++j)
+          acc[i * NTA + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[(step * CTA + i) % RING], b[step & 1][j], acc[i * NTA + j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < CTA; ++i) fragment(step * CTA + i + RING);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    block_settle(acc);
+#pragma unroll
+    for (int i = 0; i < CTA; ++i)
+#pragma unroll
+      for (int j = 0; j < NTA; ++j) {
+        int v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = clamp_uniform(acc[i * NTA + j][e], a.qa.lo, a.qa.hi);
+        *reinterpret_cast<uint32_t*>(block_lds + L::mid + (ca + i) * L::GROUP + ((pg * NTA + j) * 16 + col) * 16 + kg * 4) = shift_to_bytes(v[0], v[1], v[2], v[3], a.qa.shift);
+      }
+  }
+  block_landed<(FA < F - RING ? FA : F > RING ? F - RING : 0)>();   // the residual: all but the fragments requested since
+  block_barrier();
+
+  // ---- B: 16 channels after the other, all pixels; the result takes the residual's place.  The products of the next 16 run beside the requantisation.
+  {
+    v4i b[KA][NT], acc[2][NT];
+#pragma unroll
+    for (int k = 0; k < KA; ++k)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[k][j] = *reinterpret_cast<const v4i*>(block_lds + L::mid + (k * 4 + kg) * L::GROUP + (j * 16 + col) * 16);
+    int8_t* wide = block_lds + L::wide + wave * UB * 2 * L::GROUP + col * 16 + kg * 4;
+    auto products = [&](const int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[u & 1][j] = *reinterpret_cast<const v4i*>(block_lds + L::bias + (M + (wave * UB * 2 + u) * 16 + kg * 4) * 4);
+#pragma unroll
+      for (int k = 0; k < KA; ++k) {
+        const int f = FA + u * KA + k;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[u & 1][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[f % RING], b[k][j], acc[u & 1][j], 0, 0, 0);
+        fragment(f + RING);
+      }
+    };
+    products(0);
+#pragma unroll
+    for (int u = 0; u < 2 * UB; ++u) {
+      uint32_t res[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) res[j] = *reinterpret_cast<const uint32_t*>(wide + u * L::GROUP + j * 256);
+      if (u + 1 < 2 * UB) products(u + 1);
+      block_settle(acc[u & 1]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        int v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = clamp_uniform(acc[u & 1][j][e], a.qb.lo, a.qb.hi) >> a.qb.shift;
+          v[e] = clamp_uniform(wadd(v[e], (int32_t)(int8_t)(res[j] >> (8 * e))), a.qr.lo, a.qr.hi);
+        }
+        *reinterpret_cast<uint32_t*>(wide + u * L::GROUP + j * 256) = shift_to_bytes(v[0], v[1], v[2], v[3], a.qr.shift);
+      }
+    }
+  }
+  block_barrier();
+
+  // ---- C
+#pragma unroll
+  for (int u = 0; u < UC; ++u) {
+    v4i acc[CTA * NTA], b[2][NTA];
+    const int ct = ca + u * (M / 16);
+    const int8_t* at = block_lds + L::wide + kg * L::GROUP + (pg * NTA * 16 + col) * 16;
+#pragma unroll
+    for (int j = 0; j < NTA; ++j) b[0][j] = *reinterpret_cast<const v4i*>(at + j * 256);
+#pragma unroll
+    for (int i = 0; i < CTA; ++i)
+#pragma unroll
+      for (int j = 0; j < NTA; ++j) acc[i * NTA + j] = *reinterpret_cast<const v4i*>(block_lds + L::bias + (5 * M + (ct + i) * 16 + kg * 4) * 4);
+#pragma unroll
+    for (int k = 0; k < KC; ++k) {
+#pragma unroll
+      for (int j = 0; j < NTA; ++j)
+        if (k + 1 < KC) b[(k + 1) & 1][j] = *reinterpret_cast<const v4i*>(at + (k + 1) * 4 * L::GROUP + j * 256);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < CTA; ++i) {
+        const int f = FA + FB + (u * KC + k) * CTA + i;
+#pragma unroll
+        for (int j = 0; j < NTA; ++j) acc[i * NTA + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[f % RING], b[k & 1][j], acc[i * NTA + j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < CTA; ++i) fragment(FA + FB + (u * KC + k) * CTA + i + RING);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    block_settle(acc);
+#pragma unroll
+    for (int i = 0; i < CTA; ++i)
+#pragma unroll
+      for (int j = 0; j < NTA; ++j) {
+        int v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = clamp_uniform(acc[i * NTA + j][e], a.qc.lo, a.qc.hi);
+        const uint32_t d = shift_to_bytes(v[0], v[1], v[2], v[3], a.qc.shift);
+        const int p = p0 + (pg * NTA + j) * 16 + col, c = (ct + i) * 16;
+        if (p < a.P)
+          *reinterpret_cast<uint32_t*>(a.next + ((int64_t)(p >> 5) * (UC * M / 32) + (c >> 5)) * 1024 + ((c >> 4) & 1) * 512 + (p & 31) * 16 + kg * 4) = d;
+      }
+  }
+
+  // ---- B's result to memory, 16 bytes of 16 neighbouring pixels a quarter of a wavefront
+#pragma unroll
+  for (int k = 0; k < NT * M / 128; ++k) {
+    const int part = (k * 8 + wave) * 4 + kg, g = part / NT, p = p0 + (part - g * NT) * 16 + col;
+    const v4i v = *reinterpret_cast<const v4i*>(block_lds + L::wide + (k * 8 + wave) * 1024 + lane * 16);
+    if (p < a.P) *reinterpret_cast<v4i*>(a.out + ((int64_t)(p >> 5) * (M / 8) + (g >> 1)) * 1024 + (g & 1) * 512 + (p & 31) * 16) = v;
+  }
+}
+
+static bool block_requant(const DevChain& c, bool bytes, BlockRequant* q) {
+  return clamp_shift_of(c, &q->lo, &q->hi, &q->shift) && (!bytes || clamp_shift_narrow(q->lo, q->hi, q->shift));
+}
+
+// pixels of the longest run of the input under `pixels` consecutive output pixels (the last tile's ends with the last pixel)
+static int block_run(int n, int h, int w, int oh, int ow, int stride, int pixels) {
+  const int64_t all = (int64_t)n * oh * ow;
+  auto corner = [&](int64_t p) {
+    const int64_t im = p / (oh * ow), rem = p - im * (oh * ow), r = rem / ow;
+    return (im * h + r * stride - 1) * w + (rem - r * ow) * stride - 1;
+  };
+  if (stride == 1) return pixels + 2 * w + 2;
+  int64_t most = 0;
+  for (int64_t p = 0; p < all; p += pixels) {
+    const int64_t last = std::min(p + pixels, all) - 1;
+    most = std::max(most, corner(last) + 2 * w + 2 - corner(p) + 1);
+  }
+  return (int)most;
+}
+
+}  // namespace cvmhip
+
+using namespace cvmhip;
+
+namespace {
+
+constexpr size_t BLOCK_LDS_MOST = 160 * 1024;
+
+struct BlockForm { int nt; void (*kernel)(const BlockArgs); size_t (*lds)(int); };
+template <int M, int NT, int UC, int RING, int OCC>
+BlockForm block_form() { return {NT, k_conv_block<M, NT, UC, RING, OCC>, [](int p) { return BlockLds<M, NT, UC>::bytes(p); }}; }
+
+// The smallest tile of which the chip holds all at once with one to a compute unit; where there are more, the last.  Microseconds a launch, filters of twelve
+// layers in turn (tiles of 16, 32, 48 ... pixels):
+//   M =  64, 56 x 56:  1 image 4.3 5.1 6.3 7.3 (32, 64, 96, 128), 4 images 6.7 5.9 7.0 8.0, 7 images 9.4 8.6 7.6 8.3, 16 images 21.2 15.9 16.5 15.4,
+//                      50 images 54 37 33 31
+//   M = 128, 28 x 28:  1 image 5.6 6.3 7.7 8.7 (16, 32, 48, 64), 7 images 8.7 6.8 8.1 9.3, 12 images 11.7 10.5 8.6 9.7, 16 images 14.6 11.0 12.7 10.3,
+//                      24 images 20.6 16.3 15.7 17.4 and with 80 pixels 14.7, 50 images 40 27 27 26
+//   M = 256, 14 x 14:  1 image 12.9 14.1 15.5 17.3 (16, 32, 48, 64), 16 images 12.9 13.7 15.6 17.5, 24 images 21 14.0 15.7 17.6, 50 images 35 28 20 22
+// A number of fragments requested ahead between 9 and 40 makes no difference of more than 0.5.
+constexpr int BLOCK_SIZES = 7;
+#define BLOCK_SIZES_OF(UC)                                                                                                                        \
+  {block_form<64, 2, UC, 15, 2>(), block_form<64, 4, UC, 12, 2>(), block_form<64, 6, UC, 6, 2>(), block_form<64, 8, UC, 6, 2>()},                 \
+  {block_form<128, 1, UC, 18, 2>(), block_form<128, 2, UC, 9, 2>(), block_form<128, 3, UC, 8, 2>(), block_form<128, 4, UC, 8, 2>(),               \
+   block_form<128, 5, UC, 12, 1>(), block_form<128, 6, UC, 12, 1>(), block_form<128, 4, UC, 8, 2>()},                                             \
+  {block_form<256, 1, UC, 14, 2>(), block_form<256, 2, UC, 18, 1>(), block_form<256, 3, UC, 12, 1>(), block_form<256, 4, UC, 12, 1>()}
+const BlockForm BLOCK_FORMS[2][3][BLOCK_SIZES] = {{BLOCK_SIZES_OF(1)}, {BLOCK_SIZES_OF(2)}};
+#undef BLOCK_SIZES_OF
+
+const BlockForm* block_choose(int n, int m, int h, int w, int oc, int stride, int* run) {
+  const int oh = (h - 1) / stride + 1, ow = (w - 1) / stride + 1;
+  const int64_t p = (int64_t)n * oh * ow;
+  const BlockForm* best = nullptr;
+  for (const BlockForm& f : BLOCK_FORMS[oc / m - 1][m == 64 ? 0 : m == 128 ? 1 : 2]) {
+    if (f.nt == 0 || (best && p <= (int64_t)256 * 16 * best->nt)) break;
+    const int r = block_run(n, h, w, oh, ow, stride, 16 * f.nt);
+    if (f.lds(r) > BLOCK_LDS_MOST) continue;   // (a stride of 2 has long runs)
+    best = &f;
+    *run = r;
+  }
+  return best;
+}
+
+}  // namespace
+
+extern "C" {
+
+int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, const cvmhip_chain* chain_a, const cvmhip_chain* chain_b,
+                               const cvmhip_chain* chain_r, const cvmhip_chain* chain_c) {
+  if (n < 1 || (m != 64 && m != 128 && m != 256) || (oc != m && oc != 2 * m) || h < 1 || w < 1 || (stride != 1 && stride != 2)) return 0;
+  if ((int64_t)n * h * w > INT32_MAX / 4 - 4096 || (int64_t)n * h * w * 4 * m > (int64_t)1 << 40) return 0;
+  const cvmhip_chain* in[4] = {chain_a, chain_b, chain_r, chain_c};
+  for (int k = 0; k < 4; ++k) {
+    DevChain c;
+    BlockRequant q;
+    if (!make_chain(in[k], &c) || !block_requant(c, k != 1, &q)) return 0;
+  }
+  int run;
+  return block_choose(n, m, h, w, oc, stride, &run) != nullptr;
+}
+
+int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* bias_a, const cvmhip_chain* chain_a, const void* wb,
+                                const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual, const cvmhip_chain* chain_r, void* out,
+                                const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next, int n, int m, int h, int w, int oc,
+                                int stride, void* stream) {
+  if (!xp || !wa || !wb || !wc || !residual || !out || !next ||
+      (((uintptr_t)bias_a | (uintptr_t)bias_b | (uintptr_t)bias_c | (uintptr_t)xp | (uintptr_t)wa | (uintptr_t)wb | (uintptr_t)wc | (uintptr_t)residual | (uintptr_t)out | (uintptr_t)next) & 15) ||
+      !cvmhip_bottleneck_eligible(n, m, h, w, oc, stride, chain_a, chain_b, chain_r, chain_c))
+    return arg_error("conv2d_bottleneck_i8");
+  BlockArgs a = {};
+  DevChain c;
+  make_chain(chain_a, &c); block_requant(c, true, &a.qa);
+  make_chain(chain_b, &c); block_requant(c, false, &a.qb);
+  make_chain(chain_r, &c); block_requant(c, true, &a.qr);
+  make_chain(chain_c, &c); block_requant(c, true, &a.qc);
+  a.x = reinterpret_cast<const int8_t*>(xp);
+  a.wa = reinterpret_cast<const int8_t*>(wa);
+  a.wb = reinterpret_cast<const int8_t*>(wb);
+  a.wc = reinterpret_cast<const int8_t*>(wc);
+  a.res = reinterpret_cast<const int8_t*>(residual);
+  a.out = reinterpret_cast<int8_t*>(out);
+  a.next = reinterpret_cast<int8_t*>(next);
+  a.ba = bias_a; a.bb = bias_b; a.bc = bias_c;
+  a.H = h; a.W = w; a.S = stride;
+  const int oh = (h - 1) / stride + 1, ow = (w - 1) / stride + 1;
+  a.OHW = oh * ow;
+  a.OW = ow;
+  a.P = n * oh * ow;
+  a.in_pixels = n * h * w;
+  a.div_ohw = make_fastdiv((uint32_t)a.OHW);
+  a.div_ow = make_fastdiv((uint32_t)ow);
+  const BlockForm* f = block_choose(n, m, h, w, oc, stride, &a.patch);
+  a.div_patch = make_fastdiv((uint32_t)a.patch);
+  a.tiles = (a.P + 16 * f->nt - 1) / (16 * f->nt);
+  char desc[128] = "";
+  if (kernel_timing_enabled())
+    snprintf(desc, sizeof(desc), "3x3/%d %d + 1x1 %d +res + 1x1 %d in %dx%dx%d out %dx%d tile %d grid %d", stride, m, 4 * m, oc, n, h, w, oh, ow, 16 * f->nt, a.tiles);
+  const double px = (double)a.P;
+  KernelTimer timer("k_conv_block", 2.0 * px * m * (9.0 * m + 4.0 * m + 4.0 * oc), as_stream(stream),
+                    (double)a.in_pixels * m + px * (8.0 * m + oc) + (double)m * (13.0 * m + 4.0 * oc), desc);
+  f->kernel<<<(unsigned)a.tiles, 512, f->lds(a.patch), as_stream(stream)>>>(a);
+  return check_launch("conv_block");
+}
+
+}  // extern "C"

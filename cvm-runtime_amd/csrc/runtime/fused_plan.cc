@@ -742,6 +742,7 @@ void HipGraphRuntime::BuildPlan() {
   BuildSeparable();
   BuildStemConv();
   if (hooks_.seq) BuildSequences();
+  BuildBottlenecks();
   BuildGroups();
 }
 
@@ -855,6 +856,39 @@ void HipGraphRuntime::RunStemConv(size_t step) {
   Check(cvmhip_conv2d_stem_conv_i8(PackedImage(d), static_cast<DeviceBuffer*>(d.weights.get())->ptr, d.bias, &d.chain,
                                    static_cast<DeviceBuffer*>(p.weights.get())->ptr, p.bias, &p.chain, i8_ptr_[p.dst], d.n, d.c, d.h, d.w, p.pool2 ? 1 : 0,
                                    stream_), "conv2d_stem_conv_i8");
+}
+
+// The 3x3 layer of a bottleneck, the 1x1 layer behind it with the residual and the first layer of the next block become one launch where no
+// layer sequence runs (Launch() takes a sequence launch first where both exist).
+void HipGraphRuntime::BuildBottlenecks() {
+  if (!hooks_.separable) return;
+  auto plain = [&](size_t k) {
+    const PlanStep& st = plan_[k];
+    return !in_resident_[k] && resident_at_[k] < 0 && !InSeparable(k) && st.kind == PlanStep::CONV && st.out_i8 && !st.stem && !st.nhwc && !st.flat &&
+           !st.ws && !st.pool2 && !st.pool3 && st.dh == 1 && st.dw == 1 && st.sh == st.sw;
+  };
+  auto pointwise = [](const PlanStep& st) { return st.kh == 1 && st.kw == 1 && st.sh == 1 && st.ph == 0 && st.pw == 0; };
+  for (size_t i = 0; i + 2 < plan_.size(); ++i) {
+    PlanStep& p = plan_[i];
+    const PlanStep &q = plan_[i + 1], &r = plan_[i + 2];
+    if (!plain(i) || !plain(i + 1) || !plain(i + 2) || p.src2 != kNone || p.oc != p.c || p.kh != 3 || p.kw != 3 || p.ph != 1 || p.pw != 1) continue;
+    if (q.src != p.dst || q.src2 == kNone || q.src2 == p.dst || q.oc != 4 * p.c || !pointwise(q)) continue;
+    if (r.src != q.dst || r.src2 != kNone || !pointwise(r)) continue;
+    bool only = true;
+    for (size_t k = 0; k < plan_.size(); ++k)
+      only = only && (k == i || k == i + 1 || plan_[k].kind == PlanStep::NODE || !ReadsI8(plan_[k], i8_ptr_[p.dst]));
+    if (((reinterpret_cast<uintptr_t>(p.bias) | reinterpret_cast<uintptr_t>(q.bias) | reinterpret_cast<uintptr_t>(r.bias)) & 15) != 0) continue;
+    if (!only || !cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain)) continue;
+    p.bottleneck = true;
+    i += 2;
+  }
+}
+
+void HipGraphRuntime::RunBottleneck(size_t step) {
+  const PlanStep &p = plan_[step], &q = plan_[step + 1], &r = plan_[step + 2];
+  auto filter = [](const PlanStep& st) { return static_cast<DeviceBuffer*>(st.weights.get())->ptr; };
+  Check(cvmhip_conv2d_bottleneck_i8(i8_ptr_[p.src], filter(p), p.bias, &p.chain, filter(q), q.bias, &q.chain, i8_ptr_[q.src2], &q.chain2, i8_ptr_[q.dst],
+                                    filter(r), r.bias, &r.chain, i8_ptr_[r.dst], p.n, p.c, p.h, p.w, r.oc, p.sh, stream_), "conv2d_bottleneck_i8");
 }
 
 void HipGraphRuntime::RunSeparable(size_t step) {
@@ -992,7 +1026,7 @@ void HipGraphRuntime::BuildGroups() {
     size_t j = i;
     for (; j < plan_.size(); ++j) {
       const PlanStep& st = plan_[j];
-      if (in_resident_[j] || InSeparable(j) || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
+      if (in_resident_[j] || InSeparable(j) || InBottleneck(j) || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
       bool reads_member = false;
       for (uint32_t w : written) reads_member = reads_member || ReadsI8(st, i8_ptr_[w]);
       if (reads_member) break;

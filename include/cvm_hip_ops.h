@@ -514,6 +514,17 @@ int cvmhip_separable_eligible(int n, int c, int h, int w, int oc, int stride_h, 
 int cvmhip_conv2d_separable_i8(const void* xp, const void* wd, const int32_t* bias_d, const cvmhip_chain* chain_d, const void* wp,
                                const int32_t* bias_p, const cvmhip_chain* chain_p, void* out, int n, int c, int h, int w, int oc,
                                int stride_h, int stride_w, int pad_h, int pad_w, void* stream);
+/* Three layers of a ResNet in one launch, int8 act tensors, m = 64, 128 or 256 channels, filters from cvmhip_pack_weights:
+ *   a    = chain_a(conv3x3(x, wa, padding 1, stride 1 or 2) + bias_a)             m -> m channels, not stored
+ *   out  = chain_r(chain_b(conv1x1(a, wb) + bias_b) + residual)                   m -> 4 m
+ *   next = chain_c(conv1x1(out, wc) + bias_c)                                     4 m -> oc = m or 2 m
+ * h, w: extent of x.  Chains of one clamp and one shift each, those in front of a, out and next to int8. */
+int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, const cvmhip_chain* chain_a, const cvmhip_chain* chain_b,
+                               const cvmhip_chain* chain_r, const cvmhip_chain* chain_c);
+int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* bias_a, const cvmhip_chain* chain_a, const void* wb,
+                                const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual, const cvmhip_chain* chain_r, void* out,
+                                const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next, int n, int m, int h, int w, int oc,
+                                int stride, void* stream);
 /* depthwise conv2d (groups == channels == out channels) on int8 act tensors, filter packed by
  * cvmhip_pack_depthwise_weights into [kh*kw][cp] int8 */
 size_t cvmhip_packed_depthwise_bytes(int c, int kh, int kw);

@@ -1,0 +1,155 @@
+"""The 3x3 layer of a bottleneck, the 1x1 layer behind it with the residual and the next block's first layer in one launch, against the oracle
+running the graph node by node."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+import oracle.graph as og
+from cvm_runtime_amd import check, graphgen, hipops, lib, runtime, synth
+from cvm_runtime_amd.hipops import chain
+
+
+def _clamp_shift(lo, hi, shift):
+    c = hipops.Chain()
+    c.count = 1
+    c.stage[0] = hipops.Stage(5, 0, shift, lo, hi)
+    return c
+
+
+def _net(n, m, h, w, oc, stride, multiply=False, reader=False):
+    g = graphgen.GraphBuilder("bottleneck-%d-%d-%d" % (m, oc, stride))
+    x = g.conv_relu_q(g.var("data", (n, 32, h, w), 8), m, 1)
+    r = g.conv_relu_q(x, 4 * m, 1, stride, 0, relu=False)
+    y, k = g.conv(x, m, 3, stride, 1)
+    if multiply:   # a chain that is no clamp and shift
+        y = g.op("broadcast_mul", [y, g.param("m", (1,), 3, 3, 3)], {}, [g.shape(y)])[0]
+    y = a = g.rshift(g.relu(y), graphgen.shift_for(k) + 2 * multiply)
+    y = g.rshift(g.relu(g.add(g.conv_relu_q(y, 4 * m, 1, relu=False), r)), 1)
+    z = g.conv_relu_q(y, oc, 1)
+    # everything the launch stores is read again, as int8
+    tails = [g.conv_relu_q(z, 16, 1, relu=False), g.conv_relu_q(y, 16, 1, relu=False)] + ([g.conv_relu_q(a, 16, 1, relu=False)] if reader else [])
+    out = tails[0]
+    for t in tails[1:]:
+        out = g.concat([out, t], 1)
+    return g.build([out])
+
+
+def _run(js, pb, data, monkeypatch, calls=3):
+    """outputs of some calls (eager, captured, replayed), and the launches of a run with and without the launch in question"""
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "1")   # no layer sequences: a measurement at load would choose
+    m = runtime.HipModel(js, pb)
+    launches = [m.launch_counts()[0]]
+    got = [np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int8) for _ in range(calls)]
+    m.close()
+    monkeypatch.setenv("CVM_HIP_SEPARABLE", "0")
+    m = runtime.HipModel(js, pb)
+    launches.append(m.launch_counts()[0])
+    m.close()
+    return got, launches
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,h,w,oc,stride", [
+    (1, 64, 1, 1, 64, 1),            # one pixel: every window leaves the image on all sides
+    (1, 64, 2, 3, 128, 2),
+    (2, 64, 13, 9, 64, 1),           # tiles that span images and end in the last one
+    (5, 64, 56, 56, 128, 1),         # tiles of 64 pixels, the last one whole
+    (2, 64, 127, 97, 64, 1),         # of 96
+    (3, 64, 101, 113, 128, 1),       # of 128
+    (9, 64, 113, 111, 64, 2),
+    (1, 128, 7, 5, 256, 1),          # of 16
+    (2, 128, 56, 56, 128, 2),
+    (3, 128, 41, 37, 128, 1),        # of 32
+    (7, 128, 37, 37, 256, 1),        # of 48
+    (17, 128, 28, 28, 128, 1),       # of 64, one to a compute unit
+    (23, 128, 28, 29, 128, 1),       # of 80
+    (29, 128, 29, 28, 256, 1),       # of 96
+    (33, 128, 28, 28, 128, 1),       # of 64 again
+    (20, 128, 60, 56, 128, 2),       # stride 2: of 80
+    (1, 256, 3, 14, 256, 1),         # of 16
+    (5, 256, 28, 28, 512, 2),
+    (22, 256, 14, 15, 256, 1),       # of 32
+    (45, 256, 14, 14, 512, 1),       # of 48
+    (43, 256, 28, 28, 256, 2),       # of 48, the longest run of the input
+    (64, 256, 14, 14, 256, 1),       # of 64
+])
+def test_bottleneck_in_one_launch(n, m, h, w, oc, stride, dev):
+    import torch
+    bias = n > 1   # with one image: none
+    rng = np.random.default_rng(n * h * w + m)
+    oh, ow = (h - 1) // stride + 1, (w - 1) // stride + 1
+    shapes = {"a": (m, m, 3, 3), "b": (4 * m, m, 1, 1), "c": (oc, 4 * m, 1, 1)}
+    x, r = (rng.integers(-128, 128, v, dtype=np.int32) for v in ((n, m, h, w), (n, 4 * m, oh, ow)))
+    f = {k: rng.integers(-128, 128, v, dtype=np.int32) for k, v in shapes.items()}
+    b = {k: rng.integers(-40000, 40000, v[0], dtype=np.int32) if bias else None for k, v in shapes.items()}
+    # clamps that act, on both sides, in front of and behind the residual
+    sh = {k: graphgen.shift_for(v[1] * v[2] * v[3]) for k, v in shapes.items()}
+    q = {"a": (0, (128 << sh["a"]) - 1, sh["a"]), "b": (-300 << sh["b"], (150 << sh["b"]) + 5, sh["b"]), "r": (-200, 255, 1),
+         "c": (-(128 << sh["c"]), (127 << sh["c"]) + 3, sh["c"])}
+
+    def requant(v, k):
+        return np.clip(v, q[k][0], q[k][1]) >> q[k][2]
+
+    ya = requant(oracle.conv2d(x, f["a"], b["a"], (stride, stride), (1, 1)), "a")
+    yb = requant(requant(oracle.conv2d(ya, f["b"], b["b"]), "b") + r, "r")
+    yc = requant(oracle.conv2d(yb, f["c"], b["c"]), "c")
+
+    def dt(v):
+        return torch.from_numpy(np.ascontiguousarray(v)).to(dev)
+
+    xp, rp = hipops.pack_act_i8(dt(x)), hipops.pack_act_i8(dt(r))
+    wp = {k: hipops.pack_weights(dt(v)) for k, v in f.items()}
+    bp = {k: dt(v) if bias else None for k, v in b.items()}
+    out, nxt = hipops._act_buffer(n * oh * ow, 4 * m, dev), hipops._act_buffer(n * oh * ow, oc, dev)
+    c = {k: _clamp_shift(*v) for k, v in q.items()}
+    vp, ref = hipops._vp, ctypes.byref
+    check(lib().cvmhip_conv2d_bottleneck_i8(vp(xp), vp(wp["a"]), vp(bp["a"]), ref(c["a"]), vp(wp["b"]), vp(bp["b"]), ref(c["b"]), vp(rp), ref(c["r"]),
+                                            vp(out), vp(wp["c"]), vp(bp["c"]), ref(c["c"]), vp(nxt), n, m, h, w, oc, stride, hipops._conv_stream()))
+    assert np.array_equal(hipops.unpack_act_i8(out, n, 4 * m, oh, ow).cpu().numpy(), yb)
+    assert np.array_equal(hipops.unpack_act_i8(nxt, n, oc, oh, ow).cpu().numpy(), yc)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,h,w,oc,stride", [(2, 64, 40, 41, 64, 1), (1, 128, 57, 56, 256, 2), (3, 256, 28, 26, 256, 1)])
+def test_bottleneck_of_a_graph(n, m, h, w, oc, stride, dev, monkeypatch):
+    js, pb = _net(n, m, h, w, oc, stride)
+    data = synth.tensor("bottleneck", "data%d" % (h * w), (n, 32, h, w), -128, 127)
+    got, launches = _run(js, pb, data, monkeypatch)
+    assert launches[0] < launches[1], launches   # (of the three apart, one may share its launch with an independent layer)
+    want = og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))[0].ravel()
+    assert all(np.array_equal(v.astype(np.int32), want) for v in got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("multiply,reader", [(True, False), (False, True)])
+def test_layers_that_stay_apart(multiply, reader, dev, monkeypatch):
+    """A chain with a multiplication, and a 3x3 result that another layer reads."""
+    js, pb = _net(2, 64, 20, 20, 64, 1, multiply, reader)
+    data = synth.tensor("bottleneck", "apart", (2, 32, 20, 20), -128, 127)
+    got, launches = _run(js, pb, data, monkeypatch)
+    assert launches[1] == launches[0], launches
+    want = og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))[0].ravel()
+    assert all(np.array_equal(v.astype(np.int32), want) for v in got)
+
+
+def _eligible(n=1, m=64, h=14, w=14, oc=64, stride=1, **chains):
+    plain = _clamp_shift(-127 << 9, 127 << 9, 9)
+    c = [chains.get(k, plain) for k in ("a", "b", "r", "c")]
+    return lib().cvmhip_bottleneck_eligible(n, m, h, w, oc, stride, *[ctypes.byref(v) for v in c])
+
+
+def test_which_layers_are_taken():
+    assert _eligible() and _eligible(m=256, oc=512, stride=2, h=28, w=28, n=50) and _eligible(h=1, w=1)
+    for bad in (dict(m=32, oc=32), dict(m=512, oc=512), dict(m=96, oc=96), dict(oc=32), dict(oc=192), dict(stride=3), dict(h=0), dict(n=0),
+                dict(n=1 << 20, h=64, w=64)):
+        assert not _eligible(**bad), bad
+    wide = _clamp_shift(-128 << 9, (128 << 9) + 511, 9)   # 128 is no int8
+    assert not _eligible(a=wide) and not _eligible(r=wide) and not _eligible(c=wide)
+    assert _eligible(b=wide)                      # in front of the residual the sum is 32 bits wide
+    for two in (chain(("mul", 3)), chain(("cvm_right_shift", 8, 9)), chain(("mul", 3), ("cvm_right_shift", 8, 9))):
+        assert not any(_eligible(**{k: two}) for k in "abrc")
+    # rows so long that not even the smallest tile's run of the input fits in LDS
+    assert _eligible(m=256, oc=256, w=100) and not _eligible(m=256, oc=256, w=400)
+    assert not _eligible(m=64, oc=64, w=4000) and not _eligible(m=256, oc=256, w=200, h=200, stride=2)
