@@ -29,6 +29,8 @@ struct BlockArgs {
   int8_t *out, *next;
   int H, W, S, P, in_pixels;          // input extent, stride of A, output pixels and input pixels of all images
   int patch, tiles;                   // pixels of a tile's run of the input, tiles
+  const int8_t* ahead[3];             // filters of a launch behind this one, which the workgroups past the tiles fetch into the L2 of their XCD
+  int ahead_kib[3], helpers;          // and how many of those there are for each XCD (0: none)
   FastDiv div_ohw, div_ow, div_patch;
   int OHW, OW;
   BlockRequant qa, qb, qr, qc;        // qb in front of the residual, qr behind it
@@ -83,6 +85,14 @@ __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) 
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)block_lds;
+  if ((int)blockIdx.x >= a.tiles) {
+    const int first_kib = (((int)blockIdx.x - a.tiles) >> 3) * 8 + wave;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      for (int k = first_kib; k < a.ahead_kib[i]; k += a.helpers * 8) block_request(a.ahead[i] + (int64_t)k * 1024 + lane * 16, lds + (uint32_t)wave * 1024u);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
 
   // an eighth of the tiles to each XCD, where neighbours share the pixels between them
   int tile;
@@ -326,6 +336,7 @@ using namespace cvmhip;
 namespace {
 
 constexpr size_t BLOCK_LDS_MOST = 160 * 1024;
+constexpr int BLOCK_UNITS = 256;   // compute units
 
 struct BlockForm { int nt; void (*kernel)(const BlockArgs); size_t (*lds)(int); };
 template <int M, int NT, int UC, int RING, int OCC>
@@ -353,7 +364,7 @@ const BlockForm* block_choose(int n, int m, int h, int w, int oc, int stride, in
   const int64_t p = (int64_t)n * oh * ow;
   const BlockForm* best = nullptr;
   for (const BlockForm& f : BLOCK_FORMS[oc / m - 1][m == 64 ? 0 : m == 128 ? 1 : 2]) {
-    if (f.nt == 0 || (best && p <= (int64_t)256 * 16 * best->nt)) break;
+    if (f.nt == 0 || (best && p <= (int64_t)BLOCK_UNITS * 16 * best->nt)) break;
     const int r = block_run(n, h, w, oh, ow, stride, 16 * f.nt);
     if (f.lds(r) > BLOCK_LDS_MOST) continue;   // (a stride of 2 has long runs)
     best = &f;
@@ -383,7 +394,7 @@ int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, c
 int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* bias_a, const cvmhip_chain* chain_a, const void* wb,
                                 const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual, const cvmhip_chain* chain_r, void* out,
                                 const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next, int n, int m, int h, int w, int oc,
-                                int stride, void* stream) {
+                                int stride, const cvmhip_bottleneck_filters* ahead, void* stream) {
   if (!xp || !wa || !wb || !wc || !residual || !out || !next ||
       (((uintptr_t)bias_a | (uintptr_t)bias_b | (uintptr_t)bias_c | (uintptr_t)xp | (uintptr_t)wa | (uintptr_t)wb | (uintptr_t)wc | (uintptr_t)residual | (uintptr_t)out | (uintptr_t)next) & 15) ||
       !cvmhip_bottleneck_eligible(n, m, h, w, oc, stride, chain_a, chain_b, chain_r, chain_c))
@@ -413,13 +424,26 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   const BlockForm* f = block_choose(n, m, h, w, oc, stride, &a.patch);
   a.div_patch = make_fastdiv((uint32_t)a.patch);
   a.tiles = (a.P + 16 * f->nt - 1) / (16 * f->nt);
+  // The 1.1 MB of filters that a launch with M = 256 reads come from behind the L2 each time: all layers' are more than it holds.  Where most compute units
+  // are idle some fetch the next launch's: ResNet-50 with 1 image 199.5 -> 193.3 us a run, 2 200.8 -> 196.1, 4 214.8 -> 211.9 (49 tiles); past that the
+  // fetches are in the way (8 images 240.3 -> 241.2, 16 285 -> 288).
+  if (ahead && ahead->m == 256 && a.tiles <= BLOCK_UNITS / 4) {
+    a.helpers = 8;
+    const int m2 = ahead->m;
+    const void* filters[3] = {ahead->wa, ahead->wb, ahead->wc};
+    const int kib[3] = {m2 / 32 * (9 * m2 / 32 + 1), m2 / 8 * (m2 / 32 + 1), ahead->oc / 32 * (m2 / 8 + 1)};
+    for (int i = 0; i < 3; ++i) {
+      a.ahead[i] = reinterpret_cast<const int8_t*>(filters[i]);
+      a.ahead_kib[i] = filters[i] ? kib[i] : 0;
+    }
+  }
   char desc[128] = "";
   if (kernel_timing_enabled())
     snprintf(desc, sizeof(desc), "3x3/%d %d + 1x1 %d +res + 1x1 %d in %dx%dx%d out %dx%d tile %d grid %d", stride, m, 4 * m, oc, n, h, w, oh, ow, 16 * f->nt, a.tiles);
   const double px = (double)a.P;
   KernelTimer timer("k_conv_block", 2.0 * px * m * (9.0 * m + 4.0 * m + 4.0 * oc), as_stream(stream),
                     (double)a.in_pixels * m + px * (8.0 * m + oc) + (double)m * (13.0 * m + 4.0 * oc), desc);
-  f->kernel<<<(unsigned)a.tiles, 512, f->lds(a.patch), as_stream(stream)>>>(a);
+  f->kernel<<<(unsigned)(a.tiles + 8 * a.helpers), 512, f->lds(a.patch), as_stream(stream)>>>(a);
   return check_launch("conv_block");
 }
 

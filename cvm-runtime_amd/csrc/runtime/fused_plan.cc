@@ -887,8 +887,14 @@ void HipGraphRuntime::BuildBottlenecks() {
 void HipGraphRuntime::RunBottleneck(size_t step) {
   const PlanStep &p = plan_[step], &q = plan_[step + 1], &r = plan_[step + 2];
   auto filter = [](const PlanStep& st) { return static_cast<DeviceBuffer*>(st.weights.get())->ptr; };
+  // the next one, at most a shortcut's projection away
+  size_t later = 0;
+  for (size_t k = step + 3; k < plan_.size() && k <= step + 4 && !later; ++k) later = plan_[k].bottleneck ? k : 0;
+  cvmhip_bottleneck_filters ahead{};
+  if (later) ahead = {filter(plan_[later]), filter(plan_[later + 1]), filter(plan_[later + 2]), plan_[later].c, plan_[later + 2].oc};
   Check(cvmhip_conv2d_bottleneck_i8(i8_ptr_[p.src], filter(p), p.bias, &p.chain, filter(q), q.bias, &q.chain, i8_ptr_[q.src2], &q.chain2, i8_ptr_[q.dst],
-                                    filter(r), r.bias, &r.chain, i8_ptr_[r.dst], p.n, p.c, p.h, p.w, r.oc, p.sh, stream_), "conv2d_bottleneck_i8");
+                                    filter(r), r.bias, &r.chain, i8_ptr_[r.dst], p.n, p.c, p.h, p.w, r.oc, p.sh, later ? &ahead : nullptr, stream_),
+        "conv2d_bottleneck_i8");
 }
 
 void HipGraphRuntime::RunSeparable(size_t step) {
