@@ -73,7 +73,7 @@ __device__ __forceinline__ void block_settle(v4i (&acc)[N]) {
   }
 }
 
-template <int M, int NT, int UC, int RING, int OCC>
+template <int M, int NT, int UC, int RING, int OCC, bool HELPERS>
 __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) {
   typedef BlockLds<M, NT, UC> L;
   constexpr int CTA = M == 256 ? 2 : 1, PGA = M == 64 ? 2 : 1, NTA = NT / PGA;   // A and C: 16-channel tiles of a wavefront at a time, groups of pixels
@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) 
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)block_lds;
-  if ((int)blockIdx.x >= a.tiles) {
+  if (HELPERS && (int)blockIdx.x >= a.tiles) {
     const int first_kib = (((int)blockIdx.x - a.tiles) >> 3) * 8 + wave;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -338,9 +338,13 @@ namespace {
 constexpr size_t BLOCK_LDS_MOST = 160 * 1024;
 constexpr int BLOCK_UNITS = 256;   // compute units
 
-struct BlockForm { int nt; void (*kernel)(const BlockArgs); size_t (*lds)(int); };
+struct BlockForm { int nt; void (*kernel)(const BlockArgs); size_t (*lds)(int); void (*with_helpers)(const BlockArgs); };
 template <int M, int NT, int UC, int RING, int OCC>
-BlockForm block_form() { return {NT, k_conv_block<M, NT, UC, RING, OCC>, [](int p) { return BlockLds<M, NT, UC>::bytes(p); }}; }
+BlockForm block_form() {
+  BlockForm f = {NT, k_conv_block<M, NT, UC, RING, OCC, false>, [](int p) { return BlockLds<M, NT, UC>::bytes(p); }, nullptr};
+  if constexpr (M > 64 && NT == 1) f.with_helpers = k_conv_block<M, NT, UC, RING, OCC, true>;
+  return f;
+}
 
 // The smallest tile of which the chip holds all at once with one to a compute unit; where there are more, the last.  Microseconds a launch, filters of twelve
 // layers in turn (tiles of 16, 32, 48 ... pixels):
@@ -426,8 +430,8 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   a.tiles = (a.P + 16 * f->nt - 1) / (16 * f->nt);
   // The 1.1 MB of filters that a launch with M = 256 reads come from behind the L2 each time: all layers' are more than it holds.  Where most compute units
   // are idle some fetch the next launch's: ResNet-50 with 1 image 199.5 -> 193.3 us a run, 2 200.8 -> 196.1, 4 214.8 -> 211.9 (49 tiles); past that the
-  // fetches are in the way (8 images 240.3 -> 241.2, 16 285 -> 288).
-  if (ahead && ahead->m == 256 && a.tiles <= BLOCK_UNITS / 4) {
+  // fetches are in the way (8 images 240.3 -> 241.2, 16 285 -> 288), and the question alone costs a launch 0.2 us, hence kernels of their own.
+  if (ahead && ahead->m == 256 && f->with_helpers && a.tiles <= BLOCK_UNITS / 4) {
     a.helpers = 8;
     const int m2 = ahead->m;
     const void* filters[3] = {ahead->wa, ahead->wb, ahead->wc};
@@ -443,7 +447,7 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   const double px = (double)a.P;
   KernelTimer timer("k_conv_block", 2.0 * px * m * (9.0 * m + 4.0 * m + 4.0 * oc), as_stream(stream),
                     (double)a.in_pixels * m + px * (8.0 * m + oc) + (double)m * (13.0 * m + 4.0 * oc), desc);
-  f->kernel<<<(unsigned)(a.tiles + 8 * a.helpers), 512, f->lds(a.patch), as_stream(stream)>>>(a);
+  (a.helpers ? f->with_helpers : f->kernel)<<<(unsigned)(a.tiles + 8 * a.helpers), 512, f->lds(a.patch), as_stream(stream)>>>(a);
   return check_launch("conv_block");
 }
 
