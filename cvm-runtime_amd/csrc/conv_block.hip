@@ -24,8 +24,9 @@ __device__ const int g_block_zero[4] = {0, 0, 0, 0};
 
 struct BlockRequant { int lo, hi, shift; };
 struct BlockArgs {
-  const int8_t *x, *wa, *wb, *wc, *res;
-  const int32_t *ba, *bb, *bc;
+  const int8_t *x, *wa, *wb, *wc, *res;   // res: the residual, or what the projection reads that makes it
+  const int8_t* ws;
+  const int32_t *ba, *bb, *bc, *bs;
   int8_t *out, *next;
   int H, W, S, P, in_pixels;          // input extent, stride of A, output pixels and input pixels of all images
   int patch, tiles;                   // pixels of a tile's run of the input, tiles
@@ -33,17 +34,18 @@ struct BlockArgs {
   int ahead_kib[3], helpers;          // and how many of those there are for each XCD (0: none)
   FastDiv div_ohw, div_ow, div_patch;
   int OHW, OW;
-  BlockRequant qa, qb, qr, qc;        // qb in front of the residual, qr behind it
+  BlockRequant qa, qb, qr, qc, qs;    // qb in front of the residual, qr behind it; qs: the projection's
 };
 
 // Where things lie in LDS: sixteen zeros for windows that leave the image, biases, A's result, B's result, the run of the input.  Granules of 16 channels
 // lie pixel by pixel, channel group after channel group: a quarter of a wavefront requests, reads and writes 16 neighbouring pixels, and these are
 // neighbours in memory too.
-template <int M, int NT, int UC>
+// KS: 64-byte steps of K of the projection that makes the residual, 0: none
+template <int M, int NT, int UC, int KS>
 struct BlockLds {
   static constexpr int P = 16 * NT, GROUP = P * 16;   // bytes of a channel group of A's and B's results
-  static constexpr int bias_requests = ((5 + UC) * M * 4 + 1023) / 1024;
-  static constexpr int zero = 0, bias = 64, mid = bias + bias_requests * 1024, wide = mid + M / 16 * GROUP, patch = wide + M / 4 * GROUP;
+  static constexpr int biases = (5 + UC + (KS ? 4 : 0)) * M, bias_requests = (biases * 4 + 1023) / 1024;
+  static constexpr int zero = 0, bias = 64, mid = bias + bias_requests * 1024, wide = mid + M / 16 * GROUP, cut = wide + M / 4 * GROUP, patch = cut + KS * 4 * GROUP;
   static size_t bytes(int patch_pixels) { return (size_t)patch + (size_t)((patch_pixels * (M / 16) + 63) / 64) * 1024; }
 };
 
@@ -73,13 +75,13 @@ __device__ __forceinline__ void block_settle(v4i (&acc)[N]) {
   }
 }
 
-template <int M, int NT, int UC, int RING, int OCC, bool HELPERS>
+template <int M, int NT, int UC, int KS, int RING, int OCC, bool HELPERS>
 __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) {
-  typedef BlockLds<M, NT, UC> L;
+  typedef BlockLds<M, NT, UC, KS> L;
   constexpr int CTA = M == 256 ? 2 : 1, PGA = M == 64 ? 2 : 1, NTA = NT / PGA;   // A and C: 16-channel tiles of a wavefront at a time, groups of pixels
   constexpr int KA = M / 64, UB = M / 64, KC = M / 16;                           // 64-byte steps of K: of a tap, of B (units of 32 channels likewise), of C
-  constexpr int FA = 9 * KA * CTA, FB = UB * KA * 2, FC = UC * KC * CTA, F = FA + FB + FC;
-  constexpr int TILE_A = (9 * M / 32 + 1) * 1024, TILE_B = (M / 32 + 1) * 1024, TILE_C = (M / 8 + 1) * 1024;   // from 32 filter rows to the next
+  constexpr int FA = 9 * KA * CTA, FS = UB * KS * 2, FB = UB * KA * 2, FC = UC * KC * CTA, F = FA + FS + FB + FC;
+  constexpr int TILE_A = (9 * M / 32 + 1) * 1024, TILE_B = (M / 32 + 1) * 1024, TILE_C = (M / 8 + 1) * 1024, TILE_S = (KS * 2 + 1) * 1024;   // from 32 filter rows to the next
   static_assert(NT % PGA == 0, "pixels are split between wavefronts by 16");
   extern __shared__ __attribute__((aligned(16))) int8_t block_lds[];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kg = lane >> 4;
@@ -115,11 +117,14 @@ __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) 
   }
 
   // ---- biases, then the run of the input
-  if (wave < L::bias_requests) {
-    const int i = (wave * 64 + lane) * 4;
-    const int32_t* b = i < M ? a.ba : i < 5 * M ? a.bb : a.bc;
-    const int at = i < M ? i : i < 5 * M ? i - M : i - 5 * M;
-    block_request(b && i < (5 + UC) * M ? b + at : g_block_zero, lds + L::bias + (uint32_t)wave * 1024u);
+#pragma unroll
+  for (int k = 0; k < L::bias_requests; k += 8) {
+    if (k + wave < L::bias_requests) {
+      const int i = ((k + wave) * 64 + lane) * 4;
+      const int32_t* b = i < M ? a.ba : i < 5 * M ? a.bb : i < (5 + UC) * M ? a.bc : a.bs;
+      const int at = i < M ? i : i < 5 * M ? i - M : i < (5 + UC) * M ? i - 5 * M : i - (5 + UC) * M;
+      block_request(b && i < L::biases ? b + at : g_block_zero, lds + L::bias + (uint32_t)(k + wave) * 1024u);
+    }
   }
   const int run_requests = (a.patch * (M / 16) + 63) >> 6;
   for (int k = wave; k < run_requests; k += 8) {
@@ -135,27 +140,36 @@ __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) 
   const int8_t* fa = a.wa + (ca >> 1) * TILE_A + (ca & 1) * 256;
   const int8_t* fb = a.wb + wave * UB * TILE_B;
   const int8_t* fc = a.wc + (ca >> 1) * TILE_C + (ca & 1) * 256;
+  const int8_t* fs = KS ? a.ws + wave * UB * TILE_S : nullptr;
   const unsigned flane = (unsigned)((kg >> 1) * 1024 + (kg & 1) * 512 + col * 16);
   v4i ring[RING];
   auto fragment = [&](const int f) __attribute__((always_inline)) {
     if (f >= F) return;
     const int8_t* p;
     if (f < FA) p = fa + (f / CTA) * 2048 + (f % CTA) * 256;
-    else if (f < FA + FB) p = fb + ((f - FA) / (KA * 2)) * TILE_B + (f - FA) % KA * 2048 + ((f - FA) / KA & 1) * 256;
-    else p = fc + (f - FA - FB) / (KC * CTA) * (M / 32) * TILE_C + (f - FA - FB) / CTA % KC * 2048 + (f - FA - FB) % CTA * 256;
+    else if (f < FA + FS) p = fs + (f - FA) / (KS ? KS * 2 : 1) * TILE_S + (f - FA) / 2 % (KS ? KS : 1) * 2048 + ((f - FA) & 1) * 256;
+    else if (f < FA + FS + FB) p = fb + (f - FA - FS) / (KA * 2) * TILE_B + (f - FA - FS) % KA * 2048 + ((f - FA - FS) / KA & 1) * 256;
+    else p = fc + (f - FA - FS - FB) / (KC * CTA) * (M / 32) * TILE_C + (f - FA - FS - FB) / CTA % KC * 2048 + (f - FA - FS - FB) % CTA * 256;
     ring[f % RING] = *reinterpret_cast<const v4i*>(p + flane);
   };
 #pragma unroll
   for (int f = 0; f < RING; ++f) fragment(f);
 
-  // ---- the residual: behind the first fragments, which need not wait for it
-  constexpr int RES = NT * M / 128;
+  // ---- the residual, or the pixels that its projection reads: behind the first fragments, which need not wait for them
+  constexpr int RES = KS ? KS * NT / 8 : NT * M / 128;   // requests of every wavefront, at least
 #pragma unroll
-  for (int k = 0; k < RES; ++k) {
+  for (int k = 0; k < (KS ? (KS * NT + 7) / 8 : RES); ++k) {
     const int part = (k * 8 + wave) * 4 + kg, g = part / NT;
     int p = p0 + (part - g * NT) * 16 + col;
     p = p > a.P - 1 ? a.P - 1 : p;
-    block_request(a.res + ((int64_t)(p >> 5) * (M / 8) + (g >> 1)) * 1024 + (g & 1) * 512 + (p & 31) * 16, lds + L::wide + (uint32_t)(k * 8 + wave) * 1024u);
+    if (KS) {
+      int r, c, n;
+      corner(p, r, c, n);
+      p = (n * a.H + r + 1) * a.W + c + 1;
+    }
+    if (!KS || k * 8 + wave < KS * NT)
+      block_request(a.res + ((int64_t)(p >> 5) * (KS ? KS * 2 : M / 8) + (g >> 1)) * 1024 + (g & 1) * 512 + (p & 31) * 16,
+                    lds + (KS ? L::cut : L::wide) + (uint32_t)(k * 8 + wave) * 1024u);
   }
   if (tid < 4) *reinterpret_cast<v4i*>(block_lds + L::zero + tid * 16) = v4i{0, 0, 0, 0};
 
@@ -216,6 +230,42 @@ __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) 
   block_landed<(FA < F - RING ? FA : F > RING ? F - RING : 0)>();   // the residual: all but the fragments requested since
   block_barrier();
 
+  // ---- the projection: to where the residual would have been fetched, every wavefront the channels that it adds
+  if constexpr (KS > 0) {
+#pragma unroll
+    for (int u = 0; u < UB; ++u) {
+      v4i acc[2 * NT];
+      const int ct = (wave * UB + u) * 2;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i * NT + j] = *reinterpret_cast<const v4i*>(block_lds + L::bias + ((5 + UC) * M + (ct + i) * 16 + kg * 4) * 4);
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        v4i b[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) b[j] = *reinterpret_cast<const v4i*>(block_lds + L::cut + (k * 4 + kg) * L::GROUP + (j * 16 + col) * 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int f = FA + (u * KS + k) * 2 + i;
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[i * NT + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[f % RING], b[j], acc[i * NT + j], 0, 0, 0);
+          fragment(f + RING);
+        }
+      }
+      block_settle(acc);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          int v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = clamp_uniform(acc[i * NT + j][e], a.qs.lo, a.qs.hi);
+          *reinterpret_cast<uint32_t*>(block_lds + L::wide + (ct + i) * L::GROUP + (j * 16 + col) * 16 + kg * 4) = shift_to_bytes(v[0], v[1], v[2], v[3], a.qs.shift);
+        }
+    }
+  }
+
   // ---- B: 16 channels after the other, all pixels; the result takes the residual's place.  The products of the next 16 run beside the requantisation.
   {
     v4i b[KA][NT], acc[2][NT];
@@ -229,7 +279,7 @@ __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) 
       for (int j = 0; j < NT; ++j) acc[u & 1][j] = *reinterpret_cast<const v4i*>(block_lds + L::bias + (M + (wave * UB * 2 + u) * 16 + kg * 4) * 4);
 #pragma unroll
       for (int k = 0; k < KA; ++k) {
-        const int f = FA + u * KA + k;
+        const int f = FA + FS + u * KA + k;
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[u & 1][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[f % RING], b[k][j], acc[u & 1][j], 0, 0, 0);
         fragment(f + RING);
@@ -277,12 +327,12 @@ __global__ void __launch_bounds__(512, 2 * OCC) k_conv_block(const BlockArgs a) 
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < CTA; ++i) {
-        const int f = FA + FB + (u * KC + k) * CTA + i;
+        const int f = FA + FS + FB + (u * KC + k) * CTA + i;
 #pragma unroll
         for (int j = 0; j < NTA; ++j) acc[i * NTA + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[f % RING], b[k & 1][j], acc[i * NTA + j], 0, 0, 0);
       }
 #pragma unroll
-      for (int i = 0; i < CTA; ++i) fragment(FA + FB + (u * KC + k) * CTA + i + RING);
+      for (int i = 0; i < CTA; ++i) fragment(FA + FS + FB + (u * KC + k) * CTA + i + RING);
       __builtin_amdgcn_sched_barrier(0);
     }
     block_settle(acc);
@@ -338,11 +388,11 @@ namespace {
 constexpr size_t BLOCK_LDS_MOST = 160 * 1024;
 constexpr int BLOCK_UNITS = 256;   // compute units
 
-struct BlockForm { int nt; void (*kernel)(const BlockArgs); size_t (*lds)(int); void (*with_helpers)(const BlockArgs); };
-template <int M, int NT, int UC, int RING, int OCC>
+struct BlockForm { int nt; void (*kernel)(const BlockArgs); size_t (*lds)(int); void (*with_helpers)(const BlockArgs); };   // (lds: by the pixels of a run)
+template <int M, int NT, int UC, int KS, int RING, int OCC>
 BlockForm block_form() {
-  BlockForm f = {NT, k_conv_block<M, NT, UC, RING, OCC, false>, [](int p) { return BlockLds<M, NT, UC>::bytes(p); }, nullptr};
-  if constexpr (M > 64 && NT == 1) f.with_helpers = k_conv_block<M, NT, UC, RING, OCC, true>;
+  BlockForm f = {NT, k_conv_block<M, NT, UC, KS, RING, OCC, false>, [](int p) { return BlockLds<M, NT, UC, KS>::bytes(p); }, nullptr};
+  if constexpr (M > 64 && NT == 1) f.with_helpers = k_conv_block<M, NT, UC, KS, RING, OCC, true>;
   return f;
 }
 
@@ -355,19 +405,22 @@ BlockForm block_form() {
 //   M = 256, 14 x 14:  1 image 12.9 14.1 15.5 17.3 (16, 32, 48, 64), 16 images 12.9 13.7 15.6 17.5, 24 images 21 14.0 15.7 17.6, 50 images 35 28 20 22
 // A number of fragments requested ahead between 9 and 40 makes no difference of more than 0.5.
 constexpr int BLOCK_SIZES = 7;
-#define BLOCK_SIZES_OF(UC)                                                                                                                        \
-  {block_form<64, 2, UC, 15, 2>(), block_form<64, 4, UC, 12, 2>(), block_form<64, 6, UC, 6, 2>(), block_form<64, 8, UC, 6, 2>()},                 \
-  {block_form<128, 1, UC, 18, 2>(), block_form<128, 2, UC, 9, 2>(), block_form<128, 3, UC, 8, 2>(), block_form<128, 4, UC, 8, 2>(),               \
-   block_form<128, 5, UC, 12, 1>(), block_form<128, 6, UC, 12, 1>(), block_form<128, 4, UC, 8, 2>()},                                             \
-  {block_form<256, 1, UC, 14, 2>(), block_form<256, 2, UC, 18, 1>(), block_form<256, 3, UC, 12, 1>(), block_form<256, 4, UC, 12, 1>()}
-const BlockForm BLOCK_FORMS[2][3][BLOCK_SIZES] = {{BLOCK_SIZES_OF(1)}, {BLOCK_SIZES_OF(2)}};
+#define BLOCK_SIZES_OF(UC, CUT)                                                                                                                   \
+  {block_form<64, 2, UC, CUT, 15, 2>(), block_form<64, 4, UC, CUT, 12, 2>(), block_form<64, 6, UC, CUT, 6, 2>(),                                  \
+   block_form<64, 8, UC, CUT, 6, 2>()},                                                                                                           \
+  {block_form<128, 1, UC, 4 * CUT, 18, 2>(), block_form<128, 2, UC, 4 * CUT, 9, 2>(), block_form<128, 3, UC, 4 * CUT, 8, 2>(),                    \
+   block_form<128, 4, UC, 4 * CUT, 8, 2>(), block_form<128, 5, UC, 4 * CUT, 12, 1>(), block_form<128, 6, UC, 4 * CUT, 12, 1>(),                   \
+   block_form<128, 4, UC, 4 * CUT, 8, 2>()},                                                                                                      \
+  {block_form<256, 1, UC, 8 * CUT, 14, 2>(), block_form<256, 2, UC, 8 * CUT, 18, 1>(), block_form<256, 3, UC, 8 * CUT, 12, 1>(),                  \
+   block_form<256, 4, UC, 8 * CUT, 12, 1>()}
+const BlockForm BLOCK_FORMS[3][3][BLOCK_SIZES] = {{BLOCK_SIZES_OF(1, 0)}, {BLOCK_SIZES_OF(2, 0)}, {BLOCK_SIZES_OF(1, 1)}};   // the last: with a projection
 #undef BLOCK_SIZES_OF
 
-const BlockForm* block_choose(int n, int m, int h, int w, int oc, int stride, int* run) {
+const BlockForm* block_choose(int n, int m, int h, int w, int oc, int stride, bool projects, int* run) {
   const int oh = (h - 1) / stride + 1, ow = (w - 1) / stride + 1;
   const int64_t p = (int64_t)n * oh * ow;
   const BlockForm* best = nullptr;
-  for (const BlockForm& f : BLOCK_FORMS[oc / m - 1][m == 64 ? 0 : m == 128 ? 1 : 2]) {
+  for (const BlockForm& f : BLOCK_FORMS[projects ? 2 : oc / m - 1][m == 64 ? 0 : m == 128 ? 1 : 2]) {
     if (f.nt == 0 || (best && p <= (int64_t)BLOCK_UNITS * 16 * best->nt)) break;
     const int r = block_run(n, h, w, oh, ow, stride, 16 * f.nt);
     if (f.lds(r) > BLOCK_LDS_MOST) continue;   // (a stride of 2 has long runs)
@@ -382,26 +435,34 @@ const BlockForm* block_choose(int n, int m, int h, int w, int oc, int stride, in
 extern "C" {
 
 int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, const cvmhip_chain* chain_a, const cvmhip_chain* chain_b,
-                               const cvmhip_chain* chain_r, const cvmhip_chain* chain_c) {
+                               const cvmhip_chain* chain_r, const cvmhip_chain* chain_c, const cvmhip_bottleneck_projection* projection) {
+  if (projection && (oc != m || projection->c != (m == 64 ? 64 : 2 * m))) return 0;
   if (n < 1 || (m != 64 && m != 128 && m != 256) || (oc != m && oc != 2 * m) || h < 1 || w < 1 || (stride != 1 && stride != 2)) return 0;
   if ((int64_t)n * h * w > INT32_MAX / 4 - 4096 || (int64_t)n * h * w * 4 * m > (int64_t)1 << 40) return 0;
-  const cvmhip_chain* in[4] = {chain_a, chain_b, chain_r, chain_c};
-  for (int k = 0; k < 4; ++k) {
+  const cvmhip_chain* in[5] = {chain_a, chain_b, chain_r, chain_c, projection ? projection->chain : nullptr};
+  for (int k = 0; k < (projection ? 5 : 4); ++k) {
     DevChain c;
     BlockRequant q;
     if (!make_chain(in[k], &c) || !block_requant(c, k != 1, &q)) return 0;
   }
+  // The pixels that a projection reads take LDS beside the run of the input: where that leaves a smaller tile only, the projection is better a launch of its own
+  // (50 images, M = 256 at 28 x 28 with stride 2: 42.7 us with tiles of 32 pixels, 24.0 with 48 and 17.6 for the projection).  Elsewhere: 16 images M = 64 15.2 us
+  // against 15.5 + 7.2, M = 128 12.5 against 13.3 + 7.3, M = 256 18.0 against 13.9 + 7.5; 1 image 4.9 / 5.0 + 1, 6.4 / 6.2 + 4.0, 16.4 / 11.3 + 4.8.
   int run;
-  return block_choose(n, m, h, w, oc, stride, &run) != nullptr;
+  const BlockForm* f = block_choose(n, m, h, w, oc, stride, projection != nullptr, &run);
+  return f && (!projection || f->nt == block_choose(n, m, h, w, oc, stride, false, &run)->nt);
 }
 
 int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* bias_a, const cvmhip_chain* chain_a, const void* wb,
                                 const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual, const cvmhip_chain* chain_r, void* out,
                                 const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next, int n, int m, int h, int w, int oc,
-                                int stride, const cvmhip_bottleneck_filters* ahead, void* stream) {
+                                int stride, const cvmhip_bottleneck_projection* projection, const cvmhip_bottleneck_filters* ahead, void* stream) {
+  if (projection && (residual || !projection->w || !projection->x || (((uintptr_t)projection->w | (uintptr_t)projection->x | (uintptr_t)projection->bias) & 15)))
+    return arg_error("conv2d_bottleneck_i8 projection");
+  if (projection) residual = projection->x;
   if (!xp || !wa || !wb || !wc || !residual || !out || !next ||
       (((uintptr_t)bias_a | (uintptr_t)bias_b | (uintptr_t)bias_c | (uintptr_t)xp | (uintptr_t)wa | (uintptr_t)wb | (uintptr_t)wc | (uintptr_t)residual | (uintptr_t)out | (uintptr_t)next) & 15) ||
-      !cvmhip_bottleneck_eligible(n, m, h, w, oc, stride, chain_a, chain_b, chain_r, chain_c))
+      !cvmhip_bottleneck_eligible(n, m, h, w, oc, stride, chain_a, chain_b, chain_r, chain_c, projection))
     return arg_error("conv2d_bottleneck_i8");
   BlockArgs a = {};
   DevChain c;
@@ -409,6 +470,11 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   make_chain(chain_b, &c); block_requant(c, false, &a.qb);
   make_chain(chain_r, &c); block_requant(c, true, &a.qr);
   make_chain(chain_c, &c); block_requant(c, true, &a.qc);
+  if (projection) {
+    make_chain(projection->chain, &c); block_requant(c, true, &a.qs);
+    a.ws = reinterpret_cast<const int8_t*>(projection->w);
+    a.bs = projection->bias;
+  }
   a.x = reinterpret_cast<const int8_t*>(xp);
   a.wa = reinterpret_cast<const int8_t*>(wa);
   a.wb = reinterpret_cast<const int8_t*>(wb);
@@ -425,7 +491,7 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   a.in_pixels = n * h * w;
   a.div_ohw = make_fastdiv((uint32_t)a.OHW);
   a.div_ow = make_fastdiv((uint32_t)ow);
-  const BlockForm* f = block_choose(n, m, h, w, oc, stride, &a.patch);
+  const BlockForm* f = block_choose(n, m, h, w, oc, stride, projection != nullptr, &a.patch);
   a.div_patch = make_fastdiv((uint32_t)a.patch);
   a.tiles = (a.P + 16 * f->nt - 1) / (16 * f->nt);
   // The 1.1 MB of filters that a launch with M = 256 reads come from behind the L2 each time: all layers' are more than it holds.  Where most compute units
@@ -443,10 +509,11 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   }
   char desc[128] = "";
   if (kernel_timing_enabled())
-    snprintf(desc, sizeof(desc), "3x3/%d %d + 1x1 %d +res + 1x1 %d in %dx%dx%d out %dx%d tile %d grid %d", stride, m, 4 * m, oc, n, h, w, oh, ow, 16 * f->nt, a.tiles);
+    snprintf(desc, sizeof(desc), "3x3/%d %d + 1x1 %d %s + 1x1 %d in %dx%dx%d out %dx%d tile %d grid %d", stride, m, 4 * m, projection ? "+ projection" : "+res", oc, n, h, w, oh, ow, 16 * f->nt, a.tiles);
   const double px = (double)a.P;
-  KernelTimer timer("k_conv_block", 2.0 * px * m * (9.0 * m + 4.0 * m + 4.0 * oc), as_stream(stream),
-                    (double)a.in_pixels * m + px * (8.0 * m + oc) + (double)m * (13.0 * m + 4.0 * oc), desc);
+  const double cut = projection ? 4.0 * projection->c : 0.0;   // multiply-adds of the projection for a channel of m
+  KernelTimer timer("k_conv_block", 2.0 * px * m * (9.0 * m + 4.0 * m + 4.0 * oc + cut), as_stream(stream),
+                    (double)a.in_pixels * m + px * ((projection ? 4.0 * m + projection->c : 8.0 * m) + oc) + (double)m * (13.0 * m + 4.0 * oc + cut), desc);
   (a.helpers ? f->with_helpers : f->kernel)<<<(unsigned)(a.tiles + 8 * a.helpers), 512, f->lds(a.patch), as_stream(stream)>>>(a);
   return check_launch("conv_block");
 }

@@ -874,27 +874,46 @@ void HipGraphRuntime::BuildBottlenecks() {
     if (!plain(i) || !plain(i + 1) || !plain(i + 2) || p.src2 != kNone || p.oc != p.c || p.kh != 3 || p.kw != 3 || p.ph != 1 || p.pw != 1) continue;
     if (q.src != p.dst || q.src2 == kNone || q.src2 == p.dst || q.oc != 4 * p.c || !pointwise(q)) continue;
     if (r.src != q.dst || r.src2 != kNone || !pointwise(r)) continue;
-    bool only = true;
-    for (size_t k = 0; k < plan_.size(); ++k)
-      only = only && (k == i || k == i + 1 || plan_[k].kind == PlanStep::NODE || !ReadsI8(plan_[k], i8_ptr_[p.dst]));
-    if (((reinterpret_cast<uintptr_t>(p.bias) | reinterpret_cast<uintptr_t>(q.bias) | reinterpret_cast<uintptr_t>(r.bias)) & 15) != 0) continue;
-    if (!only || !cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain)) continue;
-    p.bottleneck = true;
+    auto read_by_next_only = [&](size_t at, size_t next) {
+      for (size_t k = 0; k < plan_.size(); ++k)
+        if (k != at && k != next && plan_[k].kind != PlanStep::NODE && ReadsI8(plan_[k], i8_ptr_[plan_[at].dst])) return false;
+      return true;
+    };
+    auto aligned = [](const PlanStep& st) { return (reinterpret_cast<uintptr_t>(st.bias) & 15) == 0; };
+    if (!aligned(p) || !aligned(q) || !aligned(r) || !read_by_next_only(i, i + 1) ||
+        !cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain, nullptr))
+      continue;
+    // the residual's own 1x1 layer in front of them
+    bool projects = false;
+    if (i > 0 && plain(i - 1) && !InBottleneck(i - 1)) {
+      const PlanStep& s = plan_[i - 1];
+      const cvmhip_bottleneck_projection projection = {nullptr, nullptr, nullptr, &s.chain, s.c};
+      projects = s.dst == q.src2 && s.src2 == kNone && s.kh == 1 && s.kw == 1 && s.sh == p.sh && s.ph == 0 && s.pw == 0 && s.h == p.h && s.w == p.w &&
+                 s.oc == q.oc && aligned(s) && read_by_next_only(i - 1, i + 1) &&
+                 cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain, &projection);
+    }
+    PlanStep& head = plan_[projects ? i - 1 : i];
+    head.bottleneck = projects ? 4 : 3;
+    for (const SeqRun& q2 : seqs_) head.bottleneck_under_seq = head.bottleneck_under_seq || (q2.first <= i + 2 && q2.last + head.bottleneck >= i + 3);
     i += 2;
   }
 }
 
 void HipGraphRuntime::RunBottleneck(size_t step) {
-  const PlanStep &p = plan_[step], &q = plan_[step + 1], &r = plan_[step + 2];
+  const bool projects = plan_[step].bottleneck == 4;
+  const PlanStep &s = plan_[step], &p = plan_[step + projects], &q = plan_[step + projects + 1], &r = plan_[step + projects + 2];
   auto filter = [](const PlanStep& st) { return static_cast<DeviceBuffer*>(st.weights.get())->ptr; };
   // the next one, at most a shortcut's projection away
+  const size_t behind = step + plan_[step].bottleneck;
   size_t later = 0;
-  for (size_t k = step + 3; k < plan_.size() && k <= step + 4 && !later; ++k) later = plan_[k].bottleneck ? k : 0;
+  for (size_t k = behind; k < plan_.size() && k <= behind + 1 && !later; ++k) later = plan_[k].bottleneck == 3 ? k : plan_[k].bottleneck == 4 ? k + 1 : 0;
   cvmhip_bottleneck_filters ahead{};
   if (later) ahead = {filter(plan_[later]), filter(plan_[later + 1]), filter(plan_[later + 2]), plan_[later].c, plan_[later + 2].oc};
-  Check(cvmhip_conv2d_bottleneck_i8(i8_ptr_[p.src], filter(p), p.bias, &p.chain, filter(q), q.bias, &q.chain, i8_ptr_[q.src2], &q.chain2, i8_ptr_[q.dst],
-                                    filter(r), r.bias, &r.chain, i8_ptr_[r.dst], p.n, p.c, p.h, p.w, r.oc, p.sh, later ? &ahead : nullptr, stream_),
-        "conv2d_bottleneck_i8");
+  cvmhip_bottleneck_projection projection{};
+  if (projects) projection = {i8_ptr_[s.src], filter(s), s.bias, &s.chain, s.c};
+  Check(cvmhip_conv2d_bottleneck_i8(i8_ptr_[p.src], filter(p), p.bias, &p.chain, filter(q), q.bias, &q.chain, projects ? nullptr : i8_ptr_[q.src2], &q.chain2,
+                                    i8_ptr_[q.dst], filter(r), r.bias, &r.chain, i8_ptr_[r.dst], p.n, p.c, p.h, p.w, r.oc, p.sh,
+                                    projects ? &projection : nullptr, later ? &ahead : nullptr, stream_), "conv2d_bottleneck_i8");
 }
 
 void HipGraphRuntime::RunSeparable(size_t step) {

@@ -808,9 +808,9 @@ void HipGraphRuntime::Launch(size_t first) {
       } else if (plan_[i].stem_conv) {
         RunStemConv(i);
         i += 2;
-      } else if (plan_[i].bottleneck) {
+      } else if (plan_[i].bottleneck && !(seq && plan_[i].bottleneck_under_seq)) {
         RunBottleneck(i);
-        i += 3;
+        i += plan_[i].bottleneck;
       } else if (!group_at_.empty() && group_at_[i] >= 0) {
         const GroupRun& r = groups_[group_at_[i]];
         if (r.i8) HipCheck(cvmhip_conv_group_launch_i8(r.table, r.nlayers, r.blocks, r.ops, r.bytes, stream_), "grouped convolutions");

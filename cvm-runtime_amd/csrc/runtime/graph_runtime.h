@@ -119,7 +119,8 @@ struct PlanStep {
   std::shared_ptr<void> pair_bias;
   std::shared_ptr<void> folded_bias;   // CONV, DWCONV: the bias with the chains' rounding terms added (device); `bias` then points here
   bool stem_conv = false;         // CONV (stem): one launch with the convolution behind it (the next step, cvmhip_conv2d_stem_conv_i8)
-  bool bottleneck = false;        // CONV: one launch with the two 1x1 convolutions behind it (the next two steps, cvmhip_conv2d_bottleneck_i8)
+  int bottleneck = 0;             // CONV: this step and the next ones, so many, are one launch (cvmhip_conv2d_bottleneck_i8): 3, or 4 with the residual's projection first
+  bool bottleneck_under_seq = false;   // a sequence launch takes some of them, and where sequences are in use the others are launches of their own
   std::shared_ptr<void> separable;   // DWCONV: its filter for one launch with the 1x1 convolution behind it (the next step)
   uint32_t wsrc = UINT32_MAX, bsrc = UINT32_MAX;   // CONV: entries of the filter and the bias (UINT32_MAX: none)
   int n = 0, c = 0, h = 0, w = 0, oc = 0, kh = 1, kw = 1, sh = 1, sw = 1, ph = 0, pw = 0, dh = 1, dw = 1, oh = 0, ow = 0;
@@ -181,12 +182,8 @@ class HipGraphRuntime {
     if (fused_)
       for (const PlanStep& st : plan_) extra += st.flat ? 1 : 0;
     for (const PlanStep& st : plan_) grouped += st.separable || st.stem_conv ? 1 : 0;
-    for (size_t k = 0; k < plan_.size(); ++k) {   // likewise for three layers in one launch
-      bool inside = false;
-      if (SeqNow())
-        for (const SeqRun& q : seqs_) inside = inside || (k >= q.first && k <= q.last);
-      if (plan_[k].bottleneck && !inside) grouped += 2;
-    }
+    for (const PlanStep& st : plan_)   // likewise the layers of a bottleneck
+      if (st.bottleneck && !(st.bottleneck_under_seq && SeqNow())) grouped += st.bottleneck - 1;
     for (const ResidentRun& r : residents_)
       if (!(r.under_seq && SeqNow())) grouped += static_cast<int>(r.last - r.first);
     if (launches) *launches = static_cast<int>(NumSteps()) - lay + seq - (fused_ ? grouped : 0) + extra;
@@ -356,8 +353,8 @@ class HipGraphRuntime {
   void BuildBottlenecks();
   void RunBottleneck(size_t step);
   bool InBottleneck(size_t step) const {
-    for (size_t k = step < 2 ? 0 : step - 2; k <= step; ++k)
-      if (plan_[k].bottleneck) return true;
+    for (size_t k = step < 3 ? 0 : step - 3; k <= step; ++k)
+      if (k + plan_[k].bottleneck > step) return true;
     return false;
   }
   bool InPair(size_t first) const { return plan_[first].separable || plan_[first].stem_conv; }

@@ -519,16 +519,23 @@ int cvmhip_conv2d_separable_i8(const void* xp, const void* wd, const int32_t* bi
  *   out  = chain_r(chain_b(conv1x1(a, wb) + bias_b) + residual)                   m -> 4 m
  *   next = chain_c(conv1x1(out, wc) + bias_c)                                     4 m -> oc = m or 2 m
  * h, w: extent of x.  Chains of one clamp and one shift each, those in front of a, out and next to int8. */
+typedef struct cvmhip_bottleneck_projection {   /* instead of a residual: chain(conv1x1(x, w, the 3x3 layer's stride) + bias), to int8 */
+  const void *x, *w;                            /* x: h x w pixels of c channels, c = 64 (m = 64) or 2 m; oc = m then */
+  const int32_t* bias;
+  const cvmhip_chain* chain;
+  int c;
+} cvmhip_bottleneck_projection;
 typedef struct cvmhip_bottleneck_filters {   /* of a later such launch: idle compute units bring them nearer */
   const void *wa, *wb, *wc;
   int m, oc;
 } cvmhip_bottleneck_filters;
 int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, const cvmhip_chain* chain_a, const cvmhip_chain* chain_b,
-                               const cvmhip_chain* chain_r, const cvmhip_chain* chain_c);
+                               const cvmhip_chain* chain_r, const cvmhip_chain* chain_c, const cvmhip_bottleneck_projection* projection /* or NULL */);
 int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* bias_a, const cvmhip_chain* chain_a, const void* wb,
-                                const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual, const cvmhip_chain* chain_r, void* out,
-                                const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next, int n, int m, int h, int w, int oc,
-                                int stride, const cvmhip_bottleneck_filters* ahead /* or NULL */, void* stream);
+                                const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual /* NULL with a projection */,
+                                const cvmhip_chain* chain_r, void* out, const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next,
+                                int n, int m, int h, int w, int oc, int stride, const cvmhip_bottleneck_projection* projection /* or NULL */,
+                                const cvmhip_bottleneck_filters* ahead /* or NULL */, void* stream);
 /* depthwise conv2d (groups == channels == out channels) on int8 act tensors, filter packed by
  * cvmhip_pack_depthwise_weights into [kh*kw][cp] int8 */
 size_t cvmhip_packed_depthwise_bytes(int c, int kh, int kw);

@@ -11,6 +11,10 @@ from cvm_runtime_amd import check, graphgen, hipops, lib, runtime, synth
 from cvm_runtime_amd.hipops import chain
 
 
+class Projection(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_void_p), ("w", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("chain", ctypes.POINTER(hipops.Chain)), ("c", ctypes.c_int)]
+
+
 def _clamp_shift(lo, hi, shift):
     c = hipops.Chain()
     c.count = 1
@@ -18,18 +22,25 @@ def _clamp_shift(lo, hi, shift):
     return c
 
 
-def _net(n, m, h, w, oc, stride, multiply=False, reader=False):
+def _net(n, m, h, w, oc, stride, multiply=False, reader=False, projects=False):
     g = graphgen.GraphBuilder("bottleneck-%d-%d-%d" % (m, oc, stride))
-    x = g.conv_relu_q(g.var("data", (n, 32, h, w), 8), m, 1)
-    r = g.conv_relu_q(x, 4 * m, 1, stride, 0, relu=False)
+    x0 = g.conv_relu_q(g.var("data", (n, 32, h, w), 8), 64 if m == 64 else 2 * m, 1)
+    x = g.conv_relu_q(x0, m, 1)
+    if not projects:   # another reader of the residual keeps its 1x1 layer apart
+        r = g.conv_relu_q(x0, 4 * m, 1, stride, 0, relu=False)
     y, k = g.conv(x, m, 3, stride, 1)
     if multiply:   # a chain that is no clamp and shift
         y = g.op("broadcast_mul", [y, g.param("m", (1,), 3, 3, 3)], {}, [g.shape(y)])[0]
     y = a = g.rshift(g.relu(y), graphgen.shift_for(k) + 2 * multiply)
-    y = g.rshift(g.relu(g.add(g.conv_relu_q(y, 4 * m, 1, relu=False), r)), 1)
+    z = g.conv_relu_q(y, 4 * m, 1, relu=False)
+    if projects:
+        r = g.conv_relu_q(x0, 4 * m, 1, stride, 0, relu=False)
+    y = g.rshift(g.relu(g.add(z, r)), 1)
     z = g.conv_relu_q(y, oc, 1)
     # everything the launch stores is read again, as int8
     tails = [g.conv_relu_q(z, 16, 1, relu=False), g.conv_relu_q(y, 16, 1, relu=False)] + ([g.conv_relu_q(a, 16, 1, relu=False)] if reader else [])
+    if not projects:
+        tails.append(g.conv_relu_q(r, 16, 1, relu=False))
     out = tails[0]
     for t in tails[1:]:
         out = g.concat([out, t], 1)
@@ -110,18 +121,41 @@ def test_bottleneck_in_one_launch(n, m, h, w, oc, stride, dev):
         _fields_ = [(k, ctypes.c_void_p) for k in ("wa", "wb", "wc")] + [("m", ctypes.c_int), ("oc", ctypes.c_int)]
     ahead = ref(Filters(wp["a"].data_ptr(), wp["b"].data_ptr(), wp["c"].data_ptr(), m, oc)) if n % 2 else None
     check(lib().cvmhip_conv2d_bottleneck_i8(vp(xp), vp(wp["a"]), vp(bp["a"]), ref(c["a"]), vp(wp["b"]), vp(bp["b"]), ref(c["b"]), vp(rp), ref(c["r"]),
-                                            vp(out), vp(wp["c"]), vp(bp["c"]), ref(c["c"]), vp(nxt), n, m, h, w, oc, stride, ahead, hipops._conv_stream()))
+                                            vp(out), vp(wp["c"]), vp(bp["c"]), ref(c["c"]), vp(nxt), n, m, h, w, oc, stride, None, ahead, hipops._conv_stream()))
+    assert np.array_equal(hipops.unpack_act_i8(out, n, 4 * m, oh, ow).cpu().numpy(), yb)
+    assert np.array_equal(hipops.unpack_act_i8(nxt, n, oc, oh, ow).cpu().numpy(), yc)
+    if oc != m or not _eligible(n, m, h, w, oc, stride, _projection(64 if m == 64 else 2 * m)):
+        return
+    # the residual made by a projection of the block's input
+    cs = 64 if m == 64 else 2 * m
+    f["s"] = rng.integers(-128, 128, (4 * m, cs, 1, 1), dtype=np.int32)
+    b["s"] = rng.integers(-40000, 40000, 4 * m, dtype=np.int32) if bias else None
+    sh = graphgen.shift_for(cs)
+    q["s"] = (-(128 << sh), (127 << sh) + 3, sh)
+    xs = rng.integers(-128, 128, (n, cs, h, w), dtype=np.int32)
+    yb = requant(requant(oracle.conv2d(ya, f["b"], b["b"]), "b") + requant(oracle.conv2d(xs, f["s"], b["s"], (stride, stride)), "s"), "r")
+    yc = requant(oracle.conv2d(yb, f["c"], b["c"]), "c")
+    xsp, ws, bs, chain_s = hipops.pack_act_i8(dt(xs)), hipops.pack_weights(dt(f["s"])), dt(b["s"]) if bias else None, _clamp_shift(*q["s"])
+
+    projection = Projection(xsp.data_ptr(), ws.data_ptr(), bs.data_ptr() if bias else None, ctypes.pointer(chain_s), cs)
+    out.zero_()
+    nxt.zero_()
+    check(lib().cvmhip_conv2d_bottleneck_i8(vp(xp), vp(wp["a"]), vp(bp["a"]), ref(c["a"]), vp(wp["b"]), vp(bp["b"]), ref(c["b"]), None, ref(c["r"]),
+                                            vp(out), vp(wp["c"]), vp(bp["c"]), ref(c["c"]), vp(nxt), n, m, h, w, oc, stride, ref(projection), ahead,
+                                            hipops._conv_stream()))
     assert np.array_equal(hipops.unpack_act_i8(out, n, 4 * m, oh, ow).cpu().numpy(), yb)
     assert np.array_equal(hipops.unpack_act_i8(nxt, n, oc, oh, ow).cpu().numpy(), yc)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,m,h,w,oc,stride", [(2, 64, 40, 41, 64, 1), (1, 128, 57, 56, 256, 2), (3, 256, 28, 26, 256, 1)])
-def test_bottleneck_of_a_graph(n, m, h, w, oc, stride, dev, monkeypatch):
-    js, pb = _net(n, m, h, w, oc, stride)
+@pytest.mark.parametrize("projects", [False, True])
+@pytest.mark.parametrize("n,m,h,w,oc,stride", [(2, 64, 40, 41, 64, 1), (1, 128, 57, 56, 128, 2), (1, 128, 57, 56, 256, 2), (3, 256, 28, 26, 256, 1)])
+def test_bottleneck_of_a_graph(n, m, h, w, oc, stride, projects, dev, monkeypatch):
+    js, pb = _net(n, m, h, w, oc, stride, projects=projects)
     data = synth.tensor("bottleneck", "data%d" % (h * w), (n, 32, h, w), -128, 127)
     got, launches = _run(js, pb, data, monkeypatch)
-    assert launches[0] < launches[1], launches   # (of the three apart, one may share its launch with an independent layer)
+    # of the layers apart, some may share a launch with one that does not depend on them
+    assert launches[0] < launches[1] and (not projects or oc != m or launches[0] <= launches[1] - 2), launches
     want = og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))[0].ravel()
     assert all(np.array_equal(v.astype(np.int32), want) for v in got)
 
@@ -138,10 +172,14 @@ def test_layers_that_stay_apart(multiply, reader, dev, monkeypatch):
     assert all(np.array_equal(v.astype(np.int32), want) for v in got)
 
 
-def _eligible(n=1, m=64, h=14, w=14, oc=64, stride=1, **chains):
+def _projection(c, chain_s=None):
+    return ctypes.byref(Projection(None, None, None, ctypes.pointer(chain_s or _clamp_shift(-128 << 5, 127 << 5, 5)), c))
+
+
+def _eligible(n=1, m=64, h=14, w=14, oc=64, stride=1, projection=None, **chains):
     plain = _clamp_shift(-127 << 9, 127 << 9, 9)
     c = [chains.get(k, plain) for k in ("a", "b", "r", "c")]
-    return lib().cvmhip_bottleneck_eligible(n, m, h, w, oc, stride, *[ctypes.byref(v) for v in c])
+    return lib().cvmhip_bottleneck_eligible(n, m, h, w, oc, stride, *[ctypes.byref(v) for v in c], projection)
 
 
 def test_which_layers_are_taken():
@@ -154,6 +192,12 @@ def test_which_layers_are_taken():
     assert _eligible(b=wide)                      # in front of the residual the sum is 32 bits wide
     for two in (chain(("mul", 3)), chain(("cvm_right_shift", 8, 9)), chain(("mul", 3), ("cvm_right_shift", 8, 9))):
         assert not any(_eligible(**{k: two}) for k in "abrc")
+    # a projection of the block's input
+    assert _eligible(projection=_projection(64)) and _eligible(m=128, oc=128, projection=_projection(256)) and _eligible(m=256, oc=256, stride=2, projection=_projection(512))
+    for bad in (dict(projection=_projection(128)), dict(oc=128, projection=_projection(64)), dict(m=128, oc=128, projection=_projection(64)), dict(projection=_projection(64, wide))):
+        assert not _eligible(**bad), bad
+    # ... which needs room beside the longest runs of the input
+    assert _eligible(n=50, m=256, oc=256, h=28, w=28, stride=2) and not _eligible(n=50, m=256, oc=256, h=28, w=28, stride=2, projection=_projection(512))
     # rows so long that not even the smallest tile's run of the input fits in LDS
     assert _eligible(m=256, oc=256, w=100) and not _eligible(m=256, oc=256, w=400)
     assert not _eligible(m=64, oc=64, w=4000) and not _eligible(m=256, oc=256, w=200, h=200, stride=2)
