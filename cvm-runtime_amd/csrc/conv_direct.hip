@@ -152,13 +152,15 @@ __global__ void __launch_bounds__(DIRECT_SPLIT * 64) k_conv_direct(const DirectA
   }
 }
 
-// More tiles than the chip has places: a workgroup packs the filter rows of 64 output channels into LDS once and then takes one
-// group of 128 pixels after another, 32 to a wavefront, with two chunks of activations in flight across the groups.
-// Bound by the int32 tensors (16 x 256 x 56 x 56 to 64 channels: 14.0 us for 64 MB) and by the chain in front of the first product.
-constexpr int SLAB_TM = 2, SLAB_AHEAD = 2;
-template <int TAPS, bool MASK>
+// More tiles than the chip has places: a workgroup packs the filter rows of 32 * TM output channels into LDS once and then takes one
+// group of 128 pixels after another, 32 to a wavefront, with four chunks of activations in flight across the groups.
+// Bound by the int32 tensors (16 x 256 x 56 x 56 to 64 channels: 14.9 us for 64 MB) and by the chain in front of the first product: filter, packing, barrier.
+// Chunks in flight, us for 2 / 3 / 4 / 6: 256 -> 320 at 8 x 96 x 96 63.2 54.2 53.8 54.6, 64 -> 256 at 16 x 56 x 56 18.7 18.0 17.0 16.2, 200 -> 128 at
+// 8 x 33 x 33 9.6 8.9 8.8 9.0, small layers the same.  Filter rows of 96 to 256 channels a workgroup: 20 to 150 % slower (fewer wavefronts wait for more).
+constexpr int SLAB_AHEAD = 4;
+template <int TAPS, bool MASK, int TM>
 __global__ void __launch_bounds__(256) k_conv_slab(const DirectArgs a) {
-  constexpr int TM = SLAB_TM, D = SLAB_AHEAD;
+  constexpr int D = SLAB_AHEAD;
   extern __shared__ __attribute__((aligned(16))) v4i s_filter[];   // [m][chunk][lane]
   const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int xcd = blockIdx.x & 7, per = gridDim.x >> 3, extra = gridDim.x & 7;
@@ -256,12 +258,12 @@ __global__ void __launch_bounds__(256) k_conv_slab(const DirectArgs a) {
 
 // Which layers, us here against packing and product (the launch that is saved is 2-3 us of host time on top).
 // 1 x 1, k_conv_direct up to 448 tiles of 32 x 32 and K of 640: 256 -> 64 at 56 x 56 3.9 / 6.6, two images of it (392 tiles) 5.1 / 6.8, four
-// (784) 8.2 / 9.0; 512 -> 128 at 28 x 28 5.0 / 6.2; K = 1024 7.2 / 6.7.  k_conv_slab beyond that up to K = 256: 64 -> 256 at 56 x 56 5.0 / 6.6,
-// 16 images 15.7 / 20.2; 256 -> 64 14.0 / 19.2; 96 -> 160 at 4 x 75 x 75 10.5 / 12.7; 256 -> 320 at 8 x 96 x 96 35.3 / 40.7; 256 -> 1024 at
+// (784) 8.2 / 9.0; 512 -> 128 at 28 x 28 5.0 / 6.2; K = 1024 7.2 / 6.7.  k_conv_slab beyond that up to K = 256: 64 -> 256 at 56 x 56 4.6 / 6.6,
+// 16 images 17.0 / 20.2; 256 -> 64 14.9 / 19.2; 96 -> 160 at 4 x 75 x 75 9.8 / 12.7; 256 -> 320 at 8 x 96 x 96, two chunks in flight, 35.3 / 40.7; 256 -> 1024 at
 // 16 x 14 x 14 11.1 / 11.2; K = 512 9.8 / 7.0.  Two workgroups to a compute unit: one round of 528 took 11.7 where two of 264 take 10.5, and
 // three of 768 15.7 -> 19.2 (64 -> 256).
 // 3 x 3, k_conv_direct up to 256 tiles and K of 640: 64 -> 64 at 56 x 56 5.6 / 6.6; two images (392 tiles) 8.2 / 6.8; K = 1152 7.8-9.9 / 8.0.
-constexpr int DIRECT_TILES = 448, DIRECT_TILES_3X3 = 256, DIRECT_K = 640, SLAB_K = 256, SLAB_GROUPS = 512;
+constexpr int DIRECT_TILES = 448, DIRECT_TILES_3X3 = 256, DIRECT_K = 640, SLAB_K = 256, SLAB_GROUPS = 512, SLAB_FEW = 264, SLAB_HALF_EMPTY = 800;
 
 static bool conv_direct(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y, int n, int ic, int h, int wd, int oc, int oh, int ow, int kh,
                  int kw, int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w, hipStream_t s, int* rc) {
@@ -308,12 +310,20 @@ static bool conv_direct(const int32_t* x, const int32_t* w, const int32_t* bias,
     else if (mask) k_conv_direct<9, true><<<blocks, DIRECT_SPLIT * 64, 0, s>>>(a);
     else k_conv_direct<9, false><<<blocks, DIRECT_SPLIT * 64, 0, s>>>(a);
   } else {
-    a.octiles = (oc + 32 * SLAB_TM - 1) / (32 * SLAB_TM);
-    const int64_t groups = (pixels + 127) / 128, rounds = (groups * a.octiles + SLAB_GROUPS - 1) / SLAB_GROUPS;
+    // 32 channels to a workgroup where 64 would leave half of the places empty, or half of the last 64 is past the layer's end and there are two rounds.  us with 64
+    // and 32: 64 -> 256 at 56 x 56 (100 workgroups of 64) 5.5 4.6, 200 -> 64 at 96 x 96 (72) 7.9 6.2, 128 -> 160 at 4 x 40 x 40 (150) 6.5 5.5, 96 -> 160 at 2 x 75 x 75
+    // (264) 7.4 6.8, 64 -> 256 at 3 x 56 x 56 (296) 7.2 7.3, 96 -> 320 at 90 x 90 (320) 8.3 8.9, 64 -> 256 at 16 x 28 x 28 (392) 7.8 8.1; the last 64 half
+    // empty: 96 -> 160 at 4 x 75 x 75 (528) 10.9 9.8, at 6 (792) 12.3 11.9, 64 -> 160 at 8 x 96 x 96 (1 728) 18.9 21.0; 128 -> 32 at 8 x 75 x 75 10.2 9.1.
+    const int64_t groups = (pixels + 127) / 128, wide = groups * ((oc + 63) / 64), past = oc % 64;
+    const int tm = oc <= 32 || wide <= SLAB_FEW || (past > 0 && past <= 32 && wide > SLAB_GROUPS && wide <= SLAB_HALF_EMPTY) ? 1 : 2;
+    a.octiles = (oc + 32 * tm - 1) / (32 * tm);
+    const int64_t rounds = (groups * a.octiles + SLAB_GROUPS - 1) / SLAB_GROUPS;
     const unsigned blocks = (unsigned)((groups + rounds - 1) / rounds * a.octiles);
-    const size_t lds = (size_t)SLAB_TM * a.chunks * 1024;
-    if (mask) k_conv_slab<1, true><<<blocks, 256, lds, s>>>(a);
-    else k_conv_slab<1, false><<<blocks, 256, lds, s>>>(a);
+    const size_t lds = (size_t)tm * a.chunks * 1024;
+    if (mask && tm == 1) k_conv_slab<1, true, 1><<<blocks, 256, lds, s>>>(a);
+    else if (mask) k_conv_slab<1, true, 2><<<blocks, 256, lds, s>>>(a);
+    else if (tm == 1) k_conv_slab<1, false, 1><<<blocks, 256, lds, s>>>(a);
+    else k_conv_slab<1, false, 2><<<blocks, 256, lds, s>>>(a);
   }
   *rc = check_launch("conv_direct");
   return true;

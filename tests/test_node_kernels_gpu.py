@@ -173,3 +173,23 @@ def test_other_threads_run_during_an_operator_call(dev):
         stop.set()
         t.join()
     assert moved >= 20
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,stride,padding", [
+    (1, 33, 130, 128, 1, (1, 1), (0, 0)),      # one channel of a tile of 32; chunks that end inside a half of the channels
+    (3, 16, 90, 91, 31, (1, 1), (0, 0)),       # one chunk; several rounds of pixels to a workgroup
+    (1, 255, 61, 60, 128, (1, 1), (0, 0)),     # 64 would be few workgroups; eight chunks, the last one short
+    (2, 160, 75, 75, 96, (1, 1), (1, 1)),      # the last 64 channels half past the end; five chunks, a border
+    (9, 96, 57, 63, 150, (1, 1), (0, 0)),      # beyond, both in rounds
+    (10, 64, 75, 75, 224, (1, 1), (0, 0)),     # 64 channels to a workgroup: two chunks, half of the four in flight
+    (8, 200, 70, 61, 192, (1, 1), (0, 1)),     # seven chunks
+    (8, 100, 95, 96, 256, (2, 2), (0, 0)),     # stride 2
+])
+def test_conv_slab_widths(n, c, h, w, oc, stride, padding, dev):
+    cid = "slab-%d-%d-%d-%d" % (c, h, w, oc)
+    x = synth.tensor(cid, "x", (n, c, h, w), -300, 300)   # narrowed like the reference narrows
+    wt = synth.tensor(cid, "w", (oc, c, 1, 1), -300, 300)
+    b = synth.tensor(cid, "b", (oc,), -2 ** 31, 2 ** 31 - 1)
+    for bias in (None, b):
+        got = hipops.conv2d(T(x, dev), T(wt, dev), None if bias is None else T(b, dev), stride, padding).cpu().numpy()
+        assert np.array_equal(got, oracle.conv2d(x, wt, bias, stride, padding))
