@@ -520,6 +520,7 @@ void HipGraphRuntime::Release() {
   if (gate_host_) { cvmhip_host_free(gate_host_); gate_host_ = nullptr; }
   if (gate_dev_) { cvmhip_free(gate_dev_); gate_dev_ = nullptr; }
   out_host_.clear();
+  out_pieces_.clear();
   own_storage_.clear();
   if (workspace_) cvmhip_free(workspace_);
   if (slab_) cvmhip_free(slab_);
@@ -964,7 +965,9 @@ void HipGraphRuntime::CheckSequences(bool requested) {
 void HipGraphRuntime::AllocOutputStage() {
   if (out_stage_host_) return;
   size_t total = 64;   // the ticket and the status word
-  for (const NodeEntry& e : outputs_) total += AlignUp(static_cast<size_t>(shape_size(shape_[entry_id(e)])) * 4, 64);
+  auto words = [&](const NodeEntry& e) { return static_cast<size_t>(shape_size(shape_[entry_id(e)])); };
+  auto table = [&](const NodeEntry& e) { return words(e) >= PIECES_FROM ? AlignUp(words(e) / CVMHIP_EXPORT_PIECE * 8, 64) : 0; };
+  for (const NodeEntry& e : outputs_) total += AlignUp(words(e) * 4, 64) + table(e);
   HipCheck(cvmhip_host_alloc(&out_stage_host_, total), "output staging buffer");
   std::memset(out_stage_host_, 0, 64);
   HipCheck(cvmhip_alloc(&out_counter_, 8), "output counter");
@@ -972,7 +975,9 @@ void HipGraphRuntime::AllocOutputStage() {
   size_t off = 64;
   for (const NodeEntry& e : outputs_) {
     out_host_.push_back(reinterpret_cast<const int32_t*>(static_cast<char*>(out_stage_host_) + off));
-    off += AlignUp(static_cast<size_t>(shape_size(shape_[entry_id(e)])) * 4, 64);
+    off += AlignUp(words(e) * 4, 64);
+    out_pieces_.push_back(table(e) ? reinterpret_cast<uint64_t*>(static_cast<char*>(out_stage_host_) + off) : nullptr);
+    off += table(e);
   }
 }
 
@@ -1027,8 +1032,30 @@ const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, 
   const cvmhip_resident_call call = {direct ? in_stage_host_ : in_stage_dev_, const_cast<int32_t*>(out_host_[0]), static_cast<uint32_t*>(out_counter_), head};
   HipCheck(cvmhip_resident_launch(r.table, r.nlayers, r.images, r.lds, &call, r.ops, r.bytes, stream_), "layers in LDS");
   ++ticket_;
+  out_in_pieces_ = false;
   AwaitTicket();
   return out_host_;
+}
+
+// An output is copied piece by piece, those of equal words are filled (a call of SSD-512, whose 590 KB are -1 but for the kept rows).
+void HipGraphRuntime::CopyFetched(size_t k, int32_t* to) const {
+  const size_t words = static_cast<size_t>(shape_size(shape_[entry_id(outputs_[k])]));
+  const int32_t* from = out_host_[k];
+  const uint64_t* table = out_in_pieces_ ? out_pieces_[k] : nullptr;
+  size_t at = 0;
+  if (table)
+    for (size_t c = 0; c < words / CVMHIP_EXPORT_PIECE; ++c, at += CVMHIP_EXPORT_PIECE) {
+      if (table[c] >> 32) std::fill_n(to + at, CVMHIP_EXPORT_PIECE, static_cast<int32_t>(table[c]));
+      else if (to != from) std::memcpy(to + at, from + at, CVMHIP_EXPORT_PIECE * 4);
+    }
+  if (to != from) std::memcpy(to + at, from + at, (words - at) * 4);
+}
+
+void HipGraphRuntime::CompleteFetched() {
+  if (!out_in_pieces_) return;
+  for (size_t k = 0; k < outputs_.size(); ++k)
+    if (out_pieces_[k]) CopyFetched(k, const_cast<int32_t*>(out_host_[k]));
+  out_in_pieces_ = false;
 }
 
 // A large image batch that only the first convolution reads, and the packing for it the first launch of a run: that launch is issued
@@ -1118,7 +1145,7 @@ void HipGraphRuntime::ExportOutputs(bool status) {
     words[k] = shape_size(shape_[eid]);
   }
   const uint32_t* word = status ? static_cast<uint32_t*>(seq_sync_) + (cvmhip_conv_seq_sync_bytes() / 4 - 64) : nullptr;
-  HipCheck(cvmhip_export_words(src, dst, words, static_cast<int>(outputs_.size()), word, word ? seq_error_host_ : nullptr,
+  HipCheck(cvmhip_export_pieces(src, dst, out_pieces_.data(), words, static_cast<int>(outputs_.size()), word, word ? seq_error_host_ : nullptr,
                                static_cast<uint32_t*>(out_counter_), static_cast<uint32_t*>(out_stage_host_), stream_), "copy output");
 }
 
@@ -1199,7 +1226,8 @@ const std::vector<const int32_t*>& HipGraphRuntime::FetchOutputs() {
 }
 
 const std::vector<const int32_t*>& HipGraphRuntime::CollectOutputs(bool status) {
-  if (outputs_.size() <= CVMHIP_EXPORT_MAX) AwaitTicket();
+  out_in_pieces_ = outputs_.size() <= CVMHIP_EXPORT_MAX;
+  if (out_in_pieces_) AwaitTicket();
   else HipCheck(cvmhip_stream_sync(stream_), "copy output");
   in_stage_busy_ = false;
   if (seq_ran_) {

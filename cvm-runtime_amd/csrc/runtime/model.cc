@@ -75,6 +75,7 @@ void HipModel::GetOutput(char* mem) {
 
 // model.cc:181-263, restated including its loop bounds
 void HipModel::SaveTensor(const std::vector<const int32_t*>& outputs, char* mem) const {
+  if (postprocess_ == "argmax" || postprocess_ == "detection" || outputs.size() > 1 || output_bytes_ != 4) rt_->CompleteFetched();
   if (postprocess_ == "argmax") {
     int32_t* cp = reinterpret_cast<int32_t*>(mem);
     for (int k = 0; k < out_num_; ++k) {
@@ -120,7 +121,7 @@ void HipModel::SaveTensor(const std::vector<const int32_t*>& outputs, char* mem)
   } else if (output_bytes_ == 4) {
     int32_t* ref = reinterpret_cast<int32_t*>(mem);
     for (size_t k = 0; k < outputs.size(); ++k) {
-      std::memcpy(ref, outputs[k], sizeof(int32_t) * static_cast<size_t>(out_size_[k]));
+      rt_->CopyFetched(k, ref);
       ref += out_size_[k];
     }
   } else {

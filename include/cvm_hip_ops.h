@@ -188,6 +188,12 @@ int cvmhip_widen_clamp_i8(const void* src, int32_t* dst, int64_t count, int32_t 
 int cvmhip_import_bytes(void* dst, const void* src_host, size_t bytes, void* stream);
 int cvmhip_export_words(const void* const* src, void* const* dst_host, const int64_t* words, int count, const uint32_t* status,
                         uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, void* stream);
+/* The same, where a destination with a table in pieces_host (may be NULL, each table too; pinned, 8-byte aligned) is written in pieces of CVMHIP_EXPORT_PIECE words:
+ * entry c of the table is 1 << 32 | the word that all of piece c are, and the piece is not written; or its upper half is 0, and the piece is.  What
+ * is left behind the last whole piece has no entry and is written. */
+#define CVMHIP_EXPORT_PIECE 1024
+int cvmhip_export_pieces(const void* const* src, void* const* dst_host, uint64_t* const* pieces_host, const int64_t* words, int count,
+                         const uint32_t* status, uint32_t* status_host, uint32_t* counter, uint32_t* flag_host, void* stream);
 /* An int8 image batch in pinned host memory (16-byte aligned, 16 readable bytes behind it) into the layout of cvmhip_pack_stem_input_i8, by a launch that may be
  * issued before the bytes are there: the host copies chunks of cvmhip_import_stem_rows image rows (0: not available for these sizes), all channels
  * of them, image by image, and stores `ticket << 32 | chunks copied` to *progress_host (pinned) behind each.  Waits are bounded by patience_us (0: gives up at once): a

@@ -1,12 +1,14 @@
 """The two ends of CVMAPIInference: the caller's bytes through the pinned buffer (pieces, odd sizes, the clamp) into the
 row-window or the plain layout, and the outputs with their ticket back -- against the oracle's graph executor."""
+import ctypes
 import json
 
 import numpy as np
 import pytest
+import torch
 
 import oracle.graph as og
-from cvm_runtime_amd import graphgen, runtime, synth
+from cvm_runtime_amd import check, graphgen, lib, runtime, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -119,4 +121,93 @@ def test_the_storage_of_the_input_lent_to_a_later_tensor(resident, dev, monkeypa
         want = og.run_graph(js, graphgen.load_params(pb), data)[0].ravel()
         got = np.frombuffer(model.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32)
         assert np.array_equal(got, want), "call %d" % call
+    model.close()
+
+
+@pytest.mark.parametrize("words", [
+    [1023], [1024], [1025], [1024 * 3 + 2],
+    [1024 * 300 + 5],                # more pieces than the workgroups load at a time
+    [70000, 0, 5, 1024 * 65],        # one array without a table among others
+])
+def test_export_in_pieces(words, dev):
+    """Pieces of equal words are told, others written; also where only the first or the last word of one differs."""
+    piece, L, align = 1024, lib(), lambda n: (n + 63) // 64 * 64
+    arrays = []
+    for k, n in enumerate(words):
+        a = np.repeat(synth.tensor("pieces", "v%d" % k, ((n + piece - 1) // piece,), -3, 3).astype(np.int32), piece)[:n].copy()
+        a[piece * 2::piece * 7] += 1
+        a[piece - 1::piece * 5] -= 1
+        arrays.append(a)
+    src = [torch.from_numpy(a).to(dev) if a.size else torch.zeros(4, dtype=torch.int32, device=dev) for a in arrays]
+    tables = [None if k == 1 else n // piece for k, n in enumerate(words)]
+    host = ctypes.c_void_p()
+    total = 64 + sum(align(n * 4 + 16) + align((t or 0) * 8 + 8) for n, t in zip(words, tables))
+    check(L.cvmhip_host_alloc(ctypes.byref(host), ctypes.c_size_t(total)))
+    raw = np.ctypeslib.as_array((ctypes.c_uint8 * total).from_address(host.value))
+    raw[:64] = 0
+    raw[64:] = 0x5a
+    at, dst, tab = 64, [], []
+    for n, t in zip(words, tables):
+        dst.append(at)
+        at += align(n * 4 + 16)
+        tab.append(None if t is None else at)
+        at += align((t or 0) * 8 + 8)
+    counter = torch.zeros(2, dtype=torch.int32, device=dev)
+    K, vp = len(words), ctypes.c_void_p
+    stream = vp(torch.cuda.current_stream().cuda_stream)
+    for ticket in (1, 2):
+        check(L.cvmhip_export_pieces((vp * K)(*[s.data_ptr() for s in src]), (vp * K)(*[host.value + d for d in dst]),
+                                     (vp * K)(*[t and host.value + t for t in tab]), (ctypes.c_int64 * K)(*words), K, None, None,
+                                     vp(counter.data_ptr()), host, stream))
+        check(L.cvmhip_export_wait(host, ctypes.c_uint32(ticket), stream))
+    for k, a in enumerate(arrays):
+        got = raw[dst[k]:dst[k] + a.size * 4].view(np.int32).copy()
+        assert np.all(raw[dst[k] + a.size * 4:dst[k] + align(a.size * 4 + 16)] == 0x5a)
+        if tab[k] is not None:
+            t = raw[tab[k]:tab[k] + tables[k] * 8].view(np.uint64)
+            assert np.all(raw[tab[k] + tables[k] * 8:tab[k] + tables[k] * 8 + 8] == 0x5a)
+            for c in range(tables[k]):
+                here = a[c * piece:(c + 1) * piece]
+                assert bool(t[c] >> np.uint64(32)) == bool(np.all(here == here[0])), c
+                if t[c] >> np.uint64(32):
+                    got[c * piece:(c + 1) * piece] = np.uint32(t[c] & np.uint64(0xffffffff)).astype(np.int32)
+        assert np.array_equal(got, a), k
+    torch.cuda.synchronize()
+    check(L.cvmhip_host_free(host))
+
+
+@pytest.mark.parametrize("heads,postprocess", [(1, None), (2, None), (1, "argmax")])
+def test_large_outputs_with_equal_pieces(heads, postprocess, dev):
+    """An int32 output of several pieces from inputs that are partly zero: read whole, beside another head, by argmax."""
+    g = graphgen.GraphBuilder("io-pieces-%d" % heads)
+    x = g.var("data", (1, 3, 132, 132), 8)
+    y, _ = g.conv(x, 8, 3, 1, 1, bias=False)
+    out = [g.reshape(y, (1, 1, 8 * 132 * 132))]
+    if heads == 2:
+        out.append(g.reshape(g.relu(y), (1, 1, 8 * 132 * 132)))
+    if postprocess:
+        out = [y]
+    js, pb = g.build(out, postprocess=postprocess)
+    model = runtime.HipModel(js, pb)
+    params = graphgen.load_params(pb)
+    for call in range(4):
+        data = synth.tensor("io-pieces", "x%d" % call, (1, 3, 132, 132), -127, 127)
+        data[:, :, 30 * call:] = 0
+        want = og.run_graph(js, params, data)
+        got = np.frombuffer(model.inference(data.astype(np.int8).tobytes()), np.int32)
+        if postprocess:
+            rows = 8 * 132
+            flat = want[0].reshape(rows, 132).ravel().astype(np.int8)
+            best = []
+            for i in range(0, rows, 132):   # the reference's loop: its row cursor advances by a row's length
+                m = 0
+                for j in range(i, i + 132):
+                    if flat[j] > flat[i + m]:
+                        m = j - i
+                best.append(m)
+            assert np.array_equal(got[:len(best)], best), "call %d" % call
+        else:
+            assert np.array_equal(got, np.concatenate([v.ravel() for v in want])), "call %d" % call
+        model.run()
+        assert np.array_equal(np.frombuffer(model.get_output(), np.int32)[:got.size], got) or postprocess, "call %d" % call
     model.close()
