@@ -198,6 +198,9 @@ void set_conv_tuning(const ConvTuning& t);
 // 3 x 3 over 64 channels with filter and input patch in LDS (conv_halo.hip): workgroups of such a launch, 0: not for this layer
 int64_t conv_halo_blocks(const ConvGeom& g, const Epilogue& ep);
 int conv_halo(const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g, const Epilogue& ep, hipStream_t s);
+// 3 x 3 over many channels of few pixels (conv_run.hip): workgroups of such a launch, 0: not for this layer
+int64_t conv_run_blocks(const ConvGeom& g, const Epilogue& ep);
+int conv_run(const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g, const Epilogue& ep, hipStream_t s);
 
 int pad_channels(int c);
 size_t packed_act_bytes(int64_t npix, int c);

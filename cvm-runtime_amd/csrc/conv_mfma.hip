@@ -2865,6 +2865,11 @@ int conv_igemm_ws(const int8_t* xp, const int8_t* wp, void* out, ConvGeom g, con
       KernelTimer timer("k_conv_halo", 2.0 * (double)g.P * g.OC * (double)g.taps * (double)(g.C ? g.C : g.Cp), s, conv_bytes(g, ep), desc.text);
       return conv_halo(xp, wp, out, g, ep, s);
     }
+    if (const int64_t nrun = conv_run_blocks(g, ep)) {
+      const ConvDesc desc(g, ep, "run", 0, 0, (long)nrun);
+      KernelTimer timer("k_conv_run", 2.0 * (double)g.P * g.OC * (double)g.taps * (double)(g.C ? g.C : g.Cp), s, conv_bytes(g, ep), desc.text);
+      return conv_run(xp, wp, out, g, ep, s);
+    }
   }
   const bool nopad = g.PH == 0 && g.PW == 0;
   const bool rows = g.row_bytes != 0;

@@ -1,0 +1,119 @@
+"""3x3 convolution over many channels of few pixels: every tile at its edges, both strides, the fused pool, against the oracle
+and against the wavefront kernel; the lines of the dispatch."""
+import ctypes
+import json
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from cvm_runtime_amd import check, hipops, lib, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def T(a, dev):
+    return torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).to(dev)
+
+
+def clamp_shift(lo, hi, shift):
+    c = hipops.Chain()
+    c.count = 1
+    c.stage[0] = hipops.Stage(5, 0, shift, lo, hi)
+    return c
+
+
+def kernel_of(run):
+    lib().cvmhip_kernel_timing_begin()
+    out = run()
+    torch.cuda.synchronize()
+    buf = ctypes.create_string_buffer(1 << 16)
+    check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
+    return out, str(json.loads(buf.value.decode())[-1])
+
+
+@pytest.mark.parametrize("n,ic,h,w,oc,stride,pool,lo,hi,shift", [
+    (1, 512, 1, 1, 64, 1, False, -508, 508, 2),      # one pixel, all its neighbours padding
+    (1, 512, 7, 7, 512, 1, False, 0, 2047, 4),       # a ResNet's last stage
+    (1, 1024, 13, 15, 128, 2, False, -128, 127, 0),  # two shares of K to a wavefront, odd extents
+    (2, 512, 8, 6, 64, 1, True, -2048, 2047, 4),
+    (1, 256, 5, 9, 64, 1, False, -127, 127, 0),      # taps dealt to wavefronts
+    (2, 128, 7, 4, 64, 2, False, -127, 127, 0),
+])
+@pytest.mark.parametrize("bias", [False, True])
+def test_against_the_oracle(n, ic, h, w, oc, stride, pool, lo, hi, shift, bias, dev):
+    cid = "run-%d-%d-%d" % (n, ic, h)
+    x = synth.tensor(cid, "x", (n, ic, h, w), -127, 127)
+    wt = synth.tensor(cid, "w", (oc, ic, 3, 3), -127, 127)
+    b = synth.tensor(cid, "b", (oc,), -2**31, 2**31 - 1) if bias else None
+    v = oracle.conv2d(x, wt, np.zeros(oc, np.int32), (stride, stride), (1, 1), (1, 1), 1)
+    if bias:
+        v = (v.astype(np.int64) + b.reshape(1, -1, 1, 1)).astype(np.int32)   # (wraps)
+    ref = np.clip(v, lo, hi) >> shift
+    if pool:
+        ref = oracle.max_pool2d(ref, (2, 2), (2, 2), (0, 0), False)
+    oh, ow = ref.shape[2:]
+    chain = clamp_shift(lo, hi, shift)
+    xp, wp = hipops.pack_act_i8(T(x, dev)), hipops.pack_weights(T(wt, dev))
+    bt = T(b, dev) if bias else None
+
+    def run():
+        if pool:
+            return hipops.conv2d_pool2_i8(xp, n, ic, h, w, wp, oc, 3, 3, bt, chain, padding=(1, 1))
+        return hipops.conv2d_i8(xp, n, ic, h, w, wp, oc, 3, 3, bt, chain, strides=(stride, stride), padding=(1, 1))
+    got, kernel = kernel_of(run)
+    assert "k_conv_run" in kernel
+    got = hipops.unpack_act_i8(got, n, oc, oh, ow)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("n,ic,h,w,oc,stride,pool,takes", [
+    (1, 512, 7, 7, 512, 1, False, True),        # 16 x 16
+    (3, 512, 7, 7, 512, 1, False, True),        # 16 channels x 32 pixels
+    (6, 512, 7, 7, 512, 1, False, True),        # 32 x 32
+    (16, 512, 7, 7, 512, 1, False, True),       # 32 x 64
+    (23, 512, 7, 7, 512, 1, False, True),       # 64 x 64
+    (1, 512, 14, 14, 512, 2, False, True),
+    (4, 512, 13, 15, 512, 2, False, True),
+    (16, 512, 14, 14, 512, 2, False, True),
+    (1, 512, 14, 14, 512, 1, True, True),       # the pool's tiles
+    (3, 512, 14, 14, 512, 1, True, True),
+    (6, 512, 14, 14, 512, 1, True, True),
+    (16, 512, 14, 14, 512, 1, True, True),
+    (2, 1536, 5, 3, 192, 1, False, True),
+    (50, 512, 14, 14, 512, 2, False, False),    # a run of more pixels than a wavefront's LDS holds
+    (50, 512, 7, 7, 512, 1, False, False),      # 312 tiles of 64 x 64
+    (1, 256, 16, 16, 512, 2, False, True),      # fewer channels: two or four wavefronts to 64 of them, each with some of the taps
+    (2, 256, 9, 5, 128, 1, False, True),
+    (5, 256, 9, 10, 256, 1, False, True),
+    (7, 768, 9, 10, 256, 1, False, True),
+    (12, 256, 9, 10, 256, 1, False, True),
+    (1, 128, 8, 8, 256, 2, False, True),
+    (1, 128, 3, 2, 64, 1, False, True),
+    (5, 128, 9, 10, 256, 1, False, True),
+    (7, 384, 9, 10, 256, 1, False, True),
+    (12, 128, 9, 10, 256, 1, False, False),
+    (2, 256, 14, 14, 256, 1, True, False),
+    (16, 64, 7, 7, 256, 1, False, False),
+    (1, 512, 7, 7, 96, 1, False, False),        # channels that are not whole groups of 64
+])
+def test_tiles_and_lines(n, ic, h, w, oc, stride, pool, takes, dev, monkeypatch):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(n * ic + h)
+    xp = hipops.pack_act_i8(torch.randint(-127, 128, (n, ic, h, w), dtype=torch.int32, device=dev, generator=gen))
+    wp = hipops.pack_weights(torch.randint(-127, 128, (oc, ic, 3, 3), dtype=torch.int32, device=dev, generator=gen))
+    bt = torch.randint(-100000, 100000, (oc,), dtype=torch.int32, device=dev, generator=gen)
+    chain = clamp_shift(0, 127 << 12, 12)
+
+    def run():
+        if pool:
+            return hipops.conv2d_pool2_i8(xp, n, ic, h, w, wp, oc, 3, 3, bt, chain, padding=(1, 1))
+        return hipops.conv2d_i8(xp, n, ic, h, w, wp, oc, 3, 3, bt, chain, strides=(stride, stride), padding=(1, 1))
+    out, kernel = kernel_of(run)
+    assert ("k_conv_run" in kernel) == takes, kernel
+    monkeypatch.setenv("CVM_HIP_CONV", "wave")
+    want, kernel = kernel_of(run)
+    assert "k_conv_run" not in kernel
+    assert torch.equal(out, want)
