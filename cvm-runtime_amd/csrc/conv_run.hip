@@ -267,3 +267,19 @@ int conv_run(const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g, c
 }
 
 }  // namespace cvmhip
+
+using namespace cvmhip;
+
+extern "C" int cvmhip_conv2d_run_eligible(const cvmhip_chain* chain, int n, int ic, int h, int w, int oc, int kh, int kw, int stride_h, int stride_w,
+                                          int pad_h, int pad_w, int dil_h, int dil_w) {
+  if (n < 1 || ic < 1 || ic % 128 != 0 || oc < 1 || h < 1 || w < 1 || kh != 3 || kw != 3 || pad_h != 1 || pad_w != 1 || stride_h < 1 || stride_w < 1) return 0;
+  ConvGeom g = {};
+  Epilogue ep = {};
+  if (!make_chain(chain, &ep.chain)) return 0;
+  g.N = n; g.H = h; g.W = w; g.Cp = ic; g.OC = oc;
+  g.OH = (h - 1) / stride_h + 1; g.OW = (w - 1) / stride_w + 1;
+  g.KH = kh; g.KW = kw; g.SH = stride_h; g.SW = stride_w; g.PH = pad_h; g.PW = pad_w; g.DH = dil_h; g.DW = dil_w;
+  ep.out_mode = OUT_I8_ACT;
+  ep.out_cp = oc;
+  return conv_run_blocks(g, ep) > 0;
+}

@@ -429,7 +429,11 @@ int cvmhip_conv_group_launch(const void* dev_table, int nlayers, int total_block
 /* The same for convolutions with int8 output that do not depend on one another (at a small batch the first 1x1 layer and
  * the shortcut projection of a ResNet block are 50-400 workgroups each): entry i describes what cvmhip_conv2d_i8 with the
  * same arguments and an int8 output would compute; a table holds either int32 entries or int8 entries, launched by
- * cvmhip_conv_group_launch or cvmhip_conv_group_launch_i8. */
+ * cvmhip_conv_group_launch or cvmhip_conv_group_launch_i8.
+ * run_eligible: cvmhip_conv2d_i8 without a residual takes such a layer by the kernel for many channels of few pixels, which is no
+ * part of a table and is faster by more than a launch. */
+int cvmhip_conv2d_run_eligible(const cvmhip_chain* chain, int n, int ic, int h, int w, int oc, int kh, int kw, int stride_h, int stride_w,
+                               int pad_h, int pad_w, int dil_h, int dil_w);
 int cvmhip_conv_group_conv_i8(void* table, int index, int first_block, int* blocks, const void* xp, const void* wp, const int32_t* bias,
                               const cvmhip_chain* chain, const void* residual, const cvmhip_chain* chain2, void* out,
                               int n, int ic, int h, int wd, int oc, int kh, int kw,

@@ -8,7 +8,8 @@ import pytest
 import torch
 
 import oracle
-from cvm_runtime_amd import check, hipops, lib, synth
+import oracle.graph as og
+from cvm_runtime_amd import check, graphgen, hipops, lib, runtime, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +118,26 @@ def test_tiles_and_lines(n, ic, h, w, oc, stride, pool, takes, dev, monkeypatch)
     want, kernel = kernel_of(run)
     assert "k_conv_run" not in kernel
     assert torch.equal(out, want)
+
+
+def test_beside_a_projection(dev, monkeypatch):
+    """Two layers of one tensor that could share a launch: the 3x3 one keeps its own kernel."""
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "0")
+    monkeypatch.setenv("CVM_HIP_SEQ", "0")
+    g = graphgen.GraphBuilder("run-pair")
+    a = g.conv_relu_q(g.var("data", (1, 64, 14, 14), 8), 512, 1)
+    b, c = g.conv_relu_q(a, 512, 3, 2, 1), g.conv_relu_q(a, 512, 1, 2, relu=False)
+    js, pb = g.build([g.clip8(g.relu(g.add(g.conv_relu_q(b, 512, 1, relu=False), c)))])
+    model = runtime.HipModel(js, pb)
+    data = synth.tensor("run-pair", "x", (1, 64, 14, 14), -127, 127)
+    want = og.run_graph(js, graphgen.load_params(pb), data)[0].ravel()
+    for call in range(3):
+        got = np.frombuffer(model.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want), call
+    lib().cvmhip_kernel_timing_begin()
+    model.run()
+    torch.cuda.synchronize()
+    buf = ctypes.create_string_buffer(1 << 16)
+    check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
+    assert sum("k_conv_run" in str(launch) for launch in json.loads(buf.value.decode())) == 1
+    model.close()
