@@ -26,16 +26,17 @@ PEAK_I8_TOPS = 5000.0   # MI355X dense int8 MFMA peak, TOP/s
 # The third field is the first 16 hex digits of the SHA-256 of the kernels' source file as it was when the counters were
 # read: a figure is only reported while that file is unchanged, otherwise `traffic` is null (measured figures go stale).
 TRAFFIC_BYTES_PER_LAUNCH = {
-    ("resnet50", "k_conv_seq", 16): (531.0e6, "profiles/k_conv_seq_resnet50_b16_traffic.txt", "38f4298682774f68"),
-    ("vgg16", "k_conv_big", 16): (27.2e6, "profiles/k_conv_big_vgg16_b16_traffic.txt", "38f4298682774f68"),
+    ("resnet50", "k_conv_block", 16): (22.2e6, "profiles/k_conv_block_resnet50_b16_traffic.txt", "c3cf7bd744974139"),
+    ("resnet50", "k_conv_seq", 16): (531.0e6, "profiles/k_conv_seq_resnet50_b16_traffic.txt", "1d4027cda118867a"),
+    ("vgg16", "k_conv_big", 16): (27.1e6, "profiles/k_conv_big_vgg16_b16_traffic.txt", "1d4027cda118867a"),
 }
-KERNEL_SOURCE = os.path.join(ROOT, "cvm-runtime_amd", "csrc", "conv_mfma.hip")
+KERNEL_SOURCES = {"k_conv_block": "conv_block.hip", "k_conv_run": "conv_run.hip"}   # others: conv_mfma.hip
 
 
-def kernel_source_hash():
+def kernel_source_hash(kernel):
     import hashlib
     try:
-        return hashlib.sha256(open(KERNEL_SOURCE, "rb").read()).hexdigest()[:16]
+        return hashlib.sha256(open(os.path.join(ROOT, "cvm-runtime_amd", "csrc", KERNEL_SOURCES.get(kernel, "conv_mfma.hip")), "rb").read()).hexdigest()[:16]
     except OSError:
         return None
 
@@ -45,7 +46,7 @@ def dominant_conv(kt, wall_s, steps):
     average launch duration with the cost of an event pair taken off, and the figures derived from it."""
     n_timed = sum(v["launches"] for v in kt.values())
     pair_cost_us = max(0.0, (sum(v["ms"] for v in kt.values()) * 1e3 - wall_s * 1e6) / max(n_timed, 1))
-    convs = {k: v for k, v in kt.items() if k in ("k_conv_wave", "k_conv_igemm", "k_conv_seq", "k_conv_big", "k_conv_block", "k_conv_group", "k_conv_halo",
+    convs = {k: v for k, v in kt.items() if k in ("k_conv_wave", "k_conv_igemm", "k_conv_seq", "k_conv_big", "k_conv_block", "k_conv_run", "k_conv_group", "k_conv_halo",
                                               "k_conv_direct", "k_conv_slab", "k_stem_pool", "k_conv_stem_pool", "k_conv_resident")}
     dom = max(convs, key=lambda k: convs[k]["ms"]) if convs else "k_conv_wave"
     conv = convs.get(dom, {"launches": 0, "ms": 0.0, "work": 0.0})
@@ -378,7 +379,7 @@ def main():
                                            ctypes.c_size_t(a.numel()), None))
         torch.cuda.synchronize()
 
-    # The implicit-GEMM kernels (same arithmetic, chosen per layer; k_conv_seq is a run of layers in one launch);
+    # The implicit-GEMM kernels (same arithmetic, chosen per layer; k_conv_block is three or four layers in one launch, k_conv_seq a run of them);
     # the roofline object is about the one that takes more of the step.  An event pair makes a launch look longer than it is.  Every launch
     # of a step is timed and the un-instrumented step is GPU-bound with its kernels back to back, so the
     # cost of one pair is (sum of all pair times - un-instrumented step time) / launches; it is taken off
@@ -392,7 +393,7 @@ def main():
     all_s = sum(v["ms"] / 1e3 - v["launches"] * pair_us["empty_us"] * 1e-6 for v in convs.values())
     step_s = wall / args.steps
     traffic = TRAFFIC_BYTES_PER_LAUNCH.get((args.workload, dom, args.batch), (None, None, None))
-    source_hash = kernel_source_hash()
+    source_hash = kernel_source_hash(dom)
     traffic_note = None
     if traffic[0] is not None:
         if traffic[2] == source_hash:
