@@ -175,13 +175,13 @@ struct RunForm { int ot, nt; };
 static const RunForm RUN_FORMS[] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}, {4, 4}}, RUN_POOL_FORMS[] = {{1, 4}, {2, 4}, {4, 4}, {4, 8}};
 
 // pixels of the longest run of input under a tile of `units` output pixels
-static int64_t run_length(const RunArgs& a, bool pool, int units) {
-  auto corner = [&](int64_t u) {
-    const int64_t n = u / a.OHW, rem = u % a.OHW;
+static int run_length(const RunArgs& a, bool pool, int units) {   // (32 bits: the tensor has fewer bytes than that; at most 256 tiles)
+  auto corner = [&](int u) {
+    const int n = u / a.OHW, rem = u % a.OHW;
     return (n * a.H + rem / a.OW * a.S - 1) * a.W + rem % a.OW * a.S - 1;
   };
-  int64_t most = 0;
-  for (int64_t u = 0; u < a.units; u += units) most = std::max(most, corner(std::min<int64_t>(u + units, a.units) - 1) - corner(u));
+  int most = 0;
+  for (int u = 0; u < a.units; u += units) most = std::max(most, corner(std::min(u + units, a.units) - 1) - corner(u));
   return most + (pool ? 3 : 2) * (a.W + 1) + 1;
 }
 
@@ -208,9 +208,8 @@ static int run_choose(const ConvGeom& g, const Epilogue& ep, RunArgs* a) {
   for (int f = 0; f < (pool ? 4 : g.Cp % 512 == 0 ? 5 : g.Cp % 256 == 0 ? 4 : 3); ++f) {
     const int units = pool ? 4 * forms[f].nt : 16 * forms[f].nt;
     if ((int64_t)((a->units + units - 1) / units) * (g.OC / (16 * forms[f].ot)) > 256) continue;
-    const int64_t run = run_length(*a, pool, units);
-    if (run > RUN_PIXELS) return -1;
-    a->run = (int)run;
+    a->run = run_length(*a, pool, units);
+    if (a->run > RUN_PIXELS) return -1;
     return f;
   }
   return -1;
@@ -241,8 +240,9 @@ int conv_run(const int8_t* xp, const int8_t* wp, void* out, const ConvGeom& g, c
   a.div_ohw = make_fastdiv((uint32_t)a.OHW);
   a.div_ow = make_fastdiv((uint32_t)a.OW);
   a.div_run = make_fastdiv((uint32_t)a.run);
-  const unsigned grid = (unsigned)conv_run_blocks(g, ep);
   const bool pool = ep.pool != 0;
+  const int units = (pool ? 4 : 16) * form.nt;
+  const unsigned grid = (unsigned)((a.units + units - 1) / units * a.octiles);
 #define RUN_CASE(OT, NT, POOL, TG, AHEAD) k_conv_run<OT, NT, POOL, TG, AHEAD><<<grid, 512, 0, s>>>(a)
   if (pool && f == 0) RUN_CASE(1, 4, true, 1, 9);
   else if (pool && f == 1) RUN_CASE(2, 4, true, 1, 9);
