@@ -46,7 +46,7 @@ struct BlockLds {
   static constexpr int P = 16 * NT, GROUP = P * 16;   // bytes of a channel group of A's and B's results
   static constexpr int biases = (5 + UC + (KS ? 4 : 0)) * M, bias_requests = (biases * 4 + 1023) / 1024;
   static constexpr int zero = 0, bias = 64, mid = bias + bias_requests * 1024, wide = mid + M / 16 * GROUP, cut = wide + M / 4 * GROUP, patch = cut + KS * 4 * GROUP;
-  static size_t bytes(int patch_pixels) { return (size_t)patch + (size_t)((patch_pixels * (M / 16) + 63) / 64) * 1024; }
+  static int64_t bytes(int64_t patch_pixels) { return patch + (patch_pixels * (M / 16) + 63) / 64 * 1024; }
 };
 
 __device__ __forceinline__ void block_request(const void* from, uint32_t lds_at) {
@@ -364,19 +364,19 @@ static bool block_requant(const DevChain& c, bool bytes, BlockRequant* q) {
 }
 
 // pixels of the longest run of the input under `pixels` consecutive output pixels (the last tile's ends with the last pixel)
-static int block_run(int n, int h, int w, int oh, int ow, int stride, int pixels) {
+static int64_t block_run(int n, int h, int w, int oh, int ow, int stride, int pixels) {
   const int64_t all = (int64_t)n * oh * ow;
   auto corner = [&](int64_t p) {
     const int64_t im = p / (oh * ow), rem = p - im * (oh * ow), r = rem / ow;
     return (im * h + r * stride - 1) * w + (rem - r * ow) * stride - 1;
   };
-  if (stride == 1) return pixels + 2 * w + 2;
+  if (stride == 1) return pixels + 2 * (int64_t)w + 2;
   int64_t most = 0;
   for (int64_t p = 0; p < all; p += pixels) {
     const int64_t last = std::min(p + pixels, all) - 1;
     most = std::max(most, corner(last) + 2 * w + 2 - corner(p) + 1);
   }
-  return (int)most;
+  return most;
 }
 
 }  // namespace cvmhip
@@ -385,13 +385,13 @@ using namespace cvmhip;
 
 namespace {
 
-constexpr size_t BLOCK_LDS_MOST = 160 * 1024;
+constexpr int64_t BLOCK_LDS_MOST = 160 * 1024;
 constexpr int BLOCK_UNITS = 256;   // compute units
 
-struct BlockForm { int nt; void (*kernel)(const BlockArgs); size_t (*lds)(int); void (*with_helpers)(const BlockArgs); };   // (lds: by the pixels of a run)
+struct BlockForm { int nt; void (*kernel)(const BlockArgs); int64_t (*lds)(int64_t); void (*with_helpers)(const BlockArgs); };   // (lds: by the pixels of a run)
 template <int M, int NT, int UC, int KS, int RING, int OCC>
 BlockForm block_form() {
-  BlockForm f = {NT, k_conv_block<M, NT, UC, KS, RING, OCC, false>, [](int p) { return BlockLds<M, NT, UC, KS>::bytes(p); }, nullptr};
+  BlockForm f = {NT, k_conv_block<M, NT, UC, KS, RING, OCC, false>, [](int64_t p) { return BlockLds<M, NT, UC, KS>::bytes(p); }, nullptr};
   if constexpr (M > 64 && NT == 1) f.with_helpers = k_conv_block<M, NT, UC, KS, RING, OCC, true>;
   return f;
 }
@@ -422,10 +422,10 @@ const BlockForm* block_choose(int n, int m, int h, int w, int oc, int stride, bo
   const BlockForm* best = nullptr;
   for (const BlockForm& f : BLOCK_FORMS[projects ? 2 : oc / m - 1][m == 64 ? 0 : m == 128 ? 1 : 2]) {
     if (f.nt == 0 || (best && p <= (int64_t)BLOCK_UNITS * 16 * best->nt)) break;
-    const int r = block_run(n, h, w, oh, ow, stride, 16 * f.nt);
+    const int64_t r = block_run(n, h, w, oh, ow, stride, 16 * f.nt);
     if (f.lds(r) > BLOCK_LDS_MOST) continue;   // (a stride of 2 has long runs)
     best = &f;
-    *run = r;
+    *run = (int)r;
   }
   return best;
 }
@@ -514,7 +514,7 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   const double cut = projection ? 4.0 * projection->c : 0.0;   // multiply-adds of the projection for a channel of m
   KernelTimer timer("k_conv_block", 2.0 * px * m * (9.0 * m + 4.0 * m + 4.0 * oc + cut), as_stream(stream),
                     (double)a.in_pixels * m + px * ((projection ? 4.0 * m + projection->c : 8.0 * m) + oc) + (double)m * (13.0 * m + 4.0 * oc + cut), desc);
-  (a.helpers ? f->with_helpers : f->kernel)<<<(unsigned)(a.tiles + 8 * a.helpers), 512, f->lds(a.patch), as_stream(stream)>>>(a);
+  (a.helpers ? f->with_helpers : f->kernel)<<<(unsigned)(a.tiles + 8 * a.helpers), 512, (size_t)f->lds(a.patch), as_stream(stream)>>>(a);
   return check_launch("conv_block");
 }
 

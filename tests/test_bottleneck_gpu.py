@@ -201,3 +201,10 @@ def test_which_layers_are_taken():
     # rows so long that not even the smallest tile's run of the input fits in LDS
     assert _eligible(m=256, oc=256, w=100) and not _eligible(m=256, oc=256, w=400)
     assert not _eligible(m=64, oc=64, w=4000) and not _eligible(m=256, oc=256, w=200, h=200, stride=2)
+
+
+@pytest.mark.parametrize("m,w", [(128, 1 << 28), (256, 1 << 27), (256, (1 << 27) + 5)])
+def test_rows_whose_bytes_do_not_fit_in_32_bits(m, w):
+    """The run of the input under the smallest tile is two rows and more: 2 * w * m bytes of LDS, next to nothing in 32 bits."""
+    assert 2 * w * m // 16 % 2**32 < 4096
+    assert not _eligible(m=m, oc=m, h=1, w=w)
