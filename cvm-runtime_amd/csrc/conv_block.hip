@@ -438,7 +438,7 @@ int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, c
                                const cvmhip_chain* chain_r, const cvmhip_chain* chain_c, const cvmhip_bottleneck_projection* projection) {
   if (projection && (oc != m || projection->c != (m == 64 ? 64 : 2 * m))) return 0;
   if (n < 1 || (m != 64 && m != 128 && m != 256) || (oc != m && oc != 2 * m) || h < 1 || w < 1 || (stride != 1 && stride != 2)) return 0;
-  if ((int64_t)n * h * w > INT32_MAX / 4 - 4096 || (int64_t)n * h * w * 4 * m > (int64_t)1 << 40) return 0;
+  if ((int64_t)n * h > INT32_MAX / 4 || (int64_t)n * h * w > INT32_MAX / 4 - 4096 || (int64_t)n * h * w * 4 * m > (int64_t)1 << 40) return 0;
   const cvmhip_chain* in[5] = {chain_a, chain_b, chain_r, chain_c, projection ? projection->chain : nullptr};
   for (int k = 0; k < (projection ? 5 : 4); ++k) {
     DevChain c;

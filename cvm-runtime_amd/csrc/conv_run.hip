@@ -273,6 +273,7 @@ using namespace cvmhip;
 extern "C" int cvmhip_conv2d_run_eligible(const cvmhip_chain* chain, int n, int ic, int h, int w, int oc, int kh, int kw, int stride_h, int stride_w,
                                           int pad_h, int pad_w, int dil_h, int dil_w) {
   if (n < 1 || ic < 1 || ic % 128 != 0 || oc < 1 || h < 1 || w < 1 || kh != 3 || kw != 3 || pad_h != 1 || pad_w != 1 || stride_h < 1 || stride_w < 1) return 0;
+  if ((int64_t)n * h > INT32_MAX || (int64_t)n * h * w > INT32_MAX || (int64_t)n * h * w * ic > INT32_MAX) return 0;   // (as cvmhip_conv2d_i8 refuses them)
   ConvGeom g = {};
   Epilogue ep = {};
   if (!make_chain(chain, &ep.chain)) return 0;

@@ -208,3 +208,12 @@ def test_rows_whose_bytes_do_not_fit_in_32_bits(m, w):
     """The run of the input under the smallest tile is two rows and more: 2 * w * m bytes of LDS, next to nothing in 32 bits."""
     assert 2 * w * m // 16 % 2**32 < 4096
     assert not _eligible(m=m, oc=m, h=1, w=w)
+
+
+def test_products_of_sizes_past_64_bits():
+    """No tensor has such sizes; in 64 bits the pixels are 0 and the bytes 2^30."""
+    assert (1 << 30) * (1 << 30) * 16 % 2**64 == 0 and 652805 * 26317 * (1 << 30) % 2**64 == 1 << 30
+    assert not _eligible(n=1 << 30, h=1 << 30, w=16) and not _eligible(n=1 << 30, h=1 << 30, w=16, stride=2)
+    c, size = _clamp_shift(0, 127 << 12, 12), dict(n=652805, ic=1 << 30, h=26317, w=1)
+    run = [lib().cvmhip_conv2d_run_eligible(ctypes.byref(c), v["n"], v["ic"], v["h"], v["w"], 64, 3, 3, 1, 1, 1, 1, 1, 1) for v in (size, dict(size, n=1, h=7, ic=512))]
+    assert not run[0] and run[1]
