@@ -12,6 +12,7 @@
 // requested RING fragments ahead across the layers.
 // v_mfma_i32_16x16x64_i8 with the filter as first operand: a lane's four results are four consecutive channels of one pixel, a dword of the operand.
 #include <algorithm>
+#include <numeric>
 
 #include "conv_mfma.h"
 #include "requant.h"
@@ -363,17 +364,19 @@ static bool block_requant(const DevChain& c, bool bytes, BlockRequant* q) {
   return clamp_shift_of(c, &q->lo, &q->hi, &q->shift) && (!bytes || clamp_shift_narrow(q->lo, q->hi, q->shift));
 }
 
-// pixels of the longest run of the input under `pixels` consecutive output pixels (the last tile's ends with the last pixel)
+// Pixels of the longest run of the input under `pixels` consecutive output pixels (the last tile's ends with the last pixel).
+// How long a run is depends on where in its image the tile begins, and that comes again after OHW / gcd(OHW, pixels) tiles: 49 of 2 450 for
+// 50 images of 56 x 56 and stride 2 in tiles of 16 (cvmhip_bottleneck_eligible with 128 channels 60 us of the host's time -> 4, 16 images 15 -> 3).
 static int64_t block_run(int n, int h, int w, int oh, int ow, int stride, int pixels) {
-  const int64_t all = (int64_t)n * oh * ow;
-  auto corner = [&](int64_t p) {
-    const int64_t im = p / (oh * ow), rem = p - im * (oh * ow), r = rem / ow;
-    return (im * h + r * stride - 1) * w + (rem - r * ow) * stride - 1;
-  };
   if (stride == 1) return pixels + 2 * (int64_t)w + 2;
+  const int image = oh * ow, all = n * image, different = image / std::gcd(image, pixels);   // (32 bits: cvmhip_bottleneck_eligible)
+  auto corner = [&](int p) {
+    const int im = p / image, rem = p - im * image, r = rem / ow;
+    return (int64_t)(im * h + r * stride - 1) * w + (rem - r * ow) * stride - 1;
+  };
   int64_t most = 0;
-  for (int64_t p = 0; p < all; p += pixels) {
-    const int64_t last = std::min(p + pixels, all) - 1;
+  for (int k = 0, p = 0; k < different && p < all; ++k, p += pixels) {
+    const int last = std::min(p + pixels, all) - 1;
     most = std::max(most, corner(last) + 2 * w + 2 - corner(p) + 1);
   }
   return most;

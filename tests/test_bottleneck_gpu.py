@@ -217,3 +217,18 @@ def test_products_of_sizes_past_64_bits():
     c, size = _clamp_shift(0, 127 << 12, 12), dict(n=652805, ic=1 << 30, h=26317, w=1)
     run = [lib().cvmhip_conv2d_run_eligible(ctypes.byref(c), v["n"], v["ic"], v["h"], v["w"], 64, 3, 3, 1, 1, 1, 1, 1, 1) for v in (size, dict(size, n=1, h=7, ic=512))]
     assert not run[0] and run[1]
+
+
+def test_longest_run_of_a_stride_2_layer():
+    """Against the runs of all tiles: whether the smallest tile's fits in LDS with the results and the biases."""
+    rng, taken = np.random.default_rng(7), 0
+    for _ in range(400):
+        m, n, h, w = int(rng.choice([64, 128, 256])), int(rng.integers(1, 6)), int(rng.integers(1, 40)), int(rng.integers(1, 90) * rng.integers(1, 12))
+        pixels, oh, ow = 32 if m == 64 else 16, (h + 1) // 2, (w + 1) // 2
+        p = np.arange(0, n * oh * ow, pixels)
+        first, last = (((q // (oh * ow)) * h + q % (oh * ow) // ow * 2 - 1) * w + q % ow * 2 - 1 for q in (p, np.minimum(p + pixels, n * oh * ow) - 1))
+        run = int((last + 2 * w + 2 - first + 1).max())
+        lds = 64 + -(-6 * m * 4 // 1024) * 1024 + 5 * m // 16 * pixels * 16 + -(-run * (m // 16) // 64) * 1024
+        assert bool(_eligible(n=n, m=m, oc=m, h=h, w=w, stride=2)) == (lds <= 160 * 1024), (n, m, h, w)
+        taken += lds <= 160 * 1024
+    assert 100 < taken < 390
