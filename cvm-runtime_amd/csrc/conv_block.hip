@@ -21,7 +21,7 @@ namespace cvmhip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-__device__ const int g_block_zero[4] = {0, 0, 0, 0};
+alignas(16) __device__ const int g_block_zero[4] = {0, 0, 0, 0};
 
 struct BlockRequant { int lo, hi, shift; };
 struct BlockArgs {

@@ -30,7 +30,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int HALO_CHUNKS = 18, HALO_FILTER = 2 * HALO_CHUNKS * 1024, HALO_PIXELS = 512;
 
-__device__ const int g_halo_zero[4] = {0, 0, 0, 0};
+alignas(16) __device__ const int g_halo_zero[4] = {0, 0, 0, 0};
 
 struct HaloGeom {
   const int8_t* x;
