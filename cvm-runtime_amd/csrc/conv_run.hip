@@ -282,5 +282,6 @@ extern "C" int cvmhip_conv2d_run_eligible(const cvmhip_chain* chain, int n, int 
   g.KH = kh; g.KW = kw; g.SH = stride_h; g.SW = stride_w; g.PH = pad_h; g.PW = pad_w; g.DH = dil_h; g.DW = dil_w;
   ep.out_mode = OUT_I8_ACT;
   ep.out_cp = oc;
-  return conv_run_blocks(g, ep) > 0;
+  RunArgs a = {};
+  return conv_run_blocks(g, ep) <= 0 ? 0 : g.Cp % 512 == 0 && run_choose(g, ep, &a) == 0 ? 2 : 1;
 }

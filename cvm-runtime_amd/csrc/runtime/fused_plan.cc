@@ -1047,13 +1047,22 @@ void HipGraphRuntime::BuildGroups() {
     table.clear();
     int blocks = 0;
     double ops = 0, bytes = 0;
+    bool has_run = false;
     std::vector<uint32_t> written;
     size_t j = i;
     for (; j < plan_.size(); ++j) {
       const PlanStep& st = plan_[j];
       if (in_resident_[j] || InSeparable(j) || InBottleneck(j) || st.kind != PlanStep::CONV || st.stem || st.nhwc || st.ws || st.flat || !st.out_i8 || st.pool2 || group_at_[j] >= 0) break;
-      // (a run of ResNet-50: 1 image with the 3x3 layer in a launch with the projection 179.4 us, for itself 174.7, 2 180.6 and 177.9, 4 198.5 and 196.5)
-      if (st.src2 == kNone && cvmhip_conv2d_run_eligible(&st.chain, st.n, st.c, st.h, st.w, st.oc, st.kh, st.kw, st.sh, st.sw, st.ph, st.pw, st.dh, st.dw)) break;
+      // A layer that has the kernel for many channels of few pixels leaves that kernel for the group's.  It stays for itself where that kernel is far ahead (512
+      // channels or a multiple, its smallest tile) or the group would be more than one workgroup to a compute unit; a group and the two launches, us with the
+      // layers around them:
+      //   3x3 512 -> 512 twice at 7 x 7, 1 image (32 workgroups in the group) 23.8 21.7, 2 24.2 22.4, 3 (96) 24.3 24.1, 6 (160) 24.9 25.9, 10 (256) 25.4 26.5, 12 (320) 31.9 28.5,
+      //   16 32.4 29.0; beside its projection at 14 x 14 stride 2, 1 image 26.6 23.1, 4 26.4 27.2, 8 (224) 28.0 29.1, 12 (320) 30.3 30.2, 16 33.7 30.8
+      //   256 channels twice at 14 x 14, 4 images (208) 25.4 26.9, 8 (400) 31.4 30.3; beside a projection, 8 (232) 26.6 28.6, 10 (280) 30.9 29.4
+      //   128 channels twice at 28 x 28, 2 images (200) 27.6 29.2; beside a projection, stride 2, 4 images (120) 25.2 27.0
+      //   in a run of ResNet-50, 512 at 14 x 14 stride 2 beside 1024 -> 2048, 1 image (80) 180.2 175.0, 2 (160) 180.5 178.5, 3 (240) 188.6 189.1, 4 (320) 199.0 197.0
+      const int run = st.src2 != kNone ? 0 : cvmhip_conv2d_run_eligible(&st.chain, st.n, st.c, st.h, st.w, st.oc, st.kh, st.kw, st.sh, st.sw, st.ph, st.pw, st.dh, st.dw);
+      if (run == 2) break;
       bool reads_member = false;
       for (uint32_t w : written) reads_member = reads_member || ReadsI8(st, i8_ptr_[w]);
       if (reads_member) break;
@@ -1064,7 +1073,8 @@ void HipGraphRuntime::BuildGroups() {
                                                static_cast<DeviceBuffer*>(st.weights.get())->ptr, st.bias, &st.chain, res, &st.chain2,
                                                i8_ptr_[st.dst], st.n, st.c, st.h, st.w, st.oc, st.kh, st.kw, st.sh, st.sw, st.ph, st.pw,
                                                st.dh, st.dw);
-      if (rc != CVMHIP_OK || blocks + nb > 512) break;
+      has_run = has_run || run;
+      if (rc != CVMHIP_OK || blocks + nb > (has_run ? 256 : 512)) break;
       blocks += nb;
       written.push_back(st.dst);
       const int oh = (st.h + 2 * st.ph - (st.dh * (st.kh - 1) + 1)) / st.sh + 1, ow = (st.w + 2 * st.pw - (st.dw * (st.kw - 1) + 1)) / st.sw + 1;

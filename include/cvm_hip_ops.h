@@ -430,8 +430,8 @@ int cvmhip_conv_group_launch(const void* dev_table, int nlayers, int total_block
  * the shortcut projection of a ResNet block are 50-400 workgroups each): entry i describes what cvmhip_conv2d_i8 with the
  * same arguments and an int8 output would compute; a table holds either int32 entries or int8 entries, launched by
  * cvmhip_conv_group_launch or cvmhip_conv_group_launch_i8.
- * run_eligible: cvmhip_conv2d_i8 without a residual takes such a layer by the kernel for many channels of few pixels, which is no
- * part of a table and is faster by more than a launch. */
+ * run_eligible: whether cvmhip_conv2d_i8 without a residual takes such a layer by the kernel for many channels of few pixels, which is no
+ * part of a table; 2: and is ahead of a launch with others of any size, 1: of one with more workgroups than compute units. */
 int cvmhip_conv2d_run_eligible(const cvmhip_chain* chain, int n, int ic, int h, int w, int oc, int kh, int kw, int stride_h, int stride_w,
                                int pad_h, int pad_w, int dil_h, int dil_w);
 int cvmhip_conv_group_conv_i8(void* table, int index, int first_block, int* blocks, const void* xp, const void* wp, const int32_t* bias,

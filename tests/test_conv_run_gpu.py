@@ -141,3 +141,37 @@ def test_beside_a_projection(dev, monkeypatch):
     check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
     assert sum("k_conv_run" in str(launch) for launch in json.loads(buf.value.decode())) == 1
     model.close()
+
+
+@pytest.mark.parametrize("n,c,hw,oc,stride,twice,shared", [
+    (2, 128, 28, 128, 1, True, True),        # 200 workgroups in the group
+    (4, 128, 28, 256, 2, False, True),
+    (4, 256, 14, 256, 1, True, True),        # 208
+    (8, 256, 14, 256, 1, True, False),       # 400: more than one to a compute unit
+    (8, 256, 14, 256, 1, False, True),       # 232
+    (2, 512, 7, 512, 1, True, False),        # the smallest tile over 512 channels
+    (3, 512, 7, 512, 1, True, True),         # 96
+    (10, 512, 7, 512, 1, True, True),        # 256
+    (12, 512, 7, 512, 1, True, False),       # 320
+])
+def test_which_layers_share_a_launch(n, c, hw, oc, stride, twice, shared, dev, monkeypatch):
+    """Two layers of one tensor, a 3x3 one and another or a 1x1 one beside it."""
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "0")
+    monkeypatch.setenv("CVM_HIP_SEQ", "0")
+    g = graphgen.GraphBuilder("share-%d-%d-%d" % (n, c, stride))
+    x = g.conv_relu_q(g.var("data", (n, 32, hw, hw), 8), c, 1)
+    a, b = g.conv_relu_q(x, oc, 3, stride, 1), g.conv_relu_q(x, oc, 3 if twice else 1, stride, 1 if twice else 0)
+    js, pb = g.build([g.concat([g.conv_relu_q(a, 32, 1), g.conv_relu_q(b, 32, 1)], 1)])
+    model = runtime.HipModel(js, pb)
+    data = synth.tensor("share", "x%d" % (n * c), (n, 32, hw, hw), -127, 127)
+    want = og.run_graph(js, graphgen.load_params(pb), data)[0].ravel()
+    for call in range(3):
+        got = np.frombuffer(model.inference(data.astype(np.int8).tobytes()), np.int8).astype(np.int32)
+        assert np.array_equal(got, want), call
+    lib().cvmhip_kernel_timing_begin()
+    model.run()
+    torch.cuda.synchronize()
+    buf = ctypes.create_string_buffer(1 << 16)
+    check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
+    assert sum("k_conv_run" in str(launch) for launch in json.loads(buf.value.decode())) == (0 if shared else 1 + twice)
+    model.close()
