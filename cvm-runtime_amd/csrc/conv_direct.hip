@@ -153,14 +153,11 @@ __global__ void __launch_bounds__(DIRECT_SPLIT * 64) k_conv_direct(const DirectA
 }
 
 // More tiles than the chip has places: a workgroup packs the filter rows of 32 * TM output channels into LDS once and then takes one
-// group of 128 pixels after another, 32 to a wavefront, with four chunks of activations in flight across the groups.
-// Bound by the int32 tensors (16 x 256 x 56 x 56 to 64 channels: 14.9 us for 64 MB) and by the chain in front of the first product: filter, packing, barrier.
-// Chunks in flight, us for 2 / 3 / 4 / 6: 256 -> 320 at 8 x 96 x 96 63.2 54.2 53.8 54.6, 64 -> 256 at 16 x 56 x 56 18.7 18.0 17.0 16.2, 200 -> 128 at
-// 8 x 33 x 33 9.6 8.9 8.8 9.0, small layers the same.  Filter rows of 96 to 256 channels a workgroup: 20 to 150 % slower (fewer wavefronts wait for more).
-constexpr int SLAB_AHEAD = 4;
-template <int TAPS, bool MASK, int TM>
+// group of 128 pixels after another, 32 to a wavefront, with D chunks of activations in flight across the groups.
+// Bound by the int32 tensors (16 x 256 x 56 x 56 to 64 channels: 15.0 us for 64 MB) and by the chain in front of the first product: filter, packing, barrier.
+// Filter rows of 96 to 256 channels a workgroup: 20 to 150 % slower (fewer wavefronts wait for more).
+template <int TAPS, bool MASK, int TM, int D>
 __global__ void __launch_bounds__(256) k_conv_slab(const DirectArgs a) {
-  constexpr int D = SLAB_AHEAD;
   extern __shared__ __attribute__((aligned(16))) v4i s_filter[];   // [m][chunk][lane]
   const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int xcd = blockIdx.x & 7, per = gridDim.x >> 3, extra = gridDim.x & 7;
@@ -256,14 +253,14 @@ __global__ void __launch_bounds__(256) k_conv_slab(const DirectArgs a) {
   }
 }
 
-// Which layers, us here against packing and product (the launch that is saved is 2-3 us of host time on top).
-// 1 x 1, k_conv_direct up to 448 tiles of 32 x 32 and K of 640: 256 -> 64 at 56 x 56 3.9 / 6.6, two images of it (392 tiles) 5.1 / 6.8, four
-// (784) 8.2 / 9.0; 512 -> 128 at 28 x 28 5.0 / 6.2; K = 1024 7.2 / 6.7.  k_conv_slab beyond that up to K = 256: 64 -> 256 at 56 x 56 4.6 / 6.6,
-// 16 images 17.0 / 20.2; 256 -> 64 14.9 / 19.2; 96 -> 160 at 4 x 75 x 75 9.8 / 12.7; 256 -> 320 at 8 x 96 x 96, two chunks in flight, 35.3 / 40.7; 256 -> 1024 at
-// 16 x 14 x 14 11.1 / 11.2; K = 512 9.8 / 7.0.  Two workgroups to a compute unit: one round of 528 took 11.7 where two of 264 take 10.5, and
-// three of 768 15.7 -> 19.2 (64 -> 256).
-// 3 x 3, k_conv_direct up to 256 tiles and K of 640: 64 -> 64 at 56 x 56 5.6 / 6.6; two images (392 tiles) 8.2 / 6.8; K = 1152 7.8-9.9 / 8.0.
-constexpr int DIRECT_TILES = 448, DIRECT_TILES_3X3 = 256, DIRECT_K = 640, SLAB_K = 256, SLAB_GROUPS = 512, SLAB_FEW = 264, SLAB_HALF_EMPTY = 800;
+// Which layers, us here against packing and product (the launch that is saved is 2-3 us of host time on top).  All figures on these kernels are us of a layer in a
+// replayed graph, with four sets of operands in turn.
+// 1 x 1, k_conv_direct up to 448 tiles of 32 x 32 and K of 640: 256 -> 64 at 56 x 56 4.2 / 6.9, two images of it (392 tiles) 5.6 / 7.9, four
+// (784) 8.9 / 9.8; 512 -> 128 at 28 x 28 5.3 / 6.5; K = 1024 9.5 / 7.0.  k_conv_slab beyond that up to K = 256: 64 -> 256 at 56 x 56 4.5 / 7.0,
+// 16 images 16.5 / 19.0; 256 -> 64, four images 7.1 / 9.8, 16 15.0 / 20.4; 96 -> 160 at 4 x 75 x 75 9.5 / 13.3; 256 -> 320 at 8 x 96 x 96 53.0 / 52.5; 256 -> 1024 at
+// 16 x 14 x 14 12.4 / 11.7, 256 -> 256 at 8 x 28 x 28 9.2 / 9.4; K = 512 at 4 x 28 x 28 9.6 / 7.9, 16 images 13.8 / 13.2.
+// 3 x 3, k_conv_direct up to 256 tiles and K of 640: 64 -> 64 at 56 x 56 5.7 / 7.0; two images (392 tiles) 8.2 / 7.2; K = 1152 at 28 x 28 7.9 / 8.3.
+constexpr int DIRECT_TILES = 448, DIRECT_TILES_3X3 = 256, DIRECT_K = 640, SLAB_K = 256, SLAB_GROUPS = 512;
 
 static bool conv_direct(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y, int n, int ic, int h, int wd, int oc, int oh, int ow, int kh,
                  int kw, int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w, hipStream_t s, int* rc) {
@@ -310,20 +307,36 @@ static bool conv_direct(const int32_t* x, const int32_t* w, const int32_t* bias,
     else if (mask) k_conv_direct<9, true><<<blocks, DIRECT_SPLIT * 64, 0, s>>>(a);
     else k_conv_direct<9, false><<<blocks, DIRECT_SPLIT * 64, 0, s>>>(a);
   } else {
-    // 32 channels to a workgroup where 64 would leave half of the places empty, or half of the last 64 is past the layer's end and there are two rounds.  us with 64
-    // and 32: 64 -> 256 at 56 x 56 (100 workgroups of 64) 5.5 4.6, 200 -> 64 at 96 x 96 (72) 7.9 6.2, 128 -> 160 at 4 x 40 x 40 (150) 6.5 5.5, 96 -> 160 at 2 x 75 x 75
-    // (264) 7.4 6.8, 64 -> 256 at 3 x 56 x 56 (296) 7.2 7.3, 96 -> 320 at 90 x 90 (320) 8.3 8.9, 64 -> 256 at 16 x 28 x 28 (392) 7.8 8.1; the last 64 half
-    // empty: 96 -> 160 at 4 x 75 x 75 (528) 10.9 9.8, at 6 (792) 12.3 11.9, 64 -> 160 at 8 x 96 x 96 (1 728) 18.9 21.0; 128 -> 32 at 8 x 75 x 75 10.2 9.1.
-    const int64_t groups = (pixels + 127) / 128, wide = groups * ((oc + 63) / 64), past = oc % 64;
-    const int tm = oc <= 32 || wide <= SLAB_FEW || (past > 0 && past <= 32 && wide > SLAB_GROUPS && wide <= SLAB_HALF_EMPTY) ? 1 : 2;
+    // The chip holds two workgroups to a compute unit at once; more take their groups in rounds (one round of 528 took 11.7 where two of 264 take 10.5).
+    // 32 channels to a workgroup, not 64, where these are no more rounds (one: more wavefronts share the wait; more: less of the last 64 channels is past the layer's
+    // end), or one more where there are several and a group is at most three chunks.  us with 64 and 32, two chunks in flight (workgroups):
+    //   64 -> 256 at 56 x 56 (100, 200) 5.4 4.5, 200 -> 64 at 96 x 96 (72, 144) 8.9 7.1, 96 -> 160 at 2 x 75 x 75 (264, 440) 7.4 6.5, 128 -> 64 at 6 x 75 x 75 (264, 528) 9.7 10.3;
+    //   96 -> 160 at 4 x 75 x 75 (528, 880) 10.6 9.8, 128 -> 96 at 5 x 91 x 91 (648, 972) 12.7 11.1, 107 -> 269 at 5 x 59 x 59 (680, 1224) 12.9 13.4, 184 -> 205 at 3 x 87 x 87 (712,
+    //   1246) 15.2 16.2; four chunks in flight: 64 -> 96 at 8 x 91 x 91 (1036, 1554) 13.0 12.1, 148 -> 277 at 8 x 64 x 64 (1280, 2304) 16.5 17.7
+    // Four chunks in flight, not two, where a compute unit has one workgroup, or in several rounds where three or more workgroups read the same pixels: elsewhere the
+    // filter waits behind the activations, and memory is what bounds.  us with two and four:
+    //   256 -> 64 at 4 x 56 x 56 (196) 8.1 7.2, 200 -> 64 at 96 x 96 (144) 7.1 6.2, 64 -> 256 at 56 x 56 (200) 4.5 4.5
+    //   256 -> 64 at 12 x 56 x 56 (294) 12.8 13.6, 128 -> 64 at 9 x 75 x 75 (396) 10.6 11.4, 128 -> 512 at 8 x 28 x 28 (392) 9.0 9.2, 96 -> 160 at 2 x 75 x 75 (440) 6.5 6.7
+    //   128 -> 64 at 12 x 75 x 75 (528) 13.9 14.9, 200 -> 64 at 13 x 75 x 75 (572) 24.8 25.8, 128 -> 96 at 10 x 91 x 91 (1294) 24.0 24.3
+    //   233 -> 214 at 5 x 88 x 88 (1212) 28.9 24.9, 148 -> 277 at 8 x 64 x 64 (1280) 18.0 16.5, 64 -> 256 at 16 x 56 x 56 (1568) 19.6 17.2, 128 -> 512 at 12 x 28 x 28 (592) 12.3 11.9
+    // (six chunks in flight: as four; of 228 layers one is slower with what the rule takes, 91 -> 206 at 8 x 61 x 61 (932) 12.3 12.7)
+    const int64_t groups = (pixels + 127) / 128;
+    auto rounds_of = [&](int tm) { return (groups * ((oc + 32 * tm - 1) / (32 * tm)) + SLAB_GROUPS - 1) / SLAB_GROUPS; };
+    const int tm = rounds_of(1) <= rounds_of(2) + (a.chunks <= 3 && rounds_of(2) > 1 ? 1 : 0) ? 1 : 2;
     a.octiles = (oc + 32 * tm - 1) / (32 * tm);
-    const int64_t rounds = (groups * a.octiles + SLAB_GROUPS - 1) / SLAB_GROUPS;
+    const int64_t rounds = rounds_of(tm), total = groups * a.octiles;
+    const bool deep = total <= SLAB_GROUPS / 2 || (a.octiles >= 3 && total > SLAB_GROUPS);
     const unsigned blocks = (unsigned)((groups + rounds - 1) / rounds * a.octiles);
     const size_t lds = (size_t)tm * a.chunks * 1024;
-    if (mask && tm == 1) k_conv_slab<1, true, 1><<<blocks, 256, lds, s>>>(a);
-    else if (mask) k_conv_slab<1, true, 2><<<blocks, 256, lds, s>>>(a);
-    else if (tm == 1) k_conv_slab<1, false, 1><<<blocks, 256, lds, s>>>(a);
-    else k_conv_slab<1, false, 2><<<blocks, 256, lds, s>>>(a);
+#define SLAB_CASE(MASK, TM, D) k_conv_slab<1, MASK, TM, D><<<blocks, 256, lds, s>>>(a)
+    if (mask) {
+      if (tm == 1) { if (deep) SLAB_CASE(true, 1, 4); else SLAB_CASE(true, 1, 2); }
+      else if (deep) SLAB_CASE(true, 2, 4);
+      else SLAB_CASE(true, 2, 2);
+    } else if (tm == 1) { if (deep) SLAB_CASE(false, 1, 4); else SLAB_CASE(false, 1, 2); }
+    else if (deep) SLAB_CASE(false, 2, 4);
+    else SLAB_CASE(false, 2, 2);
+#undef SLAB_CASE
   }
   *rc = check_launch("conv_direct");
   return true;

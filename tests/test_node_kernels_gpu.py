@@ -193,3 +193,19 @@ def test_conv_slab_widths(n, c, h, w, oc, stride, padding, dev):
     for bias in (None, b):
         got = hipops.conv2d(T(x, dev), T(wt, dev), None if bias is None else T(b, dev), stride, padding).cpu().numpy()
         assert np.array_equal(got, oracle.conv2d(x, wt, bias, stride, padding))
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,padding", [
+    (6, 24, 75, 75, 64, (0, 0)),        # 64 channels and two chunks in flight: one chunk a group, one round
+    (10, 112, 86, 80, 64, (0, 0)),      # four chunks, two rounds
+    (6, 100, 74, 75, 60, (1, 0)),       # with a border
+    (10, 48, 86, 80, 64, (0, 0)),       # 32 channels and two in flight, in rounds
+    (2, 256, 60, 60, 96, (1, 1)),       # 32 and four, with a border
+])
+def test_conv_slab_chunks_in_flight(n, c, h, w, oc, padding, dev):
+    cid = "slab-%d-%d-%d-%d" % (c, h, w, oc)
+    x = synth.tensor(cid, "x", (n, c, h, w), -300, 300)
+    wt = synth.tensor(cid, "w", (oc, c, 1, 1), -300, 300)
+    b = synth.tensor(cid, "b", (oc,), -2 ** 31, 2 ** 31 - 1)
+    got = hipops.conv2d(T(x, dev), T(wt, dev), T(b, dev), (1, 1), padding).cpu().numpy()
+    assert np.array_equal(got, oracle.conv2d(x, wt, b, (1, 1), padding))
