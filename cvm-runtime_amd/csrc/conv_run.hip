@@ -185,8 +185,25 @@ static int run_length(const RunArgs& a, bool pool, int units) {   // (32 bits: t
   return most + (pool ? 3 : 2) * (a.W + 1) + 1;
 }
 
+// Layers for which k_conv_wave, whose workgroups are larger, is ahead.  What a workgroup here fetches of each input channel, the run once for every wavefront
+// that shares the channel and the filter, goes through its L1; us with k_conv_wave / here, output pixels and these bytes (2 200 layers drawn: 183 were slower here; of 1 500 others that it still takes 31 are, 12 by more than 5 %):
+//   384, 640, 896 channels (several shares in turn, four wavefronts to each): 384 at 3 x 41 x 41 to 128 stride 2 (1 323, 1 196) 7.0 / 9.4, 896 at 37 x 37 to 64 (1 369, 576) 9.4 / 11.1, at 2 x 26 x 38
+//   to 64 stride 2 (494, 732) 9.7 / 11.9, at 2 x 40 x 40 to 192 stride 2 (800, 1 188) 14.5 / 17.0; below: 384 at 30 x 30 to 256 (900, 664) 7.4 / 6.5, at 12 x 15 x 15 to 256 stride 2 (768, 836) 9.2 / 7.8
+//   256 and 768 (two): 256 at 16 x 25 x 25 to 128 stride 2 (2 704, 886) 6.3 / 8.1, 768 at 39 x 45 to 192 (1 755, 600) 10.7 / 11.7; below: 256 at 12 x 13 x 13 to 128 (2 028, 408) 6.0 / 4.6, at
+//   45 x 45 to 128 in 32 x 32 tiles (2 025, 536) 6.0 / 5.2
+//   512 and its multiples, tiles of 64 pixels: 512 to 128 at 6 144 pixels 9.0 / 10.1, to 256 at 3 600 9.7 / 10.5, 1024 to 128 at 6 720 15.2 / 16.2; below: 512 to 512 at 1 849 10.3 / 10.0; long runs under
+//   16 x 32 tiles: 512 to 64 stride 2 at 1 352 (331) 7.5 / 8.3; with the pool in 32 x 64 tiles, 512 to 128 at 1 444 9.9 / 10.7, in 64 x 128 at 2 592 15.8 / 13.9
+static bool run_falls_behind(int c, int oc, int form, int ot, bool pool, const RunArgs& a) {
+  const int wavefronts = c % 512 == 0 ? 1 : c % 256 == 0 ? 2 : 4, bytes = wavefronts * a.run + 9 * 16 * ot;
+  if (pool) return c == 512 && form == 2 && a.units > 1000;
+  if (wavefronts == 1) return (form >= 3 && a.units > 4 * c) || (c == 512 && form == 1 && a.units > 1000 && bytes > 300);
+  if (wavefronts == 2) return a.units > 950 && bytes > (form == 2 && c == 256 ? 620 : 484);
+  return wavefronts == 4 && c > 128 && (a.units > 1200 || bytes > (oc <= 192 ? 600 : 950));
+}
+
 // Which form takes the layer, -1: none.  (g and ep as conv_prepare leaves them; fills `a`)
-// The smallest tile that makes one round of workgroups, one to a compute unit; us with k_conv_wave / here:
+// The smallest tile that makes one round of workgroups, one to a compute unit; us with k_conv_wave / here, one layer again and again in a replayed graph
+// with four sets of operands in turn (in a run of a model, by its events: 16 images at 7 x 7 8.1 / 6.8, at 14 x 14 with the pool 15.6 / 14.9):
 //   512 -> 512 at 7 x 7: 1 image 7.2 / 3.4, 3 7.7 / 4.2, 8 8.7 / 4.9, 16 8.9 / 6.1, 24 9.9 / 8.1, 32 9.9 / 8.8; 50, which would be 64 x 128, 14.0 / 14.0
 //   at 14 x 14: 1 8.4 / 4.4, 8 10.0 / 8.9, 16 (64 x 128) 14.5 / 14.6; with the pool 1 8.9 / 5.7, 8 10.3 / 8.9, 16 (64 x 128) 14.9 / 13.4; stride 2 1 7.4 / 3.7, 16 12.7 / 8.5
 //   256 channels (taps dealt to two): 1 x 7 x 7 5.8 / 3.5, 4 x 14 x 14 6.0 / 4.6, 8 x 14 x 14 (32 x 64) 6.2 / 5.8, 768 at 4 x 14 x 14 10.6 / 7.2
@@ -209,8 +226,7 @@ static int run_choose(const ConvGeom& g, const Epilogue& ep, RunArgs* a) {
     const int units = pool ? 4 * forms[f].nt : 16 * forms[f].nt;
     if ((int64_t)((a->units + units - 1) / units) * (g.OC / (16 * forms[f].ot)) > 256) continue;
     a->run = run_length(*a, pool, units);
-    if (a->run > RUN_PIXELS) return -1;
-    return f;
+    return a->run > RUN_PIXELS || run_falls_behind(g.Cp, g.OC, f, forms[f].ot, pool, *a) ? -1 : f;
   }
   return -1;
 }

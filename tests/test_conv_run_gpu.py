@@ -175,3 +175,21 @@ def test_which_layers_share_a_launch(n, c, hw, oc, stride, twice, shared, dev, m
     check(lib().cvmhip_kernel_timing_end_launches(buf, len(buf)))
     assert sum("k_conv_run" in str(launch) for launch in json.loads(buf.value.decode())) == (0 if shared else 1 + twice)
     model.close()
+
+
+@pytest.mark.parametrize("n,ic,h,w,oc,stride,pool,takes", [
+    (3, 384, 41, 41, 128, 2, False, False),     # 1 196 bytes of a channel to a workgroup
+    (1, 384, 36, 35, 512, 2, False, False),
+    (12, 384, 15, 15, 256, 2, False, True),     # 836, 768 pixels
+    (1, 896, 37, 37, 64, 1, False, False),      # 1 369 pixels
+    (16, 256, 25, 25, 128, 2, False, False),    # 2 704 pixels, 886 bytes
+    (1, 256, 45, 45, 128, 1, False, True),      # 536, in 32 x 32 tiles
+    (1, 768, 39, 45, 192, 1, False, False),
+    (32, 512, 8, 8, 256, 1, False, True),       # 2 048 pixels
+    (33, 512, 8, 8, 256, 1, False, False),
+    (4, 512, 36, 37, 64, 2, False, False),      # stride 2, long runs under small tiles
+    (3, 512, 38, 38, 128, 1, True, False),      # the pool's second largest tiles
+    (2, 512, 38, 38, 128, 1, True, True),
+])
+def test_where_the_kernel_before_is_ahead(n, ic, h, w, oc, stride, pool, takes, dev, monkeypatch):
+    test_tiles_and_lines(n, ic, h, w, oc, stride, pool, takes, dev, monkeypatch)
