@@ -1037,18 +1037,26 @@ const std::vector<const int32_t*>& HipGraphRuntime::InferI8(const int8_t* host, 
   return out_host_;
 }
 
-// An output is copied piece by piece, those of equal words are filled (a call of SSD-512, whose 590 KB are -1 but for the kept rows).
+// Pieces of equal words are filled (a call of SSD-512, whose 590 KB are -1 but for the kept rows), what lies between them is copied in runs of up to 256 KB: a longer
+// one goes past the caches (us a call whose output is of different words, one copy of the whole / copies of 4 KB / these: 544 KB 47.1 48.9 47.5, 765 KB 55.5 58.1
+// 56.4, 1 089 KB 80.5 76.5 71.9, 2 450 KB 156 137 130, 9 800 KB 551 471 454).
+constexpr size_t COPIED_AT_ONCE = 65536;   // words
 void HipGraphRuntime::CopyFetched(size_t k, int32_t* to) const {
   const size_t words = static_cast<size_t>(shape_size(shape_[entry_id(outputs_[k])]));
   const int32_t* from = out_host_[k];
   const uint64_t* table = out_in_pieces_ ? out_pieces_[k] : nullptr;
-  size_t at = 0;
+  size_t copied = 0;   // words that are in their place; others are copied up to the next piece that is filled
+  auto copy_to = [&](size_t end) {
+    for (size_t n; to != from && copied < end; copied += n) std::memcpy(to + copied, from + copied, (n = std::min(end - copied, COPIED_AT_ONCE)) * 4);
+  };
   if (table)
-    for (size_t c = 0; c < words / CVMHIP_EXPORT_PIECE; ++c, at += CVMHIP_EXPORT_PIECE) {
-      if (table[c] >> 32) std::fill_n(to + at, CVMHIP_EXPORT_PIECE, static_cast<int32_t>(table[c]));
-      else if (to != from) std::memcpy(to + at, from + at, CVMHIP_EXPORT_PIECE * 4);
+    for (size_t c = 0; c < words / CVMHIP_EXPORT_PIECE; ++c) {
+      if (!(table[c] >> 32)) continue;
+      copy_to(c * CVMHIP_EXPORT_PIECE);
+      std::fill_n(to + c * CVMHIP_EXPORT_PIECE, CVMHIP_EXPORT_PIECE, static_cast<int32_t>(table[c]));
+      copied = (c + 1) * CVMHIP_EXPORT_PIECE;
     }
-  if (to != from) std::memcpy(to + at, from + at, (words - at) * 4);
+  copy_to(words);
 }
 
 void HipGraphRuntime::CompleteFetched() {
