@@ -512,7 +512,7 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   }
   char desc[128] = "";
   if (kernel_timing_enabled())
-    snprintf(desc, sizeof(desc), "3x3/%d %d + 1x1 %d %s + 1x1 %d in %dx%dx%d out %dx%d tile %d grid %d", stride, m, 4 * m, projection ? "+ projection" : "+res", oc, n, h, w, oh, ow, 16 * f->nt, a.tiles);
+    snprintf(desc, sizeof(desc), "3x3/%d %d + 1x1 %d %s + 1x1 %d in %dx%dx%d out %dx%d tile %d grid %d + %d ahead", stride, m, 4 * m, projection ? "+ projection" : "+res", oc, n, h, w, oh, ow, 16 * f->nt, a.tiles, 8 * a.helpers);
   const double px = (double)a.P;
   const double cut = projection ? 4.0 * projection->c : 0.0;   // multiply-adds of the projection for a channel of m
   KernelTimer timer("k_conv_block", 2.0 * px * m * (9.0 * m + 4.0 * m + 4.0 * oc + cut), as_stream(stream),

@@ -452,7 +452,7 @@ void HipGraphRuntime::ReadHooks() {
                             "CVM_HIP_CONVGROUP", "CVM_HIP_FLATDENSE", "CVM_HIP_CONV", "CVM_HIP_WAVECFG", "CVM_HIP_TILE"})
     plain = plain && env(other).empty();
   hooks_.resident = hooks_.resident && plain;
-  hooks_.separable = plain && env("CVM_HIP_SEPARABLE") != "0";
+  hooks_.separable = env("CVM_HIP_SEPARABLE") == "1" || (plain && env("CVM_HIP_SEPARABLE") != "0");
   hooks_.fold_bias = env("CVM_HIP_FOLDBIAS") != "0";
   hooks_.graph = env("CVM_HIP_GRAPH") != "0";
   hooks_.seq = env("CVM_HIP_SEQ") != "0" && env("CVM_HIP_RESIDENT") != "1";

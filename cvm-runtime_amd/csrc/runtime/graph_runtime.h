@@ -295,7 +295,9 @@ class HipGraphRuntime {
     // prefer to them.  Off as well when another launch form is asked for by name
     // (any of the switches of the planner or of the kernel choice is set): those name forms of single layers.
     bool resident = true;
-    bool separable = true;    // CVM_HIP_SEPARABLE=0, or a switch as above: depthwise and 1x1 convolutions, and the first two of a VGG, stay two launches
+    // CVM_HIP_SEPARABLE=0, or a switch as above unless =1: what several layers share for being faster so has a launch each: depthwise and 1x1
+    // convolutions, the first two of a VGG, the bottlenecks of a ResNet
+    bool separable = true;
     bool flat_dense = true;   // CVM_HIP_FLATDENSE=0: a dense layer over a whole map gathers its operand from the map as it lies
     bool seq_chains = true;   // CVM_HIP_SEQ_CHAIN=0: no 1x1 layers chained behind the layer that feeds them (cvmhip_conv_seq_link)
     std::vector<std::pair<int, int>> seq_layer_cfg;   // CVM_HIP_SEQCFG: (layer of a sequence, configuration)

@@ -1,6 +1,7 @@
 """The 3x3 layer of a bottleneck, the 1x1 layer behind it with the residual and the next block's first layer in one launch, against the oracle
 running the graph node by node."""
 import ctypes
+import json
 
 import numpy as np
 import pytest
@@ -67,7 +68,7 @@ def _run(js, pb, data, monkeypatch, calls=3):
     (1, 64, 2, 3, 128, 2),
     (2, 64, 13, 9, 64, 1),           # tiles that span images and end in the last one
     (5, 64, 56, 56, 128, 1),         # tiles of 64 pixels, the last one whole
-    (2, 64, 127, 97, 64, 1),         # of 96
+    (2, 64, 127, 97, 64, 1),         # of 128
     (3, 64, 101, 113, 128, 1),       # of 128
     (9, 64, 113, 111, 64, 2),
     (1, 128, 7, 5, 256, 1),          # of 16
@@ -232,3 +233,124 @@ def test_longest_run_of_a_stride_2_layer():
         assert bool(_eligible(n=n, m=m, oc=m, h=h, w=w, stride=2)) == (lds <= 160 * 1024), (n, m, h, w)
         taken += lds <= 160 * 1024
     assert 100 < taken < 390
+
+
+def _launches(run):
+    """What the launches of `run` say of themselves"""
+    L = lib()
+    L.cvmhip_kernel_timing_begin()
+    run()
+    check(L.cvmhip_device_sync())
+    buf = ctypes.create_string_buffer(1 << 18)
+    check(L.cvmhip_kernel_timing_end_launches(buf, len(buf)))
+    return [str(v) for v in json.loads(buf.value.decode())]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,h,w,oc,tile,projected", [
+    (2, 64, 13, 9, 64, 32, 32), (2, 64, 13, 9, 128, 32, None),
+    (3, 64, 57, 61, 64, 64, 64), (3, 64, 57, 61, 128, 64, None),
+    (2, 64, 101, 99, 64, 96, 96), (2, 64, 101, 99, 128, 96, None),
+    (3, 64, 93, 91, 64, 128, 128), (3, 64, 93, 91, 128, 128, None),
+    (1, 128, 7, 5, 128, 16, 16), (1, 128, 7, 5, 256, 16, None),
+    (3, 128, 41, 37, 128, 32, 32), (3, 128, 41, 37, 256, 32, None),
+    (7, 128, 37, 37, 128, 48, 48), (7, 128, 37, 37, 256, 48, None),
+    (17, 128, 28, 28, 128, 64, 64), (17, 128, 28, 28, 256, 64, None),
+    (23, 128, 28, 29, 128, 80, 80), (23, 128, 28, 29, 256, 80, None),
+    (29, 128, 29, 28, 128, 96, 96), (29, 128, 29, 28, 256, 96, None),
+    (32, 128, 28, 28, 128, 64, 64), (32, 128, 28, 28, 256, 64, None),
+    (1, 256, 3, 14, 256, 16, 16), (1, 256, 3, 14, 512, 16, None),
+    (22, 256, 14, 15, 256, 32, 32), (22, 256, 14, 15, 512, 32, None),
+    (45, 256, 14, 14, 256, 48, 48), (45, 256, 14, 14, 512, 48, None),
+    (63, 256, 14, 14, 256, 64, 64), (63, 256, 14, 14, 512, 64, None),
+])
+def test_every_form(n, m, h, w, oc, tile, projected, dev):
+    """Each tile with each third layer, and with the projection (or without, where that leaves a smaller tile only)."""
+    said = [v for v in _launches(lambda: test_bottleneck_in_one_launch(n, m, h, w, oc, 1, dev)) if "k_conv_block" in v]
+    assert "tile %d " % tile in said[0] and "+res" in said[0], said
+    assert len(said) == 1 + (projected is not None), said
+    if projected:
+        assert "tile %d " % projected in said[1] and "+ projection" in said[1], said
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,oc,projects", [(128, 128, False), (128, 256, False), (128, 128, True), (256, 256, False), (256, 512, False), (256, 256, True)])
+@pytest.mark.parametrize("later_oc", [256, 512])
+def test_filters_of_the_next_launch(m, oc, projects, later_oc, dev):
+    """Idle compute units read the next launch's filters: the results are what they are without."""
+    import torch
+    n, h, w, gen = 2, 15, 13, torch.Generator(device=dev)
+    gen.manual_seed(m + oc)
+    c = 2 * m
+    rand = lambda *s: torch.randint(-128, 128, s, dtype=torch.int32, device=dev, generator=gen)
+    x, r, xs = hipops.pack_act_i8(rand(n, m, h, w)), hipops.pack_act_i8(rand(n, 4 * m, h, w)), hipops.pack_act_i8(rand(n, c, h, w))
+    wa, wb, wc, ws = (hipops.pack_weights(rand(*s)) for s in ((m, m, 3, 3), (4 * m, m, 1, 1), (oc, 4 * m, 1, 1), (4 * m, c, 1, 1)))
+    la, lb, lc = (hipops.pack_weights(rand(*s)) for s in ((256, 256, 3, 3), (1024, 256, 1, 1), (later_oc, 1024, 1, 1)))
+
+    class Filters(ctypes.Structure):
+        _fields_ = [(k, ctypes.c_void_p) for k in ("wa", "wb", "wc")] + [("m", ctypes.c_int), ("oc", ctypes.c_int)]
+    chains = [_clamp_shift(-(127 << s), 127 << s, s) for s in (12, 10, 1, 12, 10)]
+    ca, cb, cr, cc = (ctypes.byref(v) for v in chains[:4])
+    projection = ctypes.byref(Projection(xs.data_ptr(), ws.data_ptr(), None, ctypes.pointer(chains[4]), c)) if projects else None
+    outs = []
+    for ahead in (None, Filters(la.data_ptr(), lb.data_ptr(), lc.data_ptr(), 256, later_oc), Filters(None, lb.data_ptr(), None, 256, later_oc)):
+        out, nxt = hipops._act_buffer(n * h * w, 4 * m, dev), hipops._act_buffer(n * h * w, oc, dev)
+        vp = hipops._vp
+        said = _launches(lambda: check(lib().cvmhip_conv2d_bottleneck_i8(
+            vp(x), vp(wa), None, ca, vp(wb), None, cb, None if projects else vp(r), cr, vp(out), vp(wc), None, cc, vp(nxt), n, m, h, w, oc, 1,
+            projection, ctypes.byref(ahead) if ahead else None, hipops._conv_stream())))
+        assert "+ %d ahead" % (64 if ahead else 0) in said[-1], said
+        outs.append((hipops.unpack_act_i8(out, n, 4 * m, h, w), hipops.unpack_act_i8(nxt, n, oc, h, w)))
+    for a, b in outs[1:]:
+        assert torch.equal(a, outs[0][0]) and torch.equal(b, outs[0][1])
+
+
+@pytest.mark.gpu
+def test_several_blocks_of_a_graph(dev, monkeypatch):
+    """Blocks one behind the other, through a change of their width: every launch but the last knows the next one's filters."""
+    g, heads = graphgen.resnet50(2, blocks=(2, 2, 3, 1), size=96, classes=40, config_id="bottlenecks")
+    js, pb = g.build(heads)
+    monkeypatch.setenv("CVM_HIP_RESIDENT", "1")
+    m = runtime.HipModel(js, pb)
+    for call in range(3):
+        data = synth.tensor("bottlenecks", "data%d" % call, (2, 3, 96, 96), -127, 127)
+        want = og.run_graph(js, graphgen.load_params(pb), data)[0].ravel()
+        assert np.array_equal(np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int32), want), call
+    said = [v for v in _launches(m.run) if "k_conv_block" in v]
+    assert len(said) >= 6 and sum("+ 64 ahead" in v for v in said) >= 3, said
+    m.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spin", ["", "0"])   # "0": every wait of the sequence gives up, and the run is repeated without it
+def test_beside_a_sequence(spin, dev, monkeypatch):
+    """The block's projection is too large for a layer sequence, which begins behind it: with sequences the projection is a launch of its own, without
+    them (another such model is loaded, or the sequence gave up) all four layers are one."""
+    js, pb = _net(66, 256, 14, 14, 256, 1, projects=True)
+    inputs = [synth.tensor("bottleneck", "seq%d" % k, (66, 32, 14, 14), -128, 127).astype(np.int8) for k in range(3)]
+    monkeypatch.setenv("CVM_HIP_SEPARABLE", "0")
+    monkeypatch.setenv("CVM_HIP_SEQ", "0")
+    m = runtime.HipModel(js, pb)
+    wants = [m.inference(x.tobytes()) for x in inputs]
+    m.close()
+    monkeypatch.setenv("CVM_HIP_SEQ", "1")
+    monkeypatch.setenv("CVM_HIP_SEPARABLE", "1")
+    if spin:
+        monkeypatch.setenv("CVM_HIP_SEQ_SPIN", spin)
+    m = runtime.HipModel(js, pb)
+    counts = [m.launch_counts()]
+    assert counts[0][1] == 1 and counts[0][2] >= 3
+    for k in range(4):
+        assert m.inference(inputs[k % 3].tobytes()) == wants[k % 3], k
+    if spin:
+        assert m.launch_counts()[1] == 0
+    else:
+        assert not any("k_conv_block" in v for v in _launches(m.run))
+        other = runtime.HipModel(js, pb)
+        for k in range(4):
+            assert m.inference(inputs[k % 3].tobytes()) == wants[k % 3], k
+        assert any("+ projection" in v for v in _launches(m.run))
+        other.close()
+        for k in range(4):
+            assert m.inference(inputs[k % 3].tobytes()) == wants[k % 3], k
+    m.close()
