@@ -254,13 +254,44 @@ __global__ void __launch_bounds__(256) k_conv_slab(const DirectArgs a) {
 }
 
 // Which layers, us here against packing and product (the launch that is saved is 2-3 us of host time on top).  All figures on these kernels are us of a layer in a
-// replayed graph, with four sets of operands in turn.
+// replayed graph, with four sets of operands in turn where nothing else is said.
 // 1 x 1, k_conv_direct up to 448 tiles of 32 x 32 and K of 640: 256 -> 64 at 56 x 56 4.2 / 6.9, two images of it (392 tiles) 5.6 / 7.9, four
 // (784) 8.9 / 9.8; 512 -> 128 at 28 x 28 5.3 / 6.5; K = 1024 9.5 / 7.0.  k_conv_slab beyond that up to K = 256: 64 -> 256 at 56 x 56 4.5 / 7.0,
 // 16 images 16.5 / 19.0; 256 -> 64, four images 7.1 / 9.8, 16 15.0 / 20.4; 96 -> 160 at 4 x 75 x 75 9.5 / 13.3; 256 -> 320 at 8 x 96 x 96 53.0 / 52.5; 256 -> 1024 at
 // 16 x 14 x 14 12.4 / 11.7, 256 -> 256 at 8 x 28 x 28 9.2 / 9.4; K = 512 at 4 x 28 x 28 9.6 / 7.9, 16 images 13.8 / 13.2.
 // 3 x 3, k_conv_direct up to 256 tiles and K of 640: 64 -> 64 at 56 x 56 5.7 / 7.0; two images (392 tiles) 8.2 / 7.2; K = 1152 at 28 x 28 7.9 / 8.3.
 constexpr int DIRECT_TILES = 448, DIRECT_TILES_3X3 = 256, DIRECT_K = 640, SLAB_K = 256, SLAB_GROUPS = 512;
+
+// The chip holds two workgroups of k_conv_slab to a compute unit at once; more take their groups in rounds (one round of 528 took 11.7 where two of 264 take 10.5).
+static int64_t slab_rounds(int64_t groups, int oc, int tm) { return (groups * ((oc + 32 * tm - 1) / (32 * tm)) + SLAB_GROUPS - 1) / SLAB_GROUPS; }
+
+// 32 channels to a workgroup, not 64, where these are no more rounds (one: more wavefronts share the wait; more: less of the last 64 channels is past the layer's end).
+// us with 64 and 32, two chunks in flight (workgroups); here and below with four sets of operands in turn | with sets of 700 MB:
+//   64 -> 256 at 56 x 56 (100, 200) 5.4 4.5, 200 -> 64 at 96 x 96 (72, 144) 8.9 7.1, 96 -> 160 at 2 x 75 x 75 (264, 440) 7.4 6.5 | 8.4 8.1, 128 -> 64 at 6 x 75 x 75 (264, 528) 9.7 10.3;
+//   96 -> 160 at 4 x 75 x 75 (528, 880) 10.6 9.8 | 12.4 12.0, 128 -> 96 at 5 x 91 x 91 (648, 972) 12.7 11.1; a round more: 107 -> 269 at 5 x 59 x 59 (680, 1224) 12.9 13.4, 184 -> 205 at 3 x 87 x 87 (712,
+//   1246) 15.2 16.2, 96 -> 160 at 6 x 75 x 75 (792, 1320) 11.9 11.6 | 15.0 16.3, 64 -> 64 at 12 x 75 x 75 (528, 1056) 11.7 10.6 | 14.1 14.8; but with few channels, half of the last 64 past the end and
+//   two rounds half empty 48 -> 200 at 5 x 70 x 70 (768, 1344) 10.8 10.1 | 12.7 12.2, 46 -> 202 at 6 x 59 x 59 (656, 1148) 10.9 10.2 | 12.5 12.1, 80 -> 224 at 9 x 48 x 48 (648, 1134) 11.0 10.6
+static bool slab_narrow(int64_t groups, int ic, int oc) {
+  const int64_t wide = groups * ((oc + 63) / 64);
+  const bool half = oc % 64 > 0 && oc % 64 <= 32 && wide > SLAB_GROUPS && wide <= 800 && ic <= 80;
+  return slab_rounds(groups, oc, 1) <= slab_rounds(groups, oc, 2) + (half ? 1 : 0);
+}
+
+// Four chunks of activations in flight, not two (six: as four).  us with two and four, by how many workgroups there are and how many of them read the same pixels:
+//   at most one to a compute unit: 256 -> 64 at 4 x 56 x 56 (196) 8.1 7.2 | 11.8 8.2, 200 -> 64 at 96 x 96 (144) 7.1 6.2
+//   one round, one to its pixels: 128 -> 64 at 9 x 75 x 75 (396) 10.6 11.4 | 13.5 14.6, 200 -> 64 at 7 x 75 x 75 (308) 12.5 13.4 | 16.1 17.3, 256 -> 64 at 12 x 56 x 56 (294) 12.8 13.6 | 16.3 16.8;
+//     only 256 -> 64 at 16 x 56 x 56 (392) 15.0 15.0 | 18.4 17.9, at 20 (490) | 20.2 19.7
+//   one round, several: 256 -> 128 at 8 x 56 x 56 (392) | 15.4 15.0, 240 -> 182 at 77 x 77 (282) 8.8 9.0 | 10.8 10.0, 194 -> 133 at 7 x 52 x 52 (444) | 13.4 12.8; few channels 128 -> 64 at
+//     5 x 75 x 75 (440) 7.8 8.1, 96 -> 160 at 2 x 75 x 75 (440) 6.5 6.7 | 8.1 8.3, 77 -> 156 at 2 x 94 x 94 (417) 8.4 8.8 | 10.0 10.3
+//   rounds, one or two: 128 -> 64 at 12 x 75 x 75 (528) 13.9 14.9 | 19.8 20.0, 256 -> 64 at 24 x 56 x 56 (588) 25.9 27.4 | 25.9 27.4, 200 -> 64 at 16 x 91 x 91 (1036) 40.1 41.2 | 40.2 41.3;
+//     96 -> 64 at 12 x 96 x 96 (864) 17.8 16.9 | 18.6 18.2, 64 -> 128 at 10 x 96 x 96 (1440) 20.4 18.6 | 19.7 18.9, 128 -> 96 at 10 x 91 x 91 (1294) 24.0 24.3 | 23.3 23.8
+//   rounds, three or more: 233 -> 214 at 5 x 88 x 88 (1212) 28.9 24.9, 148 -> 277 at 8 x 64 x 64 (1280) 18.0 16.5, 64 -> 256 at 16 x 56 x 56 (1568) 19.6 17.2 | 22.7 20.8
+static bool slab_deep(int64_t workgroups, int octiles, int chunks) {
+  if (workgroups <= SLAB_GROUPS / 2) return true;
+  if (octiles >= 3) return workgroups > SLAB_GROUPS || chunks >= 5;
+  if (octiles == 2) return workgroups > 800 || chunks >= 5;
+  return workgroups > 800 ? chunks <= 4 : workgroups > 320 && workgroups <= SLAB_GROUPS && chunks >= 8;
+}
 
 static bool conv_direct(const int32_t* x, const int32_t* w, const int32_t* bias, int32_t* y, int n, int ic, int h, int wd, int oc, int oh, int ow, int kh,
                  int kw, int stride_h, int stride_w, int pad_h, int pad_w, int dil_h, int dil_w, hipStream_t s, int* rc) {
@@ -307,25 +338,11 @@ static bool conv_direct(const int32_t* x, const int32_t* w, const int32_t* bias,
     else if (mask) k_conv_direct<9, true><<<blocks, DIRECT_SPLIT * 64, 0, s>>>(a);
     else k_conv_direct<9, false><<<blocks, DIRECT_SPLIT * 64, 0, s>>>(a);
   } else {
-    // The chip holds two workgroups to a compute unit at once; more take their groups in rounds (one round of 528 took 11.7 where two of 264 take 10.5).
-    // 32 channels to a workgroup, not 64, where these are no more rounds (one: more wavefronts share the wait; more: less of the last 64 channels is past the layer's
-    // end), or one more where there are several and a group is at most three chunks.  us with 64 and 32, two chunks in flight (workgroups):
-    //   64 -> 256 at 56 x 56 (100, 200) 5.4 4.5, 200 -> 64 at 96 x 96 (72, 144) 8.9 7.1, 96 -> 160 at 2 x 75 x 75 (264, 440) 7.4 6.5, 128 -> 64 at 6 x 75 x 75 (264, 528) 9.7 10.3;
-    //   96 -> 160 at 4 x 75 x 75 (528, 880) 10.6 9.8, 128 -> 96 at 5 x 91 x 91 (648, 972) 12.7 11.1, 107 -> 269 at 5 x 59 x 59 (680, 1224) 12.9 13.4, 184 -> 205 at 3 x 87 x 87 (712,
-    //   1246) 15.2 16.2; four chunks in flight: 64 -> 96 at 8 x 91 x 91 (1036, 1554) 13.0 12.1, 148 -> 277 at 8 x 64 x 64 (1280, 2304) 16.5 17.7
-    // Four chunks in flight, not two, where a compute unit has one workgroup, or in several rounds where three or more workgroups read the same pixels: elsewhere the
-    // filter waits behind the activations, and memory is what bounds.  us with two and four:
-    //   256 -> 64 at 4 x 56 x 56 (196) 8.1 7.2, 200 -> 64 at 96 x 96 (144) 7.1 6.2, 64 -> 256 at 56 x 56 (200) 4.5 4.5
-    //   256 -> 64 at 12 x 56 x 56 (294) 12.8 13.6, 128 -> 64 at 9 x 75 x 75 (396) 10.6 11.4, 128 -> 512 at 8 x 28 x 28 (392) 9.0 9.2, 96 -> 160 at 2 x 75 x 75 (440) 6.5 6.7
-    //   128 -> 64 at 12 x 75 x 75 (528) 13.9 14.9, 200 -> 64 at 13 x 75 x 75 (572) 24.8 25.8, 128 -> 96 at 10 x 91 x 91 (1294) 24.0 24.3
-    //   233 -> 214 at 5 x 88 x 88 (1212) 28.9 24.9, 148 -> 277 at 8 x 64 x 64 (1280) 18.0 16.5, 64 -> 256 at 16 x 56 x 56 (1568) 19.6 17.2, 128 -> 512 at 12 x 28 x 28 (592) 12.3 11.9
-    // (six chunks in flight: as four; of 228 layers one is slower with what the rule takes, 91 -> 206 at 8 x 61 x 61 (932) 12.3 12.7)
     const int64_t groups = (pixels + 127) / 128;
-    auto rounds_of = [&](int tm) { return (groups * ((oc + 32 * tm - 1) / (32 * tm)) + SLAB_GROUPS - 1) / SLAB_GROUPS; };
-    const int tm = rounds_of(1) <= rounds_of(2) + (a.chunks <= 3 && rounds_of(2) > 1 ? 1 : 0) ? 1 : 2;
+    const int tm = slab_narrow(groups, ic, oc) ? 1 : 2;
     a.octiles = (oc + 32 * tm - 1) / (32 * tm);
-    const int64_t rounds = rounds_of(tm), total = groups * a.octiles;
-    const bool deep = total <= SLAB_GROUPS / 2 || (a.octiles >= 3 && total > SLAB_GROUPS);
+    const int64_t rounds = slab_rounds(groups, oc, tm);
+    const bool deep = slab_deep(groups * a.octiles, a.octiles, a.chunks);
     const unsigned blocks = (unsigned)((groups + rounds - 1) / rounds * a.octiles);
     const size_t lds = (size_t)tm * a.chunks * 1024;
 #define SLAB_CASE(MASK, TM, D) k_conv_slab<1, MASK, TM, D><<<blocks, 256, lds, s>>>(a)

@@ -859,7 +859,9 @@ void HipGraphRuntime::RunStemConv(size_t step) {
 }
 
 // The 3x3 layer of a bottleneck, the 1x1 layer behind it with the residual and the first layer of the next block become one launch where no
-// layer sequence runs (Launch() takes a sequence launch first where both exist).
+// layer sequence runs (Launch() takes a sequence launch first where both exist).  Every such block is taken; us a run of ResNet-50 with one launch per
+// layer / bottleneck launches but for 256 channels / all of them: 1 image 216 170 176, 2 232 174 178, 4 269 199 196, 8 310 235 220, 16 372 296 261, 32 536 458 391,
+// 50 774 653 559; 3 of 195 x 195 (32 tiles of 256 channels) 245 189 186.
 void HipGraphRuntime::BuildBottlenecks() {
   if (!hooks_.separable) return;
   auto plain = [&](size_t k) {

@@ -199,7 +199,9 @@ def test_conv_slab_widths(n, c, h, w, oc, stride, padding, dev):
     (6, 24, 75, 75, 64, (0, 0)),        # 64 channels and two chunks in flight: one chunk a group, one round
     (10, 112, 86, 80, 64, (0, 0)),      # four chunks, two rounds
     (6, 100, 74, 75, 60, (1, 0)),       # with a border
-    (10, 48, 86, 80, 64, (0, 0)),       # 32 channels and two in flight, in rounds
+    (10, 48, 86, 80, 32, (0, 0)),       # 32 channels and two in flight, in rounds
+    (5, 48, 70, 70, 200, (0, 0)),       # 32 and four, a round more than with 64
+    (12, 50, 96, 96, 64, (0, 0)),       # 64 and four, one workgroup to its pixels
     (2, 256, 60, 60, 96, (1, 1)),       # 32 and four, with a border
 ])
 def test_conv_slab_chunks_in_flight(n, c, h, w, oc, padding, dev):
