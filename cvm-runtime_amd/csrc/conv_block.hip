@@ -456,6 +456,24 @@ int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, c
   return f && (!projection || f->nt == block_choose(n, m, h, w, oc, stride, false, &run)->nt);
 }
 
+// us here / the layers in launches of their own, alone in a replayed graph with four sets of tensors in turn:
+//   M = 256 of few pixels, where k_conv_run has the 3x3 layer and this launch 13 to 28 workgroups, each with all filters through its L1: 256 -> 256 at 8 x 8 13.6 / 11.1, 14 x 14 13.6 / 11.0, with the
+//   projection 18.9 / 15.1, 512 out at 20 x 20 (400 pixels) 16.1 / 12.6; in a run of ResNet-50 (us with these blocks here / apart) 1 image 175.6 / 170.0, 2 (392 pixels) 178.3 / 174.2, 3 of
+//   195 x 195 (507) 185.6 / 188.9, 4 (784) 196.0 / 199.4
+//   Rows so long that LDS holds the run under a small tile only: M = 256, one 16-pixel tile where there would be two, 224 x 224 to 512 stride 2 58 / 44, 235 x 235 184 / 104, at best
+//   138 x 138 stride 2 26 / 27; otherwise several rounds of tiles whose runs are many times as long: M = 64 at 702 x 702 stride 2 (68 pixels of a run to one of the tile) 69 / 42, 684 x 684 (34)
+//   42.9 / 42.1, 654 x 654 with the projection (32.7) 40.6 / 52.6; M = 128 at 340 x 340 stride 2 (66) 50 / 36, 386 x 308 with the projection (31) 32 / 44, 328 x 516 stride 1 (33) 154 / 107, 326 x 454 (20) 116 / 101, 331 x 331 (11.4) 72.7 / 71.7,
+//   319 x 319 (11.0) 63 / 69; M = 256 at 160 x 160 to 512 (11.1) 72 / 66
+// Of 1 200 blocks drawn this keeps 126 apart, 91 of which were slower here than before there was this launch; of the others 2 are (2 %).
+int cvmhip_bottleneck_gains(int n, int m, int h, int w, int oc, int stride, const cvmhip_bottleneck_projection* projection) {
+  int run;
+  const BlockForm* f = block_choose(n, m, h, w, oc, stride, projection != nullptr, &run);
+  if (!f) return 0;
+  const int64_t p = (int64_t)n * ((h - 1) / stride + 1) * ((w - 1) / stride + 1), round = (int64_t)BLOCK_UNITS * 16 * f->nt;
+  if (m == 256 && (p <= 448 || (f->nt == 1 && p > round))) return 0;
+  return p <= 3 * round || run <= (stride == 1 ? 11 : 33) * 16 * f->nt;
+}
+
 int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* bias_a, const cvmhip_chain* chain_a, const void* wb,
                                 const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual, const cvmhip_chain* chain_r, void* out,
                                 const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next, int n, int m, int h, int w, int oc,

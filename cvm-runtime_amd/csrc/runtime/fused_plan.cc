@@ -859,9 +859,8 @@ void HipGraphRuntime::RunStemConv(size_t step) {
 }
 
 // The 3x3 layer of a bottleneck, the 1x1 layer behind it with the residual and the first layer of the next block become one launch where no
-// layer sequence runs (Launch() takes a sequence launch first where both exist).  Every such block is taken; us a run of ResNet-50 with one launch per
-// layer / bottleneck launches but for 256 channels / all of them: 1 image 216 170 176, 2 232 174 178, 4 269 199 196, 8 310 235 220, 16 372 296 261, 32 536 458 391,
-// 50 774 653 559; 3 of 195 x 195 (32 tiles of 256 channels) 245 189 186.
+// layer sequence runs (Launch() takes a sequence launch first where both exist).  us a run of ResNet-50 with one launch per layer /
+// bottleneck launches but for 256 channels / all of them: 1 image 216 170 176, 2 232 174 178, 4 269 199 196, 8 310 235 220, 16 372 296 261, 32 536 458 391, 50 774 653 559.
 void HipGraphRuntime::BuildBottlenecks() {
   if (!hooks_.separable) return;
   auto plain = [&](size_t k) {
@@ -883,7 +882,8 @@ void HipGraphRuntime::BuildBottlenecks() {
     };
     auto aligned = [](const PlanStep& st) { return (reinterpret_cast<uintptr_t>(st.bias) & 15) == 0; };
     if (!aligned(p) || !aligned(q) || !aligned(r) || !read_by_next_only(i, i + 1) ||
-        !cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain, nullptr))
+        !cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain, nullptr) ||
+        !cvmhip_bottleneck_gains(p.n, p.c, p.h, p.w, r.oc, p.sh, nullptr))
       continue;
     // the residual's own 1x1 layer in front of them
     bool projects = false;
@@ -892,7 +892,8 @@ void HipGraphRuntime::BuildBottlenecks() {
       const cvmhip_bottleneck_projection projection = {nullptr, nullptr, nullptr, &s.chain, s.c};
       projects = s.dst == q.src2 && s.src2 == kNone && s.kh == 1 && s.kw == 1 && s.sh == p.sh && s.ph == 0 && s.pw == 0 && s.h == p.h && s.w == p.w &&
                  s.oc == q.oc && aligned(s) && read_by_next_only(i - 1, i + 1) &&
-                 cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain, &projection);
+                 cvmhip_bottleneck_eligible(p.n, p.c, p.h, p.w, r.oc, p.sh, &p.chain, &q.chain, &q.chain2, &r.chain, &projection) &&
+                 cvmhip_bottleneck_gains(p.n, p.c, p.h, p.w, r.oc, p.sh, &projection);
     }
     PlanStep& head = plan_[projects ? i - 1 : i];
     head.bottleneck = projects ? 4 : 3;

@@ -541,6 +541,8 @@ typedef struct cvmhip_bottleneck_filters {   /* of a later such launch: idle com
 } cvmhip_bottleneck_filters;
 int cvmhip_bottleneck_eligible(int n, int m, int h, int w, int oc, int stride, const cvmhip_chain* chain_a, const cvmhip_chain* chain_b,
                                const cvmhip_chain* chain_r, const cvmhip_chain* chain_c, const cvmhip_bottleneck_projection* projection /* or NULL */);
+/* For sizes that are eligible: whether the launch is the faster form (few pixels, and rows too long for LDS, are better apart). */
+int cvmhip_bottleneck_gains(int n, int m, int h, int w, int oc, int stride, const cvmhip_bottleneck_projection* projection /* or NULL */);
 int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* bias_a, const cvmhip_chain* chain_a, const void* wb,
                                 const int32_t* bias_b, const cvmhip_chain* chain_b, const void* residual /* NULL with a projection */,
                                 const cvmhip_chain* chain_r, void* out, const void* wc, const int32_t* bias_c, const cvmhip_chain* chain_c, void* next,

@@ -307,17 +307,17 @@ def test_filters_of_the_next_launch(m, oc, projects, later_oc, dev):
 
 @pytest.mark.gpu
 def test_several_blocks_of_a_graph(dev, monkeypatch):
-    """Blocks one behind the other, through a change of their width: every launch but the last knows the next one's filters."""
-    g, heads = graphgen.resnet50(2, blocks=(2, 2, 3, 1), size=96, classes=40, config_id="bottlenecks")
+    """Blocks one behind the other, through a change of their width: where compute units are idle a launch has the next one's filters fetched."""
+    g, heads = graphgen.resnet50(13, blocks=(1, 2, 3, 1), size=96, classes=40, config_id="bottlenecks")   # 468 pixels of 256 channels
     js, pb = g.build(heads)
     monkeypatch.setenv("CVM_HIP_RESIDENT", "1")
     m = runtime.HipModel(js, pb)
-    for call in range(3):
-        data = synth.tensor("bottlenecks", "data%d" % call, (2, 3, 96, 96), -127, 127)
-        want = og.run_graph(js, graphgen.load_params(pb), data)[0].ravel()
-        assert np.array_equal(np.frombuffer(m.inference(data.astype(np.int8).tobytes()), np.int32), want), call
+    inputs = [synth.tensor("bottlenecks", "data%d" % k, (13, 3, 96, 96), -127, 127) for k in range(2)]
+    wants = [og.run_graph(js, graphgen.load_params(pb), x)[0].ravel() for x in inputs]
+    for call in range(4):
+        assert np.array_equal(np.frombuffer(m.inference(inputs[call % 2].astype(np.int8).tobytes()), np.int32), wants[call % 2]), call
     said = [v for v in _launches(m.run) if "k_conv_block" in v]
-    assert len(said) >= 6 and sum("+ 64 ahead" in v for v in said) >= 3, said
+    assert len(said) == 6 and sum("+ 64 ahead" in v for v in said) == 2, said
     m.close()
 
 
@@ -354,3 +354,27 @@ def test_beside_a_sequence(spin, dev, monkeypatch):
         for k in range(4):
             assert m.inference(inputs[k % 3].tobytes()) == wants[k % 3], k
     m.close()
+
+
+@pytest.mark.gpu
+def test_few_pixels_stay_apart(dev, monkeypatch):
+    js, pb = _net(2, 256, 14, 14, 256, 1, projects=True)
+    data = synth.tensor("bottleneck", "few", (2, 32, 14, 14), -128, 127)
+    got, launches = _run(js, pb, data, monkeypatch)
+    assert launches[0] == launches[1], launches
+    want = og.run_graph(js, graphgen.load_params(pb), data.astype(np.int32))[0].ravel()
+    assert all(np.array_equal(v.astype(np.int32), want) for v in got)
+
+
+def test_which_launches_gain():
+    def gains(n, m, h, w, oc, stride, projection=None):
+        assert _eligible(n, m, h, w, oc, stride, projection)
+        return bool(lib().cvmhip_bottleneck_gains(n, m, h, w, oc, stride, projection))
+    for n, m, h, w, oc, stride in ((3, 256, 14, 14, 256, 1), (50, 256, 28, 28, 512, 2), (1, 256, 59, 59, 256, 1), (1, 128, 7, 7, 128, 1), (1, 64, 1, 1, 64, 1), (256, 64, 56, 56, 128, 1),
+                                   (256, 128, 56, 56, 128, 2), (1, 128, 266, 266, 256, 2), (1, 128, 319, 319, 128, 1), (1, 64, 654, 654, 64, 2)):
+        assert gains(n, m, h, w, oc, stride), (n, m, h, w)
+    for n, m, h, w, oc, stride in ((1, 256, 14, 14, 256, 1), (2, 256, 28, 28, 512, 2), (1, 256, 224, 224, 512, 2), (1, 256, 235, 235, 256, 1), (1, 64, 702, 702, 64, 2), (1, 128, 340, 340, 256, 2),
+                                   (1, 128, 328, 516, 128, 1), (1, 128, 331, 331, 128, 1)):
+        assert not gains(n, m, h, w, oc, stride), (n, m, h, w)
+    assert gains(3, 256, 28, 28, 256, 2, _projection(512)) and not gains(1, 256, 14, 14, 256, 1, _projection(512))
+    assert not lib().cvmhip_bottleneck_gains(1, 256, 1, 400, 256, 1, None)   # fits nowhere
