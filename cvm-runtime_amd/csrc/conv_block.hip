@@ -516,7 +516,7 @@ int cvmhip_conv2d_bottleneck_i8(const void* xp, const void* wa, const int32_t* b
   a.div_patch = make_fastdiv((uint32_t)a.patch);
   a.tiles = (a.P + 16 * f->nt - 1) / (16 * f->nt);
   // The 1.1 MB of filters that a launch with M = 256 reads come from behind the L2 each time: all layers' are more than it holds.  Where most compute units
-  // are idle some fetch the next launch's: ResNet-50 with 1 image 199.5 -> 193.3 us a run, 2 200.8 -> 196.1, 4 214.8 -> 211.9 (49 tiles); past that the
+  // are idle some fetch the next launch's: ResNet-50, all blocks in one launch each, with 1 image 199.5 -> 193.3 us a run, 2 200.8 -> 196.1, 4 214.8 -> 211.9 (49 tiles); past that the
   // fetches are in the way (8 images 240.3 -> 241.2, 16 285 -> 288), and the question alone costs a launch 0.2 us, hence kernels of their own.
   if (ahead && ahead->m == 256 && f->with_helpers && a.tiles <= BLOCK_UNITS / 4) {
     a.helpers = 8;
